@@ -71,8 +71,10 @@ k_rope(const uint16_t* __restrict__ in, const uint16_t* __restrict__ cosv, const
       whi = pack8(oh);
     }
     if (TO_HEADS) {
-      *reinterpret_cast<uint4*>(out_heads + heads_off) = wlo;
-      *reinterpret_cast<uint4*>(out_heads + heads_off + half) = whi;
+      if (out_heads) {
+        *reinterpret_cast<uint4*>(out_heads + heads_off) = wlo;
+        *reinterpret_cast<uint4*>(out_heads + heads_off + half) = whi;
+      }
       if (out_rows) {
         *reinterpret_cast<uint4*>(out_rows + rows_off) = wlo;
         *reinterpret_cast<uint4*>(out_rows + rows_off + half) = whi;
@@ -112,7 +114,7 @@ int hyc_rope_to_heads(const void* x, int64_t x_pitch, const void* cosv, const vo
   if (x_pitch < heads * head_dim || x_pitch % 8 != 0)
     return fail(HYC_EINVAL, "hyc_rope_to_heads: token pitch %lld (at least heads*head_dim, a multiple of 8)", (long long)x_pitch);
   if (B == 0 || S == 0) return HYC_OK;
-  if (!x || !out_heads || ((cosv == nullptr) != (sinv == nullptr))) return fail(HYC_EFAULT, "hyc_rope_to_heads: null buffer");
+  if (!x || (!out_heads && !out_rows) || ((cosv == nullptr) != (sinv == nullptr))) return fail(HYC_EFAULT, "hyc_rope_to_heads: null buffer");
   if (!aligned16(x) || !aligned16(out_heads) || !aligned16(out_rows) || !aligned16(cosv) || !aligned16(sinv))
     return fail(HYC_EINVAL, "hyc_rope_to_heads: buffers must be 16-byte aligned");
   const int64_t items = B * S * heads * (head_dim / 16);

@@ -352,9 +352,9 @@ class _AttentionFunc(torch.autograd.Function):
 
 
 class _FlashAttentionFunc(torch.autograd.Function):
-    """The design of the reference's flash-attention operator (operators/efficient_flashattention.py:10-135): the
-    fused attention kernel of the library runs the forward, what is kept is q, k (after RoPE), v and the attention
-    output as codes plus the fp32 log-sum-exp of every row, and the library's backward kernel runs on the restored
+    """The design of the reference's flash-attention operator (operators/efficient_flashattention.py:10-135): a fused
+    attention kernel (hyc_attn_fwd; the library's for head sizes other than 64 and 128) runs the forward, what is kept is q, k (after RoPE), v and the attention
+    output as codes plus the fp32 log-sum-exp of every row, and the fused backward runs on the restored
     tensors.  No [S, S] matrix exists at any time.  The backward kernel rebuilds the probabilities from the restored
     q and k with the exact log-sum-exp, and takes its row term sum(dO * O) from the restored output."""
 
@@ -364,14 +364,20 @@ class _FlashAttentionFunc(torch.autograd.Function):
         b, s, H = q.shape
         nh, hd = cfg.heads, cfg.head_dim
         scale = 1.0 / math.sqrt(hd)
-        qh, q_rows = K.rope_to_heads(q, nh, cos, sin, want_rows=True)
-        kh, k_rows = K.rope_to_heads(k, nh, cos, sin, want_rows=True)
-        vh = K.rope_to_heads(v, nh)
-        out_h, lse, _, _, _, _, seed, offset, _ = torch.ops.aten._scaled_dot_product_flash_attention(
-            qh, kh, vh, 0.0, True, False, scale=scale)
-        del qh, kh, vh
-        out = K.rope_from_heads(out_h)                              # [B, S, H]
-        del out_h
+        ctx.rows = K.attn_supported(hd, s, max(v.stride(1), H))
+        seed = offset = None
+        if ctx.rows:                                                # the kernels read and write the rows as they are
+            q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
+            out, lse = K.attn_fwd(q_rows, k_rows, v, nh, scale)
+        else:
+            qh, q_rows = K.rope_to_heads(q, nh, cos, sin, want_rows=True)
+            kh, k_rows = K.rope_to_heads(k, nh, cos, sin, want_rows=True)
+            vh = K.rope_to_heads(v, nh)
+            out_h, lse, _, _, _, _, seed, offset, _ = torch.ops.aten._scaled_dot_product_flash_attention(
+                qh, kh, vh, 0.0, True, False, scale=scale)
+            del qh, kh, vh
+            out = K.rope_from_heads(out_h)                          # [B, S, H]
+            del out_h
         rows = [t.reshape(b * s, H) for t in (q_rows, k_rows, v, out)]
         it = mod.iteration
         if cfg.compress:
@@ -393,6 +399,10 @@ class _FlashAttentionFunc(torch.autograd.Function):
         b, nh, s, hd = ctx.geom
         cos, sin, lse = ctx.saved_tensors
         restore = (lambda c: K.decompress_channel(c)) if ctx.compress else (lambda c: c)
+        if ctx.rows:
+            qq, kk, vv, oo = (restore(c).view(b, s, nh * hd) for c in ctx.saved)
+            ctx.saved = None
+            return K.attn_bwd(g.to(BF16).contiguous(), qq, kk, vv, oo, lse, nh, 1.0 / math.sqrt(hd), cos, sin) + (None, None, None)
         to_heads = lambda rows: K.rope_to_heads(rows.view(b, s, nh * hd), nh)
         gh = K.rope_to_heads(g.to(BF16).contiguous(), nh)
         qq, kk, vv, oo = (to_heads(restore(c)) for c in ctx.saved)

@@ -991,6 +991,29 @@ def rope_to_heads(x, heads, cos=None, sin=None, want_rows=False):
     return (out_heads, out_rows) if want_rows else out_heads
 
 
+def _need_tokens(x, name):
+    """(B, S, H, pitch) of a bf16 [B, S, H] tensor with contiguous channels and evenly spaced tokens"""
+    if not isinstance(x, torch.Tensor) or not x.is_cuda or x.dtype != BF16 or x.dim() != 3:
+        raise ValueError("%s must be a bfloat16 [B, S, H] tensor on the GPU" % name)
+    B, S, H = x.shape
+    pitch = x.stride(1) if S > 1 else (x.stride(0) if B > 1 else H)
+    if x.stride(2) != 1 or (B > 1 and x.stride(0) != S * pitch):
+        raise ValueError("%s must have contiguous channels and evenly spaced tokens" % name)
+    return B, S, H, pitch
+
+
+def rope_rows(x, heads, cos, sin):
+    """x bf16 [B, S, heads*hd], possibly a column slice of a wider matrix -> the rotated rows, contiguous"""
+    B, S, H, pitch = _need_tokens(x, "x")
+    if heads <= 0 or H % heads:
+        raise ValueError("%d channels do not split into %d heads" % (H, heads))
+    hd = H // heads
+    _need_tables(cos, sin, S, hd)
+    out = torch.empty((B, S, H), dtype=BF16, device=x.device)
+    check(_abi.load().hyc_rope_to_heads(_p(x), pitch, _p(cos), _p(sin), B, S, heads, hd, None, _p(out), _stream()))
+    return out
+
+
 def rope_from_heads(g, cos=None, sin=None):
     """gradient bf16 [B, heads, S, hd] -> [B, S, heads*hd] through the transposed rotation"""
     _need(g, BF16, "g")
@@ -999,6 +1022,45 @@ def rope_from_heads(g, cos=None, sin=None):
     out = torch.empty((B, S, heads * hd), dtype=BF16, device=g.device)
     check(_abi.load().hyc_rope_from_heads(_p(g), _p(cos), _p(sin), B, S, heads, hd, _p(out), _stream()))
     return out
+
+
+# ----------------------------------------------------------------------------------------------------
+# fused causal attention
+# ----------------------------------------------------------------------------------------------------
+def attn_supported(head_dim, S, widest_pitch):
+    """shapes hyc_attn_fwd / hyc_attn_bwd cover (the library's fused attention serves the others)"""
+    return head_dim in (64, 128) and S * widest_pitch < 1 << 30
+
+
+def attn_fwd(q, k, v, heads, scale):
+    """causal softmax(scale q k^T) v on [B, S, heads*hd] rows -> (out [B, S, heads*hd], lse fp32 [B, heads, S])"""
+    B, S, H, pq = _need_tokens(q, "q")
+    pk, pv = _need_tokens(k, "k")[3], _need_tokens(v, "v")[3]
+    if tuple(k.shape) != (B, S, H) or tuple(v.shape) != (B, S, H) or H % heads:
+        raise ValueError("q, k, v must be [B, S, heads*hd] alike, got %s, %s, %s" % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
+    out = torch.empty((B, S, H), dtype=BF16, device=q.device)
+    lse = torch.empty((B, heads, S), dtype=torch.float32, device=q.device)
+    check(_abi.load().hyc_attn_fwd(_p(q), pq, _p(k), pk, _p(v), pv, B, S, heads, H // heads, float(scale), _p(out), H, _p(lse),
+                                   _stream()))
+    return out, lse
+
+
+def attn_bwd(g, q, k, v, out, lse, heads, scale, cos=None, sin=None):
+    """(dq, dk, dv) of attn_fwd at the given q, k, v, out and lse; with cos / sin the gradients of q and k before their
+    rotation"""
+    B, S, H, pg = _need_tokens(g, "g")
+    ptrs = []
+    for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):
+        if tuple(t.shape) != (B, S, H):
+            raise ValueError("%s is %s, the gradient is %s" % (name, tuple(t.shape), tuple(g.shape)))
+        ptrs += [_p(t), _need_tokens(t, name)[3]]
+    _need_vec(lse, torch.float32, B * heads * S, "lse")
+    _need_tables(cos, sin, S, H // heads)
+    dq, dk, dv = (torch.empty((B, S, H), dtype=BF16, device=g.device) for _ in range(3))
+    ws = torch.empty(2 * B * heads * S, dtype=torch.float32, device=g.device)
+    check(_abi.load().hyc_attn_bwd(_p(g), pg, *ptrs, _p(lse), _p(cos), _p(sin), B, S, heads, H // heads, float(scale),
+                                   _p(dq), H, _p(dk), H, _p(dv), H, _p(ws), _stream()))
+    return dq, dk, dv
 
 
 # ----------------------------------------------------------------------------------------------------

@@ -300,7 +300,7 @@ int hyc_low_rank_update(const void* L, const void* R, const void* x, void* out, 
 
 /* ---- rotary embedding + attention layout ----------------------------------------------------- */
 /* x bf16 [B, S, heads, head_dim] (what the projections produce) -> the rotated tensor as [B, heads, S, head_dim] in
- * out_heads (what the batched attention GEMMs consume) and, when out_rows is not NULL, also in the input's layout
+ * out_heads (what the batched attention GEMMs consume) and / or in the input's layout in out_rows; either may be NULL
  * (apply_rotary_pos_emb, models/modeling_llama.py:236-260, with the .view().transpose(1, 2) of :423-425).
  *   y[i] = x[i] cos[i] - x[i+h] sin[i],  y[i+h] = x[i+h] cos[i+h] + x[i] sin[i+h],  h = head_dim / 2
  * cos / sin bf16 [S, head_dim]; both NULL = layout change only (the value tensor).  fp32 arithmetic, one rounding.
@@ -313,6 +313,21 @@ int hyc_rope_to_heads(const void* x, int64_t x_pitch, const void* cosv, const vo
                       int64_t heads, int64_t head_dim, void* out_heads, void* out_rows, void* stream);
 int hyc_rope_from_heads(const void* g, const void* cosv, const void* sinv, int64_t B, int64_t S, int64_t heads,
                         int64_t head_dim, void* out_rows, void* stream);
+
+/* ---- fused causal attention ------------------------------------------------------------------ */
+/* On the rows layout [B, S, heads, head_dim] of the projections, every operand with its own token pitch (elements between
+ * consecutive tokens, a multiple of 8; batch elements are S tokens apart); bf16, fp32 accumulation, head_dim 64 or 128.
+ *   out = softmax(scale q k^T + causal mask) v,  lse fp32 [B, heads, S] = log of each row's sum of exponentials
+ * hyc_attn_bwd: gradients at the given q, k, v and out, with probabilities exp(scale q.k - lse); with cos / sin (bf16
+ * [S, head_dim]) dq and dk leave through the transposed rotation of hyc_rope_from_heads.  workspace: 2 * B * heads * S
+ * floats.  No atomics: results repeat bit for bit.
+ * (operators/efficient_flashattention.py:10-135 reaches the same computation through flash_attn.) */
+int hyc_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, int64_t B, int64_t S,
+                 int64_t heads, int64_t head_dim, float scale, void* out, int64_t ldo, float* lse, void* stream);
+int hyc_attn_bwd(const void* dout, int64_t ldg, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                 const void* out, int64_t ldo, const float* lse, const void* cosv, const void* sinv, int64_t B, int64_t S,
+                 int64_t heads, int64_t head_dim, float scale, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv,
+                 int64_t lddv, float* workspace, void* stream);
 
 /* ---- seeded dropout ----------------------------------------------------------------------------- */
 /* EfficientMemoryDropoutFunc, operators/efficient_dropout.py:56-79: the keep mask of element i is
