@@ -84,6 +84,14 @@ SIGNATURES = {
     "hyc_kth_value": (c_i32, [c_ptr, c_i32, c_i64, c_i64, c_ptr, c_ptr, c_ptr]),
     "hyc_rope_to_heads": (c_i32, [c_ptr, c_i64, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_ptr]),
     "hyc_rope_from_heads": (c_i32, [c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_i64, c_ptr, c_ptr]),
+    "hyc_gated_act_bwd_rows": (c_i32, [c_i32, c_ptr, c_ptr, c_ptr, c_ptr, ctypes.POINTER(HycDesc), c_ptr, c_ptr, c_ptr, ctypes.POINTER(HycDesc),
+                                       c_ptr, c_ptr, c_ptr, ctypes.POINTER(HycDesc), c_i64, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr]),
+    "hyc_lora_down": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i32, c_i32, c_ptr, c_ptr]),
+    "hyc_lora_up": (c_i32, [c_ptr, c_i64, c_ptr, c_ptr, c_i32, c_i32, c_f32, c_ptr, c_ptr]),
+    "hyc_lora_weight_t": (c_i32, [c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_i32, c_i32, c_i64, c_ptr, c_ptr]),
+    "hyc_lora_up_bwd_workspace_bytes": (c_i64, [c_i64, c_ptr, c_i32, c_i32]),
+    "hyc_lora_up_bwd": (c_i32, [c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_i32, c_i32, c_f32, c_ptr, c_ptr, c_i64, c_i64, c_i32, c_ptr,
+                                c_ptr, c_ptr]),
     "hyc_attn_fwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_ptr, c_i64, c_ptr, c_ptr]),
     "hyc_attn_bwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64,
                              c_i64, c_f32, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr]),

@@ -418,8 +418,8 @@ k_gated_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__
                      const uint16_t* __restrict__ s_a, ChanArgs c_a, const uint8_t* __restrict__ st_u,
                      const uint16_t* __restrict__ v_u, const uint16_t* __restrict__ s_u, ChanArgs c_u,
                      const uint8_t* __restrict__ st_g, const uint16_t* __restrict__ v_g, const uint16_t* __restrict__ s_g,
-                     ChanArgs c_g, int64_t M, int64_t H, int CPS, int cps_wg, uint16_t* __restrict__ d_gate,
-                     uint16_t* __restrict__ d_up, int use_lut) {
+                     ChanArgs c_g, int64_t M, int64_t H, int CPS, int cps_wg, uint16_t* __restrict__ d_gate, int64_t ld_dg,
+                     uint16_t* __restrict__ d_up, int64_t ld_du, int use_lut) {
   constexpr int NSEG = Q<BITS>::NSEG;
   __shared__ uint16_t lut[LUT_NEG + LUT_N];             // the activation's derivative, see lut_fill
   if (use_lut) {
@@ -438,9 +438,9 @@ k_gated_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__
   U.init(st_u, v_u, s_u, c_u, c, CPS, row, stride);
   G.init(st_g, v_g, s_g, c_g, c, CPS, row, stride);
   const uint16_t* gp = g + row * H + 8 * c;
-  uint16_t* dgp = d_gate + row * H + 8 * c;
-  uint16_t* dup = d_up + row * H + 8 * c;
-  const int64_t xstep = stride * H;
+  uint16_t* dgp = d_gate + row * ld_dg + 8 * c;
+  uint16_t* dup = d_up + row * ld_du + 8 * c;
+  const int64_t xstep = stride * H, dgstep = stride * ld_dg, dustep = stride * ld_du;
   uint4 graw[NSEG];
   if (row < M) {
 #pragma unroll
@@ -471,7 +471,7 @@ k_gated_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__
     }
 #pragma unroll
     for (int i = 0; i < NSEG; ++i) graw[i] = g_n[i];
-    gp += xstep; dgp += xstep; dup += xstep;
+    gp += xstep; dgp += dgstep; dup += dustep;
   }
 }
 
@@ -956,6 +956,18 @@ int hyc_gated_act_bwd(int32_t act, const void* g, const void* stored_a, const vo
                       const hyc_desc* d_a, const void* stored_u, const void* vals_u, const void* scales_u,
                       const hyc_desc* d_u, const void* stored_g, const void* vals_g, const void* scales_g,
                       const hyc_desc* d_g, int64_t M, int64_t H, void* d_gate, void* d_up, void* stream) {
+  return hyc_gated_act_bwd_rows(act, g, stored_a, vals_a, scales_a, d_a, stored_u, vals_u, scales_u, d_u, stored_g, vals_g, scales_g,
+                                d_g, M, H, d_gate, H, d_up, H, stream);
+}
+
+int hyc_gated_act_bwd_rows(int32_t act, const void* g, const void* stored_a, const void* vals_a, const void* scales_a,
+                           const hyc_desc* d_a, const void* stored_u, const void* vals_u, const void* scales_u,
+                           const hyc_desc* d_u, const void* stored_g, const void* vals_g, const void* scales_g,
+                           const hyc_desc* d_g, int64_t M, int64_t H, void* d_gate, int64_t ld_dgate, void* d_up, int64_t ld_dup,
+                           void* stream) {
+  if (ld_dgate < H || ld_dup < H || ld_dgate % 8 != 0 || ld_dup % 8 != 0)
+    return fail(HYC_EINVAL, "hyc_gated_act_bwd: row pitches %lld, %lld (at least H=%lld, multiples of 8)", (long long)ld_dgate,
+                (long long)ld_dup, (long long)H);
   if (act != HYC_ACT_SILU && act != HYC_ACT_GELU_TANH) return fail(HYC_EINVAL, "hyc_gated_act_bwd: act=%d", act);
   if (!d_a || !d_u || !d_g) return fail(HYC_EFAULT, "hyc_gated_act_bwd: null descriptor");
   if (M < 0) return fail(HYC_EINVAL, "hyc_gated_act_bwd: M=%lld", (long long)M);
@@ -1001,7 +1013,7 @@ int hyc_gated_act_bwd(int32_t act, const void* g, const void* stored_a, const vo
                      static_cast<const uint8_t*>(stored_u), static_cast<const uint16_t*>(vals_u),                  \
                      static_cast<const uint16_t*>(scales_u), c_u, static_cast<const uint8_t*>(stored_g),           \
                      static_cast<const uint16_t*>(vals_g), static_cast<const uint16_t*>(scales_g), c_g, M, H,      \
-                     geo.cps, cps_wg, static_cast<uint16_t*>(d_gate), static_cast<uint16_t*>(d_up), use_lut)
+                     geo.cps, cps_wg, static_cast<uint16_t*>(d_gate), ld_dgate, static_cast<uint16_t*>(d_up), ld_dup, use_lut)
 #define HYC_GATED_T(B_, A_)                                                       \
   do {                                                                            \
     if (threads <= 256) HYC_GATED(B_, A_, 256);                                   \

@@ -1,0 +1,550 @@
+// The rank-r terms of LoRA projections beside a frozen NF4 base (the reference: peft `Linear.forward` around
+// bitsandbytes_fix/_function.py:509-540, once per projection), a group of projections of one input at a time:
+//
+//   forward     h = x A^T;  y = s h B^T, onto which the base product accumulates (the rank-r term is rounded to bf16 before
+//               it is added, as it is when it is a tensor of its own)
+//   backward    dX = [dY | dh] [W^T | A^T]^T: ONE product over all projections of the group, the rank-r columns as R further
+//               columns of its reduction;  dh = s dY B and dB = s dY^T h both from ONE read of dY
+//
+// The transient weight of the backward is written transposed: the library's GEMMs with both operands contiguous along the
+// reduction are 10-20 % faster (dX of a 3 x 4096 group at 4096 tokens: three accumulating products 318 us, one 293, one with
+// the transposed weight 252; 2 x 11008: 551 / 525 / 460).
+#include <type_traits>
+
+#include "abi_util.hpp"
+#include "row_kernels.hpp"
+
+namespace hyc {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+#define HYC_MFMA16(a_, b_, c_) __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_, b_, c_, 0, 0, 0)
+
+constexpr int LORA_MAX = 4;                              // projections of a group
+
+// the same 16 NormalFloat4 levels as nf4.hip
+__device__ __constant__ float kLoraNF4[16] = {
+    -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f, -0.28444138169288635f,
+    -0.18477343022823334f, -0.09105003625154495f, 0.0f, 0.07958029955625534f, 0.16093020141124725f,
+    0.24611230194568634f, 0.33791524171829224f, 0.44070982933044434f, 0.5626170039176941f, 0.7229568362236023f,
+    1.0f};
+
+struct LoraGroup {
+  const uint16_t* f[LORA_MAX];                           // the LoRA factors (A [r, K] or B [out, r])
+  int end[LORA_MAX];                                     // first row of the stacked weight after projection i
+  int n, r;
+};
+
+// out[k, n] = the dequantised W[n, k] for n < rows, A_i[j, k] for n = rows + i r + j, zeros in the rest of the room.  A
+// workgroup turns a tile of 128 n x 64 k in LDS: a lane decodes the 16 weights of two neighbouring n and writes them as
+// pairs (64 lanes = consecutive banks), rows of k leave as whole 256-byte runs.
+__global__ void __launch_bounds__(256)
+k_lora_weight_t(const uint8_t* __restrict__ packed, const float* __restrict__ absmax, int rows, int K, int room, LoraGroup g,
+                uint16_t* __restrict__ out) {
+  __shared__ float lut[16];
+  __shared__ __align__(16) uint32_t T[64][64 + 4];       // [k][n / 2]
+  if (threadIdx.x < 16) lut[threadIdx.x] = kLoraNF4[threadIdx.x];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n0 = blockIdx.y * 128, k0 = blockIdx.x * 64, N = rows + room;
+  const int64_t pitch = N;
+  float v[2][16];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int n = n0 + 2 * lane + a, k = k0 + 16 * wave;
+    if (n < rows) {
+      const int64_t at = (int64_t)n * K + k;
+      const uint2 w = *reinterpret_cast<const uint2*>(packed + at / 2);
+      const float s = absmax[at >> 6];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const uint32_t byte = ((b < 4 ? w.x : w.y) >> (8 * (b & 3))) & 0xFFu;
+        v[a][2 * b] = lut[byte >> 4] * s;
+        v[a][2 * b + 1] = lut[byte & 15u] * s;
+      }
+    } else {
+      const int t = n - rows, p = t / g.r;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[a][j] = 0.f;
+      if (p < g.n) {
+        const uint16_t* A = g.f[p] + (int64_t)(t - p * g.r) * K + k;
+        float lo[8], hi[8];
+        unpack8(*reinterpret_cast<const uint4*>(A), lo);
+        unpack8(*reinterpret_cast<const uint4*>(A + 8), hi);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { v[a][j] = lo[j]; v[a][8 + j] = hi[j]; }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 16; ++j) T[16 * wave + j][lane] = pack_bf16(v[0][j], v[1][j]);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int at = threadIdx.x + 256 * u, k = at / 16, c = at % 16;
+    if (n0 + 8 * c < N)
+      *reinterpret_cast<uint4*>(out + (int64_t)(k0 + k) * pitch + n0 + 8 * c) = *reinterpret_cast<const uint4*>(&T[k][4 * c]);
+  }
+}
+
+// h[m, i r + j] = sum_k x[m, k] A_i[j, k].  Eight waves share 16 tokens, each taking every eighth 32-channel step, so a row
+// is read in runs of 512 bytes; A stays in L2.  Bound by the read of x (4096 x 4096: 33.5 MB; stacking the A_i and the
+// library's thin GEMM took 5 + 14 us).
+template <int CT>
+__global__ void __launch_bounds__(512)
+k_lora_down(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int K, LoraGroup g, uint16_t* __restrict__ h) {
+  __shared__ __align__(16) float red[8][CT][256];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t m0 = (int64_t)blockIdx.x * 16;
+  const int kq = 8 * (lane >> 4), nr = g.n * g.r;
+  const int64_t m = m0 + (lane & 15) < M ? m0 + (lane & 15) : M - 1;
+  const uint16_t* xp = x + m * ldx + kq;
+  const uint16_t* ap[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const int f = 16 * c + (lane & 15), ff = f < nr ? f : 0, p = ff / g.r;
+    ap[c] = g.f[p] + (int64_t)(ff - p * g.r) * K + kq;
+  }
+  floatx4_t acc[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) acc[c] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int U = CT <= 3 ? 4 : 2;
+  const int steps = K / 32;
+  auto run = [&](int s, auto uno) __attribute__((always_inline)) {      // UU steps, all loads ahead of the products
+    constexpr int UU = decltype(uno)::value;
+    bf16x8_t a[UU], b[UU][CT];
+#pragma unroll
+    for (int u = 0; u < UU; ++u) {
+      a[u] = *reinterpret_cast<const bf16x8_t*>(xp + 32 * (s + 8 * u));
+#pragma unroll
+      for (int c = 0; c < CT; ++c) b[u][c] = *reinterpret_cast<const bf16x8_t*>(ap[c] + 32 * (s + 8 * u));
+    }
+#pragma unroll
+    for (int u = 0; u < UU; ++u)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[c] = HYC_MFMA16(a[u], b[u][c], acc[c]);
+  };
+  int s = wave;
+  for (; s + 8 * (U - 1) < steps; s += 8 * U) run(s, std::integral_constant<int, U>{});
+  for (; s < steps; s += 8) run(s, std::integral_constant<int, 1>{});
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave][c][(4 * (lane >> 4) + i) * 16 + (lane & 15)] = acc[c][i];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 16 * nr; e += 512) {
+    const int t = e / nr, f = e - t * nr;
+    if (m0 + t >= M) break;
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) sum += red[w][f >> 4][t * 16 + (f & 15)];
+    h[(m0 + t) * nr + f] = f_to_bf(sum);
+  }
+}
+
+// ---- y = s h B^T ----------------------------------------------------------------------------------------------------
+struct LoraOut {
+  const uint16_t* B[LORA_MAX];                           // [n_out_i, r]
+  int n_out[LORA_MAX], fb0[LORA_MAX + 1], row0[LORA_MAX + 1];   // first feature block / first column of projection i
+  int n, r;
+};
+constexpr int LO_F = 256, LO_M = 128;                    // features and tokens of a workgroup
+
+// A pure write (4096 tokens x 12288: 100 MB), so the point is full 16-byte stores: the products are taken with the features
+// as rows in the order that gives a lane eight neighbouring features of its token over two MFMAs.  Ordinary stores: the base
+// product reads y next, from the last-level cache.
+__global__ void __launch_bounds__(256)
+k_lora_up(const uint16_t* __restrict__ h, int64_t M, LoraOut a, float scale, uint16_t* __restrict__ y) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, lq = lane >> 4;
+  int p = 0;
+  while (p + 1 < a.n && (int)blockIdx.x >= a.fb0[p + 1]) ++p;
+  const int f0 = ((int)blockIdx.x - a.fb0[p]) * LO_F + 64 * wave, r = a.r, nr = a.n * r, n_out = a.n_out[p];
+  const int64_t m_begin = (int64_t)blockIdx.y * LO_M, pitch = a.row0[a.n];
+  const bool on = 8 * lq < r;                            // (r is a multiple of 8)
+  bf16x8_t bf[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int f = f0 + 32 * (q >> 1) + 8 * (l15 >> 2) + 4 * (q & 1) + (l15 & 3);
+    const uint4 v = on && f < n_out ? *reinterpret_cast<const uint4*>(a.B[p] + (int64_t)f * r + 8 * lq) : make_uint4(0, 0, 0, 0);
+    bf[q] = __builtin_bit_cast(bf16x8_t, v);
+  }
+#pragma unroll 4
+  for (int t = 0; t < LO_M; t += 16) {
+    const int64_t m = m_begin + t + l15;
+    const uint4 v = on && m < M ? *reinterpret_cast<const uint4*>(h + m * nr + p * r + 8 * lq) : make_uint4(0, 0, 0, 0);
+    const bf16x8_t hf = __builtin_bit_cast(bf16x8_t, v);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const floatx4_t z = {0.f, 0.f, 0.f, 0.f};
+      const floatx4_t d0 = HYC_MFMA16(bf[2 * g], hf, z), d1 = HYC_MFMA16(bf[2 * g + 1], hf, z);
+      const int f = f0 + 32 * g + 8 * lq;
+      if (m < M && f < n_out) {
+        const float o[8] = {d0[0] * scale, d0[1] * scale, d0[2] * scale, d0[3] * scale, d1[0] * scale, d1[1] * scale, d1[2] * scale, d1[3] * scale};
+        *reinterpret_cast<uint4*>(y + m * pitch + a.row0[p] + f) = pack8(o);
+      }
+    }
+  }
+}
+
+// ---- dh = s dY B and dB = s dY^T h from one read of dY -----------------------------------------------------------------
+struct LoraUp {
+  const uint16_t* g[LORA_MAX];                           // dY_i [M, n_out_i], rows ldg_i apart
+  int64_t ldg[LORA_MAX];
+  const uint16_t* B[LORA_MAX];                           // [n_out_i, r]
+  uint16_t* dB[LORA_MAX];
+  int n_out[LORA_MAX], fb0[LORA_MAX + 1], row0[LORA_MAX + 1];   // first feature block / first stacked row of projection i
+  int n, r;
+};
+constexpr int LU_F = 256, LU_M = 64;                     // features of a workgroup, tokens of a tile
+
+__device__ __forceinline__ int lu_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+
+// A workgroup owns 256 features and a range of tokens, walked in tiles of 64 that go from memory straight to LDS (two
+// buffers of 32 KB, two workgroups per CU).  From a tile, wave w takes the 16 tokens 16 w .. for dh (all 256 features, the
+// B factors in registers) and the 64 features 64 w .. for dB (all 64 tokens): dY rows as stored are the operand of the
+// first, the transposing read gives that of the second, and no sum crosses a wave.  dh leaves as one fp32 partial per
+// feature block, dB as one per token range; k_lora_up_finish adds them in a fixed order.  Bound by the read of dY.
+template <int RT>
+__global__ void __launch_bounds__(256, 2)
+k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, float* __restrict__ dhp, float* __restrict__ dbp,
+              uint16_t* __restrict__ copy, int64_t ld_copy) {
+  constexpr int RC = 16 * RT;                            // columns of the factor, padded
+  __shared__ __align__(1024) uint16_t tile[2][LU_M * LU_F];
+  __shared__ __align__(1024) uint16_t ht[2][LU_M * RC];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, lq = lane >> 4;
+  const int fb = blockIdx.x;
+  int p = 0;
+  while (p + 1 < a.n && fb >= a.fb0[p + 1]) ++p;
+  const int f0 = (fb - a.fb0[p]) * LU_F, n_out = a.n_out[p], r = a.r, nr = a.n * r;
+  const int64_t m_begin = (int64_t)blockIdx.y * tokens, m_end = m_begin + tokens < M ? m_begin + tokens : M;
+  const int count = (int)(m_end - m_begin), tiles = (count + LU_M - 1) / LU_M;
+  const uint32_t pitch = (uint32_t)a.ldg[p] * 2u;
+  const uint16_t* base = a.g[p] + m_begin * a.ldg[p] + f0;
+  // (the resource ends with the last row's last feature of this block)
+  const int fl = n_out - f0 < LU_F ? n_out - f0 : LU_F;  // features this block really has, a multiple of 8
+  const uint64_t ba = (uint64_t)(uintptr_t)base;
+  u32x4_t rs;
+  rs.x = __builtin_amdgcn_readfirstlane((uint32_t)ba);
+  rs.y = __builtin_amdgcn_readfirstlane((uint32_t)(ba >> 32) & 0xFFFFu);
+  rs.z = __builtin_amdgcn_readfirstlane((uint32_t)(count - 1) * pitch + 2u * (uint32_t)fl);
+  rs.w = 0x00020000u;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)&tile[0][0];
+  const int ir = lane >> 5, ic = lane & 31;              // an instruction brings two rows of 32 chunks
+  auto issue = [&](int t, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int row = 2 * (wave + 4 * u) + ir;           // row of the tile; its chunk c lies at position c ^ swz(row)
+      int c = ic ^ lu_swz(row & 15);
+      c = 8 * c < fl ? c : 0;                            // features past the end: any finite values (their factors are zero)
+      const int m = t * LU_M + row < count ? t * LU_M + row : count - 1;
+      const uint32_t dst = lds0 + (uint32_t)(buf * LU_M * LU_F * 2 + (wave + 4 * u) * 1024);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                   :: "s"(dst), "v"((uint32_t)m * pitch + 16u * c), "s"(rs));
+    }
+  };
+  // the tile's rows of h (this projection's r columns, zeros behind them and past the range): registers, then LDS
+  constexpr int HC = LU_M * RC / 8;                      // 16-byte chunks: one per thread at RT = 2, half the threads at 1
+  const int hrow = threadIdx.x / (RC / 8), hcol = 8 * (threadIdx.x % (RC / 8));
+  auto load_h = [&](int t) __attribute__((always_inline)) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    const int m = t * LU_M + hrow;
+    if (threadIdx.x < HC && m < count && hcol < r) v = *reinterpret_cast<const uint4*>(h + (m_begin + m) * nr + p * r + hcol);
+    return v;
+  };
+  auto store_h = [&](int buf, const uint4& v) __attribute__((always_inline)) {
+    if (threadIdx.x < HC) *reinterpret_cast<uint4*>(&ht[buf][hrow * RC + hcol]) = v;
+  };
+  issue(0, 0);
+  uint4 hv = load_h(0);
+  // B as the second operand of dh: lane = column l % 16, 8 consecutive features per reduction step
+  bf16x8_t bf[8][RT];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int f = f0 + 32 * ks + 8 * lq + j, c = 16 * rt + l15;
+        const uint16_t v = f < n_out && c < r ? a.B[p][(int64_t)f * r + c] : (uint16_t)0;
+        bf[ks][rt][j] = __builtin_bit_cast(__bf16, v);
+      }
+  store_h(0, hv);
+  floatx4_t db[4][RT];
+#pragma unroll
+  for (int ft = 0; ft < 4; ++ft)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) db[ft][rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  typedef bf16x4_t __attribute__((address_space(3))) * lds_b64;
+  auto tr8 = [](const uint16_t* q0, const uint16_t* q1) __attribute__((always_inline)) {
+    const bf16x4_t x = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_b64)const_cast<uint16_t*>(q0));
+    const bf16x4_t y = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_b64)const_cast<uint16_t*>(q1));
+    bf16x8_t f;
+    f[0] = x[0]; f[1] = x[1]; f[2] = x[2]; f[3] = x[3]; f[4] = y[0]; f[5] = y[1]; f[6] = y[2]; f[7] = y[3];
+    return f;
+  };
+  for (int t = 0; t < tiles; ++t) {
+    const int buf = t & 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const bool more = t + 1 < tiles;
+    if (more) { issue(t + 1, buf ^ 1); hv = load_h(t + 1); }
+    const uint16_t* T = tile[buf];
+    if (copy) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int at = threadIdx.x + 256 * u, row = at / 32, c = at % 32;
+        if (t * LU_M + row < count && 8 * c < fl)
+          *reinterpret_cast<uint4*>(copy + (m_begin + t * LU_M + row) * ld_copy + a.row0[p] + f0 + 8 * c) =
+              *reinterpret_cast<const uint4*>(T + row * LU_F + 8 * (c ^ lu_swz(row & 15)));
+      }
+    }
+    floatx4_t dh[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) dh[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    const uint16_t* arow = T + (16 * wave + l15) * LU_F;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const bf16x8_t x = *reinterpret_cast<const bf16x8_t*>(arow + 8 * ((4 * ks + lq) ^ lu_swz(l15)));
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) dh[rt] = HYC_MFMA16(x, bf[ks][rt], dh[rt]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = t * LU_M + 16 * wave + 4 * lq + i;
+      if (m < count) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) dhp[((int64_t)fb * M + m_begin + m) * RC + 16 * rt + l15] = dh[rt][i];
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int r0 = 32 * kk + 8 * lq + (l15 >> 2), r1 = r0 + 4;
+      bf16x8_t hb[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const uint16_t* q = &ht[buf][16 * rt + 4 * (l15 & 3)];
+        hb[rt] = tr8(q + r0 * RC, q + r1 * RC);
+      }
+#pragma unroll
+      for (int ft = 0; ft < 4; ++ft) {
+        const int col = 64 * wave + 16 * ft + 4 * (l15 & 3);
+        const bf16x8_t x = tr8(T + r0 * LU_F + 8 * ((col >> 3) ^ lu_swz(r0 & 15)) + (col & 7),
+                               T + r1 * LU_F + 8 * ((col >> 3) ^ lu_swz(r1 & 15)) + (col & 7));
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) db[ft][rt] = HYC_MFMA16(x, hb[rt], db[ft][rt]);
+      }
+    }
+    if (more) store_h(buf ^ 1, hv);
+  }
+  float* o = dbp + ((int64_t)blockIdx.y * a.row0[a.n] + a.row0[p] + f0) * RC;
+#pragma unroll
+  for (int ft = 0; ft < 4; ++ft)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int f = 64 * wave + 16 * ft + 4 * lq + i;
+      if (f < fl) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) o[(int64_t)f * RC + 16 * rt + l15] = db[ft][rt][i];
+      }
+    }
+}
+
+// adds the partial results: dh (scaled, bf16) to dh [M, n r] and to the columns behind the dY in ext, dB to each dB_i
+__global__ void __launch_bounds__(256)
+k_lora_up_finish(LoraUp a, int64_t M, int RC, const float* __restrict__ dhp, const float* __restrict__ dbp, int ranges, float scale,
+                 uint16_t* __restrict__ dh, uint16_t* __restrict__ tail, int64_t ld_tail, int room, int64_t dh_items) {
+  const int nr = a.n * a.r;
+  int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e < dh_items) {                                    // dh_items = M * room, padded to whole workgroups by the launch
+    const int64_t m = e / room;
+    const int c = (int)(e - m * room);
+    if (m >= M) return;
+    uint16_t v = 0;
+    if (c < nr) {
+      const int p = c / a.r, j = c - p * a.r;
+      float s = 0.f;
+      for (int f = a.fb0[p]; f < a.fb0[p + 1]; ++f) s += dhp[((int64_t)f * M + m) * RC + j];
+      v = f_to_bf(s * scale);
+      dh[m * nr + c] = v;
+    }
+    tail[m * ld_tail + c] = v;
+    return;
+  }
+  e -= dh_items;
+  const int64_t row = e / a.r;
+  const int j = (int)(e - row * a.r), rows = a.row0[a.n];
+  if (row >= rows) return;
+  int p = 0;
+  while (p + 1 < a.n && row >= a.row0[p + 1]) ++p;
+  float s = 0.f;
+  for (int t = 0; t < ranges; ++t) s += dbp[((int64_t)t * rows + row) * RC + j];
+  a.dB[p][(row - a.row0[p]) * a.r + j] = f_to_bf(s * scale);
+}
+
+static int lora_group(const char* who, const void* const* factors, const int64_t* n_out, int32_t n, int32_t r, int64_t K, LoraGroup* g) {
+  if (n < 1 || n > LORA_MAX) return fail(HYC_ENOTSUP, "%s: %d projections (1 to %d)", who, n, LORA_MAX);
+  if (r < 8 || r > 32 || r % 8 != 0) return fail(HYC_ENOTSUP, "%s: rank %d (8, 16, 24 or 32)", who, r);
+  if (K <= 0 || K % 64 != 0 || K > (1 << 24)) return fail(HYC_ENOTSUP, "%s: %lld input features (a multiple of 64)", who, (long long)K);
+  if (!factors || !n_out) return fail(HYC_EFAULT, "%s: null buffer", who);
+  int64_t at = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!factors[i]) return fail(HYC_EFAULT, "%s: null factor", who);
+    if (!aligned16(factors[i])) return fail(HYC_EINVAL, "%s: factors must be 16-byte aligned", who);
+    if (n_out[i] <= 0 || n_out[i] % 8 != 0) return fail(HYC_ENOTSUP, "%s: %lld output features (a multiple of 8)", who, (long long)n_out[i]);
+    at += n_out[i];
+    if (at > (1 << 24)) return fail(HYC_ENOTSUP, "%s: too many output features", who);
+    g->f[i] = static_cast<const uint16_t*>(factors[i]);
+    g->end[i] = (int)at;
+  }
+  for (int i = n; i < LORA_MAX; ++i) { g->f[i] = nullptr; g->end[i] = (int)at; }
+  g->n = n; g->r = r;
+  return HYC_OK;
+}
+
+// token ranges of k_lora_up_bwd: enough workgroups for two per CU, whole tiles each, at most 32 (the partial dB)
+static int lora_up_ranges(int64_t M, int fblocks) {
+  int64_t want = (512 + fblocks - 1) / fblocks, most = (M + LU_M - 1) / LU_M;
+  if (want > most) want = most;
+  if (want > 32) want = 32;
+  return (int)(want < 1 ? 1 : want);
+}
+static int lora_up_blocks(const int64_t* n_out, int n) {
+  int64_t b = 0;
+  for (int i = 0; i < n; ++i) b += (n_out[i] + LU_F - 1) / LU_F;
+  return (int)b;
+}
+
+}  // namespace hyc
+
+using namespace hyc;
+
+extern "C" {
+
+int hyc_lora_weight_t(const void* packed, const float* absmax, int64_t K, const void* const* A, const int64_t* n_out, int32_t n,
+                      int32_t r, int64_t room, void* out, void* stream) {
+  LoraGroup g;
+  int rc = lora_group("hyc_lora_weight_t", A, n_out, n, r, K, &g);
+  if (rc) return rc;
+  if (room < (int64_t)n * r || room % 8 != 0 || room > 4096) return fail(HYC_EINVAL, "hyc_lora_weight_t: room=%lld for %d columns", (long long)room, n * r);
+  if (!packed || !absmax || !out) return fail(HYC_EFAULT, "hyc_lora_weight_t: null buffer");
+  if (!aligned16(packed) || !aligned16(out)) return fail(HYC_EINVAL, "hyc_lora_weight_t: packed and out must be 16-byte aligned");
+  const int rows = g.end[n - 1];
+  if ((rows + room + 127) / 128 > 65535) return fail(HYC_ENOTSUP, "hyc_lora_weight_t: too many output features");
+  hipStream_t st = begin_launch(stream);
+  hipLaunchKernelGGL(k_lora_weight_t, dim3((unsigned)(K / 64), (unsigned)((rows + room + 127) / 128)), dim3(256), 0, st,
+                     static_cast<const uint8_t*>(packed), absmax, rows, (int)K, (int)room, g, static_cast<uint16_t*>(out));
+  return check_launch("hyc_lora_weight_t");
+}
+
+int hyc_lora_down(const void* x, int64_t ldx, int64_t M, int64_t K, const void* const* A, int32_t n, int32_t r, void* h, void* stream) {
+  LoraGroup g;
+  const int64_t ones[LORA_MAX] = {8, 8, 8, 8};
+  int rc = lora_group("hyc_lora_down", A, ones, n, r, K, &g);
+  if (rc) return rc;
+  const int nr = n * r;
+  if (M < 0 || ldx < K || ldx % 8 != 0) return fail(HYC_EINVAL, "hyc_lora_down: M=%lld, row pitch %lld", (long long)M, (long long)ldx);
+  if (nr > 96) return fail(HYC_ENOTSUP, "hyc_lora_down: %d columns (at most 96)", nr);
+  if (M == 0) return HYC_OK;
+  if (!x || !h) return fail(HYC_EFAULT, "hyc_lora_down: null buffer");
+  if (!aligned16(x)) return fail(HYC_EINVAL, "hyc_lora_down: x must be 16-byte aligned");
+  hipStream_t st = begin_launch(stream);
+  const dim3 grid((unsigned)((M + 15) / 16));
+#define HYC_GO(CT_)                                                                                                        \
+  hipLaunchKernelGGL((k_lora_down<CT_>), grid, dim3(512), 0, st, static_cast<const uint16_t*>(x), ldx, M, (int)K, g,       \
+                     static_cast<uint16_t*>(h))
+  switch ((nr + 15) / 16) {
+    case 1: HYC_GO(1); break;
+    case 2: HYC_GO(2); break;
+    case 3: HYC_GO(3); break;
+    case 4: HYC_GO(4); break;
+    case 5: HYC_GO(5); break;
+    default: HYC_GO(6); break;
+  }
+#undef HYC_GO
+  return check_launch("hyc_lora_down");
+}
+
+int hyc_lora_up(const void* h, int64_t M, const void* const* B, const int64_t* n_out, int32_t n, int32_t r, float scale, void* y,
+                void* stream) {
+  LoraGroup g;
+  int rc = lora_group("hyc_lora_up", B, n_out, n, r, 64, &g);
+  if (rc) return rc;
+  if (M < 0) return fail(HYC_EINVAL, "hyc_lora_up: M=%lld", (long long)M);
+  if (M == 0) return HYC_OK;
+  if (!h || !y) return fail(HYC_EFAULT, "hyc_lora_up: null buffer");
+  if (!aligned16(h) || !aligned16(y)) return fail(HYC_EINVAL, "hyc_lora_up: buffers must be 16-byte aligned");
+  if ((M + LO_M - 1) / LO_M > 65535) return fail(HYC_ENOTSUP, "hyc_lora_up: too many tokens");
+  LoraOut a = {};
+  a.n = n; a.r = r;
+  for (int i = 0; i < n; ++i) {
+    a.B[i] = g.f[i];
+    a.n_out[i] = (int)n_out[i];
+    a.fb0[i + 1] = a.fb0[i] + (int)((n_out[i] + LO_F - 1) / LO_F);
+    a.row0[i + 1] = a.row0[i] + (int)n_out[i];
+  }
+  hipLaunchKernelGGL(k_lora_up, dim3((unsigned)a.fb0[n], (unsigned)((M + LO_M - 1) / LO_M)), dim3(256), 0, begin_launch(stream),
+                     static_cast<const uint16_t*>(h), M, a, scale, static_cast<uint16_t*>(y));
+  return check_launch("hyc_lora_up");
+}
+
+int64_t hyc_lora_up_bwd_workspace_bytes(int64_t M, const int64_t* n_out, int32_t n, int32_t r) {
+  if (M <= 0 || !n_out || n < 1 || n > LORA_MAX || r < 1) return 0;
+  int64_t rows = 0;
+  for (int i = 0; i < n; ++i) rows += n_out[i];
+  const int fblocks = lora_up_blocks(n_out, n);
+  const int64_t RC = r <= 16 ? 16 : 32;
+  return 4 * RC * ((int64_t)fblocks * M + (int64_t)lora_up_ranges(M, fblocks) * rows);
+}
+
+int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const int64_t* n_out, const void* const* B, const void* h,
+                    int32_t n, int32_t r, float scale, void* dh, void* ext, int64_t ld_ext, int64_t room, int32_t copy_dy, void* const* dB,
+                    void* workspace, void* stream) {
+  LoraGroup g;
+  int rc = lora_group("hyc_lora_up_bwd", B, n_out, n, r, 64, &g);
+  if (rc) return rc;
+  const int nr = n * r;
+  const int64_t rows = g.end[n - 1];
+  if (M < 0 || room < nr || ld_ext < rows + room || ld_ext % 8 != 0)
+    return fail(HYC_EINVAL, "hyc_lora_up_bwd: M=%lld, row pitch %lld, room=%lld for %d columns behind %lld", (long long)M, (long long)ld_ext,
+                (long long)room, nr, (long long)rows);
+  if (!dy || !ldg || !dB || (M > 0 && (!h || !dh || !ext || !workspace))) return fail(HYC_EFAULT, "hyc_lora_up_bwd: null buffer");
+  if (!aligned16(h) || !aligned16(ext) || !aligned16(workspace)) return fail(HYC_EINVAL, "hyc_lora_up_bwd: buffers must be 16-byte aligned");
+  LoraUp a = {};
+  a.n = n; a.r = r;
+  for (int i = 0; i < n; ++i) {
+    if (!dy[i] || !dB[i]) return fail(HYC_EFAULT, "hyc_lora_up_bwd: null buffer");
+    if (!aligned16(dy[i]) || ldg[i] < n_out[i] || ldg[i] % 8 != 0)
+      return fail(HYC_EINVAL, "hyc_lora_up_bwd: dy must be 16-byte aligned, rows a multiple of 8 (at least n_out) apart");
+    a.g[i] = static_cast<const uint16_t*>(dy[i]);
+    a.ldg[i] = ldg[i];
+    a.B[i] = g.f[i];
+    a.dB[i] = static_cast<uint16_t*>(dB[i]);
+    a.n_out[i] = (int)n_out[i];
+    a.fb0[i + 1] = a.fb0[i] + (int)((n_out[i] + LU_F - 1) / LU_F);
+    a.row0[i + 1] = a.row0[i] + (int)n_out[i];
+  }
+  if (M == 0) return HYC_OK;
+  const int fblocks = a.fb0[n], ranges = lora_up_ranges(M, fblocks);
+  int64_t tokens = (M + ranges - 1) / ranges;
+  tokens = (tokens + LU_M - 1) / LU_M * LU_M;
+  for (int i = 0; i < n; ++i)
+    if (tokens * ldg[i] >= ((int64_t)1 << 30)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: a token range of dy must stay below 2 GiB");
+  const int used = (int)((M + tokens - 1) / tokens);
+  const int RC = r <= 16 ? 16 : 32;
+  float *dhp = static_cast<float*>(workspace), *dbp = dhp + (int64_t)fblocks * M * RC;
+  uint16_t* cp = copy_dy ? static_cast<uint16_t*>(ext) : nullptr;
+  hipStream_t st = begin_launch(stream);
+  const dim3 grid((unsigned)fblocks, (unsigned)used);
+  if (RC == 16) hipLaunchKernelGGL((k_lora_up_bwd<1>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
+  else hipLaunchKernelGGL((k_lora_up_bwd<2>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
+  if ((rc = check_launch("hyc_lora_up_bwd"))) return rc;
+  const int64_t dh_items = (M * room + 255) / 256 * 256;
+  const int64_t blocks = dh_items / 256 + (rows * r + 255) / 256;
+  if (blocks >= ((int64_t)1 << 31)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: too many tokens");
+  hipLaunchKernelGGL(k_lora_up_finish, dim3((unsigned)blocks), dim3(256), 0, st, a, M, RC, dhp, dbp, used, scale, static_cast<uint16_t*>(dh),
+                     static_cast<uint16_t*>(ext) + rows, ld_ext, (int)room, dh_items);
+  return check_launch("hyc_lora_up_bwd (finish)");
+}
+
+}  // extern "C"

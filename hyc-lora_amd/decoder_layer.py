@@ -24,7 +24,7 @@ import torch
 from . import kernels as K
 from .operators._calibration import CompressionSite, running_mean
 from .operators.compress_function import get_statistics_softmax
-from .operators.efficient_hadamard import EfficientMemoryGatedAct
+from .operators.efficient_hadamard import EfficientMemoryGatedAct, _row_view
 from .operators.efficient_rmsnorm import EfficientMemoryRMSNorm
 
 BF16 = torch.bfloat16
@@ -86,89 +86,73 @@ class LoRAProjections(torch.nn.Module):
             row += out
         self.site = CompressionSite(cfg.outlier_ratio, 1.0, cfg.linear_bits, "per-token", 0, "hyc", cfg.linear_group,
                                     cfg.scale_rule)
+        self.room = K.lora_room(len(self.out_features), cfg.lora_r)
         self.iteration = 0
         self.record = None
-        self._fused_choice = {}
-
-    def fuse_base_gemm(self, x2, w_all):
-        """whether the group's base GEMM runs faster as one wide GEMM or as one per projection: measured once per
-        token count (the library's kernel selection favours either, depending on the shape: at 2048 tokens the
-        fused gate/up GEMM is 30 % slower than two, at 4096 tokens 20 % faster)"""
-        M = x2.shape[0]
-        if len(self.out_features) == 1:
-            return True
-        if M not in self._fused_choice:
-            scratch = torch.empty((M, sum(self.out_features)), dtype=BF16, device=x2.device)
-            times = []
-            for fused in (True, False):
-                _base_gemm(scratch, x2, w_all, self.out_features, fused)                      # warm-up
-                e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                e0.record()
-                for _ in range(3):
-                    _base_gemm(scratch, x2, w_all, self.out_features, fused)
-                e1.record()
-                e1.synchronize()
-                times.append(e0.elapsed_time(e1))
-            self._fused_choice[M] = times[0] <= times[1]
-        return self._fused_choice[M]
 
     def forward(self, x):
         x2 = x.reshape(-1, self.in_features)
         plan = self.site.channel_plan(x2, self.iteration) if self.cfg.compress else None
         self.iteration += 1
-        n = len(self.out_features)
         outs = _LoRAProjectionsFunc.apply(x, self, plan, *self.lora_A, *self.lora_B)
-        return outs if n > 1 else outs[0]
+        return outs if len(self.out_features) > 1 else outs[0]
 
 
-def _base_gemm(y_all, x2, w_all, out_features, fused):
-    """y_all += x2 @ w_all^T, as one GEMM or as one GEMM per projection writing its column slice of y_all"""
-    if fused or len(out_features) == 1:
-        y_all.addmm_(x2, w_all.t())
-        return
-    row = 0
-    for out in out_features:
-        y_all[:, row:row + out].addmm_(x2, w_all[row:row + out].t())
-        row += out
+def _product(out, a, b, accumulate=False):
+    """out [M, N] (+)= a @ b^T, both operands contiguous along the reduction.  The library's kernels for output widths that
+    are not whole multiples of 4096 waste up to a third of the chip from about six rounds of its 256-wide tiles on; cut at
+    8192 (4096) columns both parts run at the rate of the round widths: N = 22016, K = 4160 at 1536 / 2048 / 3093 / 4096
+    tokens 308 -> 221, 402 -> 260, 528 -> 421, 638 -> 505 us (but 332 -> 369 at 2560), N = 11008: 132 -> 122, 260 -> 143,
+    331 -> 232, 404 -> 264; N = 5632, K = 2112 at 3093 / 4096: 85 -> 75, 94 -> 79 (2048: 52 -> 54, so not below 3072)."""
+    M, N = out.shape
+    cut = 0
+    if N % 4096:
+        cut = 8192 if N > 8192 and M >= 1536 else 4096 if 4096 < N < 8192 and M >= 3072 else 0
+    for lo, hi in (((0, cut), (cut, N)) if cut else ((0, N),)):
+        part = out[:, lo:hi]
+        if accumulate:
+            part.addmm_(a, b[lo:hi].t())
+        else:
+            torch.mm(a, b[lo:hi].t(), out=part)
+
+
+def _room_behind(rows, tensors, total, room):
+    """`rows` if it is the [M, total + room] buffer whose first columns `tensors` are, side by side, else None"""
+    if not isinstance(rows, torch.Tensor) or rows.dtype != BF16 or rows.dim() != 2 or not rows.is_contiguous():
+        return None
+    if rows.shape[1] != total + room or any(t.dtype != BF16 or t.numel() != rows.shape[0] * t.shape[-1] for t in tensors):
+        return None
+    at = rows.data_ptr()
+    for t in tensors:
+        t2 = t.flatten(0, -2) if t.dim() > 2 else t
+        if t2.data_ptr() != at or t2.stride(1) != 1 or (t2.shape[0] > 1 and t2.stride(0) != total + room):
+            return None
+        at += 2 * t.shape[-1]
+    return rows
 
 
 class _LoRAProjectionsFunc(torch.autograd.Function):
+    """A group is one library product each way: forward y = s h B^T (h = x A^T), onto which the base product accumulates in
+    its epilogue; backward dX = [dY | s dY B] [W^T | A^T]^T with the rank-r terms as mod.room further columns of the
+    reduction (kernels.lora_down / lora_up / lora_up_bwd / lora_weight_t)."""
+
     @staticmethod
     def forward(ctx, x, mod, plan, *ab):
         n = len(mod.out_features)
         A, B = ab[:n], ab[n:]
-        r = A[0].shape[0]
-        x2 = x.reshape(-1, mod.in_features)
-        if not x2.is_contiguous():
-            x2 = x2.contiguous()
-        s = mod.scaling
-        zero = x2.new_zeros(1)                                   # ignored (beta = 0), only has to broadcast
-        total = sum(mod.out_features)
-        # h = x A^T for every projection of the group at once; the rank-r terms s * h_i B_i^T as one thin GEMM with
-        # the B_i on a block diagonal; then the base GEMM accumulates onto that in its epilogue (the other order
-        # costs a separate read-modify-write pass over y)
-        h_all = x2 @ (A[0] if n == 1 else torch.cat(list(A), dim=0)).t()                      # [M, n*r]
-        if n == 1:
-            b_all = B[0]
-        else:
-            b_all = x2.new_zeros((total, n * r))
-            row = 0
-            for i, out in enumerate(mod.out_features):
-                b_all[row:row + out, i * r:(i + 1) * r] = B[i]
-                row += out
-        y_all = torch.addmm(zero, h_all, b_all.t(), beta=0.0, alpha=s)                         # [M, sum(out)]
-        w_all = K.nf4_dequantize(mod.base_all)
-        _base_gemm(y_all, x2, w_all, mod.out_features, mod.fuse_base_gemm(x2, w_all))
-        del w_all, b_all
+        x2 = _row_view(x)
+        h = K.lora_down(x2, A)
+        y_all = K.lora_up(h, B, mod.scaling)
+        _product(y_all, x2, K.nf4_dequantize(mod.base_all), accumulate=True)
         outs, row = [], 0
         for out in mod.out_features:                            # column slices: no copies, consumers take the pitch
             outs.append(y_all[:, row:row + out].unflatten(0, x.shape[:-1]))
             row += out
         cfg = mod.cfg
-        ctx.saved_x = K.compress_channel(x2, plan, cfg.linear_bits, cfg.linear_group) if cfg.compress else x2
+        ctx.saved_x = K.compress_channel(x2, plan, cfg.linear_bits, cfg.linear_group) if cfg.compress else x2.contiguous()
         if mod.record is not None:
             mod.record["x"], mod.record["saved"] = x2.detach().clone(), ctx.saved_x
-        ctx.mod, ctx.h_all = mod, h_all
+        ctx.mod, ctx.h = mod, h
         ctx.save_for_backward(*ab)
         return tuple(outs)
 
@@ -176,38 +160,20 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
     def backward(ctx, *gs):
         mod = ctx.mod
         n = len(mod.out_features)
-        ab = ctx.saved_tensors
-        A, B = ab[:n], ab[n:]
-        r = A[0].shape[0]
-        s = mod.scaling
-        dA, dB, dhs, grads = [], [], [], []
-        zero = ab[0].new_zeros(1)
-        for i in range(n):
-            g = gs[i].reshape(-1, mod.out_features[i]).to(BF16)
-            if not g.is_contiguous():
-                g = g.contiguous()
-            grads.append(g)
-            dh = torch.addmm(zero, g, B[i], beta=0.0, alpha=s)    # [M, r]
-            dhs.append(dh)
-            dB.append(torch.addmm(zero, g.t(), ctx.h_all[:, i * r:(i + 1) * r], beta=0.0, alpha=s))
-        dh_all = dhs[0] if n == 1 else torch.cat(dhs, dim=1)         # [M, n*r]
+        A, B = ctx.saved_tensors[:n], ctx.saved_tensors[n:]
+        r, total = A[0].shape[0], sum(mod.out_features)
+        rows = _room_behind(getattr(gs[0], "_hyc_rows", None), gs, total, mod.room)
+        ext, dh, dB = K.lora_up_bwd([_row_view(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, mod.room, rows)
         # dA_i = dh_i^T @ x_hat: the projections of a group read the same saved activation, so their dh go through
         # the weight-gradient kernel side by side (32 output rows per call, the widest its LoRA-shaped form takes)
         # and x_hat is decoded once per call instead of once per projection
-        per_call = max(1, 32 // r) * r
+        dA, per_call = [], max(1, 32 // r) * r
         for c0 in range(0, n * r, per_call):
-            block = K.gradw_gemm(dh_all[:, c0:c0 + per_call], ctx.saved_x, out_dtype=A[0].dtype)
+            block = K.gradw_gemm(dh[:, c0:c0 + per_call], ctx.saved_x, out_dtype=A[0].dtype)
             dA.extend(block[j:j + r] for j in range(0, block.shape[0], r))
-        # dX: all rank-r terms as one thin GEMM, then each base GEMM accumulates onto it in its epilogue
-        dx = dh_all @ (A[0] if n == 1 else torch.cat(list(A), dim=0))
-        w_all = K.nf4_dequantize(mod.base_all)
-        row = 0
-        for i, out in enumerate(mod.out_features):
-            dx.addmm_(grads[i], w_all[row:row + out])
-            row += out
-        del w_all, grads, dhs
-        ctx.h_all = None
-        ctx.saved_x = None
+        dx = torch.empty((ext.shape[0], mod.in_features), dtype=BF16, device=ext.device)
+        _product(dx, ext, K.lora_weight_t(mod.base_all, A, mod.out_features, mod.room))
+        ctx.h = ctx.saved_x = None
         return (dx.reshape(gs[0].shape[:-1] + (mod.in_features,)), None, None) + tuple(dA) + tuple(dB)
 
 
@@ -237,9 +203,11 @@ class CompressedAttention(torch.nn.Module):
         self.static_value = None          # probability threshold, as in EfficientMemorySoftmax
         self.record = None
 
-    def forward(self, q, k, v, cos, sin):
+    def forward(self, q, k, v, cos, sin, grad_room=0):
+        """grad_room: columns to leave free behind the gradients of q, k and v side by side, where one kernel writes them (they
+        are handed on as `_hyc_rows` of the three, see _LoRAProjectionsFunc)"""
         func = _FlashAttentionFunc if self.cfg.attention == "flash" else _AttentionFunc
-        return func.apply(q, k, v, cos, sin, self)
+        return func.apply(q, k, v, cos, sin, self, grad_room)
 
 
 def _matrices_per_group(total, s, budget_bytes):
@@ -251,7 +219,7 @@ def _matrices_per_group(total, s, budget_bytes):
 
 class _AttentionFunc(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, k, v, cos, sin, mod):
+    def forward(ctx, q, k, v, cos, sin, mod, grad_room):
         cfg = mod.cfg
         b, s, H = q.shape
         nh, hd = cfg.heads, cfg.head_dim
@@ -348,7 +316,7 @@ class _AttentionFunc(torch.autograd.Function):
         dq = K.rope_from_heads(dq.view(b, nh, s, hd), cos, sin)
         dk = K.rope_from_heads(dk.view(b, nh, s, hd), cos, sin)
         dv = K.rope_from_heads(dv.view(b, nh, s, hd))
-        return dq, dk, dv, None, None, None
+        return dq, dk, dv, None, None, None, None
 
 
 class _FlashAttentionFunc(torch.autograd.Function):
@@ -359,7 +327,7 @@ class _FlashAttentionFunc(torch.autograd.Function):
     q and k with the exact log-sum-exp, and takes its row term sum(dO * O) from the restored output."""
 
     @staticmethod
-    def forward(ctx, q, k, v, cos, sin, mod):
+    def forward(ctx, q, k, v, cos, sin, mod, grad_room):
         cfg = mod.cfg
         b, s, H = q.shape
         nh, hd = cfg.heads, cfg.head_dim
@@ -369,6 +337,7 @@ class _FlashAttentionFunc(torch.autograd.Function):
         if ctx.rows:                                                # the kernels read and write the rows as they are
             q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
             out, lse = K.attn_fwd(q_rows, k_rows, v, nh, scale)
+            ctx.grad_room = grad_room
         else:
             qh, q_rows = K.rope_to_heads(q, nh, cos, sin, want_rows=True)
             kh, k_rows = K.rope_to_heads(k, nh, cos, sin, want_rows=True)
@@ -402,7 +371,10 @@ class _FlashAttentionFunc(torch.autograd.Function):
         if ctx.rows:
             qq, kk, vv, oo = (restore(c).view(b, s, nh * hd) for c in ctx.saved)
             ctx.saved = None
-            return K.attn_bwd(g.to(BF16).contiguous(), qq, kk, vv, oo, lse, nh, 1.0 / math.sqrt(hd), cos, sin) + (None, None, None)
+            grads = K.attn_bwd(g.to(BF16).contiguous(), qq, kk, vv, oo, lse, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
+            for t in grads[:3]:
+                t._hyc_rows = grads[3]
+            return grads[:3] + (None,) * 4
         to_heads = lambda rows: K.rope_to_heads(rows.view(b, s, nh * hd), nh)
         gh = K.rope_to_heads(g.to(BF16).contiguous(), nh)
         qq, kk, vv, oo = (to_heads(restore(c)) for c in ctx.saved)
@@ -413,7 +385,7 @@ class _FlashAttentionFunc(torch.autograd.Function):
         dq = K.rope_from_heads(dq.contiguous(), cos, sin)
         dk = K.rope_from_heads(dk.contiguous(), cos, sin)
         dv = K.rope_from_heads(dv.contiguous())
-        return dq, dk, dv, None, None, None
+        return dq, dk, dv, None, None, None, None
 
 
 # ---- the layer --------------------------------------------------------------------------------------------------
@@ -461,12 +433,12 @@ class DecoderLayer(torch.nn.Module):
             self._rope = rope_tables(s, cfg.head_dim, cfg.rope_theta, x.device)
         cos, sin = self._rope
         # no names for the wide intermediates: each is released as soon as its consumer has run
-        x = x + self.o_proj(self.attention(*self.qkv_proj(self.input_layernorm(x)), cos, sin))
+        x = x + self.o_proj(self.attention(*self.qkv_proj(self.input_layernorm(x)), cos, sin, self.qkv_proj.room))
         return x + self.down_proj(self._gated(*self.gate_up_proj(self.post_attention_layernorm(x))))
 
     def _gated(self, gate, up):
         if self.act is not None:
-            return self.act(gate, up)
+            return self.act(gate, up, grad_room=self.gate_up_proj.room)
         return torch.nn.functional.silu(gate) * up
 
     def saved_activation_bytes(self, batch, seq):

@@ -642,19 +642,25 @@ def hadamard_bwd(g2d, src1, src2):
     return dx1, dx2
 
 
-def gated_act_bwd(act, g2d, src_act, src_up, src_gate):
-    """backward of act(gate) * up in one pass -> (d_gate, d_up); the three sources are ChannelCompressed"""
+def gated_act_bwd(act, g2d, src_act, src_up, src_gate, room=None):
+    """backward of act(gate) * up in one pass -> (d_gate, d_up); the three sources are ChannelCompressed.  With `room` (a
+    number of columns, 0 included) the two are the halves of one [M, 2 H + room] matrix, returned as a third value."""
     _need(g2d, BF16, "grad_output")
     M, H = g2d.shape
     sa, va, ca, da = _source(src_act, M, H)
     su, vu, cu, du = _source(src_up, M, H)
     sg, vg, cg, dg = _source(src_gate, M, H)
-    d_gate, d_up = torch.empty_like(g2d), torch.empty_like(g2d)
+    both = None
+    if room is None:
+        d_gate, d_up, pitch = torch.empty_like(g2d), torch.empty_like(g2d), H
+    else:
+        both = torch.empty((M, 2 * H + room), dtype=BF16, device=g2d.device)
+        d_gate, d_up, pitch = both[:, :H], both[:, H:2 * H], 2 * H + room
     code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
-    check(_abi.load().hyc_gated_act_bwd(code, _p(g2d), _p(sa), _p(va), _p(ca), ctypes.byref(da), _p(su), _p(vu), _p(cu),
-                                        ctypes.byref(du), _p(sg), _p(vg), _p(cg), ctypes.byref(dg), M, H, _p(d_gate),
-                                        _p(d_up), _stream()))
-    return d_gate, d_up
+    check(_abi.load().hyc_gated_act_bwd_rows(code, _p(g2d), _p(sa), _p(va), _p(ca), ctypes.byref(da), _p(su), _p(vu), _p(cu),
+                                             ctypes.byref(du), _p(sg), _p(vg), _p(cg), ctypes.byref(dg), M, H, _p(d_gate), pitch,
+                                             _p(d_up), pitch, _stream()))
+    return (d_gate, d_up) if room is None else (d_gate, d_up, both)
 
 
 def _row_kernel_fits(H, bits, group, widths):
@@ -960,6 +966,102 @@ def nf4_dequantize(q: NF4Weight, out=None):
 
 
 # ----------------------------------------------------------------------------------------------------
+# LoRA beside a frozen NF4 base
+# ----------------------------------------------------------------------------------------------------
+def lora_room(n, r):
+    """columns appended to the reduction of a group's input gradient for its n * r rank columns: whole steps of 64"""
+    return -(-n * r // 64) * 64
+
+
+def _lora_kernels_cover(factors, K, outs, r):
+    return (len(factors) <= 4 and r in (8, 16, 24, 32) and len(factors) * r <= 96 and K % 64 == 0 and all(o % 8 == 0 for o in outs)
+            and all(f.dtype == BF16 and f.is_contiguous() for f in factors))
+
+
+def _ptrs(ts):
+    return (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+
+
+def _i64s(vs):
+    return (ctypes.c_int64 * len(vs))(*vs)
+
+
+def lora_down(x2d, A):
+    """h [M, n r] = x A_i^T side by side"""
+    _need_rows(x2d, "x")
+    M, Kf = x2d.shape
+    n, r = len(A), A[0].shape[0]
+    if not _lora_kernels_cover(A, Kf, [8], r):
+        return x2d @ torch.cat(list(A), dim=0).t()
+    h = torch.empty((M, n * r), dtype=BF16, device=x2d.device)
+    check(_abi.load().hyc_lora_down(_p(x2d), x2d.stride(0) if M > 1 else Kf, M, Kf, _ptrs(A), n, r, _p(h), _stream()))
+    return h
+
+
+def lora_up(h, B, scale):
+    """y [M, sum(out_i)] = scale * h_i B_i^T side by side"""
+    M, n, r = h.shape[0], len(B), B[0].shape[1]
+    outs = [b.shape[0] for b in B]
+    y = torch.empty((M, sum(outs)), dtype=BF16, device=h.device)
+    if _lora_kernels_cover(B, 64, outs, r):
+        check(_abi.load().hyc_lora_up(_p(_need(h, BF16, "h")), M, _ptrs(B), _i64s(outs), n, r, float(scale), _p(y), _stream()))
+        return y
+    zero, col = h.new_zeros(1), 0
+    for i, (b, o) in enumerate(zip(B, outs)):
+        torch.addmm(zero, h[:, i * r:(i + 1) * r], b.t(), beta=0.0, alpha=scale, out=y[:, col:col + o])
+        col += o
+    return y
+
+
+def lora_up_bwd(gs, B, h, scale, room, ext=None):
+    """(ext, dh, [dB_i]) from the gradients gs[i] [M, out_i] of a group: dB_i = scale * gs[i]^T h_i, dh = scale * gs[i] B_i
+    side by side [M, n r] and, with zeros behind them, as the columns [sum(outs), + room) of ext.  ext: the buffer the gs
+    already are the first columns of, side by side; None: they are copied into a new one."""
+    M, n, r = gs[0].shape[0], len(gs), B[0].shape[1]
+    outs = [g.shape[1] for g in gs]
+    total = sum(outs)
+    copy = ext is None
+    if copy:
+        ext = torch.empty((M, total + room), dtype=BF16, device=gs[0].device)
+    if _lora_kernels_cover(B, 64, outs, r):
+        for g in gs:
+            _need_rows(g, "grad_output")
+        lib = _abi.load()
+        dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
+        dB = [torch.empty_like(b) for b in B]
+        outs_c = _i64s(outs)
+        ws = torch.empty(lib.hyc_lora_up_bwd_workspace_bytes(M, outs_c, n, r) // 4, dtype=torch.float32, device=h.device)
+        pitches = _i64s([g.stride(0) if M > 1 else o for g, o in zip(gs, outs)])
+        check(lib.hyc_lora_up_bwd(_ptrs(gs), pitches, M, outs_c, _ptrs(B), _p(h), n, r, float(scale), _p(dh), _p(ext), total + room, room,
+                                  1 if copy else 0, _ptrs(dB), _p(ws), _stream()))
+        return ext, dh, dB
+    zero = h.new_zeros(1)
+    dh = torch.cat([torch.addmm(zero, g, b, beta=0.0, alpha=scale) for g, b in zip(gs, B)], dim=1)
+    dB = [torch.addmm(zero, g.t(), h[:, i * r:(i + 1) * r], beta=0.0, alpha=scale) for i, g in enumerate(gs)]
+    if copy:
+        col = 0
+        for g, o in zip(gs, outs):
+            ext[:, col:col + o] = g
+            col += o
+    ext[:, total:] = 0
+    ext[:, total:total + n * r] = dh
+    return ext, dh, dB
+
+
+def lora_weight_t(q: NF4Weight, A, outs, room):
+    """[K, sum(outs) + room] = [W^T | A_i^T side by side | zeros]: the transposed weight of the group's input gradient"""
+    total, Kf = q.shape
+    n, r = len(A), A[0].shape[0]
+    out = torch.empty((Kf, total + room), dtype=BF16, device=q.packed.device)
+    if _lora_kernels_cover(A, Kf, outs, r):
+        check(_abi.load().hyc_lora_weight_t(_p(q.packed), _p(q.absmax), Kf, _ptrs(A), _i64s(outs), n, r, room, _p(out), _stream()))
+        return out
+    out[:, :total], out[:, total:] = nf4_dequantize(q).t(), 0
+    out[:, total:total + n * r] = torch.cat(list(A), dim=0).t()
+    return out
+
+
+# ----------------------------------------------------------------------------------------------------
 # rotary embedding + attention layout
 # ----------------------------------------------------------------------------------------------------
 def _need_tables(cos, sin, S, hd):
@@ -1045,9 +1147,10 @@ def attn_fwd(q, k, v, heads, scale):
     return out, lse
 
 
-def attn_bwd(g, q, k, v, out, lse, heads, scale, cos=None, sin=None):
+def attn_bwd(g, q, k, v, out, lse, heads, scale, cos=None, sin=None, room=None):
     """(dq, dk, dv) of attn_fwd at the given q, k, v, out and lse; with cos / sin the gradients of q and k before their
-    rotation"""
+    rotation.  With `room` (a number of columns, 0 included) the three lie side by side in one [B*S, 3 H + room] matrix,
+    returned as a fourth value."""
     B, S, H, pg = _need_tokens(g, "g")
     ptrs = []
     for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):
@@ -1056,11 +1159,17 @@ def attn_bwd(g, q, k, v, out, lse, heads, scale, cos=None, sin=None):
         ptrs += [_p(t), _need_tokens(t, name)[3]]
     _need_vec(lse, torch.float32, B * heads * S, "lse")
     _need_tables(cos, sin, S, H // heads)
-    dq, dk, dv = (torch.empty((B, S, H), dtype=BF16, device=g.device) for _ in range(3))
+    if room is None:
+        pitch = H
+        dq, dk, dv = (torch.empty((B, S, H), dtype=BF16, device=g.device) for _ in range(3))
+    else:
+        pitch = 3 * H + room
+        both = torch.empty((B * S, pitch), dtype=BF16, device=g.device)
+        dq, dk, dv = (both[:, i * H:(i + 1) * H].unflatten(0, (B, S)) for i in range(3))
     ws = torch.empty(2 * B * heads * S, dtype=torch.float32, device=g.device)
     check(_abi.load().hyc_attn_bwd(_p(g), pg, *ptrs, _p(lse), _p(cos), _p(sin), B, S, heads, H // heads, float(scale),
-                                   _p(dq), H, _p(dk), H, _p(dv), H, _p(ws), _stream()))
-    return dq, dk, dv
+                                   _p(dq), pitch, _p(dk), pitch, _p(dv), pitch, _p(ws), _stream()))
+    return (dq, dk, dv) if room is None else (dq, dk, dv, both)
 
 
 # ----------------------------------------------------------------------------------------------------

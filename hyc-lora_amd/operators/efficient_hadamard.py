@@ -113,8 +113,8 @@ class _ChannelGatedActFunc(torch.autograd.Function):
     (gate; act(gate) and up), and one backward pass over them."""
 
     @staticmethod
-    def forward(ctx, gate, up, act, sites, iteration, bits, group):
-        ctx.act = act
+    def forward(ctx, gate, up, act, sites, iteration, bits, group, grad_room=None):
+        ctx.act, ctx.grad_room = act, grad_room
         calibrated = iteration >= 2 and all(site.plan is not None for site in sites)
         if calibrated and K.gated_act_fwd_supported(gate.shape[-1], bits, group):
             # steady state: one pass over gate and up writes the product and the three compressed activations;
@@ -133,8 +133,11 @@ class _ChannelGatedActFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         g2, _ = as_rows(grad_output.to(torch.bfloat16))
-        d_gate, d_up = K.gated_act_bwd(ctx.act, g2, *ctx.saved)
-        return d_gate.reshape(grad_output.shape), d_up.reshape(grad_output.shape), None, None, None, None, None
+        grads = K.gated_act_bwd(ctx.act, g2, *ctx.saved, room=ctx.grad_room)
+        d_gate, d_up = (t.reshape(grad_output.shape) for t in grads[:2])
+        if ctx.grad_room is not None:
+            d_gate._hyc_rows = d_up._hyc_rows = grads[2]
+        return d_gate, d_up, None, None, None, None, None, None
 
 
 class EfficientMemoryGatedAct(torch.nn.Module):
@@ -155,8 +158,10 @@ class EfficientMemoryGatedAct(torch.nn.Module):
         self.site_act, self.site_up, self.site_gate = mk(), mk(), mk()
         self.iteration = 0
 
-    def forward(self, gate, up):
+    def forward(self, gate, up, grad_room=None):
+        """grad_room: write the gradients of gate and up side by side into one matrix with that many free columns behind them,
+        and hand the matrix on as `_hyc_rows` of both, so that the projections they go to can append to its rows"""
         out = _ChannelGatedActFunc.apply(gate, up, self.act, (self.site_act, self.site_up, self.site_gate), self.iteration,
-                                         self.sub_outlier_bit, self.group_size)
+                                         self.sub_outlier_bit, self.group_size, grad_room)
         self.iteration += 1
         return out

@@ -226,6 +226,12 @@ int hyc_gated_act_bwd(int32_t act, const void* g, const void* stored_a, const vo
                       const hyc_desc* d_a, const void* stored_u, const void* vals_u, const void* scales_u,
                       const hyc_desc* d_u, const void* stored_g, const void* vals_g, const void* scales_g,
                       const hyc_desc* d_g, int64_t M, int64_t H, void* d_gate, void* d_up, void* stream);
+/* the same with row pitches for the two results (e.g. the halves of one [M, 2 H + room] matrix) */
+int hyc_gated_act_bwd_rows(int32_t act, const void* g, const void* stored_a, const void* vals_a, const void* scales_a,
+                           const hyc_desc* d_a, const void* stored_u, const void* vals_u, const void* scales_u,
+                           const hyc_desc* d_u, const void* stored_g, const void* vals_g, const void* scales_g,
+                           const hyc_desc* d_g, int64_t M, int64_t H, void* d_gate, int64_t ld_dgate, void* d_up, int64_t ld_dup,
+                           void* stream);
 
 /* Forward of the same product with its three saves fused in: h = bf16(bf16(act(gate)) * up), plus the channel-compressed
  * forms of act(gate), up and gate (what EfficientMemorySiLU/GELU.forward, efficient_silu.py:13-40 / efficient_gelu.py:13-40,
@@ -313,6 +319,30 @@ int hyc_rope_to_heads(const void* x, int64_t x_pitch, const void* cosv, const vo
                       int64_t heads, int64_t head_dim, void* out_heads, void* out_rows, void* stream);
 int hyc_rope_from_heads(const void* g, const void* cosv, const void* sinv, int64_t B, int64_t S, int64_t heads,
                         int64_t head_dim, void* out_rows, void* stream);
+
+/* ---- LoRA beside a frozen NF4 base --------------------------------------------------------------- */
+/* A group of n (1 to 4) projections of one input, rank r (8, 16, 24 or 32) each, K input features (a multiple of 64),
+ * n_out[i] output features (multiples of 8); A_i bf16 [r, K], B_i bf16 [n_out_i, r]; `packed` / `absmax` hold the stacked
+ * base [sum n_out, K] as hyc_nf4_quantize writes it.  What stands beside the products with the base weight:
+ *   hyc_lora_down      h bf16 [M, n r] = x A_i^T side by side
+ *   hyc_lora_up        y bf16 [M, sum n_out] = scale * h_i B_i^T side by side (the base product accumulates onto it)
+ *   hyc_lora_up_bwd    from one read of dY_i [M, n_out_i] (rows ldg[i] apart): dh = bf16(scale * dY_i B_i) to dh [M, n r] and,
+ *                      with zeros behind them, to the `room` columns [sum n_out, + room) of ext (rows ld_ext apart);
+ *                      dB_i = scale * dY_i^T h_i; with copy_dy the dY_i side by side to the first sum n_out columns of ext.
+ *                      workspace: hyc_lora_up_bwd_workspace_bytes()
+ *   hyc_lora_weight_t  out bf16 [K, sum n_out + room] = [W^T | A_i^T side by side | zeros]: dX = ext out^T is the whole input
+ *                      gradient of the group, base and rank-r terms
+ * fp32 accumulation in a fixed order throughout; room >= n r, a multiple of 8.
+ * (peft's Linear.forward around bitsandbytes_fix/_function.py:509-540 computes the same per projection.) */
+int hyc_lora_down(const void* x, int64_t ldx, int64_t M, int64_t K, const void* const* A, int32_t n, int32_t r, void* h, void* stream);
+int hyc_lora_up(const void* h, int64_t M, const void* const* B, const int64_t* n_out, int32_t n, int32_t r, float scale, void* y,
+                void* stream);
+int64_t hyc_lora_up_bwd_workspace_bytes(int64_t M, const int64_t* n_out, int32_t n, int32_t r);
+int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const int64_t* n_out, const void* const* B, const void* h,
+                    int32_t n, int32_t r, float scale, void* dh, void* ext, int64_t ld_ext, int64_t room, int32_t copy_dy, void* const* dB,
+                    void* workspace, void* stream);
+int hyc_lora_weight_t(const void* packed, const float* absmax, int64_t K, const void* const* A, const int64_t* n_out, int32_t n,
+                      int32_t r, int64_t room, void* out, void* stream);
 
 /* ---- fused causal attention ------------------------------------------------------------------ */
 /* On the rows layout [B, S, heads, head_dim] of the projections, every operand with its own token pitch (elements between

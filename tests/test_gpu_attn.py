@@ -48,11 +48,12 @@ def test_attention_against_fp32(K, hd, B, S, heads):
     out, lse = K.attn_fwd(q, k, v, heads, scale)
     leaves = [t.float().detach().contiguous().requires_grad_(True) for t in (q, k, v)]
     want, want_lse = attention_fp32(*leaves, heads, scale)
-    # probabilities are rounded to bf16 for the second product and the result once more: 2 * 2^-9 at most
+    # probabilities are rounded to bf16 for the second product and the result once more; a rounding is 2^-8 / sqrt(3) of the
+    # leading binade in the root mean square, below 2^-9 over a norm
     close(out, want.detach(), 2 * 2.0 ** -9)
     assert (lse - want_lse.detach()).abs().max() < 1e-4        # fp32 sums of at most 1030 terms
     grads = torch.autograd.grad(want, leaves, g.float())
-    # P or dS, the stored output inside delta, and the result: 3 * 2^-9 at most
+    # P or dS, the stored output inside delta, and the result: three such roundings
     for got, ref in zip(K.attn_bwd(g, q, k, v, out, lse, heads, scale), grads):
         close(got, ref, 3 * 2.0 ** -9)
 

@@ -1,0 +1,74 @@
+"""The kernels beside the frozen base of a LoRA projection group against the same products in fp32, at the sizes where a
+tile of tokens (16, 64, 128), a block of features (256) or a factor (8 of 16 / 24 of 32 columns) is cut, and the torch form
+that serves the ranks they do not cover."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K(hyc):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return hyc.kernels
+
+
+def close(got, want):
+    """one rounding of an fp32 sum to bf16 (8 bits of significand: at most 2^-8 of the element), plus the sums' own error (fp32,
+    a few thousand terms)"""
+    want = want.double()
+    bound = 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max().clamp_min(1e-30)
+    assert ((got.double() - want).abs() <= bound).all(), float(((got.double() - want).abs() / bound).max())
+
+
+CASES = [(1, 64, [8], 8), (16, 256, [256, 64, 128], 16), (65, 512, [1000, 24], 24), (157, 1024, [320], 32), (130, 2816, [1024, 1024, 1024], 32),
+         (300, 4096, [4096, 512], 16), (33, 256, [256, 256], 64)]                   # rank 64: the torch form
+
+
+@pytest.mark.parametrize("M,Kf,outs,r", CASES)
+def test_lora_group_products(K, M, Kf, outs, r):
+    n, total, room, s = len(outs), sum(outs), K.lora_room(len(outs), r), 1.5
+    assert room >= n * r and room % 64 == 0
+    gen = torch.Generator(device="cuda").manual_seed(M + Kf)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    A, B = [mk(r, Kf) for _ in outs], [mk(o, r) for o in outs]
+    wide = mk(M, Kf + 8)
+    x = wide[:, :Kf]                                                                # rows with a pitch of their own
+    h = K.lora_down(x, A)
+    close(h, torch.cat([x.float() @ a.float().t().contiguous() for a in A], 1))
+    y = K.lora_up(h, B, s)
+    close(y, torch.cat([s * (h[:, i * r:(i + 1) * r].float() @ b.float().t().contiguous()) for i, b in enumerate(B)], 1))
+    gs = [mk(M, o) for o in outs]
+    ext, dh, dB = K.lora_up_bwd(gs, B, h, s, room)
+    close(dh, torch.cat([s * (g.float() @ b.float()) for g, b in zip(gs, B)], 1))
+    for i, (g, d) in enumerate(zip(gs, dB)):
+        close(d, s * (g.float().t().contiguous() @ h[:, i * r:(i + 1) * r].float()))
+    assert torch.equal(ext[:, :total], torch.cat(gs, 1))                            # the copy, dh, zeros
+    assert torch.equal(ext[:, total:total + n * r], dh) and not ext[:, total + n * r:].any()
+    # the gradients already in front of the room: nothing is copied, the rest is the same bit for bit
+    buf = torch.full_like(ext, float("nan"))
+    buf[:, :total] = ext[:, :total]
+    cuts = [sum(outs[:i]) for i in range(n + 1)]
+    ext2, dh2, dB2 = K.lora_up_bwd([buf[:, a:b] for a, b in zip(cuts, cuts[1:])], B, h, s, room, buf)
+    assert ext2 is buf and torch.equal(ext2, ext) and torch.equal(dh2, dh) and all(torch.equal(a, b) for a, b in zip(dB2, dB))
+    # the transposed weight: the dequantised values and the factors themselves
+    q = K.nf4_quantize(mk(total, Kf))
+    wt = K.lora_weight_t(q, A, outs, room)
+    assert torch.equal(wt[:, :total], K.nf4_dequantize(q).t()) and torch.equal(wt[:, total:total + n * r], torch.cat(A, 0).t())
+    assert not wt[:, total + n * r:].any()
+
+
+def test_gradients_side_by_side_are_recognised_only_when_they_are(hyc):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import importlib
+    DL = importlib.import_module(hyc.__name__ + ".decoder_layer")
+    buf = torch.zeros(6, 64 + 32 + 64, dtype=torch.bfloat16, device="cuda")
+    a, b = buf[:, :64].unflatten(0, (2, 3)), buf[:, 64:96].unflatten(0, (2, 3))
+    assert DL._room_behind(buf, [a, b], 96, 64) is buf
+    assert DL._room_behind(None, [a, b], 96, 64) is None
+    assert DL._room_behind(buf, [b, a], 96, 64) is None
+    assert DL._room_behind(buf, [a, b.clone()], 96, 64) is None
+    assert DL._room_behind(buf, [a, b], 96, 128) is None
+    assert DL._room_behind(buf[:, :160].float(), [a, b], 96, 64) is None
