@@ -60,6 +60,8 @@ SIGNATURES = {
                                        ctypes.POINTER(HycDesc), c_i32, c_ptr, c_ptr, c_ptr]),
     "hyc_layernorm_bwd": (c_i32, [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i32, c_ptr, c_ptr, c_i64, c_i64,
                                   ctypes.POINTER(HycDesc), c_ptr, c_ptr, c_ptr, c_ptr]),
+    "hyc_bias_grad_partials": (c_i64, [c_i64, c_i64]),
+    "hyc_bias_grad": (c_i32, [c_ptr, c_i64, c_i64, c_ptr, c_ptr, c_i32, c_ptr]),
     "hyc_act_bwd": (c_i32, [c_i32, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_i64, ctypes.POINTER(HycDesc), c_ptr, c_ptr]),
     "hyc_hadamard_bwd": (c_i32, [c_ptr, c_ptr, c_ptr, c_ptr, ctypes.POINTER(HycDesc), c_ptr, c_ptr, c_ptr,
                                  ctypes.POINTER(HycDesc), c_i64, c_i64, c_ptr, c_ptr, c_ptr]),

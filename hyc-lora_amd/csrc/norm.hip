@@ -942,6 +942,59 @@ k_colsum(const float* __restrict__ partials, int64_t P, int64_t H, void* __restr
   }
 }
 
+// Column sums of a bf16 [M, H] matrix (the bias gradient: dy summed over the tokens) as fp32 partial rows for k_colsum.
+// Bound by the one read of dy.  A workgroup takes a block of rows of 256 columns: 32 lanes side by side (512 contiguous
+// bytes of a row), eight rows at a time, four such steps requested before the first is added; its eight row lanes meet in
+// LDS.  Replaces a conversion to fp32, the library's sum of that copy and a conversion back (10 bytes an element instead
+// of 2): 3627 x 1024 30 -> 7 us with the sum of the partial rows.
+constexpr int BIAS_COLS = 256, BIAS_LANES = BIAS_COLS / 8, BIAS_ROWS = 8, BIAS_STEPS = 4;
+__global__ void __launch_bounds__(256)
+k_bias_partials(const uint16_t* __restrict__ dy, int64_t M, int64_t H, int64_t rows_per_block, float* __restrict__ partials) {
+  __shared__ __align__(16) float part[BIAS_ROWS][BIAS_COLS];
+  const int cl = threadIdx.x & (BIAS_LANES - 1), rl = threadIdx.x / BIAS_LANES;
+  const int64_t col = (int64_t)blockIdx.x * BIAS_COLS + 8 * cl;
+  const int64_t r0 = (int64_t)blockIdx.y * rows_per_block;
+  const int64_t r1 = r0 + rows_per_block < M ? r0 + rows_per_block : M;
+  float acc[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+  if (col < H) {                                           // H is a multiple of 8: a chunk is whole or absent
+    for (int64_t r = r0 + rl; r < r1; r += BIAS_ROWS * BIAS_STEPS) {
+      uint4 raw[BIAS_STEPS];
+#pragma unroll
+      for (int t = 0; t < BIAS_STEPS; ++t)
+        raw[t] = r + t * BIAS_ROWS < r1 ? *reinterpret_cast<const uint4*>(dy + (r + t * BIAS_ROWS) * H + col) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < BIAS_STEPS; ++t) {
+        float v[8];
+        unpack8(raw[t], v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] += v[j];
+      }
+    }
+  }
+  float4* o = reinterpret_cast<float4*>(&part[rl][8 * cl]);
+  o[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  o[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  __syncthreads();
+  const int64_t c = (int64_t)blockIdx.x * BIAS_COLS + threadIdx.x;
+  float s = 0.f;
+#pragma unroll
+  for (int l = 0; l < BIAS_ROWS; ++l) s += part[l][threadIdx.x];
+  if (c < H) partials[(int64_t)blockIdx.y * H + c] = s;
+}
+
+// rows a workgroup of k_bias_partials sums: one round of 32 at least, and so many that about 1024 workgroups are launched and
+// the partial rows stay at 256 (what k_colsum reads in one trip)
+static inline int64_t bias_rows_per_block(int64_t M, int64_t H) {
+  const int64_t across = (H + BIAS_COLS - 1) / BIAS_COLS;
+  int64_t blocks = 1024 / across;
+  blocks = blocks < 1 ? 1 : blocks > 256 ? 256 : blocks;
+  const int64_t round = BIAS_ROWS * BIAS_STEPS;
+  const int64_t rows = (M + blocks - 1) / blocks;
+  return (rows + round - 1) / round * round;
+}
+
 // Row-slot geometry of the fused norm kernels: T threads per row, ITERS chunks per thread and segment.
 struct NormGeom {
   int T, iters, iters_t;   // iters_t = the template value (1, 2 or 4) that covers `iters`
@@ -1356,6 +1409,32 @@ int hyc_layernorm_bwd(const void* dy, const void* stored, const void* vals, cons
                       void* dx, float* dw_partials, void* dw, void* stream) {
   if (M > 0 && !mean) return fail(HYC_EFAULT, "hyc_layernorm_bwd: null mean");
   return norm_bwd_impl(dy, stored, vals, scales, w, w_dtype, rstd, mean, M, H, d, 1, dx, dw_partials, dw, stream);
+}
+
+int64_t hyc_bias_grad_partials(int64_t M, int64_t H) {
+  if (M <= 0 || H <= 0) return 0;
+  const int64_t rpb = bias_rows_per_block(M, H);
+  return (M + rpb - 1) / rpb;
+}
+
+int hyc_bias_grad(const void* dy, int64_t M, int64_t H, float* partials, void* db, int32_t db_dtype, void* stream) {
+  if (M < 0 || H <= 0 || H % 8 != 0 || H > 65536)
+    return fail(HYC_EINVAL, "hyc_bias_grad: M=%lld H=%lld (H a multiple of 8, at most 65536)", (long long)M, (long long)H);
+  if (db_dtype != HYC_DTYPE_BF16 && db_dtype != HYC_DTYPE_F32) return fail(HYC_EINVAL, "hyc_bias_grad: db_dtype=%d", db_dtype);
+  if (!db || (M > 0 && (!dy || !partials))) return fail(HYC_EFAULT, "hyc_bias_grad: null buffer");
+  if (M > 0 && !aligned16(dy)) return fail(HYC_EINVAL, "hyc_bias_grad: dy must be 16-byte aligned");
+  hipStream_t st = begin_launch(stream);
+  int64_t P = 0;
+  if (M > 0) {
+    const int64_t rpb = bias_rows_per_block(M, H);
+    P = (M + rpb - 1) / rpb;
+    hipLaunchKernelGGL(k_bias_partials, dim3((unsigned)((H + BIAS_COLS - 1) / BIAS_COLS), (unsigned)P), dim3(256), 0, st,
+                       static_cast<const uint16_t*>(dy), M, H, rpb, partials);
+    const int rc = check_launch("hyc_bias_grad");
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(k_colsum, dim3((unsigned)((H + 31) / 32)), dim3(256), 0, st, partials, P, H, db, db_dtype == HYC_DTYPE_F32);
+  return check_launch("hyc_bias_grad (sum)");
 }
 
 }  // extern "C"

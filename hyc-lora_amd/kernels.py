@@ -603,6 +603,17 @@ def layernorm_bwd(dy2d, src, w, mean, rstd):
     return dx, dw
 
 
+def bias_grad(dy2d, dtype):
+    """the sum of dy bf16 [M, H] over its rows, accumulated in fp32, as a vector of `dtype` (bf16 or fp32)"""
+    _need(dy2d, BF16, "dy")
+    M, H = dy2d.shape
+    lib = _abi.load()
+    partials = torch.empty((max(lib.hyc_bias_grad_partials(M, H), 1), H), dtype=torch.float32, device=dy2d.device)
+    db = torch.empty(H, dtype=dtype, device=dy2d.device)
+    check(lib.hyc_bias_grad(_p(dy2d), M, H, _p(partials), _p(db), _wdtype(db), _stream()))
+    return db
+
+
 def rmsnorm_bwd_partial(dy2d, src, w, rstd, c2_quirk=True):
     """-> (dx bf16 [M,H], fp32 partial rows [P,H] whose column sum is dw); the caller does the last reduction"""
     _need(dy2d, BF16, "dy")

@@ -3,7 +3,7 @@ backward :66-148, Function :203-330, module :333-405).
 
 The forward is one kernel (statistics, y and the compressed x from a single read of x, the RMSNorm forward kernel
 with the row mean added); the backward is the fused decompress + dx + dw kernel of the RMSNorm path with the row mean
-folded in (xn = (x_hat - mean) * rstd), and db = sum of dy.  Rows too long for the one-pass forward (more than 1024
+folded in (xn = (x_hat - mean) * rstd), and db = sum of dy (K.bias_grad).  Rows too long for the one-pass forward (more than 1024
 chunks per segment) take the framework's layer norm followed by the compress kernel."""
 import torch
 
@@ -32,7 +32,9 @@ def _affine(weight, bias):
 def _backward(ctx, dy):
     dy2, _ = as_rows(dy.to(torch.bfloat16))
     dx, dw = K.layernorm_bwd(dy2, ctx.saved, ctx.weight.detach().contiguous(), ctx.mean, ctx.rstd)
-    db = dy2.float().sum(0).to(ctx.bias.dtype) if ctx.bias is not None else None
+    db = None
+    if ctx.bias is not None:
+        db = K.bias_grad(dy2, ctx.bias.dtype if ctx.bias.dtype == torch.bfloat16 else torch.float32).to(ctx.bias.dtype)
     return dx.reshape(dy.shape), dw, db
 
 

@@ -203,11 +203,16 @@ int hyc_layernorm_fwd_compress(const void* x, const void* w, const void* bias, i
                                void* scales, int32_t* row_counts, void* stream);
 
 /* LayerNorm backward (efficient_layernorm.py:66-148, 262-330): xn = (xhat - mean)*rstd, dx as above with both
- * means (c1, c2), dw = sum_m dy*xn.  db = sum_m dy is a plain reduction left to the caller.  Buffers as for
+ * means (c1, c2), dw = sum_m dy*xn.  db = sum_m dy: hyc_bias_grad.  Buffers as for
  * hyc_rmsnorm_bwd. */
 int hyc_layernorm_bwd(const void* dy, const void* stored, const void* vals, const void* scales, const void* w,
                       int32_t w_dtype, const float* mean, const float* rstd, int64_t M, int64_t H, const hyc_desc* d,
                       void* dx, float* dw_partials, void* dw, void* stream);
+
+/* db[c] = sum over the rows of dy bf16 [M, H], accumulated in fp32, in bf16 or fp32.  partials: fp32
+ * [hyc_bias_grad_partials(M, H), H] scratch.  H a multiple of 8, at most 65536; dy 16-byte aligned. */
+int64_t hyc_bias_grad_partials(int64_t M, int64_t H);
+int hyc_bias_grad(const void* dy, int64_t M, int64_t H, float* partials, void* db, int32_t db_dtype, void* stream);
 
 /* ---- activation backward ------------------------------------------------------------------- */
 /* dx = act'(xhat) * g evaluated op by op in bf16 as the reference expressions are. */

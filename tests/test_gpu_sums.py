@@ -1,0 +1,27 @@
+"""Sums over the tokens (kernels.bias_grad) against fp64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    import importlib
+    return importlib.import_module("hyc-lora_amd").kernels
+
+
+# one row; around a round of 32 rows and a block of 256 columns; a last chunk alone; several rounds per block; wide rows
+@pytest.mark.parametrize("M,H", [(0, 64), (1, 8), (31, 256), (33, 264), (257, 248), (3627, 1024), (9000, 4104), (40, 16384)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_bias_grad(K, M, H, dtype):
+    gen = torch.Generator().manual_seed(M + H)
+    dy = torch.randn(M, H, generator=gen).to(torch.bfloat16)
+    got = K.bias_grad(dy.cuda(), dtype).cpu()
+    assert got.dtype == dtype and got.shape == (H,)
+    want = dy.double().sum(0)
+    # every partial sum is at most sum |dy|; each of fewer than M / 8 + 300 additions in a chain rounds by 2^-24 of that
+    bound = dy.double().abs().sum(0) * (M / 8 + 300) * 2.0 ** -24
+    if dtype == torch.bfloat16:
+        bound = bound + want.abs() * 2.0 ** -8
+    assert bool(((got.double() - want).abs() <= bound).all())
