@@ -64,10 +64,13 @@ k_softmax_fwd(const uint16_t* __restrict__ x, int64_t rows, int64_t N, float thr
 // CAUSAL: row r belongs to query position r % period and sees columns 0..position only; the rest of the row is
 // neither read (x may hold anything there) nor exponentiated, and comes out as exact zeros.
 // FULL: the row is exactly 512 CPL entries, every lane owns CPL chunks and nothing is predicated on that.
-template <int CPL, bool CAUSAL, bool FULL>
+// SLAB: the row's first `cap` kept entries go to slab + row * cap in column order (one word each: column low, bf16 bits
+// high) while the row is in registers, so that the CSR arrays are filled from there and not from a second read of y: at
+// 65 536 x 2048 with 1 % kept this kernel 90 -> 104 us (the compaction's scans), the fill 49 -> 12.
+template <int CPL, bool CAUSAL, bool FULL, bool SLAB>
 __global__ void __launch_bounds__(256)
 k_softmax_fwd_wave(const uint16_t* x, int64_t rows, int64_t N, float thr, uint16_t* y,   // y may be x (in place)
-                   int32_t* __restrict__ counts, int64_t period) {
+                   int32_t* __restrict__ counts, int64_t period, uint32_t* __restrict__ slab, int cap) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int nch = (int)(N / 8);
@@ -137,21 +140,55 @@ k_softmax_fwd_wave(const uint16_t* x, int64_t rows, int64_t N, float thr, uint16
     l = wave_sum(l);
     const float inv = 1.0f / l;
     int kept = 0;
+    uint4 out[CPL];
+    uint32_t above[SLAB ? CPL : 1];                        // one bit per kept entry of the chunk
 #pragma unroll
     for (int u = 0; u < CPL; ++u) {
+      out[u] = make_uint4(0, 0, 0, 0);
+      uint32_t bits = 0;
       if (live[u]) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           v[u][j] = bfr(v[u][j] * inv);
-          kept += (v[u][j] > thr) ? 1 : 0;
+          if (SLAB) bits |= (v[u][j] > thr) ? 1u << j : 0u;
+          else kept += (on[u] && v[u][j] > thr) ? 1 : 0;    // (a lane past the row holds zeros: above a negative threshold)
         }
-        if (on[u]) store_stream(y + row * N + 8 * (lane + 64 * u), pack8(v[u]));
+        out[u] = pack8(v[u]);
       } else if (on[u]) {
-        kept += 0.f > thr ? 8 : 0;
-        store_stream(y + row * N + 8 * (lane + 64 * u), make_uint4(0, 0, 0, 0));
+        if (SLAB) bits = 0.f > thr ? 0xFFu : 0u;
+        else kept += 0.f > thr ? 8 : 0;
       }
+      if (on[u]) store_stream(y + row * N + 8 * (lane + 64 * u), out[u]);
+      if (SLAB) above[u] = on[u] ? bits : 0u;
     }
-    if (counts) {
+    if (SLAB) {
+      // where a chunk's entries start: two chunks' counts share a register through the scan (at most 512 in 16 bits each)
+      uint32_t* srow = slab + row * cap;
+      int first = 0;
+#pragma unroll
+      for (int u = 0; u < CPL; u += 2) {
+        const uint32_t hi = u + 1 < CPL ? above[(u + 1) % CPL] : 0u;
+        const int both = __popc(above[u]) | (__popc(hi) << 16);
+        const int incl = wave_inclusive_scan(both), all = __builtin_amdgcn_readlane(incl, 63);
+        const int excl = incl - both;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          if (u + t >= CPL) break;
+          const int uu = (u + t) % CPL;
+          int pos = first + (t ? excl >> 16 : excl & 0xFFFF);
+          // (nearly always one or two rounds: 1 % of 512 entries over 64 lanes)
+          for (uint32_t m = above[uu]; m; m &= m - 1, ++pos) {
+            const int j = __builtin_ctz(m);
+            const uint32_t lo2 = j & 2 ? out[uu].y : out[uu].x, hi2 = j & 2 ? out[uu].w : out[uu].z;
+            const uint32_t two = j & 4 ? hi2 : lo2, val = j & 1 ? two >> 16 : two & 0xFFFFu;
+            if (pos < cap) srow[pos] = (uint32_t)(8 * (lane + 64 * uu) + j) | (val << 16);
+          }
+          first += t ? all >> 16 : all & 0xFFFF;
+        }
+      }
+      if (lane == 0) counts[row] = first;
+    }
+    if (!SLAB && counts) {
       const float total = wave_sum((float)kept);
       if (lane == 0) counts[row] = (int32_t)total;
     }
@@ -238,6 +275,113 @@ k_csr_offsets(const int32_t* __restrict__ counts, int64_t rows, int64_t capacity
   if (tid == 0) {
     row_ptr[rows] = (int32_t)(carry < capacity ? carry : capacity);
     if (total) *total = carry;
+  }
+}
+
+// The same over several workgroups, 4096 rows each: a workgroup adds up the counts before its own by itself (they lie in
+// L2; at most 256 KB per 65 536 rows) instead of waiting for its neighbours.  The one-workgroup form walks its rounds one
+// after the other: 65 536 rows 15.1 -> 5.4 us, 32 768 rows 8.7 -> 4.9.  What all workgroups read together grows by
+// the square of the rows, so it stays below OFFS_MULTI_MAX of them (where the last one reads 1 MB).
+constexpr int64_t OFFS_MULTI_MAX = 262144;
+template <bool VEC>
+__global__ void __launch_bounds__(OFFS_THREADS)
+k_csr_offsets_multi(const int32_t* __restrict__ counts, int64_t rows, int64_t capacity, int32_t* __restrict__ row_ptr,
+                    int64_t* __restrict__ total) {
+  __shared__ long long before_w[OFFS_THREADS / 64];
+  __shared__ int tot[OFFS_THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t i = (int64_t)blockIdx.x * OFFS_TILE + 4 * tid;
+  int c[4];
+  if (VEC && i + 3 < rows) {
+    const int4 v = *reinterpret_cast<const int4*>(counts + i);
+    c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e] = i + e < rows ? counts[i + e] : 0;
+  }
+  long long part = 0;                                       // the counts before this workgroup's: whole tiles of 4096
+  const int tiles = blockIdx.x;
+  for (int t0 = 0; t0 < tiles; t0 += OFFS_SUB) {
+    int4 w[OFFS_SUB];
+#pragma unroll
+    for (int t = 0; t < OFFS_SUB; ++t) {
+      const int32_t* at = counts + (int64_t)(t0 + t) * OFFS_TILE + 4 * tid;
+      w[t] = make_int4(0, 0, 0, 0);
+      if (t0 + t < tiles) w[t] = VEC ? *reinterpret_cast<const int4*>(at) : make_int4(at[0], at[1], at[2], at[3]);
+    }
+#pragma unroll
+    for (int t = 0; t < OFFS_SUB; ++t) part += (w[t].x + w[t].y) + (w[t].z + w[t].w);
+  }
+#pragma unroll
+  for (int d = 32; d; d >>= 1) part += __shfl_xor(part, d, 64);
+  const int sum = (c[0] + c[1]) + (c[2] + c[3]), incl = wave_inclusive_scan(sum);
+  if (lane == 0) before_w[wave] = part;
+  if (lane == 63) tot[wave] = incl;
+  __syncthreads();
+  long long at = 0, end = 0;
+#pragma unroll
+  for (int w = 0; w < OFFS_THREADS / 64; ++w) { end += before_w[w] + tot[w]; at += before_w[w] + (w < wave ? tot[w] : 0); }
+  at += incl - sum;
+  int o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { o[e] = (int32_t)(at < capacity ? at : capacity); at += c[e]; }
+  if (VEC && i + 3 < rows) {
+    *reinterpret_cast<int4*>(row_ptr + i) = make_int4(o[0], o[1], o[2], o[3]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) if (i + e < rows) row_ptr[i + e] = o[e];
+  }
+  if (tid == 0 && blockIdx.x == gridDim.x - 1) {
+    row_ptr[rows] = (int32_t)(end < capacity ? end : capacity);
+    if (total) *total = end;
+  }
+}
+
+// The kept entries from the forward's slab, one wave per row: a copy of a few words.  A row that kept more than the slab
+// holds is read again, as k_softmax_fill does.
+__global__ void __launch_bounds__(256)
+k_softmax_fill_slab(const uint16_t* __restrict__ y, int64_t rows, int64_t N, float thr, const int32_t* __restrict__ counts,
+                    const uint32_t* __restrict__ slab, int cap, const int32_t* __restrict__ row_ptr, int32_t* __restrict__ cols,
+                    uint16_t* __restrict__ vals) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int n = counts[row];
+  const int64_t base = row_ptr[row];
+  const int limit = row_ptr[row + 1] - (int)base;           // the row's room in cols / vals
+  if (n <= cap) {
+    const int m = n < limit ? n : limit;
+    for (int e = lane; e < m; e += 64) {
+      const uint32_t w = slab[row * cap + e];
+      cols[base + e] = (int32_t)(w & 0xFFFFu);
+      vals[base + e] = (uint16_t)(w >> 16);
+    }
+    return;
+  }
+  const uint16_t* yr = y + row * N;
+  int running = 0;
+  for (int64_t c0 = 0; c0 < N / 8; c0 += 64) {
+    const int64_t c = c0 + lane;
+    uint4 raw = make_uint4(0, 0, 0, 0);
+    uint32_t m = 0;
+    if (c < N / 8) {
+      raw = *reinterpret_cast<const uint4*>(yr + 8 * c);
+      float v[8];
+      unpack8(raw, v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) m |= (v[j] > thr) ? (1u << j) : 0u;
+    }
+    const int cnt = __popc(m), incl = wave_inclusive_scan(cnt);
+    int pos = running + incl - cnt;
+    for (; m; m &= m - 1, ++pos) {
+      const int j = __builtin_ctz(m);
+      const uint32_t lo2 = j & 2 ? raw.y : raw.x, hi2 = j & 2 ? raw.w : raw.z, two = j & 4 ? hi2 : lo2;
+      if (pos < limit) {
+        cols[base + pos] = (int32_t)(8 * c + j);
+        vals[base + pos] = (uint16_t)(j & 1 ? two >> 16 : two & 0xFFFFu);
+      }
+    }
+    running += __builtin_amdgcn_readlane(incl, 63);
   }
 }
 
@@ -395,8 +539,8 @@ int hyc_softmax_fwd(const void* x, int64_t rows, int64_t N, float threshold, voi
     const int64_t blocks = (rows + 3) / 4, cap = blocks;
     const dim3 grid((unsigned)(blocks < cap ? blocks : cap));
 #define HYC_SMW_F(C_, F_)                                                                                          \
-  hipLaunchKernelGGL((k_softmax_fwd_wave<C_, false, F_>), grid, dim3(256), 0, st, static_cast<const uint16_t*>(x), rows, N, \
-                     thr, static_cast<uint16_t*>(y), counts, (int64_t)1)
+  hipLaunchKernelGGL((k_softmax_fwd_wave<C_, false, F_, false>), grid, dim3(256), 0, st, static_cast<const uint16_t*>(x), rows, N, \
+                     thr, static_cast<uint16_t*>(y), counts, (int64_t)1, static_cast<uint32_t*>(nullptr), 0)
 #define HYC_SMW(C_) do { if ((C_) > 1 && N == 512 * (C_)) HYC_SMW_F(C_, true); else HYC_SMW_F(C_, false); } while (0)
     if (cpl <= 1) HYC_SMW(1); else if (cpl <= 2) HYC_SMW(2); else if (cpl <= 4) HYC_SMW(4); else HYC_SMW(8);
 #undef HYC_SMW
@@ -429,8 +573,8 @@ int hyc_softmax_causal_fwd(const void* x, int64_t rows, int64_t N, int64_t perio
   const int64_t blocks = (rows + 3) / 4, cap = blocks;        // one row per wave, see hyc_softmax_fwd
   const dim3 grid((unsigned)(blocks < cap ? blocks : cap));
 #define HYC_SMC_F(C_, F_)                                                                                         \
-  hipLaunchKernelGGL((k_softmax_fwd_wave<C_, true, F_>), grid, dim3(256), 0, st, static_cast<const uint16_t*>(x), rows, N, \
-                     thr, static_cast<uint16_t*>(y), counts, period)
+  hipLaunchKernelGGL((k_softmax_fwd_wave<C_, true, F_, false>), grid, dim3(256), 0, st, static_cast<const uint16_t*>(x), rows, N, \
+                     thr, static_cast<uint16_t*>(y), counts, period, static_cast<uint32_t*>(nullptr), 0)
 #define HYC_SMC(C_) do { if ((C_) > 1 && N == 512 * (C_)) HYC_SMC_F(C_, true); else HYC_SMC_F(C_, false); } while (0)
   if (cpl <= 1) HYC_SMC(1); else if (cpl <= 2) HYC_SMC(2); else if (cpl <= 4) HYC_SMC(4); else HYC_SMC(8);
 #undef HYC_SMC
@@ -438,11 +582,61 @@ int hyc_softmax_causal_fwd(const void* x, int64_t rows, int64_t N, int64_t perio
   return check_launch("hyc_softmax_causal_fwd");
 }
 
+int hyc_softmax_fwd_slab(const void* x, int64_t rows, int64_t N, int64_t period, float threshold, void* y, int32_t* counts,
+                         uint32_t* slab, int64_t cap, void* stream) {
+  int rc = softmax_shape("hyc_softmax_fwd_slab", rows, N);
+  if (rc) return rc;
+  if (N > 4096) return fail(HYC_ENOTSUP, "hyc_softmax_fwd_slab: N=%lld (rows of at most 4096 entries)", (long long)N);
+  if (period < 0 || period > N)
+    return fail(HYC_EINVAL, "hyc_softmax_fwd_slab: period=%lld must be in 0..N=%lld", (long long)period, (long long)N);
+  if (cap <= 0 || cap > N) return fail(HYC_EINVAL, "hyc_softmax_fwd_slab: cap=%lld must be in 1..N=%lld", (long long)cap, (long long)N);
+  if (rows == 0) return HYC_OK;
+  if (!x || !y || !counts || !slab) return fail(HYC_EFAULT, "hyc_softmax_fwd_slab: null buffer");
+  if (!aligned16(x) || !aligned16(y)) return fail(HYC_EINVAL, "hyc_softmax_fwd_slab: x and y must be 16-byte aligned");
+  hipStream_t st = begin_launch(stream);
+  const float thr = round_to_bf16(threshold);
+  const int cpl = (int)((N / 8 + 63) / 64);
+  const dim3 grid((unsigned)((rows + 3) / 4));                 // one row per wave, see hyc_softmax_fwd
+#define HYC_SMS_F(C_, K_, F_)                                                                                     \
+  hipLaunchKernelGGL((k_softmax_fwd_wave<C_, K_, F_, true>), grid, dim3(256), 0, st, static_cast<const uint16_t*>(x), rows, N, \
+                     thr, static_cast<uint16_t*>(y), counts, period ? period : (int64_t)1, slab, (int)cap)
+#define HYC_SMS(C_)                                                                                               \
+  do {                                                                                                            \
+    const bool full_ = (C_) > 1 && N == 512 * (C_);                                                               \
+    if (period) { if (full_) HYC_SMS_F(C_, true, true); else HYC_SMS_F(C_, true, false); }                        \
+    else { if (full_) HYC_SMS_F(C_, false, true); else HYC_SMS_F(C_, false, false); }                             \
+  } while (0)
+  if (cpl <= 1) HYC_SMS(1); else if (cpl <= 2) HYC_SMS(2); else if (cpl <= 4) HYC_SMS(4); else HYC_SMS(8);
+#undef HYC_SMS
+#undef HYC_SMS_F
+  return check_launch("hyc_softmax_fwd_slab");
+}
+
+int hyc_softmax_fill_slab(const void* y, int64_t rows, int64_t N, float threshold, const int32_t* counts, const uint32_t* slab,
+                          int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals, void* stream) {
+  int rc = softmax_shape("hyc_softmax_fill_slab", rows, N);
+  if (rc) return rc;
+  if (cap <= 0 || cap > N) return fail(HYC_EINVAL, "hyc_softmax_fill_slab: cap=%lld must be in 1..N=%lld", (long long)cap, (long long)N);
+  if (rows == 0) return HYC_OK;
+  if (!y || !counts || !slab || !row_ptr) return fail(HYC_EFAULT, "hyc_softmax_fill_slab: null buffer");
+  if (!aligned16(y)) return fail(HYC_EINVAL, "hyc_softmax_fill_slab: y must be 16-byte aligned");
+  hipLaunchKernelGGL(k_softmax_fill_slab, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, begin_launch(stream),
+                     static_cast<const uint16_t*>(y), rows, N, round_to_bf16(threshold), counts, slab, (int)cap, row_ptr, cols,
+                     static_cast<uint16_t*>(vals));
+  return check_launch("hyc_softmax_fill_slab");
+}
+
 int hyc_csr_offsets(const int32_t* counts, int64_t rows, int64_t capacity, int32_t* row_ptr, int64_t* total, void* stream) {
   if (rows < 0) return fail(HYC_EINVAL, "hyc_csr_offsets: rows=%lld", (long long)rows);
   if (!row_ptr || (rows > 0 && !counts)) return fail(HYC_EFAULT, "hyc_csr_offsets: null buffer");
   if (capacity < 0 || capacity > 0x7FFFFFFFll) capacity = 0x7FFFFFFFll;          // row_ptr is int32
-  if (aligned16(counts) && aligned16(row_ptr))
+  if (rows > OFFS_TILE && rows <= OFFS_MULTI_MAX) {
+    const dim3 grid((unsigned)((rows + OFFS_TILE - 1) / OFFS_TILE));
+    if (aligned16(counts) && aligned16(row_ptr))
+      hipLaunchKernelGGL(k_csr_offsets_multi<true>, grid, dim3(OFFS_THREADS), 0, begin_launch(stream), counts, rows, capacity, row_ptr, total);
+    else
+      hipLaunchKernelGGL(k_csr_offsets_multi<false>, grid, dim3(OFFS_THREADS), 0, begin_launch(stream), counts, rows, capacity, row_ptr, total);
+  } else if (aligned16(counts) && aligned16(row_ptr))
     hipLaunchKernelGGL(k_csr_offsets<true>, dim3(1), dim3(OFFS_THREADS), 0, begin_launch(stream), counts, rows, capacity, row_ptr, total);
   else
     hipLaunchKernelGGL(k_csr_offsets<false>, dim3(1), dim3(OFFS_THREADS), 0, begin_launch(stream), counts, rows, capacity, row_ptr, total);

@@ -810,12 +810,26 @@ class SparseRows:
         return self.row_ptr.numel() - 1
 
 
-def _csr_from_counts(lib, y2d, threshold, counts, budget=None):
+def _slab_entries(budget, N):
+    """entries per row of the forward's slab of kept probabilities, or 0 to read y a second time instead.  A slab entry is
+    written and read (8 bytes) where the second read of y costs 2 N bytes a row: worth it while twice the share seen before
+    fits an eighth of the row (N / 2 bytes of traffic for the average row)."""
+    if budget is None or not budget.ready or N > 4096:
+        return 0
+    cap = max(32, (int(2 * budget.per_row) + 31) // 32 * 32)
+    return cap if cap <= max(32, N // 8) and cap <= N else 0
+
+
+def _csr_from_counts(lib, y2d, threshold, counts, budget=None, slab=None):
     rows, N = y2d.shape
     dev = y2d.device
     row_ptr, nnz, total = _csr_offsets(lib, counts, rows, budget)
     cols = torch.empty(nnz, dtype=torch.int32, device=dev)
     vals = torch.empty(nnz, dtype=BF16, device=dev)
+    if slab is not None and nnz:
+        check(lib.hyc_softmax_fill_slab(_p(y2d), rows, N, float(threshold), _p(counts), _p(slab), slab.shape[1], _p(row_ptr),
+                                        _p(cols), _p(vals), _stream()))
+        return row_ptr, cols, vals, total
     check(lib.hyc_softmax_fill(_p(y2d), rows, N, float(threshold), _p(row_ptr), _p(cols) if nnz else None,
                                _p(vals) if nnz else None, _stream()))
     return row_ptr, cols, vals, total
@@ -837,13 +851,17 @@ def softmax_fwd(x, threshold=None, causal_period=None, inplace=False, budget=Non
     y = x2 if inplace else torch.empty_like(x2)
     counts = None if threshold is None else torch.empty(rows, dtype=torch.int32, device=x.device)
     thr = 0.0 if threshold is None else float(threshold)
-    if causal_period is None:
+    slab, cap = None, 0 if threshold is None or rows == 0 else _slab_entries(budget, N)
+    if cap and (causal_period is None or 0 < int(causal_period) <= N):
+        slab = torch.empty((rows, cap), dtype=torch.int32, device=x.device)
+        check(lib.hyc_softmax_fwd_slab(_p(x2), rows, N, int(causal_period or 0), thr, _p(y), _p(counts), _p(slab), cap, _stream()))
+    elif causal_period is None:
         check(lib.hyc_softmax_fwd(_p(x2), rows, N, thr, _p(y), _p(counts), _stream()))
     else:
         check(lib.hyc_softmax_causal_fwd(_p(x2), rows, N, int(causal_period), thr, _p(y), _p(counts), _stream()))
     if threshold is None:
         return y.reshape(x.shape), None
-    row_ptr, cols, vals, total = _csr_from_counts(lib, y, threshold, counts, budget)
+    row_ptr, cols, vals, total = _csr_from_counts(lib, y, threshold, counts, budget, slab)
     return y.reshape(x.shape), SparseRows(row_ptr, cols, vals, tuple(x.shape), total)
 
 

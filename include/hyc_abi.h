@@ -276,6 +276,13 @@ int hyc_softmax_fwd(const void* x, int64_t rows, int64_t N, float threshold, voi
  * out as exact zeros.  1 <= period <= N <= 4096. */
 int hyc_softmax_causal_fwd(const void* x, int64_t rows, int64_t N, int64_t period, float threshold, void* y,
                            int32_t* counts, void* stream);
+/* The same (period 0: no mask; rows of at most 4096 entries) that also leaves the first `cap` kept entries of every row, in
+ * column order, in slab [rows, cap] (column in the low half of a word, bf16 bits in the high half; what lies behind a row's
+ * entries is not written), and hyc_softmax_fill from that slab: y is read only for rows that kept more than cap. */
+int hyc_softmax_fwd_slab(const void* x, int64_t rows, int64_t N, int64_t period, float threshold, void* y, int32_t* counts,
+                         uint32_t* slab, int64_t cap, void* stream);
+int hyc_softmax_fill_slab(const void* y, int64_t rows, int64_t N, float threshold, const int32_t* counts, const uint32_t* slab,
+                          int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals, void* stream);
 /* Row offsets from per-row counts (of hyc_softmax_fwd, hyc_ref_outlier_count or the fused forwards), without the host:
  * row_ptr int32 [rows+1], row_ptr[r] = min(capacity, counts[0] + ... + counts[r-1]); *total (int64, may be NULL) = the
  * uncut sum.  capacity = the entries the caller's cols / vals buffers hold (negative: no limit).  With the offsets cut
