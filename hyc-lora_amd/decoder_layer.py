@@ -131,6 +131,15 @@ def _room_behind(rows, tensors, total, room):
     return rows
 
 
+def _kernel_rows(t):
+    """[..., H] -> the [M, H] rows the kernels read as they lie (16-byte aligned, evenly spaced by a multiple of 8 elements, none
+    on top of another), copied where they do not: a gradient broadcast over the tokens, an odd slice, a view at an odd offset"""
+    t = _row_view(t)
+    if t.data_ptr() % 16 or (t.shape[0] > 1 and (t.stride(0) < t.shape[1] or t.stride(0) % 8)):
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t
+
+
 class _LoRAProjectionsFunc(torch.autograd.Function):
     """A group is one library product each way: forward y = s h B^T (h = x A^T), onto which the base product accumulates in
     its epilogue; backward dX = [dY | s dY B] [W^T | A^T]^T with the rank-r terms as mod.room further columns of the
@@ -140,7 +149,7 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
     def forward(ctx, x, mod, plan, *ab):
         n = len(mod.out_features)
         A, B = ab[:n], ab[n:]
-        x2 = _row_view(x)
+        x2 = _kernel_rows(x)
         h = K.lora_down(x2, A)
         y_all = K.lora_up(h, B, mod.scaling)
         _product(y_all, x2, K.nf4_dequantize(mod.base_all), accumulate=True)
@@ -163,7 +172,7 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
         A, B = ctx.saved_tensors[:n], ctx.saved_tensors[n:]
         r, total = A[0].shape[0], sum(mod.out_features)
         rows = _room_behind(getattr(gs[0], "_hyc_rows", None), gs, total, mod.room)
-        ext, dh, dB = K.lora_up_bwd([_row_view(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, mod.room, rows)
+        ext, dh, dB = K.lora_up_bwd([_kernel_rows(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, mod.room, rows)
         # dA_i = dh_i^T @ x_hat: the projections of a group read the same saved activation, so their dh go through
         # the weight-gradient kernel side by side (32 output rows per call, the widest its LoRA-shaped form takes)
         # and x_hat is decoded once per call instead of once per projection

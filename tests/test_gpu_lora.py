@@ -72,3 +72,29 @@ def test_gradients_side_by_side_are_recognised_only_when_they_are(hyc):
     assert DL._room_behind(buf, [a, b.clone()], 96, 64) is None
     assert DL._room_behind(buf, [a, b], 96, 128) is None
     assert DL._room_behind(buf[:, :160].float(), [a, b], 96, 64) is None
+
+
+def _group(hyc, outs=(128, 64), compress=False):
+    import importlib
+    DL = importlib.import_module(hyc.__name__ + ".decoder_layer")
+    return DL, DL.LoRAProjections(256, list(outs), DL.LayerConfig(hidden=256, lora_r=16, compress=compress), "cuda")
+
+
+def _gradients(mod, x, gs):
+    x = x.detach().requires_grad_(True)
+    return torch.autograd.grad(mod(x), [x] + list(mod.parameters()), gs)
+
+
+def test_rows_that_do_not_lie_as_the_kernels_read_them(K, hyc):
+    """gradients broadcast over the tokens, inputs and gradients at odd pitches and offsets: the results of their copies, bit for bit"""
+    DL, mod = _group(hyc)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    x, g = mk(1, 33, 256), [mk(1, 1, o).expand(1, 33, o) for o in (128, 64)]
+    pitch, offset = mk(1, 33, 259)[..., :256], mk(33 * 256 + 1)[1:].view(1, 33, 256)
+    cases = [(x, g), (x, [mk(1, 33, o + 3)[..., :o] for o in (128, 64)]), (x, [mk(33 * o + 1)[1:].view(1, 33, o) for o in (128, 64)]),
+             (pitch, [mk(1, 33, o) for o in (128, 64)]), (offset, [mk(1, 33, o) for o in (128, 64)])]
+    for xi, gi in cases:
+        got = _gradients(mod, xi, gi)
+        want = _gradients(mod, xi.clone(memory_format=torch.contiguous_format), [t.clone(memory_format=torch.contiguous_format) for t in gi])
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
