@@ -1004,7 +1004,7 @@ def lora_room(n, r):
 
 def _lora_kernels_cover(factors, K, outs, r):
     return (len(factors) <= 4 and r in (8, 16, 24, 32) and len(factors) * r <= 96 and K % 64 == 0 and all(o % 8 == 0 for o in outs)
-            and all(f.dtype == BF16 and f.is_contiguous() for f in factors))
+            and all(f.dtype == BF16 and f.is_contiguous() and f.data_ptr() % 16 == 0 for f in factors))
 
 
 def _ptrs(ts):

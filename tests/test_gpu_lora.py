@@ -98,3 +98,20 @@ def test_rows_that_do_not_lie_as_the_kernels_read_them(K, hyc):
         got = _gradients(mod, xi, gi)
         want = _gradients(mod, xi.clone(memory_format=torch.contiguous_format), [t.clone(memory_format=torch.contiguous_format) for t in gi])
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_factors_at_an_odd_address(K, hyc):
+    """factors that are views into a flat parameter buffer at an offset the kernels do not take go through the general products"""
+    DL, mod = _group(hyc)
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    x, gs = mk(2, 17, 256), [mk(2, 17, o) for o in (128, 64)]
+    want = _gradients(mod, x, gs)
+    for p in mod.parameters():
+        flat = torch.empty(p.numel() + 1, dtype=p.dtype, device="cuda")
+        flat[1:] = p.data.flatten()
+        p.data = flat[1:].view(p.shape)
+    got = _gradients(mod, x, gs)
+    for a, b in zip(got, want):                            # products in another order: a rounding to bf16 of h, of dh and of the result
+        bound = 3 * 2.0 ** -8 * (b.float().abs() + b.float().abs().max())
+        assert ((a.float() - b.float()).abs() <= bound).all()
