@@ -1057,7 +1057,7 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
             _need_rows(g, "grad_output")
         lib = _abi.load()
         dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
-        dB = [torch.empty_like(b) for b in B]
+        dB = [torch.empty_like(b) if M else torch.zeros_like(b) for b in B]      # (no tokens: nothing is launched)
         outs_c = _i64s(outs)
         ws = torch.empty(lib.hyc_lora_up_bwd_workspace_bytes(M, outs_c, n, r) // 4, dtype=torch.float32, device=h.device)
         pitches = _i64s([g.stride(0) if M > 1 else o for g, o in zip(gs, outs)])

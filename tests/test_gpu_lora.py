@@ -115,3 +115,11 @@ def test_factors_at_an_odd_address(K, hyc):
     for a, b in zip(got, want):                            # products in another order: a rounding to bf16 of h, of dh and of the result
         bound = 3 * 2.0 ** -8 * (b.float().abs() + b.float().abs().max())
         assert ((a.float() - b.float()).abs() <= bound).all()
+
+
+def test_no_tokens(K):
+    B = [torch.ones(64, 16, dtype=torch.bfloat16, device="cuda")]
+    empty = lambda w: torch.empty(0, w, dtype=torch.bfloat16, device="cuda")
+    K.lora_up_bwd([torch.ones(8, 64, dtype=torch.bfloat16, device="cuda")], B, torch.ones(8, 16, dtype=torch.bfloat16, device="cuda"), 1.0, 64)
+    ext, dh, dB = K.lora_up_bwd([empty(64)], B, empty(16), 1.0, 64)
+    assert ext.shape == (0, 128) and dh.shape == (0, 16) and not dB[0].any()
