@@ -1052,12 +1052,12 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
     copy = ext is None
     if copy:
         ext = torch.empty((M, total + room), dtype=BF16, device=gs[0].device)
-    if _lora_kernels_cover(B, 64, outs, r):
+    if M and _lora_kernels_cover(B, 64, outs, r):
         for g in gs:
             _need_rows(g, "grad_output")
         lib = _abi.load()
         dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
-        dB = [torch.empty_like(b) if M else torch.zeros_like(b) for b in B]      # (no tokens: nothing is launched)
+        dB = [torch.empty_like(b) for b in B]
         outs_c = _i64s(outs)
         ws = torch.empty(lib.hyc_lora_up_bwd_workspace_bytes(M, outs_c, n, r) // 4, dtype=torch.float32, device=h.device)
         pitches = _i64s([g.stride(0) if M > 1 else o for g, o in zip(gs, outs)])
