@@ -433,11 +433,13 @@ static int lora_group(const char* who, const void* const* factors, const int64_t
   return HYC_OK;
 }
 
-// token ranges of k_lora_up_bwd: enough workgroups for two per CU, whole tiles each, at most 32 (the partial dB)
+// token ranges of k_lora_up_bwd: enough workgroups for two per CU, whole tiles each, at most 32 (the partial dB) unless that
+// leaves a range more than 32768 tokens (its offsets into dY are 31-bit numbers of bytes up to row pitches of 32760)
 static int lora_up_ranges(int64_t M, int fblocks) {
   int64_t want = (512 + fblocks - 1) / fblocks, most = (M + LU_M - 1) / LU_M;
   if (want > most) want = most;
   if (want > 32) want = 32;
+  if (want < (M + 32767) / 32768) want = (M + 32767) / 32768;
   return (int)(want < 1 ? 1 : want);
 }
 static int lora_up_blocks(const int64_t* n_out, int n) {

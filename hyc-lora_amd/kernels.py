@@ -1052,7 +1052,7 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
     copy = ext is None
     if copy:
         ext = torch.empty((M, total + room), dtype=BF16, device=gs[0].device)
-    if M and _lora_kernels_cover(B, 64, outs, r):
+    if M and min(M, 32768) * max(max(g.stride(0), o) for g, o in zip(gs, outs)) < 1 << 30 and _lora_kernels_cover(B, 64, outs, r):
         for g in gs:
             _need_rows(g, "grad_output")
         lib = _abi.load()

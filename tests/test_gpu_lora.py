@@ -123,3 +123,15 @@ def test_no_tokens(K):
     K.lora_up_bwd([torch.ones(8, 64, dtype=torch.bfloat16, device="cuda")], B, torch.ones(8, 16, dtype=torch.bfloat16, device="cuda"), 1.0, 64)
     ext, dh, dB = K.lora_up_bwd([empty(64)], B, empty(16), 1.0, 64)
     assert ext.shape == (0, 128) and dh.shape == (0, 16) and not dB[0].any()
+
+
+def test_more_tokens_than_a_range_takes_in_32(K):
+    """past 32 x 32768 tokens there are more ranges, each short enough for its offsets"""
+    M, r = (1 << 20) + 33, 8
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    g, h, B = mk(M, 8), mk(M, r), [mk(8, r)]
+    ext, dh, dB = K.lora_up_bwd([g], B, h, 0.5, 64)
+    close(dh, 0.5 * (g.float() @ B[0].float()))
+    close(dB[0], 0.5 * (g.double().t().contiguous() @ h.double()))
+    assert torch.equal(ext[:, :8], g) and torch.equal(ext[:, 8:16], dh) and not ext[:, 16:].any()
