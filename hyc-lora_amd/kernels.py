@@ -21,12 +21,13 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 def _stream():
     """handle of torch's current stream on the current device (the kernels are launched on it)"""
     if _raw_stream is not None:                    # no Stream object is built: 0.5 us instead of 5 per launch
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """device address for a pointer argument of the library (the prototypes turn the number into a pointer)"""
+    return None if t is None else t.data_ptr()
 
 
 def _need(t, dtype, name):
@@ -249,7 +250,7 @@ def _check_plan(plan, device=None):
                              "calibration state to the GPU (load_calibration_state does)" % name)
         if t.dtype != torch.int32 or not t.is_contiguous() or t.numel() != n:
             raise ValueError("%s must be a contiguous int32 tensor of %d elements" % (name, n))
-        if device is not None:
+        if device is not None and t.device != device:      # (a device without an index means the current one)
             want = torch.device(device)
             index = want.index if want.index is not None else torch.cuda.current_device()
             if t.device.type != want.type or t.device.index != index:
@@ -260,6 +261,11 @@ def _check_plan(plan, device=None):
 
 def channel_desc(plan: ChannelPlan, bits, group, device=None):
     _check_plan(plan, device)
+    return _checked_desc(plan, bits, group)
+
+
+def _checked_desc(plan, bits, group):
+    """channel_desc of a plan that _check_plan has just passed"""
     d = HycDesc()
     d.mode, d.bits, d.group, d.k = _abi.MODE_CHANNEL, bits, group, plan.k
     d.chan_plan = plan.plan.data_ptr()
@@ -318,7 +324,7 @@ def compress_channel(x2d, plan, bits, group):
     lib = _abi.load()
     check(lib.hyc_check_shape(H, bits, group, _abi.MODE_CHANNEL))
     out = alloc_channel(M, H, plan, bits, group, x2d.device)
-    d = out.desc()
+    d = _checked_desc(plan, bits, group)
     pitch = x2d.stride(0) if M > 1 else H
     check(lib.hyc_compress_rows(_p(x2d), pitch, M, H, ctypes.byref(d), _p(out.stored), _p(out.vals), _p(out.scales), None,
                                 _stream()))
@@ -463,7 +469,7 @@ def rmsnorm_fwd_compress_channel(x2d, w, eps, plan, bits, group):
     y = torch.empty_like(x2d)
     rstd = torch.empty(M, dtype=torch.float32, device=x2d.device)
     c = alloc_channel(M, H, plan, bits, group, x2d.device)
-    d = c.desc()
+    d = _checked_desc(plan, bits, group)
     check(lib.hyc_rmsnorm_fwd_compress(_p(x2d), _p(w), _wdtype(w), float(eps), M, H, ctypes.byref(d), _p(y), _p(rstd),
                                        _p(c.stored), _p(c.vals), _p(c.scales), None, _stream()))
     return y, rstd, c
@@ -520,7 +526,7 @@ def layernorm_fwd_compress_channel(x2d, w, bias, eps, plan, bits, group):
     mean = torch.empty(M, dtype=torch.float32, device=x2d.device)
     rstd = torch.empty(M, dtype=torch.float32, device=x2d.device)
     c = alloc_channel(M, H, plan, bits, group, x2d.device)
-    d = c.desc()
+    d = _checked_desc(plan, bits, group)
     check(lib.hyc_layernorm_fwd_compress(_p(x2d), _p(w), _p(bias), _wdtype(w), float(eps), M, H, ctypes.byref(d), _p(y),
                                          _p(mean), _p(rstd), _p(c.stored), _p(c.vals), _p(c.scales), None, _stream()))
     return y, mean, rstd, c
@@ -694,7 +700,7 @@ def act_fwd_compress(act, x2d, plan, bits, group):
     _need_rows(x2d, "x")
     M, H = x2d.shape
     c = alloc_channel(M, H, plan, bits, group, x2d.device)
-    d = c.desc()
+    d = _checked_desc(plan, bits, group)
     y = torch.empty((M, H), dtype=BF16, device=x2d.device)
     code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
     check(_abi.load().hyc_act_fwd_compress(code, _p(x2d), x2d.stride(0) if M > 1 else H, M, H, ctypes.byref(d), _p(y),
@@ -711,7 +717,7 @@ def hadamard_fwd_compress(a2d, b2d, plan_a, plan_b, bits, group):
     M, H = a2d.shape
     ca = alloc_channel(M, H, plan_a, bits, group, a2d.device)
     cb = alloc_channel(M, H, plan_b, bits, group, a2d.device)
-    da, db = ca.desc(), cb.desc()
+    da, db = _checked_desc(plan_a, bits, group), _checked_desc(plan_b, bits, group)
     y = torch.empty((M, H), dtype=BF16, device=a2d.device)
     check(_abi.load().hyc_hadamard_fwd_compress(_p(a2d), a2d.stride(0) if M > 1 else H, _p(b2d), b2d.stride(0) if M > 1 else H,
                                                 M, H, ctypes.byref(da), ctypes.byref(db), _p(y), _p(ca.stored), _p(ca.vals),
@@ -740,7 +746,7 @@ def gated_act_fwd(act, gate2d, up2d, plan_act, plan_up, plan_gate, bits, group):
     M, H = gate2d.shape
     dev = gate2d.device
     outs = [alloc_channel(M, H, p, bits, group, dev) for p in (plan_act, plan_up, plan_gate)]
-    descs = [o.desc() for o in outs]
+    descs = [_checked_desc(p, bits, group) for p in (plan_act, plan_up, plan_gate)]
     h = torch.empty((M, H), dtype=BF16, device=dev)
     code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
     flat = []

@@ -79,10 +79,8 @@ class EfficientMemoryHadamard(torch.nn.Module):
 
     def forward(self, x1, x2):
         if self.mode == "hyc":
-            a, _ = as_rows(x1)
-            b, _ = as_rows(x2)
-            p1 = self.site_1.channel_plan(a, self.iteration)
-            p2 = self.site_2.channel_plan(b, self.iteration)
+            p1 = self.site_1.channel_plan(x1, self.iteration)
+            p2 = self.site_2.channel_plan(x2, self.iteration)
             result = _ChannelHadamardFunc.apply(x1, x2, p1, p2, self.sub_outlier_bit_1, self.sub_outlier_bit_2, self.group_size)
             self.iteration += 1
             return result

@@ -112,8 +112,7 @@ class EfficientMemoryLayerNorm(torch.nn.LayerNorm):
 
     def forward(self, x):
         if self.mode == "hyc":
-            x2, _ = as_rows(x)
-            plan = self.site.channel_plan(x2, self.iteration)
+            plan = self.site.channel_plan(x, self.iteration)
             y = _ChannelLayerNormFunc.apply(x, self.weight, self.bias, self.eps, plan, self.sub_outlier_bit, self.group_size)
             self.iteration += 1
             return y

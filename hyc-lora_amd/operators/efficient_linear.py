@@ -91,8 +91,7 @@ class EfficientMemoryLinear(torch.nn.Linear):
 
     def forward(self, input: torch.Tensor):
         if self.mode == "hyc":
-            x2, _ = as_rows(input)
-            plan = self.site.channel_plan(x2, self.iteration)
+            plan = self.site.channel_plan(input, self.iteration)
             result = _ChannelLinearFunc.apply(input, self.weight, self.bias, plan, self.sub_outlier_bit, self.group_size)
             self.iteration += 1
             return result

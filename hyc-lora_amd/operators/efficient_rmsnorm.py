@@ -119,8 +119,7 @@ class EfficientMemoryRMSNorm(torch.nn.LayerNorm):
 
     def forward(self, x):
         if self.mode == "hyc":
-            x2, _ = as_rows(x)
-            plan = self.site.channel_plan(x2, self.iteration)
+            plan = self.site.channel_plan(x, self.iteration)
             y = _ChannelRMSNormFunc.apply(x, self.weight, self.eps, plan, self.sub_outlier_bit, self.group_size,
                                           self.ref_c2_quirk, self._func.weight_offset)
             self.iteration += 1

@@ -89,8 +89,7 @@ class _ActModule(torch.nn.Module):
 
     def forward(self, input):
         if self.mode == "hyc":
-            x2, _ = as_rows(input)
-            plan = self.site.channel_plan(x2, self.iteration)
+            plan = self.site.channel_plan(input, self.iteration)
             result = _ChannelActFunc.apply(input, self._act, plan, self.sub_outlier_bit, self.group_size)
             self.iteration += 1
             return result
