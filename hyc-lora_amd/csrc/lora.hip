@@ -119,57 +119,91 @@ k_lora_weight_t(const uint8_t* __restrict__ packed, const float* __restrict__ ab
   }
 }
 
-// h[m, i r + j] = sum_k x[m, k] A_i[j, k].  Eight waves share 16 tokens, each taking every eighth 32-channel step, so a row
-// is read in runs of 512 bytes; A stays in L2.  Bound by the read of x (4096 x 4096: 33.5 MB; stacking the A_i and the
-// library's thin GEMM took 5 + 14 us).
+// h[m, i r + j] = sum_k x[m, k] A_i[j, k].  Eight waves share 16 tokens, each taking every eighth block of 64 channels; A stays
+// in L2.  Should be bound by the read of x (4096 x 4096: 33.5 MB).  Loading the operands of the products straight from memory
+// puts neighbouring lanes into different rows, which the load path takes far longer for than for whole lines: 4 us per 16 columns
+// of h, however many tokens there are (and however many loads are under way).  So a wave loads 16 rows x 128 bytes as lines and turns them in 2 KB of LDS of
+// its own (no barrier: a wave's LDS operations are in order); the swizzle puts the 16 lanes of a read and of a write on all
+// banks.  4096 x 4096 with 16 / 32 / 48 columns 10.9 / 15.5 / 19.6 -> 8.4 / 12.2 / 14.8 us, 4096 x 11008 with 16 31.4 -> 26.0 (2048 tokens: 10.9 / 15.2 /
+// 19.4 / 27.6 -> 8.2 / 10.8 / 13.5 / 18.5).  Starting every workgroup at another block gave 5 % more at most, for sums that depend
+// on a token's place in the batch: not taken.
 template <int CT>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, 2)
 k_lora_down(const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int K, LoraGroup g, uint16_t* __restrict__ h) {
-  __shared__ __align__(16) float red[8][CT][256];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int TILE = 16 * 64;                          // 16 rows of 64 channels
+  __shared__ __align__(16) uint16_t lds[8][(1 + CT) * TILE];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, lq = lane >> 4;
   const int64_t m0 = (int64_t)blockIdx.x * 16;
-  const int kq = 8 * (lane >> 4), nr = g.n * g.r;
-  const int64_t m = m0 + (lane & 15) < M ? m0 + (lane & 15) : M - 1;
-  const uint16_t* xp = x + m * ldx + kq;
-  const uint16_t* ap[CT];
+  const int nr = g.n * g.r, lr = lane >> 3, lc = lane & 7;   // a load brings eight rows of eight chunks
+  const uint16_t *xp[2], *ap[CT][2];
 #pragma unroll
-  for (int c = 0; c < CT; ++c) {
-    const int f = 16 * c + (lane & 15), ff = f < nr ? f : 0, p = ff / g.r;
-    ap[c] = g.f[p] + (int64_t)(ff - p * g.r) * K + kq;
+  for (int u = 0; u < 2; ++u) {
+    const int64_t m = m0 + 8 * u + lr < M ? m0 + 8 * u + lr : M - 1;
+    xp[u] = x + m * ldx + 8 * lc;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int f = 16 * c + 8 * u + lr, ff = f < nr ? f : 0, p = ff / g.r;
+      ap[c][u] = g.f[p] + (int64_t)(ff - p * g.r) * K + 8 * lc;
+    }
   }
   floatx4_t acc[CT];
 #pragma unroll
   for (int c = 0; c < CT; ++c) acc[c] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-  constexpr int U = CT <= 3 ? 4 : 2;
-  const int steps = K / 32;
-  auto run = [&](int s, auto uno) __attribute__((always_inline)) {      // UU steps, all loads ahead of the products
+  constexpr int U = CT == 1 ? 8 : CT <= 3 ? 4 : 2;       // blocks whose loads are under way together (at most 128 registers)
+  const int blocks = K / 64;
+  uint16_t* T = lds[wave];
+  auto run = [&](int s, auto uno) __attribute__((always_inline)) {
     constexpr int UU = decltype(uno)::value;
-    bf16x8_t a[UU], b[UU][CT];
-#pragma unroll
-    for (int u = 0; u < UU; ++u) {
-      a[u] = *reinterpret_cast<const bf16x8_t*>(xp + 32 * (s + 8 * u));
-#pragma unroll
-      for (int c = 0; c < CT; ++c) b[u][c] = *reinterpret_cast<const bf16x8_t*>(ap[c] + 32 * (s + 8 * u));
-    }
+    bf16x8_t a[UU][2], b[UU][CT][2];
 #pragma unroll
     for (int u = 0; u < UU; ++u)
 #pragma unroll
-      for (int c = 0; c < CT; ++c) acc[c] = HYC_MFMA16(a[u], b[u][c], acc[c]);
+      for (int i = 0; i < 2; ++i) {
+        a[u][i] = *reinterpret_cast<const bf16x8_t*>(xp[i] + 64 * (s + 8 * u));
+#pragma unroll
+        for (int c = 0; c < CT; ++c) b[u][c][i] = *reinterpret_cast<const bf16x8_t*>(ap[c][i] + 64 * (s + 8 * u));
+      }
+    __builtin_amdgcn_sched_barrier(0);                   // (the scheduler would trade loads in flight for occupancy)
+#pragma unroll
+    for (int u = 0; u < UU; ++u) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = 8 * i + lr, at = row * 64 + 8 * (lc ^ ((row >> 1) & 7));
+        *reinterpret_cast<bf16x8_t*>(T + at) = a[u][i];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) *reinterpret_cast<bf16x8_t*>(T + (1 + c) * TILE + at) = b[u][c][i];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const int at = l15 * 64 + 8 * ((4 * ks + lq) ^ ((l15 >> 1) & 7));
+        const bf16x8_t av = *reinterpret_cast<const bf16x8_t*>(T + at);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[c] = HYC_MFMA16(av, *reinterpret_cast<const bf16x8_t*>(T + (1 + c) * TILE + at), acc[c]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
   };
   int s = wave;
-  for (; s + 8 * (U - 1) < steps; s += 8 * U) run(s, std::integral_constant<int, U>{});
-  for (; s < steps; s += 8) run(s, std::integral_constant<int, 1>{});
+  for (; s + 8 * (U - 1) < blocks; s += 8 * U) run(s, std::integral_constant<int, U>{});
+  if constexpr (U > 4)
+    if (s + 8 * 3 < blocks) { run(s, std::integral_constant<int, 4>{}); s += 8 * 4; }
+  if constexpr (U > 2)
+    if (s + 8 < blocks) { run(s, std::integral_constant<int, 2>{}); s += 8 * 2; }
+  if (s < blocks) run(s, std::integral_constant<int, 1>{});
+  // the waves' sums meet in the same memory: a wave's CT * 256 floats fit its own tiles
+  float* red = reinterpret_cast<float*>(T);
 #pragma unroll
   for (int c = 0; c < CT; ++c)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][c][(4 * (lane >> 4) + i) * 16 + (lane & 15)] = acc[c][i];
+    for (int i = 0; i < 4; ++i) red[c * 256 + (4 * lq + i) * 16 + l15] = acc[c][i];
   __syncthreads();
   for (int e = threadIdx.x; e < 16 * nr; e += 512) {
     const int t = e / nr, f = e - t * nr;
     if (m0 + t >= M) break;
     float sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < 8; ++w) sum += red[w][f >> 4][t * 16 + (f & 15)];
+    for (int w = 0; w < 8; ++w) sum += reinterpret_cast<const float*>(lds[w])[(f >> 4) * 256 + t * 16 + (f & 15)];
     h[(m0 + t) * nr + f] = f_to_bf(sum);
   }
 }
