@@ -49,7 +49,7 @@ class LayerConfig:
     scale_rule: str = "absmax"       # how a (token, group) scale is formed, see kernels.ChannelPlan
     compress: bool = True            # False: the same functions keep their activations in bf16 (formula check)
     attention: str = "eager"         # "eager": scores, softmax, p @ v with the kept probabilities (the path the
-                                     # reference wires into its models); "flash": the library's fused attention with
+                                     # reference wires into its models); "flash": fused attention kernels with
                                      # q, k, v and the output saved as codes (operators/efficient_flashattention.py)
     attn_group_bytes: int = 128 << 20  # attention is walked in groups of [S, S] score matrices of at most this size
 
@@ -330,8 +330,8 @@ class _AttentionFunc(torch.autograd.Function):
 
 class _FlashAttentionFunc(torch.autograd.Function):
     """The design of the reference's flash-attention operator (operators/efficient_flashattention.py:10-135): a fused
-    attention kernel (hyc_attn_fwd; the library's for head sizes other than 64 and 128) runs the forward, what is kept is q, k (after RoPE), v and the attention
-    output as codes plus the fp32 log-sum-exp of every row, and the fused backward runs on the restored
+    attention kernel (hyc_attn_fwd; the library's for head sizes other than 64 and 128) runs the forward, what is kept is
+    q, k (after RoPE), v and the attention output as codes plus the fp32 log-sum-exp of every row, and the fused backward runs on the restored
     tensors.  No [S, S] matrix exists at any time.  The backward kernel rebuilds the probabilities from the restored
     q and k with the exact log-sum-exp, and takes its row term sum(dO * O) from the restored output."""
 
