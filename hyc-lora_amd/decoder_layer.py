@@ -151,7 +151,7 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
         A, B = ab[:n], ab[n:]
         x2 = _kernel_rows(x)
         h = K.lora_down(x2, A)
-        y_all = K.lora_up(h, B, mod.scaling)
+        y_all = K.lora_up(h, B, mod.scaling, mod.out_features)
         _product(y_all, x2, K.nf4_dequantize(mod.base_all), accumulate=True)
         outs, row = [], 0
         for out in mod.out_features:                            # column slices: no copies, consumers take the pitch

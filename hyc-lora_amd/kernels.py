@@ -1008,9 +1008,22 @@ def lora_room(n, r):
     return -(-n * r // 64) * 64
 
 
-def _lora_kernels_cover(factors, K, outs, r):
-    return (len(factors) <= 4 and r in (8, 16, 24, 32) and len(factors) * r <= 96 and K % 64 == 0 and all(o % 8 == 0 for o in outs)
-            and all(f.dtype == BF16 and f.is_contiguous() and f.data_ptr() % 16 == 0 for f in factors))
+def _lora_factors(factors, shapes, device, name):
+    """every factor of a group is a bf16 matrix of its shape on `device` (the kernels index them by those shapes alone), else
+    ValueError; True if all of them also lie as the kernels read them: contiguous, at multiples of 16 bytes"""
+    if len(factors) != len(shapes):
+        raise ValueError("%d factors %s for %d projections" % (len(factors), name, len(shapes)))
+    as_read = True
+    for f, shape in zip(factors, shapes):
+        if not isinstance(f, torch.Tensor) or f.device != device or f.dtype != BF16 or f.shape != shape:
+            what = "%s %s on %s" % (f.dtype, tuple(f.shape), f.device) if isinstance(f, torch.Tensor) else type(f).__name__
+            raise ValueError("%s must be bfloat16 %s on %s, got %s" % (name, tuple(shape), device, what))
+        as_read = as_read and f.is_contiguous() and f.data_ptr() % 16 == 0
+    return as_read
+
+
+def _lora_kernels_cover(n, r, K, outs):
+    return n <= 4 and r in (8, 16, 24, 32) and n * r <= 96 and K % 64 == 0 and all(o % 8 == 0 for o in outs)
 
 
 def _ptrs(ts):
@@ -1026,20 +1039,31 @@ def lora_down(x2d, A):
     _need_rows(x2d, "x")
     M, Kf = x2d.shape
     n, r = len(A), A[0].shape[0]
-    if not _lora_kernels_cover(A, Kf, [8], r):
+    as_read = _lora_factors(A, [(r, Kf)] * n, x2d.device, "A")
+    if not as_read or not _lora_kernels_cover(n, r, Kf, ()):
         return x2d @ torch.cat(list(A), dim=0).t()
     h = torch.empty((M, n * r), dtype=BF16, device=x2d.device)
     check(_abi.load().hyc_lora_down(_p(x2d), x2d.stride(0) if M > 1 else Kf, M, Kf, _ptrs(A), n, r, _p(h), _stream()))
     return h
 
 
-def lora_up(h, B, scale):
-    """y [M, sum(out_i)] = scale * h_i B_i^T side by side"""
-    M, n, r = h.shape[0], len(B), B[0].shape[1]
-    outs = [b.shape[0] for b in B]
+def _need_h(h, M, width):
+    _need(h, BF16, "h")
+    if h.shape != (M, width):
+        raise ValueError("h must be [%d, %d], got %s" % (M, width, tuple(h.shape)))
+    return h
+
+
+def lora_up(h, B, scale, outs=None):
+    """y [M, sum(out_i)] = scale * h_i B_i^T side by side.  outs: the widths out_i the factors must have (None: as they come)"""
+    n, r = len(B), B[0].shape[-1]
+    outs = [b.shape[0] for b in B] if outs is None else list(outs)
+    M = h.shape[0]
+    _need_h(h, M, n * r)
+    as_read = _lora_factors(B, [(o, r) for o in outs], h.device, "B")
     y = torch.empty((M, sum(outs)), dtype=BF16, device=h.device)
-    if _lora_kernels_cover(B, 64, outs, r):
-        check(_abi.load().hyc_lora_up(_p(_need(h, BF16, "h")), M, _ptrs(B), _i64s(outs), n, r, float(scale), _p(y), _stream()))
+    if as_read and _lora_kernels_cover(n, r, 64, outs):
+        check(_abi.load().hyc_lora_up(_p(h), M, _ptrs(B), _i64s(outs), n, r, float(scale), _p(y), _stream()))
         return y
     zero, col = h.new_zeros(1), 0
     for i, (b, o) in enumerate(zip(B, outs)):
@@ -1052,15 +1076,26 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
     """(ext, dh, [dB_i]) from the gradients gs[i] [M, out_i] of a group: dB_i = scale * gs[i]^T h_i, dh = scale * gs[i] B_i
     side by side [M, n r] and, with zeros behind them, as the columns [sum(outs), + room) of ext.  ext: the buffer the gs
     already are the first columns of, side by side; None: they are copied into a new one."""
-    M, n, r = gs[0].shape[0], len(gs), B[0].shape[1]
+    M, n, r = gs[0].shape[0], len(gs), B[0].shape[-1]
+    for g in gs:
+        _need_rows(g, "grad_output")
+        if g.shape[0] != M or g.device != h.device:
+            raise ValueError("the gradients of a group must have the same rows, on the device of h")
     outs = [g.shape[1] for g in gs]
     total = sum(outs)
+    as_read = _lora_factors(B, [(o, r) for o in outs], h.device, "B")
+    _need_h(h, M, n * r)
+    if room < n * r:
+        raise ValueError("room for %d columns, the group has %d" % (room, n * r))
     copy = ext is None
     if copy:
-        ext = torch.empty((M, total + room), dtype=BF16, device=gs[0].device)
-    if M and min(M, 32768) * max(max(g.stride(0), o) for g, o in zip(gs, outs)) < 1 << 30 and _lora_kernels_cover(B, 64, outs, r):
-        for g in gs:
-            _need_rows(g, "grad_output")
+        ext = torch.empty((M, total + room), dtype=BF16, device=h.device)
+    else:
+        _need(ext, BF16, "ext")
+        if ext.shape != (M, total + room) or ext.device != h.device:
+            raise ValueError("ext must be [%d, %d] on %s, got %s on %s" % (M, total + room, h.device, tuple(ext.shape), ext.device))
+    if M and as_read and _lora_kernels_cover(n, r, 64, outs) and \
+            min(M, 32768) * max(max(g.stride(0), o) for g, o in zip(gs, outs)) < 1 << 30:
         lib = _abi.load()
         dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
         dB = [torch.empty_like(b) for b in B]
@@ -1087,8 +1122,15 @@ def lora_weight_t(q: NF4Weight, A, outs, room):
     """[K, sum(outs) + room] = [W^T | A_i^T side by side | zeros]: the transposed weight of the group's input gradient"""
     total, Kf = q.shape
     n, r = len(A), A[0].shape[0]
+    if sum(outs) != total or len(outs) != n:
+        raise ValueError("%d projections of %s features in a weight of %s with %d factors" % (len(outs), list(outs), tuple(q.shape), n))
+    _need_vec(q.packed, torch.uint8, total * Kf // 2, "packed")
+    _need_vec(q.absmax, torch.float32, total * Kf // 64, "absmax")
+    as_read = _lora_factors(A, [(r, Kf)] * n, q.packed.device, "A")
+    if room < n * r:
+        raise ValueError("room for %d columns, the group has %d" % (room, n * r))
     out = torch.empty((Kf, total + room), dtype=BF16, device=q.packed.device)
-    if _lora_kernels_cover(A, Kf, outs, r):
+    if as_read and _lora_kernels_cover(n, r, Kf, outs):
         check(_abi.load().hyc_lora_weight_t(_p(q.packed), _p(q.absmax), Kf, _ptrs(A), _i64s(outs), n, r, room, _p(out), _stream()))
         return out
     out[:, :total], out[:, total:] = nf4_dequantize(q).t(), 0

@@ -135,3 +135,56 @@ def test_more_tokens_than_a_range_takes_in_32(K):
     close(dh, 0.5 * (g.float() @ B[0].float()))
     close(dB[0], 0.5 * (g.double().t().contiguous() @ h.double()))
     assert torch.equal(ext[:, :8], g) and torch.equal(ext[:, 8:16], dh) and not ext[:, 16:].any()
+
+
+def test_factors_that_do_not_fit_are_refused(K, hyc):
+    """a factor of another shape, type or device raises before anything is launched, in every function that hands its address on"""
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    M, Kf, outs, r = 20, 128, [128, 64], 16
+    x, A, B, h, gs = mk(M, Kf), [mk(r, Kf) for _ in outs], [mk(o, r) for o in outs], mk(M, 2 * r), [mk(M, o) for o in outs]
+    q = K.nf4_quantize(mk(sum(outs), Kf))
+    for bad in ([A[0], A[1].cpu()], [A[0], mk(8, Kf)], [A[0], mk(r, 64)], [A[0], A[1].float()], [A[0], A[1].flatten()]):
+        with pytest.raises(ValueError):
+            K.lora_down(x, bad)
+        with pytest.raises(ValueError):
+            K.lora_weight_t(q, bad, outs, 64)
+    for bad in ([B[0], B[1].cpu()], [B[0], mk(64, 8)], [B[0], B[1].float()], [B[1], B[0]], [B[0]], [B[0], mk(72, r)]):
+        with pytest.raises(ValueError):
+            K.lora_up(h, bad, 1.0, outs)
+        with pytest.raises(ValueError):
+            K.lora_up_bwd(gs, bad, h, 1.0, 64)
+    for bad in (h[:, :r], h[:-1], h.float(), h.cpu(), mk(M, 3 * r)):
+        with pytest.raises(ValueError):
+            K.lora_up(bad, B, 1.0, outs) if bad.shape[0] == M else K.lora_up_bwd(gs, B, bad, 1.0, 64)
+        with pytest.raises(ValueError):
+            K.lora_up_bwd(gs, B, bad, 1.0, 64)
+    for ext in (mk(M, 192), mk(M, 256).float(), mk(M - 1, 256), mk(M, 257)[:, :256], mk(M, 256).cpu()):
+        with pytest.raises(ValueError):
+            K.lora_up_bwd(gs, B, h, 1.0, 64, ext)
+    for args in (([gs[0], gs[1][:-1]], B, h, 1.0, 64), ([gs[0], gs[1].cpu()], B, h, 1.0, 64), (gs, B, h, 1.0, 24)):
+        with pytest.raises(ValueError):
+            K.lora_up_bwd(*args)
+    for args in ((q, A, outs[::-1] + [8], 64), (q, A, [128, 128], 64), (q, A, outs, 24),
+                 (K.NF4Weight(q.packed[:-32], q.absmax, q.shape), A, outs, 64), (K.NF4Weight(q.packed, q.absmax.cpu(), q.shape), A, outs, 64)):
+        with pytest.raises(ValueError):
+            K.lora_weight_t(*args)
+
+
+def test_a_group_whose_factors_do_not_fit_is_refused(K, hyc):
+    """adapters on the host, of two ranks, or in the wrong order: the call raises as the products used to"""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(2, 17, 256, generator=gen, device="cuda").bfloat16()
+    for change in (lambda m: m.lora_A.cpu(), lambda m: m.lora_B.cpu(),
+                   lambda m: setattr(m.lora_A[1], "data", m.lora_A[1].data[:8].clone()),
+                   lambda m: [setattr(p, "data", d) for p, d in zip(m.lora_B, [m.lora_B[1].data, m.lora_B[0].data])]):
+        DL, mod = _group(hyc)
+        change(mod)
+        with pytest.raises(ValueError):
+            mod(x)
+    DL, mod = _group(hyc)                                  # between forward and backward
+    ys = mod(x.requires_grad_(True))
+    for p, d in zip(mod.lora_B, [mod.lora_B[1].data, mod.lora_B[0].data]):
+        p.data = d
+    with pytest.raises((ValueError, RuntimeError)):
+        torch.autograd.grad(ys, [x], [torch.ones_like(y) for y in ys])

@@ -1,0 +1,29 @@
+"""What the LoRA functions check about a group's factors before an address leaves Python (no GPU needed)."""
+import importlib
+
+import pytest
+import torch
+
+K = importlib.import_module("hyc-lora_amd").kernels
+CPU = torch.device("cpu")
+
+
+def factors(*shapes, dtype=torch.bfloat16):
+    return [torch.zeros(s, dtype=dtype) for s in shapes]
+
+
+def test_factors_must_have_their_shape_type_and_device():
+    shapes = [(16, 128), (16, 128)]
+    assert K._lora_factors(factors(*shapes), shapes, CPU, "A") is True
+    for bad in (factors((16, 128), (8, 128)), factors((16, 128), (16, 64)), factors((16, 128)), factors((16, 128), (2048,)),
+                factors(*shapes, dtype=torch.float32), [torch.zeros(16, 128, dtype=torch.bfloat16), None],
+                [torch.zeros(16, 128, dtype=torch.bfloat16), torch.zeros(16, 128, dtype=torch.bfloat16, device="meta")]):
+        with pytest.raises(ValueError):
+            K._lora_factors(bad, shapes, CPU, "A")
+    with pytest.raises(ValueError):                        # the second factor of a swapped pair
+        K._lora_factors(factors((64, 16), (128, 16)), [(128, 16), (64, 16)], CPU, "B")
+
+
+def test_factors_the_kernels_cannot_read_as_they_lie_go_elsewhere():
+    assert K._lora_factors([torch.zeros(128, 16, dtype=torch.bfloat16).t()], [(16, 128)], CPU, "A") is False
+    assert K._lora_factors([torch.zeros(16 * 128 + 1, dtype=torch.bfloat16)[1:].view(16, 128)], [(16, 128)], CPU, "A") is False
