@@ -1026,6 +1026,12 @@ def _lora_kernels_cover(n, r, K, outs):
     return n <= 4 and r in (8, 16, 24, 32) and n * r <= 96 and K % 64 == 0 and all(o % 8 == 0 for o in outs)
 
 
+def _lora_range_fits(M, pitch):
+    """a token range of hyc_lora_up_bwd (whole tiles of 64 tokens, at most 32768) stays below 2 GiB of rows `pitch` apart, however
+    many ranges there are"""
+    return (min(M, 32768) + 63) // 64 * 64 * pitch < 1 << 30
+
+
 def _ptrs(ts):
     return (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
 
@@ -1094,8 +1100,7 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
         _need(ext, BF16, "ext")
         if ext.shape != (M, total + room) or ext.device != h.device:
             raise ValueError("ext must be [%d, %d] on %s, got %s on %s" % (M, total + room, h.device, tuple(ext.shape), ext.device))
-    if M and as_read and _lora_kernels_cover(n, r, 64, outs) and \
-            min(M, 32768) * max(max(g.stride(0), o) for g, o in zip(gs, outs)) < 1 << 30:
+    if M and as_read and _lora_kernels_cover(n, r, 64, outs) and _lora_range_fits(M, max(max(g.stride(0), o) for g, o in zip(gs, outs))):
         lib = _abi.load()
         dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
         dB = [torch.empty_like(b) for b in B]

@@ -188,3 +188,15 @@ def test_a_group_whose_factors_do_not_fit_is_refused(K, hyc):
         p.data = d
     with pytest.raises((ValueError, RuntimeError)):
         torch.autograd.grad(ys, [x], [torch.ones_like(y) for y in ys])
+
+
+def test_a_range_that_only_its_last_tile_takes_past_2_gib(K):
+    """one range (as many feature blocks as the chip has places), whose length is rounded up to whole tiles: the general products"""
+    M, out, r = 7050, 151936, 8                            # 7050 * 151936 < 2^30 <= 7104 * 151936
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    g, h, B = mk(M, out), mk(M, r), [mk(out, r)]
+    ext, dh, dB = K.lora_up_bwd([g], B, h, 0.5, 64)
+    assert torch.equal(ext[:, :out], g) and torch.equal(ext[:, out:out + r], dh) and not ext[:, out + r:].any()
+    close(dh[:64], 0.5 * (g[:64].float() @ B[0].float()))
+    close(dB[0][:64], 0.5 * (g[:, :64].float().t().contiguous() @ h.float()))

@@ -27,3 +27,10 @@ def test_factors_must_have_their_shape_type_and_device():
 def test_factors_the_kernels_cannot_read_as_they_lie_go_elsewhere():
     assert K._lora_factors([torch.zeros(128, 16, dtype=torch.bfloat16).t()], [(16, 128)], CPU, "A") is False
     assert K._lora_factors([torch.zeros(16 * 128 + 1, dtype=torch.bfloat16)[1:].view(16, 128)], [(16, 128)], CPU, "A") is False
+
+
+def test_token_ranges_are_bounded_with_their_last_tile():
+    fits = K._lora_range_fits
+    for M, pitch in ((7041, 151936), (7050, 151936), (7067, 151936)):          # the last tile takes the range past 2^30 elements
+        assert M * pitch < 1 << 30 <= (M + 63) // 64 * 64 * pitch and not fits(M, pitch)
+    assert fits(7040, 151936) and fits(1 << 20, 32760) and not fits(1 << 20, 32768) and fits(1, 1 << 23) and not fits(1, 1 << 24)
