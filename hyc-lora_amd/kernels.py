@@ -1022,8 +1022,10 @@ def _lora_factors(factors, shapes, device, name):
     return as_read
 
 
-def _lora_kernels_cover(n, r, K, outs):
-    return n <= 4 and r in (8, 16, 24, 32) and n * r <= 96 and K % 64 == 0 and all(o % 8 == 0 for o in outs)
+def _lora_kernels_cover(M, n, r, K, outs):
+    """what the hyc_lora_* entries take: up to 4 factors of rank 8 to 32, and no more tokens and features than their launches count"""
+    return (n <= 4 and r in (8, 16, 24, 32) and n * r <= 96 and K % 64 == 0 and K <= 1 << 24 and M <= 65535 * 128
+            and sum(outs) <= 65535 * 128 - 4096 and all(o % 8 == 0 and o for o in outs))
 
 
 def _lora_range_fits(M, pitch):
@@ -1046,7 +1048,7 @@ def lora_down(x2d, A):
     M, Kf = x2d.shape
     n, r = len(A), A[0].shape[0]
     as_read = _lora_factors(A, [(r, Kf)] * n, x2d.device, "A")
-    if not as_read or not _lora_kernels_cover(n, r, Kf, ()):
+    if not as_read or not _lora_kernels_cover(M, n, r, Kf, ()):
         return x2d @ torch.cat(list(A), dim=0).t()
     h = torch.empty((M, n * r), dtype=BF16, device=x2d.device)
     check(_abi.load().hyc_lora_down(_p(x2d), x2d.stride(0) if M > 1 else Kf, M, Kf, _ptrs(A), n, r, _p(h), _stream()))
@@ -1068,7 +1070,7 @@ def lora_up(h, B, scale, outs=None):
     _need_h(h, M, n * r)
     as_read = _lora_factors(B, [(o, r) for o in outs], h.device, "B")
     y = torch.empty((M, sum(outs)), dtype=BF16, device=h.device)
-    if as_read and _lora_kernels_cover(n, r, 64, outs):
+    if as_read and _lora_kernels_cover(M, n, r, 64, outs):
         check(_abi.load().hyc_lora_up(_p(h), M, _ptrs(B), _i64s(outs), n, r, float(scale), _p(y), _stream()))
         return y
     zero, col = h.new_zeros(1), 0
@@ -1100,7 +1102,7 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
         _need(ext, BF16, "ext")
         if ext.shape != (M, total + room) or ext.device != h.device:
             raise ValueError("ext must be [%d, %d] on %s, got %s on %s" % (M, total + room, h.device, tuple(ext.shape), ext.device))
-    if M and as_read and _lora_kernels_cover(n, r, 64, outs) and _lora_range_fits(M, max(max(g.stride(0), o) for g, o in zip(gs, outs))):
+    if M and as_read and _lora_kernels_cover(M, n, r, 64, outs) and _lora_range_fits(M, max(max(g.stride(0), o) for g, o in zip(gs, outs))):
         lib = _abi.load()
         dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
         dB = [torch.empty_like(b) for b in B]
@@ -1135,7 +1137,7 @@ def lora_weight_t(q: NF4Weight, A, outs, room):
     if room < n * r:
         raise ValueError("room for %d columns, the group has %d" % (room, n * r))
     out = torch.empty((Kf, total + room), dtype=BF16, device=q.packed.device)
-    if as_read and _lora_kernels_cover(n, r, Kf, outs):
+    if as_read and _lora_kernels_cover(0, n, r, Kf, outs):
         check(_abi.load().hyc_lora_weight_t(_p(q.packed), _p(q.absmax), Kf, _ptrs(A), _i64s(outs), n, r, room, _p(out), _stream()))
         return out
     out[:, :total], out[:, total:] = nf4_dequantize(q).t(), 0

@@ -34,3 +34,11 @@ def test_token_ranges_are_bounded_with_their_last_tile():
     for M, pitch in ((7041, 151936), (7050, 151936), (7067, 151936)):          # the last tile takes the range past 2^30 elements
         assert M * pitch < 1 << 30 <= (M + 63) // 64 * 64 * pitch and not fits(M, pitch)
     assert fits(7040, 151936) and fits(1 << 20, 32760) and not fits(1 << 20, 32768) and fits(1, 1 << 23) and not fits(1, 1 << 24)
+
+
+def test_sizes_past_what_a_launch_counts_take_the_general_products():
+    cover = K._lora_kernels_cover
+    assert cover(4096, 3, 16, 4096, [4096] * 3) and cover(65535 * 128, 1, 8, 64, [8])
+    for args in ((65535 * 128 + 1, 1, 8, 64, [8]), (1, 1, 8, 64, [65535 * 128]), (1, 1, 8, (1 << 24) + 64, [8]), (1, 5, 8, 64, [8] * 5),
+                 (1, 1, 64, 64, [8]), (1, 1, 8, 32, [8]), (1, 1, 8, 64, [12]), (1, 2, 8, 64, [8, 0])):
+        assert not cover(*args)
