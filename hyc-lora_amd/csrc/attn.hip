@@ -534,9 +534,12 @@ k_attn_delta(AttnRows G, AttnRows O, const float* __restrict__ lse, float* __res
   }
 }
 
-static int attn_args(const char* who, int64_t B, int64_t S, int64_t heads, int64_t hd, const int64_t* pitches, int n) {
+static int attn_args(const char* who, int64_t B, int64_t S, int64_t heads, int64_t hd, float scale, const int64_t* pitches, int n) {
   if (B < 0 || S < 0 || heads <= 0) return fail(HYC_EINVAL, "%s: B=%lld S=%lld heads=%lld", who, (long long)B, (long long)S, (long long)heads);
   if (hd != 64 && hd != 128) return fail(HYC_ENOTSUP, "%s: head_dim=%lld (64 or 128)", who, (long long)hd);
+  // (the running maximum and the mask are taken before the scores are scaled, and the backward divides by the scale)
+  if (!(scale > 0.f) || !(1.0f / scale > 0.f) || !isfinite(1.0f / scale))
+    return fail(HYC_EINVAL, "%s: scale=%g must be positive, and so must its reciprocal, both finite", who, (double)scale);
   for (int i = 0; i < n; ++i) {
     if (pitches[i] < heads * hd || pitches[i] % 8 != 0)
       return fail(HYC_EINVAL, "%s: token pitch %lld (at least heads*head_dim, a multiple of 8)", who, (long long)pitches[i]);
@@ -557,7 +560,7 @@ extern "C" {
 int hyc_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, int64_t B, int64_t S,
                  int64_t heads, int64_t head_dim, float scale, void* out, int64_t ldo, float* lse, void* stream) {
   const int64_t pitches[4] = {ldq, ldk, ldv, ldo};
-  int rc = attn_args("hyc_attn_fwd", B, S, heads, head_dim, pitches, 4);
+  int rc = attn_args("hyc_attn_fwd", B, S, heads, head_dim, scale, pitches, 4);
   if (rc) return rc;
   if (B == 0 || S == 0) return HYC_OK;
   if (!q || !k || !v || !out || !lse) return fail(HYC_EFAULT, "hyc_attn_fwd: null buffer");
@@ -578,8 +581,7 @@ int hyc_attn_bwd(const void* dout, int64_t ldg, const void* q, int64_t ldq, cons
                  int64_t heads, int64_t head_dim, float scale, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv,
                  int64_t lddv, float* workspace, void* stream) {
   const int64_t pitches[8] = {ldg, ldq, ldk, ldv, lddq, lddk, lddv, ldo};
-  int rc = attn_args("hyc_attn_bwd", B, S, heads, head_dim, pitches, 8);
-  if (rc == HYC_OK && scale == 0.f) rc = fail(HYC_EINVAL, "hyc_attn_bwd: scale = 0");
+  int rc = attn_args("hyc_attn_bwd", B, S, heads, head_dim, scale, pitches, 8);
   if (rc) return rc;
   if (B == 0 || S == 0) return HYC_OK;
   if (!dout || !q || !k || !v || !out || !lse || !workspace || !dq || !dk || !dv || ((cosv == nullptr) != (sinv == nullptr)))

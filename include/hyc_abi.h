@@ -358,7 +358,8 @@ int hyc_lora_weight_t(const void* packed, const float* absmax, int64_t K, const 
 
 /* ---- fused causal attention ------------------------------------------------------------------ */
 /* On the rows layout [B, S, heads, head_dim] of the projections, every operand with its own token pitch (elements between
- * consecutive tokens, a multiple of 8; batch elements are S tokens apart); bf16, fp32 accumulation, head_dim 64 or 128.
+ * consecutive tokens, a multiple of 8; batch elements are S tokens apart); bf16, fp32 accumulation, head_dim 64 or 128,
+ * scale > 0 (finite, as its reciprocal).
  *   out = softmax(scale q k^T + causal mask) v,  lse fp32 [B, heads, S] = log of each row's sum of exponentials
  * hyc_attn_bwd: gradients at the given q, k, v and out, with probabilities exp(scale q.k - lse); with cos / sin (bf16
  * [S, head_dim]) dq and dk leave through the transposed rotation of hyc_rope_from_heads.  workspace: 2 * B * heads * S

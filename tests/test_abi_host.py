@@ -393,3 +393,16 @@ def test_header_is_plain_c_and_links_from_a_c_program(abi, tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
     assert "%d entry points" % len(names) in r.stdout
+
+
+def test_attention_takes_positive_scales_only(abi):
+    """both directions, before anything is launched (no tokens: a call that is accepted does nothing)"""
+    lib = abi.load()
+    fwd = lambda scale: lib.hyc_attn_fwd(None, 64, None, 64, None, 64, 0, 8, 1, 64, scale, None, 64, None, None)
+    bwd = lambda scale: lib.hyc_attn_bwd(None, 64, None, 64, None, 64, None, 64, None, 64, None, None, None, 0, 8, 1, 64, scale,
+                                         None, 64, None, 64, None, 64, None, None)
+    for call in (fwd, bwd):
+        assert call(0.125) == 0 and call(1e-30) == 0 and call(1e30) == 0
+        for scale in (0.0, -0.0, -0.125, float("inf"), float("-inf"), float("nan"), 1e-45):
+            assert call(scale) == abi.EINVAL, scale
+        assert b"scale" in lib.hyc_last_error()

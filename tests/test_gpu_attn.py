@@ -101,3 +101,9 @@ def test_attention_refuses_what_it_does_not_cover(K):
         K.attn_fwd(q, q, q, 2, 0.1)
     with pytest.raises(ValueError):
         K.attn_fwd(q, q[:, :4], q, 1, 0.1)
+    out, lse = K.attn_fwd(q, q, q, 1, 0.1)
+    for scale in (0.0, -0.1):
+        with pytest.raises(ValueError):
+            K.attn_fwd(q, q, q, 1, scale)
+        with pytest.raises(ValueError):
+            K.attn_bwd(q, q, q, q, out, lse, 1, scale)
