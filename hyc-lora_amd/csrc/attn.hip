@@ -547,7 +547,8 @@ static int attn_args(const char* who, int64_t B, int64_t S, int64_t heads, int64
       return fail(HYC_ENOTSUP, "%s: S * pitch = %lld elements (a batch element must stay below 2 GiB)", who, (long long)(S * pitches[i]));
   }
   const int64_t blocks = (S + AT_OWN - 1) / AT_OWN;
-  if (B * heads * blocks >= ((int64_t)1 << 31)) return fail(HYC_ENOTSUP, "%s: B * heads * S too large", who);
+  if (B * heads * blocks >= ((int64_t)1 << 24))          // (a launch counts its threads in 32 bits)
+    return fail(HYC_ENOTSUP, "%s: B * heads * S = %lld matrices of %lld blocks", who, (long long)(B * heads), (long long)blocks);
   return HYC_OK;
 }
 

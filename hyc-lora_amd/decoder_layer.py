@@ -341,7 +341,7 @@ class _FlashAttentionFunc(torch.autograd.Function):
         b, s, H = q.shape
         nh, hd = cfg.heads, cfg.head_dim
         scale = 1.0 / math.sqrt(hd)
-        ctx.rows = K.attn_supported(hd, s, max(v.stride(1), 3 * H + grad_room))        # (the pitch the gradients get)
+        ctx.rows = K.attn_supported(hd, s, max(v.stride(1), 3 * H + grad_room), b * nh)        # (the pitch the gradients get)
         seed = offset = None
         if ctx.rows:                                                # the kernels read and write the rows as they are
             q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)

@@ -1213,9 +1213,9 @@ def rope_from_heads(g, cos=None, sin=None):
 # ----------------------------------------------------------------------------------------------------
 # fused causal attention
 # ----------------------------------------------------------------------------------------------------
-def attn_supported(head_dim, S, widest_pitch):
-    """shapes hyc_attn_fwd / hyc_attn_bwd cover (the library's fused attention serves the others)"""
-    return head_dim in (64, 128) and S * widest_pitch < 1 << 30
+def attn_supported(head_dim, S, widest_pitch, matrices=1):
+    """shapes hyc_attn_fwd / hyc_attn_bwd cover (the library's fused attention serves the others); matrices: B * heads"""
+    return head_dim in (64, 128) and S * widest_pitch < 1 << 30 and matrices * -(-S // 128) < 1 << 24
 
 
 def attn_fwd(q, k, v, heads, scale):

@@ -406,3 +406,13 @@ def test_attention_takes_positive_scales_only(abi):
         for scale in (0.0, -0.0, -0.125, float("inf"), float("-inf"), float("nan"), 1e-45):
             assert call(scale) == abi.EINVAL, scale
         assert b"scale" in lib.hyc_last_error()
+
+
+def test_attention_launch_limit(abi, hyc):
+    """as many matrices and blocks as one launch counts; the layer's shape rule draws the same line"""
+    lib, ok = abi.load(), hyc.kernels.attn_supported
+    call = lambda B, S: lib.hyc_attn_fwd(None, 64, None, 64, None, 64, B, S, 1, 64, 0.1, None, 64, None, None)
+    for B, S in ((1 << 24, 1), (1 << 23, 129), (1 << 12, 1 << 19)):
+        assert call(B, S) == abi.ENOTSUP and not ok(64, S, 64, B)
+    for B, S in (((1 << 24) - 1, 1), ((1 << 23) - 1, 129)):
+        assert call(B, S) == abi.EFAULT and ok(64, S, 64, B)               # (null buffers: past the shape checks)
