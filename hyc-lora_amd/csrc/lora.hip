@@ -601,7 +601,7 @@ int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const 
   LoraUp a = {};
   a.n = n; a.r = r;
   for (int i = 0; i < n; ++i) {
-    if (!dy[i] || !dB[i]) return fail(HYC_EFAULT, "hyc_lora_up_bwd: null buffer");
+    if ((M > 0 && !dy[i]) || !dB[i]) return fail(HYC_EFAULT, "hyc_lora_up_bwd: null buffer");
     if (!aligned16(dy[i]) || ldg[i] < n_out[i] || ldg[i] % 8 != 0)
       return fail(HYC_EINVAL, "hyc_lora_up_bwd: dy must be 16-byte aligned, rows a multiple of 8 (at least n_out) apart");
     a.g[i] = static_cast<const uint16_t*>(dy[i]);
@@ -612,19 +612,19 @@ int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const 
     a.fb0[i + 1] = a.fb0[i] + (int)((n_out[i] + LU_F - 1) / LU_F);
     a.row0[i + 1] = a.row0[i] + (int)n_out[i];
   }
-  if (M == 0) return HYC_OK;
   const int fblocks = a.fb0[n], ranges = lora_up_ranges(M, fblocks);
   int64_t tokens = (M + ranges - 1) / ranges;
   tokens = (tokens + LU_M - 1) / LU_M * LU_M;
   for (int i = 0; i < n; ++i)
     if (tokens * ldg[i] >= ((int64_t)1 << 30)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: a token range of dy must stay below 2 GiB");
-  const int used = (int)((M + tokens - 1) / tokens);
+  const int used = M ? (int)((M + tokens - 1) / tokens) : 0;   // (no tokens: the sums below are empty and dB is zero)
   const int RC = r <= 16 ? 16 : 32;
   float *dhp = static_cast<float*>(workspace), *dbp = dhp + (int64_t)fblocks * M * RC;
   uint16_t* cp = copy_dy ? static_cast<uint16_t*>(ext) : nullptr;
   hipStream_t st = begin_launch(stream);
   const dim3 grid((unsigned)fblocks, (unsigned)used);
-  if (RC == 16) hipLaunchKernelGGL((k_lora_up_bwd<1>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
+  if (M == 0) {}
+  else if (RC == 16) hipLaunchKernelGGL((k_lora_up_bwd<1>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
   else hipLaunchKernelGGL((k_lora_up_bwd<2>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
   if ((rc = check_launch("hyc_lora_up_bwd"))) return rc;
   const int64_t per = 256 / RC, token_blocks = (M + per - 1) / per, blocks = n * token_blocks + (rows + per - 1) / per;

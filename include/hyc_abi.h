@@ -341,7 +341,7 @@ int hyc_rope_from_heads(const void* g, const void* cosv, const void* sinv, int64
  *   hyc_lora_up_bwd    from one read of dY_i [M, n_out_i] (rows ldg[i] apart): dh = bf16(scale * dY_i B_i) to dh [M, n r] and,
  *                      with zeros behind them, to the `room` columns [sum n_out, + room) of ext (rows ld_ext apart);
  *                      dB_i = scale * dY_i^T h_i; with copy_dy the dY_i side by side to the first sum n_out columns of ext.
- *                      workspace: hyc_lora_up_bwd_workspace_bytes()
+ *                      workspace: hyc_lora_up_bwd_workspace_bytes().  Without tokens (M = 0) only the dB_i are used: zero
  *   hyc_lora_weight_t  out bf16 [K, sum n_out + room] = [W^T | A_i^T side by side | zeros]: dX = ext out^T is the whole input
  *                      gradient of the group, base and rank-r terms
  * fp32 accumulation in a fixed order throughout; room >= n r, a multiple of 8.

@@ -125,6 +125,22 @@ def test_no_tokens(K):
     assert ext.shape == (0, 128) and dh.shape == (0, 16) and not dB[0].any()
 
 
+@pytest.mark.parametrize("r", [16, 32])
+def test_no_tokens_at_the_c_entry(hyc, r):
+    """dB of an empty batch is written (zero), with no other buffer given; nothing behind it is touched"""
+    import ctypes
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    K, lib = hyc.kernels, hyc._abi.load()
+    outs = [72, 264]
+    B = [torch.ones(o, r, dtype=torch.bfloat16, device="cuda") for o in outs]
+    dB = [torch.full((o + 1, r), 7.0, dtype=torch.bfloat16, device="cuda") for o in outs]
+    none = (ctypes.c_void_p * 2)(None, None)
+    rc = lib.hyc_lora_up_bwd(none, K._i64s(outs), 0, K._i64s(outs), K._ptrs(B), None, 2, r, 1.0, None, None, 336 + 64, 64, 1, K._ptrs(dB), None,
+                             K._stream())
+    assert rc == 0 and all(not d[:-1].any() and (d[-1] == 7).all() for d in dB)
+
+
 def test_more_tokens_than_a_range_takes_in_32(K):
     """past 32 x 32768 tokens there are more ranges, each short enough for its offsets"""
     M, r = (1 << 20) + 33, 8
