@@ -98,16 +98,37 @@ class LoRAProjections(torch.nn.Module):
         return outs if len(self.out_features) > 1 else outs[0]
 
 
+def _cut_columns(M, N):
+    """columns at which _product cuts an [M, N] result in two, 0 to leave it whole.  The library's kernels are chosen for
+    256-wide tiles here, and where they do not come out even it takes ones that run at down to half the rate.  A cut behind the
+    first 8192 columns (4096 of up to 8192) costs nothing where the two parts take no more rounds of 256 tiles over the 256
+    CUs than the whole does, and gains where the first part fills its rounds and the rest is short, or where the width is a
+    multiple of 256 that no 192- or 224-wide tile divides.  Measured at 22 widths from 4608 to 37888 and 25 token counts from
+    1024 to 16384, both with and without accumulation: 328 products that this rule cuts take 1.23 times as long whole on
+    average, and one of them 0.93 times (the next 0.97).  In us, whole -> cut: N = 22016, K = 4096 at 1536 / 2048 / 3093 /
+    4096 tokens 288 -> 213, 401 -> 253, 536 -> 421, 625 -> 497; N = 11008, K = 4160: 130 -> 121, 260 -> 142, 328 -> 228,
+    404 -> 266; N = 5632, K = 2112 at 3093 / 4096: 80 -> 74, 94 -> 79.  Left whole for the rounds a cut adds: N = 22016 at
+    2560 and 5120 tokens 326 (361 cut) and 736 (860), N = 11008 at 2560 160 (189), N = 5632 at 2048 52 (54); for its width:
+    N = 13824, K = 5120 at 2048 tokens 207 (212), N = 27648, K = 4096 the same 332 (443)."""
+    if N % 256 or N % 4096 == 0 or N <= 4096 or M * N <= 256 * 256 * 256:
+        return 0
+    cut = 8192 if N > 8192 else 4096
+    rest, row_tiles = N - cut, -(-M // 256)
+    rounds = lambda columns: -(-row_tiles * (columns // 256) // 256)
+    first = row_tiles * (cut // 256)                                # tiles of the first part
+    if rounds(cut) > 4 or rounds(cut) + rounds(rest) > rounds(N):
+        return 0
+    even = first % 256 == 0
+    if even and 2 * rest <= cut:
+        return cut
+    filled = even or (rounds(cut) <= 2 and 4 * first >= 3 * 256 * rounds(cut))
+    return cut if filled and (N // 256) % 3 and (N // 256) % 7 else 0
+
+
 def _product(out, a, b, accumulate=False):
-    """out [M, N] (+)= a @ b^T, both operands contiguous along the reduction.  The library's kernels for output widths that
-    are not whole multiples of 4096 waste up to a third of the chip from about six rounds of its 256-wide tiles on; cut at
-    8192 (4096) columns both parts run at the rate of the round widths: N = 22016, K = 4160 at 1536 / 2048 / 3093 / 4096
-    tokens 308 -> 221, 402 -> 260, 528 -> 421, 638 -> 505 us (but 332 -> 369 at 2560), N = 11008: 132 -> 122, 260 -> 143,
-    331 -> 232, 404 -> 264; N = 5632, K = 2112 at 3093 / 4096: 85 -> 75, 94 -> 79 (2048: 52 -> 54, so not below 3072)."""
+    """out [M, N] (+)= a @ b^T, both operands contiguous along the reduction, in one product or two (_cut_columns)"""
     M, N = out.shape
-    cut = 0
-    if N % 4096:
-        cut = 8192 if N > 8192 and M >= 1536 else 4096 if 4096 < N < 8192 and M >= 3072 else 0
+    cut = _cut_columns(M, N)
     for lo, hi in (((0, cut), (cut, N)) if cut else ((0, N),)):
         part = out[:, lo:hi]
         if accumulate:
