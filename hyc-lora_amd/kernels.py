@@ -4,6 +4,7 @@ torch is used for device memory and the current stream only.  Nothing here compu
 nothing falls back to torch ops for the hot path: inputs that are not CUDA tensors raise.
 """
 import ctypes
+import functools
 from dataclasses import dataclass
 from typing import Optional
 
@@ -1015,13 +1016,15 @@ def _lora_factors(factors, shapes, device, name):
         raise ValueError("%d factors %s for %d projections" % (len(factors), name, len(shapes)))
     as_read = True
     for f, shape in zip(factors, shapes):
-        if not isinstance(f, torch.Tensor) or f.device != device or f.dtype != BF16 or f.shape != shape:
+        if not isinstance(f, torch.Tensor) or f.dtype is not BF16 or f.device != device or f.shape != shape:
             what = "%s %s on %s" % (f.dtype, tuple(f.shape), f.device) if isinstance(f, torch.Tensor) else type(f).__name__
             raise ValueError("%s must be bfloat16 %s on %s, got %s" % (name, tuple(shape), device, what))
-        as_read = as_read and f.is_contiguous() and f.data_ptr() % 16 == 0
+        if f.data_ptr() % 16 or not f.is_contiguous():
+            as_read = False
     return as_read
 
 
+@functools.lru_cache(maxsize=256)
 def _lora_kernels_cover(M, n, r, K, outs):
     """what the hyc_lora_* entries take: up to 4 factors of rank 8 to 32, and no more tokens and features than their launches count"""
     return (n <= 4 and r in (8, 16, 24, 32) and n * r <= 96 and K % 64 == 0 and K <= 1 << 24 and M <= 65535 * 128
@@ -1070,7 +1073,7 @@ def lora_up(h, B, scale, outs=None):
     _need_h(h, M, n * r)
     as_read = _lora_factors(B, [(o, r) for o in outs], h.device, "B")
     y = torch.empty((M, sum(outs)), dtype=BF16, device=h.device)
-    if as_read and _lora_kernels_cover(M, n, r, 64, outs):
+    if as_read and _lora_kernels_cover(M, n, r, 64, tuple(outs)):
         check(_abi.load().hyc_lora_up(_p(h), M, _ptrs(B), _i64s(outs), n, r, float(scale), _p(y), _stream()))
         return y
     zero, col = h.new_zeros(1), 0
@@ -1102,7 +1105,7 @@ def lora_up_bwd(gs, B, h, scale, room, ext=None):
         _need(ext, BF16, "ext")
         if ext.shape != (M, total + room) or ext.device != h.device:
             raise ValueError("ext must be [%d, %d] on %s, got %s on %s" % (M, total + room, h.device, tuple(ext.shape), ext.device))
-    if M and as_read and _lora_kernels_cover(M, n, r, 64, outs) and _lora_range_fits(M, max(max(g.stride(0), o) for g, o in zip(gs, outs))):
+    if M and as_read and _lora_kernels_cover(M, n, r, 64, tuple(outs)) and _lora_range_fits(M, max(max(g.stride(0), o) for g, o in zip(gs, outs))):
         lib = _abi.load()
         dh = torch.empty((M, n * r), dtype=BF16, device=h.device)
         dB = [torch.empty_like(b) for b in B]
@@ -1137,7 +1140,7 @@ def lora_weight_t(q: NF4Weight, A, outs, room):
     if room < n * r:
         raise ValueError("room for %d columns, the group has %d" % (room, n * r))
     out = torch.empty((Kf, total + room), dtype=BF16, device=q.packed.device)
-    if as_read and _lora_kernels_cover(0, n, r, Kf, outs):
+    if as_read and _lora_kernels_cover(0, n, r, Kf, tuple(outs)):
         check(_abi.load().hyc_lora_weight_t(_p(q.packed), _p(q.absmax), Kf, _ptrs(A), _i64s(outs), n, r, room, _p(out), _stream()))
         return out
     out[:, :total], out[:, total:] = nf4_dequantize(q).t(), 0

@@ -38,7 +38,7 @@ def test_token_ranges_are_bounded_with_their_last_tile():
 
 def test_sizes_past_what_a_launch_counts_take_the_general_products():
     cover = K._lora_kernels_cover
-    assert cover(4096, 3, 16, 4096, [4096] * 3) and cover(65535 * 128, 1, 8, 64, [8])
-    for args in ((65535 * 128 + 1, 1, 8, 64, [8]), (1, 1, 8, 64, [65535 * 128]), (1, 1, 8, (1 << 24) + 64, [8]), (1, 5, 8, 64, [8] * 5),
-                 (1, 1, 64, 64, [8]), (1, 1, 8, 32, [8]), (1, 1, 8, 64, [12]), (1, 2, 8, 64, [8, 0])):
+    assert cover(4096, 3, 16, 4096, (4096,) * 3) and cover(65535 * 128, 1, 8, 64, (8,))
+    for args in ((65535 * 128 + 1, 1, 8, 64, (8,)), (1, 1, 8, 64, (65535 * 128,)), (1, 1, 8, (1 << 24) + 64, (8,)), (1, 5, 8, 64, (8,) * 5),
+                 (1, 1, 64, 64, (8,)), (1, 1, 8, 32, (8,)), (1, 1, 8, 64, (12,)), (1, 2, 8, 64, (8, 0))):
         assert not cover(*args)
