@@ -58,26 +58,6 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 
-// 16 bytes per lane from memory to LDS (lane i lands at lds_base + 16 i).  Written as an instruction instead of the
-// compiler's builtin because the compiler then makes every later LDS read wait for it, buffer it fills or not; the kernels
-// below wait themselves (vmcnt 0 in front of the barrier that publishes a tile).
-__device__ __forceinline__ void dma_b128(u32x4_t rsrc, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_base), "v"(voff), "s"(rsrc));
-}
-__device__ __forceinline__ void dma_b32(u32x4_t rsrc, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-               :: "s"(lds_base), "v"(voff), "s"(rsrc));
-}
-__device__ __forceinline__ u32x4_t uniform_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t a = (uint64_t)(uintptr_t)base;
-  u32x4_t r;
-  r.x = __builtin_amdgcn_readfirstlane((uint32_t)a);
-  r.y = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xFFFFu);
-  r.z = __builtin_amdgcn_readfirstlane(bytes);
-  r.w = 0x00020000u;
-  return r;
-}
 // every load to LDS of this wave has landed, then the workgroup meets
 __device__ __forceinline__ void tile_barrier() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -288,12 +288,7 @@ k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, f
   const uint16_t* base = a.g[p] + m_begin * a.ldg[p] + f0;
   // (the resource ends with the last row's last feature of this block)
   const int fl = n_out - f0 < LU_F ? n_out - f0 : LU_F;  // features this block really has, a multiple of 8
-  const uint64_t ba = (uint64_t)(uintptr_t)base;
-  u32x4_t rs;
-  rs.x = __builtin_amdgcn_readfirstlane((uint32_t)ba);
-  rs.y = __builtin_amdgcn_readfirstlane((uint32_t)(ba >> 32) & 0xFFFFu);
-  rs.z = __builtin_amdgcn_readfirstlane((uint32_t)(count - 1) * pitch + 2u * (uint32_t)fl);
-  rs.w = 0x00020000u;
+  const u32x4_t rs = uniform_rsrc(base, (uint32_t)(count - 1) * pitch + 2u * (uint32_t)fl);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)&tile[0][0];
   const int ir = lane >> 5, ic = lane & 31;              // an instruction brings two rows of 32 chunks
   auto issue = [&](int t, int buf) __attribute__((always_inline)) {
@@ -304,8 +299,7 @@ k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, f
       c = 8 * c < fl ? c : 0;                            // features past the end: any finite values (their factors are zero)
       const int m = t * LU_M + row < count ? t * LU_M + row : count - 1;
       const uint32_t dst = lds0 + (uint32_t)(buf * LU_M * LU_F * 2 + (wave + 4 * u) * 1024);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                   :: "s"(dst), "v"((uint32_t)m * pitch + 16u * c), "s"(rs));
+      dma_b128(rs, (uint32_t)m * pitch + 16u * c, dst);
     }
   };
   // the tile's rows of h (this projection's r columns, zeros behind them and past the range): registers, then LDS

@@ -93,6 +93,32 @@ __device__ __forceinline__ void store_b32(BufferRsrc r, uint32_t off, uint32_t v
 __device__ __forceinline__ void store_b16(BufferRsrc r, uint32_t off, uint16_t v) {
   __builtin_amdgcn_raw_buffer_store_b16((short)v, r, (int)off, 0, 0);
 }
+
+// The same resource in four scalar registers, for an instruction written out.
+__device__ __forceinline__ u32x4_t uniform_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  u32x4_t r;
+  r.x = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  r.y = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xFFFFu);
+  r.z = __builtin_amdgcn_readfirstlane(bytes);
+  r.w = 0x00020000u;
+  return r;
+}
+// 16 (4) bytes per lane from memory to LDS (lane i lands at lds_base + 16 i (4 i)).  Written as an instruction instead of the
+// compiler's builtin because the compiler then makes every later LDS read wait for it, buffer it fills or not; the kernels
+// that use it wait themselves (vmcnt 0 in front of the barrier that publishes a tile).  m0 is named as overwritten, for
+// whatever the compiler may have put there; it warns because it reserves that register, whose old value nothing needs back.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma_b128(u32x4_t rsrc, uint32_t voff, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_base), "v"(voff), "s"(rsrc) : "m0");
+}
+__device__ __forceinline__ void dma_b32(u32x4_t rsrc, uint32_t voff, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               :: "s"(lds_base), "v"(voff), "s"(rsrc) : "m0");
+}
+#pragma clang diagnostic pop
 // 16 bytes per lane from memory straight into LDS: lane i of the wave lands at `lds_wave_base` + 16 i
 __device__ __forceinline__ void load_b128_to_lds(BufferRsrc r, uint32_t off, void* lds_wave_base) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_wave_base, 16, (int)off, 0, 0, 0);

@@ -416,3 +416,15 @@ def test_attention_launch_limit(abi, hyc):
         assert call(B, S) == abi.ENOTSUP and not ok(64, S, 64, B)
     for B, S in (((1 << 24) - 1, 1), ((1 << 23) - 1, 129)):
         assert call(B, S) == abi.EFAULT and ok(64, S, 64, B)               # (null buffers: past the shape checks)
+
+
+def test_inline_assembly_names_the_registers_it_overwrites():
+    """an instruction sequence that sets m0 says so: the compiler may keep a value of its own there"""
+    import glob
+    seen = 0
+    for path in sorted(glob.glob(os.path.join(ROOT, "hyc-lora_amd", "csrc", "*.h*"))):
+        for stmt in re.findall(r"\basm\b[^;]*;", open(path).read()):
+            if re.search(r"\bs_mov_b32 m0\b", stmt):
+                seen += 1
+                assert stmt.rsplit(":", 1)[-1].count('"m0"') == 1, (path, stmt)
+    assert seen >= 2
