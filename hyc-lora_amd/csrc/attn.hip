@@ -185,6 +185,7 @@ __device__ __forceinline__ void store_own(floatx16_t (&o)[HD / 32], uint16_t* T,
       const uint2 w = make_uint2(pack_bf16(o[db][4 * b], o[db][4 * b + 1]), pack_bf16(o[db][4 * b + 2], o[db][4 * b + 3]));
       *reinterpret_cast<uint2*>(T + r * HD + 8 * (c ^ swz<HD>(r)) + 4 * hi) = w;
     }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the other lanes' writes before these reads
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
   for (int u = 0; u < 32 * CH / 64; ++u) {
@@ -193,6 +194,7 @@ __device__ __forceinline__ void store_own(floatx16_t (&o)[HD / 32], uint16_t* T,
       *reinterpret_cast<uint4*>(out + (int64_t)(row0 + rr) * pitch + 8 * c) =
           *reinterpret_cast<const uint4*>(T + rr * HD + 8 * (c ^ swz<HD>(rr)));
   }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // and the reads before what is written there next
   __builtin_amdgcn_wave_barrier();
 }
 

@@ -428,3 +428,16 @@ def test_inline_assembly_names_the_registers_it_overwrites():
                 seen += 1
                 assert stmt.rsplit(":", 1)[-1].count('"m0"') == 1, (path, stmt)
     assert seen >= 2
+
+
+def test_lanes_that_meet_in_lds_order_their_memory():
+    """a wave barrier keeps the lanes together and orders nothing by itself: a fence stands in front of each"""
+    import glob
+    seen = 0
+    for path in sorted(glob.glob(os.path.join(ROOT, "hyc-lora_amd", "csrc", "*.h*"))):
+        lines = [l.split("//")[0] for l in open(path).read().splitlines()]
+        for i, line in enumerate(lines):
+            if "__builtin_amdgcn_wave_barrier" in line:
+                seen += 1
+                assert "__builtin_amdgcn_fence" in lines[i - 1] and '"wavefront"' in lines[i - 1], (path, i + 1)
+    assert seen >= 4
