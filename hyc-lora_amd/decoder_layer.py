@@ -192,17 +192,39 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
         n = len(mod.out_features)
         A, B = ctx.saved_tensors[:n], ctx.saved_tensors[n:]
         r, total = A[0].shape[0], sum(mod.out_features)
+        if torch.is_grad_enabled():                             # create_graph: products that leave one
+            return _LoRAProjectionsFunc._backward_with_graph(ctx, A, B, gs)
         rows = _room_behind(getattr(gs[0], "_hyc_rows", None), gs, total, mod.room)
         ext, dh, dB = K.lora_up_bwd([_kernel_rows(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, mod.room, rows)
-        # dA_i = dh_i^T @ x_hat: the projections of a group read the same saved activation, so their dh go through
-        # the weight-gradient kernel side by side (32 output rows per call, the widest its LoRA-shaped form takes)
-        # and x_hat is decoded once per call instead of once per projection
-        dA, per_call = [], max(1, 32 // r) * r
-        for c0 in range(0, n * r, per_call):
-            block = K.gradw_gemm(dh[:, c0:c0 + per_call], ctx.saved_x, out_dtype=A[0].dtype)
-            dA.extend(block[j:j + r] for j in range(0, block.shape[0], r))
+        dA = _LoRAProjectionsFunc._grad_A(ctx, dh, A)
         dx = torch.empty((ext.shape[0], mod.in_features), dtype=BF16, device=ext.device)
         _product(dx, ext, K.lora_weight_t(mod.base_all, A, mod.out_features, mod.room))
+        ctx.h = ctx.saved_x = None
+        return (dx.reshape(gs[0].shape[:-1] + (mod.in_features,)), None, None) + tuple(dA) + tuple(dB)
+
+    @staticmethod
+    def _grad_A(ctx, dh, A):
+        """dA_i = dh_i^T @ x_hat: the projections of a group read the same saved activation, so their dh go through the
+        weight-gradient kernel side by side (32 output rows per call, the widest its LoRA-shaped form takes) and x_hat is
+        decoded once per call instead of once per projection"""
+        r, dA = A[0].shape[0], []
+        per_call = max(1, 32 // r) * r
+        for c0 in range(0, dh.shape[1], per_call):
+            block = K.gradw_gemm(dh[:, c0:c0 + per_call], ctx.saved_x, out_dtype=A[0].dtype)
+            dA.extend(block[j:j + r] for j in range(0, block.shape[0], r))
+        return dA
+
+    @staticmethod
+    def _backward_with_graph(ctx, A, B, gs):
+        """the same gradients through torch's own products, so that dx and dB can be differentiated again with respect to the
+        gradients and the factors (dA comes from the compressed input by a kernel and is a constant there)"""
+        mod, s, r = ctx.mod, ctx.mod.scaling, A[0].shape[0]
+        gs2 = [g.reshape(-1, o).to(BF16) for g, o in zip(gs, mod.out_features)]
+        dhs = [s * (g @ b) for g, b in zip(gs2, B)]
+        dB = [s * (g.t() @ ctx.h[:, i * r:(i + 1) * r]) for i, g in enumerate(gs2)]
+        dh = torch.cat(dhs, dim=1)
+        dA = _LoRAProjectionsFunc._grad_A(ctx, dh.detach(), A)
+        dx = dh @ torch.cat(list(A), dim=0) + torch.cat(gs2, dim=1) @ K.nf4_dequantize(mod.base_all)
         ctx.h = ctx.saved_x = None
         return (dx.reshape(gs[0].shape[:-1] + (mod.in_features,)), None, None) + tuple(dA) + tuple(dB)
 

@@ -216,3 +216,27 @@ def test_a_range_that_only_its_last_tile_takes_past_2_gib(K):
     assert torch.equal(ext[:, :out], g) and torch.equal(ext[:, out:out + r], dh) and not ext[:, out + r:].any()
     close(dh[:64], 0.5 * (g[:64].float() @ B[0].float()))
     close(dB[0][:64], 0.5 * (g[:, :64].float().t().contiguous() @ h.float()))
+
+
+@pytest.mark.parametrize("rank", [16, 64])                 # the kernels' and the general products' backward
+def test_a_gradient_of_a_gradient(K, hyc, rank):
+    """create_graph: dx and dB can be differentiated with respect to the factors and the upstream gradients, as through plain
+    products (the first gradients are the ordinary ones)"""
+    import importlib
+    DL = importlib.import_module(hyc.__name__ + ".decoder_layer")
+    outs = (128, 64)
+    mod = DL.LoRAProjections(256, list(outs), DL.LayerConfig(hidden=256, lora_r=rank, compress=False), "cuda")
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    x, gs, v = mk(2, 9, 256), [mk(2, 9, o) for o in outs], mk(2, 9, 256)
+    plain = _gradients(mod, x, gs)
+    xl, gl = x.clone().requires_grad_(True), [g.clone().requires_grad_(True) for g in gs]
+    first = torch.autograd.grad(mod(xl), [xl] + list(mod.parameters()), gl, create_graph=True)
+    for a, b in zip(first, plain):
+        assert (a - b).abs().max() <= 4 * 2.0 ** -8 * b.abs().max()       # up to four roundings in place of one
+    second = torch.autograd.grad(first[0], gl + list(mod.parameters()), v, allow_unused=True)
+    A, B = ([p.detach().double().requires_grad_(True) for p in ps] for ps in (mod.lora_A, mod.lora_B))
+    G = [g.double().requires_grad_(True) for g in gs]
+    dx = sum(g @ (K.nf4_dequantize(w).double() + mod.scaling * b @ a) for g, w, a, b in zip(G, mod.base, A, B))
+    for a, b in zip(second, torch.autograd.grad(dx, G + A + B, v.double())):
+        assert (a.double() - b).norm() <= 1e-2 * b.norm()
