@@ -33,7 +33,9 @@ def _backward(ctx, dy):
     dy2, _ = as_rows(dy.to(torch.bfloat16))
     dx, dw = K.layernorm_bwd(dy2, ctx.saved, ctx.weight.detach().contiguous(), ctx.mean, ctx.rstd)
     db = None
-    if ctx.bias is not None:
+    if ctx.bias is not None and torch.is_grad_enabled():           # create_graph: a sum that can be differentiated again
+        db = dy2.float().sum(0).to(ctx.bias.dtype)
+    elif ctx.bias is not None:
         db = K.bias_grad(dy2, ctx.bias.dtype if ctx.bias.dtype == torch.bfloat16 else torch.float32).to(ctx.bias.dtype)
     return dx.reshape(dy.shape), dw, db
 

@@ -25,3 +25,17 @@ def test_bias_grad(K, M, H, dtype):
     if dtype == torch.bfloat16:
         bound = bound + want.abs() * 2.0 ** -8
     assert bool(((got.double() - want).abs() <= bound).all())
+
+
+def test_bias_gradient_of_a_gradient(K):
+    """create_graph: the bias gradient can be differentiated with respect to the upstream gradient"""
+    import importlib
+    ops = importlib.import_module("hyc-lora_amd").operators
+    mod = ops.EfficientMemoryLayerNorm(256, mode="hyc", rank=0, group_size=32).cuda().bfloat16()
+    x = torch.randn(2, 9, 256, device="cuda").bfloat16()
+    for _ in range(3):
+        y = mod(x)
+    g = torch.randn(2, 9, 256, device="cuda").bfloat16().requires_grad_(True)
+    (db,) = torch.autograd.grad(y, [mod.bias], g, create_graph=True)
+    (dg,) = torch.autograd.grad(db, [g], torch.arange(256, device="cuda").bfloat16())
+    assert torch.equal(dg, torch.arange(256, device="cuda").bfloat16().expand(2, 9, 256))
