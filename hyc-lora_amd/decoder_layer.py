@@ -86,9 +86,13 @@ class LoRAProjections(torch.nn.Module):
             row += out
         self.site = CompressionSite(cfg.outlier_ratio, 1.0, cfg.linear_bits, "per-token", 0, "hyc", cfg.linear_group,
                                     cfg.scale_rule)
-        self.room = K.lora_room(len(self.out_features), cfg.lora_r)
         self.iteration = 0
         self.record = None
+
+    @property
+    def room(self):
+        """columns for the group's rank columns behind its gradients (of the factors as they are now: a rank may be changed)"""
+        return K.lora_room(len(self.out_features), self.lora_A[0].shape[0])
 
     def forward(self, x):
         x2 = x.reshape(-1, self.in_features)
@@ -163,7 +167,7 @@ def _kernel_rows(t):
 
 class _LoRAProjectionsFunc(torch.autograd.Function):
     """A group is one library product each way: forward y = s h B^T (h = x A^T), onto which the base product accumulates in
-    its epilogue; backward dX = [dY | s dY B] [W^T | A^T]^T with the rank-r terms as mod.room further columns of the
+    its epilogue; backward dX = [dY | s dY B] [W^T | A^T]^T with the rank-r terms as further columns of the
     reduction (kernels.lora_down / lora_up / lora_up_bwd / lora_weight_t)."""
 
     @staticmethod
@@ -194,11 +198,12 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
         r, total = A[0].shape[0], sum(mod.out_features)
         if torch.is_grad_enabled():                             # create_graph: products that leave one
             return _LoRAProjectionsFunc._backward_with_graph(ctx, A, B, gs)
-        rows = _room_behind(getattr(gs[0], "_hyc_rows", None), gs, total, mod.room)
-        ext, dh, dB = K.lora_up_bwd([_kernel_rows(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, mod.room, rows)
+        room = K.lora_room(n, r)
+        rows = _room_behind(getattr(gs[0], "_hyc_rows", None), gs, total, room)
+        ext, dh, dB = K.lora_up_bwd([_kernel_rows(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, room, rows)
         dA = _LoRAProjectionsFunc._grad_A(ctx, dh, A)
         dx = torch.empty((ext.shape[0], mod.in_features), dtype=BF16, device=ext.device)
-        _product(dx, ext, K.lora_weight_t(mod.base_all, A, mod.out_features, mod.room))
+        _product(dx, ext, K.lora_weight_t(mod.base_all, A, mod.out_features, room))
         ctx.h = ctx.saved_x = None
         return (dx.reshape(gs[0].shape[:-1] + (mod.in_features,)), None, None) + tuple(dA) + tuple(dB)
 

@@ -240,3 +240,22 @@ def test_a_gradient_of_a_gradient(K, hyc, rank):
     dx = sum(g @ (K.nf4_dequantize(w).double() + mod.scaling * b @ a) for g, w, a, b in zip(G, mod.base, A, B))
     for a, b in zip(second, torch.autograd.grad(dx, G + A + B, v.double())):
         assert (a.double() - b).norm() <= 1e-2 * b.norm()
+
+
+@pytest.mark.parametrize("rank", [32, 8])
+def test_factors_of_another_rank(K, hyc, rank):
+    """adapters replaced by ones of another rank: the results of a group that was made with that rank"""
+    import importlib
+    DL = importlib.import_module(hyc.__name__ + ".decoder_layer")
+    outs = (128, 64, 64)
+    make = lambda r: DL.LoRAProjections(256, list(outs), DL.LayerConfig(hidden=256, lora_r=r, lora_alpha=2.0 * r, compress=False), "cuda")
+    mod, want = make(16), make(rank)
+    for ours, theirs in ((mod.lora_A, want.lora_A), (mod.lora_B, want.lora_B)):
+        for i, p in enumerate(theirs):
+            ours[i] = torch.nn.Parameter(p.detach().clone())
+    mod.base_all, mod.base = want.base_all, want.base
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    mk = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").bfloat16()
+    x, gs = mk(2, 9, 256), [mk(2, 9, o) for o in outs]
+    assert mod.room == K.lora_room(3, rank) == want.room
+    assert all(torch.equal(a, b) for a, b in zip(_gradients(mod, x, gs), _gradients(want, x, gs)))
