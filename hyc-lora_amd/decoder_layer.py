@@ -248,6 +248,10 @@ class CompressedAttention(torch.nn.Module):
     threshold.  Composition of apply_rotary_pos_emb and the reference's gemm1, softmax and gemm2 modules
     (models/modeling_llama.py:423-462, operators/efficient_gemm.py, operators/efficient_softmax.py)."""
 
+    # columns to leave free behind the gradients of q, k and v side by side, where one kernel writes them (they are handed on as
+    # `_hyc_rows` of the three, see _LoRAProjectionsFunc)
+    grad_room = 0
+
     def __init__(self, cfg: LayerConfig):
         super().__init__()
         if cfg.attention not in ("eager", "flash"):
@@ -260,9 +264,8 @@ class CompressedAttention(torch.nn.Module):
         self.static_value = None          # probability threshold, as in EfficientMemorySoftmax
         self.record = None
 
-    def forward(self, q, k, v, cos, sin, grad_room=0):
-        """grad_room: columns to leave free behind the gradients of q, k and v side by side, where one kernel writes them (they
-        are handed on as `_hyc_rows` of the three, see _LoRAProjectionsFunc)"""
+    def forward(self, q, k, v, cos, sin, grad_room=None):
+        grad_room = self.grad_room if grad_room is None else grad_room
         func = _FlashAttentionFunc if self.cfg.attention == "flash" else _AttentionFunc
         return func.apply(q, k, v, cos, sin, self, grad_room)
 
@@ -481,6 +484,10 @@ class DecoderLayer(torch.nn.Module):
         self.attention = CompressedAttention(cfg)
         self.act = EfficientMemoryGatedAct("silu", cfg.outlier_ratio, 1.0, cfg.act_bits, "per-token", 0,
                                            group_size=cfg.act_group, scale_rule=cfg.scale_rule) if cfg.compress else None
+        # (as attributes: what the layer calls its modules with is what their hooks and replacements see)
+        self.attention.grad_room = self.qkv_proj.room
+        if self.act is not None:
+            self.act.grad_room = self.gate_up_proj.room
         self._rope = None
 
     def forward(self, x):
@@ -490,12 +497,12 @@ class DecoderLayer(torch.nn.Module):
             self._rope = rope_tables(s, cfg.head_dim, cfg.rope_theta, x.device)
         cos, sin = self._rope
         # no names for the wide intermediates: each is released as soon as its consumer has run
-        x = x + self.o_proj(self.attention(*self.qkv_proj(self.input_layernorm(x)), cos, sin, self.qkv_proj.room))
+        x = x + self.o_proj(self.attention(*self.qkv_proj(self.input_layernorm(x)), cos, sin))
         return x + self.down_proj(self._gated(*self.gate_up_proj(self.post_attention_layernorm(x))))
 
     def _gated(self, gate, up):
         if self.act is not None:
-            return self.act(gate, up, grad_room=self.gate_up_proj.room)
+            return self.act(gate, up)
         return torch.nn.functional.silu(gate) * up
 
     def saved_activation_bytes(self, batch, seq):

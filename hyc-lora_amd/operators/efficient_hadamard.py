@@ -144,6 +144,10 @@ class EfficientMemoryGatedAct(torch.nn.Module):
     module saves the same three compressed activations and gives bit-identical gradients, but its backward reads the
     incoming gradient once and never writes the gradient of act(gate) to memory."""
 
+    # a number of columns: the gradients of gate and up are written side by side into one matrix with that many free columns
+    # behind them, which is handed on as `_hyc_rows` of both, so that the projections they go to can append to its rows
+    grad_room = None
+
     def __init__(self, act: str = "silu", outlier_ratio: float = 0.01, sub_outlier_ratio: float = 1.0,
                  sub_outlier_bit: int = 4, sub_outlier_quantize_method: str = 'per-token', rank: int = 0, *,
                  group_size: int = 128, scale_rule: str = "absmax"):
@@ -157,8 +161,7 @@ class EfficientMemoryGatedAct(torch.nn.Module):
         self.iteration = 0
 
     def forward(self, gate, up, grad_room=None):
-        """grad_room: write the gradients of gate and up side by side into one matrix with that many free columns behind them,
-        and hand the matrix on as `_hyc_rows` of both, so that the projections they go to can append to its rows"""
+        grad_room = self.grad_room if grad_room is None else grad_room
         out = _ChannelGatedActFunc.apply(gate, up, self.act, (self.site_act, self.site_up, self.site_gate), self.iteration,
                                          self.sub_outlier_bit, self.group_size, grad_room)
         self.iteration += 1

@@ -360,3 +360,29 @@ def test_layer_at_its_own_size(DL, K, B, S):
     analytic = layer.saved_activation_bytes(B, S)
     assert 0.9 * analytic < held < 1.25 * analytic, (held, analytic)
     y.sum().backward()
+
+
+def test_the_layer_calls_its_modules_with_what_they_compute_from(DL, K):
+    """hooks and replacements of the attention and the gated product see (q, k, v, cos, sin) and (gate, up) and nothing else"""
+    cfg = small_cfg(DL, attention="flash")
+    layer = DL.DecoderLayer(cfg)
+    gen = torch.Generator().manual_seed(11)
+    x = make_input(gen, 2, 32, cfg.hidden).cuda().requires_grad_(True)
+    seen = []
+    for mod in (layer.attention, layer.act):
+        mod.register_forward_pre_hook(lambda m, args, kwargs: seen.append((len(args), sorted(kwargs))), with_kwargs=True)
+    layer(x)
+    assert seen == [(5, []), (2, [])]
+
+    class Plain(torch.nn.Module):
+        def forward(self, gate, up):
+            return torch.nn.functional.silu(gate) * up
+
+    class Pass(torch.nn.Module):
+        def forward(self, q, k, v, cos, sin):
+            return v
+
+    layer.act, layer.attention = Plain(), Pass()
+    y = layer(x)
+    y.backward(torch.ones_like(y))
+    assert torch.isfinite(x.grad).all()
