@@ -248,9 +248,10 @@ class CompressedAttention(torch.nn.Module):
     threshold.  Composition of apply_rotary_pos_emb and the reference's gemm1, softmax and gemm2 modules
     (models/modeling_llama.py:423-462, operators/efficient_gemm.py, operators/efficient_softmax.py)."""
 
-    # columns to leave free behind the gradients of q, k and v side by side, where one kernel writes them (they are handed on as
-    # `_hyc_rows` of the three, see _LoRAProjectionsFunc)
-    grad_room = 0
+    # a number of columns: where one kernel writes the gradients of q, k and v, they lie side by side in one matrix with that many
+    # free columns behind them, which is handed on as `_hyc_rows` of the three (see _LoRAProjectionsFunc); None: three
+    # contiguous tensors
+    grad_room = None
 
     def __init__(self, cfg: LayerConfig):
         super().__init__()
@@ -392,7 +393,8 @@ class _FlashAttentionFunc(torch.autograd.Function):
         b, s, H = q.shape
         nh, hd = cfg.heads, cfg.head_dim
         scale = 1.0 / math.sqrt(hd)
-        ctx.rows = K.attn_supported(hd, s, max(v.stride(1), 3 * H + grad_room), b * nh)        # (the pitch the gradients get)
+        pitch = H if grad_room is None else 3 * H + grad_room       # of the gradients
+        ctx.rows = K.attn_supported(hd, s, max(v.stride(1), pitch), b * nh)
         seed = offset = None
         if ctx.rows:                                                # the kernels read and write the rows as they are
             q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
@@ -432,8 +434,9 @@ class _FlashAttentionFunc(torch.autograd.Function):
             qq, kk, vv, oo = (restore(c).view(b, s, nh * hd) for c in ctx.saved)
             ctx.saved = None
             grads = K.attn_bwd(g.to(BF16).contiguous(), qq, kk, vv, oo, lse, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
-            for t in grads[:3]:
-                t._hyc_rows = grads[3]
+            if ctx.grad_room is not None:
+                for t in grads[:3]:
+                    t._hyc_rows = grads[3]
             return grads[:3] + (None,) * 4
         to_heads = lambda rows: K.rope_to_heads(rows.view(b, s, nh * hd), nh)
         gh = K.rope_to_heads(g.to(BF16).contiguous(), nh)

@@ -386,3 +386,17 @@ def test_the_layer_calls_its_modules_with_what_they_compute_from(DL, K):
     y = layer(x)
     y.backward(torch.ones_like(y))
     assert torch.isfinite(x.grad).all()
+
+
+@pytest.mark.parametrize("attention", ["eager", "flash"])
+def test_attention_by_itself_returns_contiguous_gradients(DL, attention):
+    """outside a layer nothing asks for room behind the gradients: each is a tensor of its own that can be viewed flat"""
+    cfg = small_cfg(DL, attention=attention)
+    mod = DL.CompressedAttention(cfg)
+    gen = torch.Generator().manual_seed(12)
+    q, k, v = (torch.randn(2, 32, cfg.hidden, generator=gen).bfloat16().cuda().requires_grad_(True) for _ in range(3))
+    cos, sin = DL.rope_tables(32, cfg.head_dim, cfg.rope_theta, "cuda")
+    y = mod(q, k, v, cos, sin)
+    grads = torch.autograd.grad(y, (q, k, v), torch.ones_like(y))
+    assert all(t.is_contiguous() and t.view(-1).numel() == t.numel() for t in grads)
+    assert len({t.untyped_storage().data_ptr() for t in grads}) == 3
