@@ -239,8 +239,10 @@ k_attn_fwd(AttnRows Q, AttnRows K, AttnRows V, AttnOut O, float* __restrict__ ls
   floatx16_t o[NB];
 #pragma unroll
   for (int d = 0; d < NB; ++d) o[d] = zero16();
-  float m = -INFINITY, l = 0.f;
   const float c = scale * LOG2E;
+  // the running maximum starts below every score but finite, also once scaled: a row that has met only scores of -inf so far
+  // (masked keys, products past the range) keeps it, and weights them 0
+  float m = -3e38f / __builtin_fmaxf(c, 1.f), l = 0.f;
   const int my_q = w0 + (lane & 31);
   for (int t = 0; t < tiles; ++t) {
     tile_barrier();
@@ -270,7 +272,7 @@ k_attn_fwd(AttnRows Q, AttnRows K, AttnRows V, AttnOut O, float* __restrict__ ls
       for (int i = 0; i < 16; ++i) mx = __builtin_fmaxf(mx, s[kb][i]);
     mx = __builtin_fmaxf(mx, other_half(mx));
     if (__ballot(mx > m)) {
-      // (mx is -inf where a row of the wave lies wholly above this tile: m keeps its value, and is finite from the first tile on)
+      // (mx is -inf where a row of the wave lies wholly above this tile: m keeps its value)
       const float mn = __builtin_fmaxf(m, mx), f = __builtin_amdgcn_exp2f((m - mn) * c);
       m = mn;
       l *= f;

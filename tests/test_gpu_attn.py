@@ -94,6 +94,26 @@ def test_attention_stays_inside_its_batch_element(K, hd):
         assert torch.equal(a[0], b[0])
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("scale", [0.1, 3.0])
+@pytest.mark.parametrize("dead", [64, 130])
+def test_scores_of_minus_infinity_have_no_weight(K, hd, scale, dead):
+    """whole tiles of keys that score -inf: later queries attend to the keys behind them, as in the softmax written out; queries
+    that see nothing else are NaN there and here"""
+    S, heads = 200, 2
+    H = heads * hd
+    gen = torch.Generator(device="cuda").manual_seed(10)
+    q, k, v = (torch.randn(1, S, H, generator=gen, device="cuda").bfloat16() for _ in range(3))
+    q[..., ::hd] = 1.0
+    k[:, :dead, ::hd] = float("-inf")
+    out, lse = K.attn_fwd(q, k, v, heads, scale)
+    want, want_lse = attention_fp32(q.float(), k.float(), v.float(), heads, scale)
+    assert torch.isfinite(want[:, dead:]).all()
+    close(out[:, dead:], want[:, dead:], 2 * 2.0 ** -9)
+    assert (lse[..., dead:] - want_lse[..., dead:]).abs().max() < 1e-4 * max(1.0, scale / 0.1)
+    assert out[:, :dead].isnan().all() and (lse[..., :dead] == float("-inf")).all()
+
+
 def test_attention_refuses_what_it_does_not_cover(K):
     assert not K.attn_supported(32, 64, 128) and not K.attn_supported(128, 1 << 18, 1 << 12)
     q = torch.zeros(1, 8, 64, dtype=torch.bfloat16, device="cuda")
