@@ -911,6 +911,8 @@ k_rmsnorm_bwd(const uint16_t* __restrict__ dy, const uint8_t* __restrict__ store
 // p = lane, lane+8, ... and the 8 lane sums are added in lane order.  The kernel is one round trip to memory long, so
 // a lane asks for all of its rows at once (32 loads in flight cover the 256 partial rows of the fast backward; rows
 // past the end lie beyond the buffer resource and read zeros).
+// PAIRS: lane sums and rounds of rows are added as a tree, for sums of few rounding errors (the bias gradient in fp32).
+template <bool PAIRS = false>
 __global__ void __launch_bounds__(256)
 k_colsum(const float* __restrict__ partials, int64_t P, int64_t H, void* __restrict__ dw, bool wf32) {
   __shared__ float part[8][33];
@@ -928,8 +930,12 @@ k_colsum(const float* __restrict__ partials, int64_t P, int64_t H, void* __restr
     for (int i = 0; i < BATCH; ++i) t[i] = __uint_as_float(load_b32(rs, off + (uint32_t)i * (uint32_t)(8 * H * 4)));
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
 #pragma unroll
-    for (int i = 0; i < BATCH; i += 4) { s0 += t[i]; s1 += t[i + 1]; s2 += t[i + 2]; s3 += t[i + 3]; }
-    s += (s0 + s1) + (s2 + s3);
+    for (int d = 1; PAIRS && d < BATCH; d *= 2)
+#pragma unroll
+      for (int i = 0; i < BATCH; i += 2 * d) t[i] += t[i + d];
+#pragma unroll
+    for (int i = 0; !PAIRS && i < BATCH; i += 4) { s0 += t[i]; s1 += t[i + 1]; s2 += t[i + 2]; s3 += t[i + 3]; }
+    s += PAIRS ? t[0] : (s0 + s1) + (s2 + s3);
   }
   part[lane][cx] = s;
   __syncthreads();
@@ -937,6 +943,8 @@ k_colsum(const float* __restrict__ partials, int64_t P, int64_t H, void* __restr
     float tot = 0.f;
 #pragma unroll
     for (int l = 0; l < 8; ++l) tot += part[l][cx];
+    if (PAIRS)
+      tot = ((part[0][cx] + part[1][cx]) + (part[2][cx] + part[3][cx])) + ((part[4][cx] + part[5][cx]) + (part[6][cx] + part[7][cx]));
     if (wf32) static_cast<float*>(dw)[c] = tot;
     else static_cast<uint16_t*>(dw)[c] = f_to_bf(tot);
   }
@@ -965,11 +973,12 @@ k_bias_partials(const uint16_t* __restrict__ dy, int64_t M, int64_t H, int64_t r
       for (int t = 0; t < BIAS_STEPS; ++t)
         raw[t] = r + t * BIAS_ROWS < r1 ? *reinterpret_cast<const uint4*>(dy + (r + t * BIAS_ROWS) * H + col) : make_uint4(0, 0, 0, 0);
 #pragma unroll
-      for (int t = 0; t < BIAS_STEPS; ++t) {
-        float v[8];
-        unpack8(raw[t], v);
+      for (int t = 0; t < BIAS_STEPS; t += 4) {
+        float v[4][8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] += v[j];
+        for (int u = 0; u < 4; ++u) unpack8(raw[t + u], v[u]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] += (v[0][j] + v[1][j]) + (v[2][j] + v[3][j]);
       }
     }
   }
@@ -978,10 +987,10 @@ k_bias_partials(const uint16_t* __restrict__ dy, int64_t M, int64_t H, int64_t r
   o[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
   __syncthreads();
   const int64_t c = (int64_t)blockIdx.x * BIAS_COLS + threadIdx.x;
-  float s = 0.f;
+  float s[BIAS_ROWS];
 #pragma unroll
-  for (int l = 0; l < BIAS_ROWS; ++l) s += part[l][threadIdx.x];
-  if (c < H) partials[(int64_t)blockIdx.y * H + c] = s;
+  for (int l = 0; l < BIAS_ROWS; ++l) s[l] = part[l][threadIdx.x];
+  if (c < H) partials[(int64_t)blockIdx.y * H + c] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
 // rows a workgroup of k_bias_partials sums: one round of 32 at least, and so many that about 1024 workgroups are launched and
@@ -1339,7 +1348,7 @@ static int norm_bwd_impl(const void* dy, const void* stored, const void* vals, c
     }
   }
   if (!dw) return HYC_OK;                        // the caller adds up the partial rows itself
-  hipLaunchKernelGGL(k_colsum, dim3((unsigned)((H + 31) / 32)), dim3(256), 0, st, dw_partials, used_P, H, dw, wf32);
+  hipLaunchKernelGGL(k_colsum<false>, dim3((unsigned)((H + 31) / 32)), dim3(256), 0, st, dw_partials, used_P, H, dw, wf32);
   return check_launch("hyc_rmsnorm_bwd (dw)");
 }
 
@@ -1433,7 +1442,7 @@ int hyc_bias_grad(const void* dy, int64_t M, int64_t H, float* partials, void* d
     const int rc = check_launch("hyc_bias_grad");
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_colsum, dim3((unsigned)((H + 31) / 32)), dim3(256), 0, st, partials, P, H, db, db_dtype == HYC_DTYPE_F32);
+  hipLaunchKernelGGL(k_colsum<true>, dim3((unsigned)((H + 31) / 32)), dim3(256), 0, st, partials, P, H, db, db_dtype == HYC_DTYPE_F32);
   return check_launch("hyc_bias_grad (sum)");
 }
 

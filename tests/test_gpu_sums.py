@@ -39,3 +39,15 @@ def test_bias_gradient_of_a_gradient(K):
     (db,) = torch.autograd.grad(y, [mod.bias], g, create_graph=True)
     (dg,) = torch.autograd.grad(db, [g], torch.arange(256, device="cuda").bfloat16())
     assert torch.equal(dg, torch.arange(256, device="cuda").bfloat16().expand(2, 9, 256))
+
+
+@pytest.mark.parametrize("M,H", [(3627, 1024), (9700, 13824), (2048, 65536), (16384, 4096)])
+@pytest.mark.parametrize("mean", [0.0, 0.05])
+def test_bias_grad_rounds_no_more_than_the_plain_sum(K, M, H, mean):
+    """in fp32 the error against fp64 (over the whole vector) is that of torch's own fp32 sum or less (5 %: two samples of the
+    same size differ by 1 / sqrt(2 H))"""
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    dy = (mean + 0.02 * torch.randn(M, H, generator=gen, device="cuda")).bfloat16()
+    want = dy.double().sum(0)
+    error = lambda t: float((t.double() - want).norm() / want.norm())
+    assert error(K.bias_grad(dy, torch.float32)) <= 1.05 * error(dy.float().sum(0))
