@@ -29,16 +29,17 @@ def attention_fp32(q, k, v, heads, scale):
     return torch.matmul(torch.softmax(s, -1), v).transpose(1, 2).reshape(B, S, H), torch.logsumexp(s, -1)
 
 
-def close(got, want, bound):
-    # (absolute where the exact result is zero: the first query attends to itself alone, its dq and dk vanish)
+def close(got, want, bound, zero=0.0):
+    # zero: an element's error where the exact result vanishes
     err = (got.double() - want.double()).norm()
-    assert err <= bound * want.double().norm() + 1e-3 * math.sqrt(want.numel()), float(err / want.double().norm())
+    assert err <= bound * want.double().norm() + zero * math.sqrt(want.numel()), float(err / want.double().norm())
 
 
-# a walked tile is 64 rows, a wave owns 32, a workgroup 128; 513 and more walk several tiles on both sides of the diagonal
+# a walked tile is 64 rows, a wave owns 32, a workgroup 128; 513 and more walk several tiles on both sides of the diagonal; 13
+# batches of 8 heads and 5 blocks are more workgroups than two per CU, where the order of the blocks is another
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("B,S,heads", [(1, 1, 1), (2, 31, 3), (1, 33, 2), (2, 64, 1), (1, 65, 8), (1, 127, 2), (3, 129, 2), (1, 513, 5),
-                                       (2, 1030, 2)])
+                                       (2, 1030, 2), (13, 513, 8)])
 def test_attention_against_fp32(K, hd, B, S, heads):
     H, scale = heads * hd, 1.0 / math.sqrt(hd)
     gen = torch.Generator(device="cuda").manual_seed(S * hd)
@@ -54,8 +55,9 @@ def test_attention_against_fp32(K, hd, B, S, heads):
     assert (lse - want_lse.detach()).abs().max() < 1e-4        # fp32 sums of at most 1030 terms
     grads = torch.autograd.grad(want, leaves, g.float())
     # P or dS, the stored output inside delta, and the result: three such roundings
+    # (a single query attends to itself alone and its dq and dk vanish: fp32 sums of hd products in two orders, about 1e-6 each)
     for got, ref in zip(K.attn_bwd(g, q, k, v, out, lse, heads, scale), grads):
-        close(got, ref, 3 * 2.0 ** -9)
+        close(got, ref, 3 * 2.0 ** -9, 1e-5 if S == 1 else 0.0)
 
 
 @pytest.mark.parametrize("hd,S", [(128, 77), (64, 200)])

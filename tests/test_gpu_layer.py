@@ -23,9 +23,13 @@ def DL(hyc):
     return importlib.import_module(hyc.__name__ + ".decoder_layer")
 
 
-def small_cfg(DL, **kw):
-    return DL.LayerConfig(hidden=256, heads=4, head_dim=64, intermediate=512, lora_r=16, lora_alpha=32.0,
+def small_cfg(DL, heads=4, **kw):
+    return DL.LayerConfig(hidden=256, heads=heads, head_dim=256 // heads, intermediate=512, lora_r=16, lora_alpha=32.0,
                           outlier_ratio=0.02, softmax_ratio=0.05, **kw)
+
+
+# heads of 64 and 128 channels take the layer's own attention kernels, of 32 the library's
+ATTENTION = [("eager", 4), ("flash", 4), ("flash", 2), ("flash", 8)]
 
 
 def oracle_params(K, layer):
@@ -80,12 +84,12 @@ def check_grads(layer, groups, xg, P, xo, tol):
     return errs
 
 
-@pytest.mark.parametrize("attention", ["eager", "flash"])
-def test_layer_formulas_without_compression(DL, K, attention):
+@pytest.mark.parametrize("attention,heads", ATTENTION)
+def test_layer_formulas_without_compression(DL, K, attention, heads):
     """compress=False: the layer's own backward (LoRA composite, attention) against the oracle with exact activations,
     whose gradients are pinned against plain float64 autograd"""
     B, S = 2, 64
-    cfg = small_cfg(DL, compress=False, attn_group_bytes=5 * 2 * 64 * 64, attention=attention)
+    cfg = small_cfg(DL, heads, compress=False, attn_group_bytes=5 * 2 * 64 * 64, attention=attention)
     layer = DL.DecoderLayer(cfg)
     gen = torch.Generator().manual_seed(3)
     x = make_input(gen, B, S, cfg.hidden)
@@ -110,14 +114,14 @@ def K(hyc):
     return hyc.kernels
 
 
-@pytest.mark.parametrize("attention", ["eager", "flash"])
-def test_layer_with_compression(DL, K, attention):
+@pytest.mark.parametrize("attention,heads", ATTENTION)
+def test_layer_with_compression(DL, K, attention, heads):
     """three steps (two calibrating, one steady); on each: every site restores what the oracle restores, the kept
     probabilities are the oracle's set (eager attention; the fused attention keeps its output instead), and the
     gradients equal the oracle layer's at those restored activations (relative error of each gradient tensor below
     1e-2)"""
     B, S = 2, 64
-    cfg = small_cfg(DL, attn_group_bytes=3 * 2 * 64 * 64, attention=attention)   # 8 score matrices in groups of 3, 3, 2
+    cfg = small_cfg(DL, heads, attn_group_bytes=3 * 2 * 64 * 64, attention=attention)   # 8 score matrices in groups of 3, 3, 2
     layer = DL.DecoderLayer(cfg)
     H, I, nh = cfg.hidden, cfg.intermediate, cfg.heads
     gen = torch.Generator().manual_seed(4)
@@ -242,16 +246,17 @@ def test_training_tracks_the_uncompressed_layer(DL, K):
     assert abs(c[-1] - u[-1]) < 0.15 * u[0], (c[-1], u[-1], u[0])
 
 
+@pytest.mark.parametrize("attention", ["eager", "flash"])
 @pytest.mark.parametrize("B,S", [(1, 2048), (4, 1024)])
-def test_layer_at_its_own_size(DL, K, B, S):
+def test_layer_at_its_own_size(DL, K, B, S, attention):
     """The fifth configuration at its real size (hidden 4096, 32 heads x 128, intermediate 11008, NF4 base, LoRA r = 16,
     1 % outlier channels, INT2 linear inputs, INT4 elsewhere), batch 1 x 2048 and 4 x 1024 tokens, three steps (two
     calibrating, one steady).  On each step: every compressed site restores, bit for bit on a 48-row sample, what the
     oracle's compress / decompress gives for the activation the device saw; the kept probabilities are the oracle's
-    set; the layer's output and every gradient are within 1e-2 (relative norm) of the oracle layer evaluated at the
+    set (eager attention); the layer's output and every gradient are within 1e-2 (relative norm) of the oracle layer evaluated at the
     restored activations (the oracle, plain fp32 torch, runs on the GPU here: its matrix products at this size take
     minutes on the host).  After the steps: what a forward keeps matches the analytic count."""
-    cfg = DL.LayerConfig()
+    cfg = DL.LayerConfig(attention=attention)
     layer = DL.DecoderLayer(cfg)
     H, I, nh = cfg.hidden, cfg.intermediate, cfg.heads
     gen = torch.Generator().manual_seed(B * 1000 + S)
@@ -301,18 +306,22 @@ def test_layer_at_its_own_size(DL, K, B, S):
         R["gate"] = restore_and_check(gate.reshape(-1, I), c_gate, ab, ag).reshape(B, S, I)
         R["up"] = restore_and_check(up.reshape(-1, I), c_up, ab, ag).reshape(B, S, I)
         R["act"] = restore_and_check(torch.nn.functional.silu(gate).reshape(-1, I), c_act, ab, ag).reshape(B, S, I)
-        p_dev = rec["attn"]["p"]
-        thr = O.get_statistics_softmax(p_dev, step, cfg.softmax_ratio) if step < 2 else layer.attention.static_value
-        R["p"] = torch.cat([K.softmax_dense(sp) for sp in rec["attn"]["sparse"]]).reshape(p_dev.shape)
-        assert bits_equal(R["p"], O.prune_softmax(p_dev, thr))
-        kept = float((R["p"] > 0).float().mean())
-        assert 0.002 < kept < 0.03, kept
+        p_dev = None
+        if attention == "flash":
+            R["o"] = restore_and_check(rec["attn"]["o"].contiguous(), rec["attn"]["saved"][3], ab, ag).reshape(B, S, H)
+        else:
+            p_dev = rec["attn"]["p"]
+            thr = O.get_statistics_softmax(p_dev, step, cfg.softmax_ratio) if step < 2 else layer.attention.static_value
+            R["p"] = torch.cat([K.softmax_dense(sp) for sp in rec["attn"]["sparse"]]).reshape(p_dev.shape)
+            assert bits_equal(R["p"], O.prune_softmax(p_dev, thr))
+            kept = float((R["p"] > 0).float().mean())
+            assert 0.002 < kept < 0.03, kept
 
         for t in P.values():
             t.grad = None
         xo = x.float().cuda().requires_grad_(True)
         yo = LO.decoder_layer(xo, P, R, nh, cfg.rms_eps, cfg.lora_alpha / cfg.lora_r, cos, sin, quirk=True, probs=p_dev,
-                              attention="eager")
+                              attention=attention)
         yo.backward(g.float().cuda())
         errs = {"y": err(y.detach(), yo.detach()), "dx": err(xg.grad, xo.grad),
                 "w_in": err(layer.input_layernorm.weight.grad, P["w_in"].grad),
@@ -400,3 +409,75 @@ def test_attention_by_itself_returns_contiguous_gradients(DL, attention):
     grads = torch.autograd.grad(y, (q, k, v), torch.ones_like(y))
     assert all(t.is_contiguous() and t.view(-1).numel() == t.numel() for t in grads)
     assert len({t.untyped_storage().data_ptr() for t in grads}) == 3
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_a_hook_on_one_gradient_of_a_group(DL, K, which):
+    """a hook that scales, replaces or rewrites in place one gradient of q, k, v or of gate, up: the results are those of the
+    layer whose attention and gated product return separate gradients, bit for bit"""
+    cfg = small_cfg(DL, attention="flash")
+    layer = DL.DecoderLayer(cfg)
+    gen = torch.Generator().manual_seed(13)
+    x = make_input(gen, 2, 48, cfg.hidden).cuda()
+    g = (0.05 * torch.randn(2, 48, cfg.hidden, generator=gen)).bfloat16().cuda()
+    for _ in range(2):
+        layer(x)
+    changes = [lambda t: 2 * t, lambda t: torch.full_like(t, 0.01), lambda t: t.mul_(0.5)]
+
+    def hooked(change):
+        for mod in (layer.qkv_proj, layer.gate_up_proj):
+            yield mod.register_forward_hook(lambda m, i, outs: outs[which % len(outs)].register_hook(change) and None)
+
+    def gradients(change):
+        handles = list(hooked(change))
+        leaf = x.clone().requires_grad_(True)
+        out = torch.autograd.grad(layer(leaf), [leaf] + list(layer.parameters()), g)
+        for h in handles:
+            h.remove()
+        return out
+
+    for change in changes:
+        got = gradients(change)
+        room = layer.attention.grad_room, layer.act.grad_room
+        layer.attention.grad_room = layer.act.grad_room = None
+        want = gradients(change)
+        layer.attention.grad_room, layer.act.grad_room = room
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    plain = gradients(lambda t: None)
+    assert not torch.equal(plain[0], got[0])
+
+
+def test_layer_captured_in_a_graph(DL, K):
+    """a calibrated layer's forward and backward as one graph: every replay, with eager work between, gives what the same step
+    gives eagerly on that input"""
+    cfg = small_cfg(DL, attention="flash")
+    layer = DL.DecoderLayer(cfg)
+    gen = torch.Generator().manual_seed(14)
+    mk = lambda: (make_input(gen, 2, 48, cfg.hidden).cuda(), (0.05 * torch.randn(2, 48, cfg.hidden, generator=gen)).bfloat16().cuda())
+    x, g = mk()
+    x.requires_grad_(True)
+
+    def step():
+        y = layer(x)
+        return (y,) + torch.autograd.grad(y, [x] + list(layer.parameters()), g)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for _ in range(4):
+        xi, gi = mk()
+        with torch.no_grad():
+            x.copy_(xi)
+            g.copy_(gi)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.detach().clone() for t in out]
+        want = step()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        torch.cuda.synchronize()

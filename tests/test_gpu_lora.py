@@ -23,7 +23,13 @@ def close(got, want):
 
 
 CASES = [(1, 64, [8], 8), (16, 256, [256, 64, 128], 16), (65, 512, [1000, 24], 24), (157, 1024, [320], 32), (130, 2816, [1024, 1024, 1024], 32),
-         (300, 4096, [4096, 512], 16), (33, 256, [256, 256], 64)]                   # rank 64: the torch form
+         (300, 4096, [4096, 512], 16), (33, 256, [256, 256], 64),                   # rank 64: the torch form
+         # token ranges of three tiles each (32 ranges of 192 tokens), both buffers refilled, with 24 and 32 of 32 columns
+         (4200, 256, [512, 264], 24), (4200, 256, [512, 264], 32),
+         # four and five tiles of 16 columns of h
+         (200, 512, [64, 64], 32), (200, 512, [64, 64, 64], 24),
+         # the transposed weight by four scale groups at a time (104 x 5 workgroups), the last of them cut at K = 1088
+         (33, 1088, [13248], 16)]
 
 
 @pytest.mark.parametrize("M,Kf,outs,r", CASES)
