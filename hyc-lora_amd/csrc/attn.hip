@@ -9,7 +9,7 @@
 // What bounds these kernels is that a wave's steps follow each other: scores, exponentials, second product.  No unit is full; as
 // shares of the kernel's cycles at 4 x 1024 x 32 heads x 128 (55, 66 and 87 us; counters): matrix cores 0.34 forward, 0.44 dQ,
 // 0.42 dK / dV; the other vector instructions 0.40, 0.24 and 0.21, the exponentials' slower rate not counted (about 0.1
-// more); LDS 0.20, 0.25 and 0.30, of which 6 % at most bank conflicts.  The registers leave room for two waves per SIMD to
+// more); LDS 0.20, 0.25 and 0.30, of which 7 % at most bank conflicts.  The registers leave room for two waves per SIMD to
 // overlap them, so everything that can stay in registers does, and every fragment is read as few times as it can be:
 //  * A wave owns 32 queries (forward, dQ) or 32 keys (dK / dV) and keeps their rows as MFMA operands for the whole loop.
 //  * The score tile is produced with the owned index in the lane (column) and the walked index in the registers (row), so
