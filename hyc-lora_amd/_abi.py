@@ -99,6 +99,11 @@ SIGNATURES = {
     "hyc_attn_fwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_ptr, c_i64, c_ptr, c_ptr]),
     "hyc_attn_bwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64,
                              c_i64, c_f32, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr]),
+    "hyc_attn_kept_fwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_ptr, c_i64, c_ptr, c_ptr]),
+    "hyc_attn_kept": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_f32, c_f32, c_i64, c_i64, c_ptr, c_ptr, c_i64, c_ptr]),
+    "hyc_attn_kept_fill": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_f32, c_f32, c_i64, c_i64, c_ptr, c_ptr, c_i64,
+                                   c_ptr, c_ptr, c_ptr, c_ptr]),
+    "hyc_attn_kept_bwd": (c_i32, [c_ptr, c_i64] * 4 + [c_ptr] * 5 + [c_i64] * 4 + [c_f32, c_i64, c_i64] + [c_ptr, c_i64] * 3 + [c_ptr, c_ptr]),
     "hyc_dropout": (c_i32, [c_ptr, c_ptr, c_i64, c_f32, ctypes.c_uint64, c_i32, c_ptr]),
     "hyc_nf4_quantize": (c_i32, [c_ptr, c_i64, c_ptr, c_ptr, c_ptr]),
     "hyc_nf4_dequantize": (c_i32, [c_ptr, c_ptr, c_i64, c_ptr, c_ptr]),

@@ -5,6 +5,7 @@
 //   dense     yh as a dense matrix (what true_decompress_softmax returns)
 // Reference: operators/efficient_softmax.py:10-45, operators/compress_function.py:264-275.
 #include "abi_util.hpp"
+#include "softmax_slab.hpp"
 #include "wave_scan.hpp"
 
 namespace hyc {
@@ -338,7 +339,7 @@ k_csr_offsets_multi(const int32_t* __restrict__ counts, int64_t rows, int64_t ca
 }
 
 // The kept entries from the forward's slab, one wave per row: a copy of a few words.  A row that kept more than the slab
-// holds is read again, as k_softmax_fill does.
+// holds is read again, as k_softmax_fill does (without a y it is left to the caller).
 __global__ void __launch_bounds__(256)
 k_softmax_fill_slab(const uint16_t* __restrict__ y, int64_t rows, int64_t N, float thr, const int32_t* __restrict__ counts,
                     const uint32_t* __restrict__ slab, int cap, const int32_t* __restrict__ row_ptr, int32_t* __restrict__ cols,
@@ -358,6 +359,7 @@ k_softmax_fill_slab(const uint16_t* __restrict__ y, int64_t rows, int64_t N, flo
     }
     return;
   }
+  if (!y) return;
   const uint16_t* yr = y + row * N;
   int running = 0;
   for (int64_t c0 = 0; c0 < N / 8; c0 += 64) {
@@ -510,6 +512,12 @@ k_softmax_rows(const uint16_t* g, int64_t rows, int64_t N, const int32_t* __rest
   // 16-byte pieces, for the kept entries to pick from a second LDS row was 3 % slower at 2048 entries and 20 % at 8192.)
   uint16_t* orow = out + row * N;
   for (int64_t c = lane; c < N / 8; c += 64) store_stream(orow + 8 * c, *reinterpret_cast<const uint4*>(buf + 8 * c));
+}
+
+void launch_slab_copy(int64_t rows, const int32_t* counts, const uint32_t* slab, int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals,
+                      hipStream_t stream) {
+  hipLaunchKernelGGL(k_softmax_fill_slab, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, static_cast<const uint16_t*>(nullptr), rows,
+                     (int64_t)0, 0.f, counts, slab, (int)cap, row_ptr, cols, static_cast<uint16_t*>(vals));
 }
 
 static int softmax_shape(const char* who, int64_t rows, int64_t N) {

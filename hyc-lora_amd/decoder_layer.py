@@ -285,6 +285,10 @@ class _AttentionFunc(torch.autograd.Function):
         b, s, H = q.shape
         nh, hd = cfg.heads, cfg.head_dim
         scale = 1.0 / math.sqrt(hd)
+        cap = _AttentionFunc._kept_entries(q, k, v, mod, grad_room)
+        ctx.rows = cap > 0
+        if ctx.rows:                                                # a calibrated site: no score matrix is formed
+            return _AttentionFunc._forward_kept(ctx, q, k, v, cos, sin, mod, grad_room, cap)
         # one pass per tensor: rotate, and write both the head-major copy the batched GEMMs need and the rows that
         # are compressed
         qh, q_rows = K.rope_to_heads(q, nh, cos, sin, want_rows=True)
@@ -343,9 +347,52 @@ class _AttentionFunc(torch.autograd.Function):
         return out
 
     @staticmethod
+    def _kept_entries(q, k, v, mod, grad_room):
+        """see kernels.attn_kept_entries; 0 also while the threshold is measured, where all probabilities are kept or recorded and
+        for rows the attention kernels do not cover"""
+        cfg = mod.cfg
+        if not cfg.compress or mod.iteration < 2 or mod.record is not None or q.dim() != 3 or v.data_ptr() % 16 or v.shape != q.shape:
+            return 0
+        b, s, H = q.shape
+        pitch = H if grad_room is None else 3 * H + grad_room
+        if not b or v.stride(2) != 1 or v.stride(1) % 8 or not K.attn_supported(cfg.head_dim, s, max(v.stride(1), pitch), b * cfg.heads):
+            return 0
+        return K.attn_kept_entries(K.kept_budget(mod.static_value), K.threshold_value(mod.static_value), s, cfg.head_dim)
+
+    @staticmethod
+    def _forward_kept(ctx, q, k, v, cos, sin, mod, grad_room, cap):
+        cfg = mod.cfg
+        b, s, H = q.shape
+        nh = cfg.heads
+        scale = 1.0 / math.sqrt(cfg.head_dim)
+        q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
+        out, lse = K.attn_fwd(q_rows, k_rows, v, nh, scale, round_scores=True)
+        thr, budget = K.threshold_value(mod.static_value), K.kept_budget(mod.static_value)
+        # (the slab of kept entries is what grows with the number of matrices here)
+        group = max(1, min(b * nh, cfg.attn_group_bytes // (4 * s * cap)))
+        ctx.kept = [K.attn_kept(q_rows, k_rows, lse, nh, scale, thr, budget, cap, c0, min(group, b * nh - c0))
+                    for c0 in range(0, b * nh, group)]
+        ctx.saved = []
+        for site, r in zip((mod.site_q, mod.site_k, mod.site_v), (q_rows, k_rows, v)):
+            r = r.reshape(b * s, H)
+            ctx.saved.append(K.compress_channel(r, site.channel_plan(r, mod.iteration), cfg.act_bits, cfg.act_group))
+        mod.iteration += 1
+        ctx.geom, ctx.grad_room = (b, nh, s, cfg.head_dim), grad_room
+        ctx.save_for_backward(cos, sin)
+        return out
+
+    @staticmethod
     def backward(ctx, g):
         b, nh, s, hd = ctx.geom
         cos, sin = ctx.saved_tensors
+        if ctx.rows:
+            qq, kk, vv = (K.decompress_channel(c).view(b, s, nh * hd) for c in ctx.saved)
+            grads = K.attn_kept_bwd(g.to(BF16).contiguous(), qq, kk, vv, ctx.kept, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
+            ctx.saved = ctx.kept = None
+            if ctx.grad_room is not None:
+                for t in grads[:3]:
+                    t._hyc_rows = grads[3]
+            return grads[:3] + (None,) * 4
         restore = (lambda c: K.decompress_channel(c)) if ctx.compress else (lambda c: c)
         to_heads = lambda rows: K.rope_to_heads(rows.view(b, s, nh * hd), nh).view(b * nh, s, hd)
         gh = K.rope_to_heads(g.to(BF16).contiguous(), nh).view(b * nh, s, hd)

@@ -1221,17 +1221,28 @@ def attn_supported(head_dim, S, widest_pitch, matrices=1):
     return head_dim in (64, 128) and S * widest_pitch < 1 << 30 and matrices * -(-S // 128) < 1 << 24
 
 
-def attn_fwd(q, k, v, heads, scale):
-    """causal softmax(scale q k^T) v on [B, S, heads*hd] rows -> (out [B, S, heads*hd], lse fp32 [B, heads, S])"""
+def attn_fwd(q, k, v, heads, scale, round_scores=False):
+    """causal softmax(scale q k^T) v on [B, S, heads*hd] rows -> (out [B, S, heads*hd], lse fp32 [B, heads, S]); round_scores: from
+    scores rounded to bf16, as attn_kept takes them"""
     B, S, H, pq = _need_tokens(q, "q")
     pk, pv = _need_tokens(k, "k")[3], _need_tokens(v, "v")[3]
     if tuple(k.shape) != (B, S, H) or tuple(v.shape) != (B, S, H) or H % heads:
         raise ValueError("q, k, v must be [B, S, heads*hd] alike, got %s, %s, %s" % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
     out = torch.empty((B, S, H), dtype=BF16, device=q.device)
     lse = torch.empty((B, heads, S), dtype=torch.float32, device=q.device)
-    check(_abi.load().hyc_attn_fwd(_p(q), pq, _p(k), pk, _p(v), pv, B, S, heads, H // heads, float(scale), _p(out), H, _p(lse),
-                                   _stream()))
+    lib = _abi.load()
+    entry = lib.hyc_attn_kept_fwd if round_scores else lib.hyc_attn_fwd
+    check(entry(_p(q), pq, _p(k), pk, _p(v), pv, B, S, heads, H // heads, float(scale), _p(out), H, _p(lse), _stream()))
     return out, lse
+
+
+def _grad_rows(g, room):
+    """((dq, dk, dv), pitch): empty gradients like g, or with `room` side by side in a matrix that comes as a fourth"""
+    B, S, H = g.shape
+    if room is None:
+        return tuple(torch.empty((B, S, H), dtype=BF16, device=g.device) for _ in range(3)), H
+    both = torch.empty((B * S, 3 * H + room), dtype=BF16, device=g.device)
+    return tuple(both[:, i * H:(i + 1) * H].unflatten(0, (B, S)) for i in range(3)) + (both,), 3 * H + room
 
 
 def attn_bwd(g, q, k, v, out, lse, heads, scale, cos=None, sin=None, room=None):
@@ -1246,17 +1257,69 @@ def attn_bwd(g, q, k, v, out, lse, heads, scale, cos=None, sin=None, room=None):
         ptrs += [_p(t), _need_tokens(t, name)[3]]
     _need_vec(lse, torch.float32, B * heads * S, "lse")
     _need_tables(cos, sin, S, H // heads)
-    if room is None:
-        pitch = H
-        dq, dk, dv = (torch.empty((B, S, H), dtype=BF16, device=g.device) for _ in range(3))
-    else:
-        pitch = 3 * H + room
-        both = torch.empty((B * S, pitch), dtype=BF16, device=g.device)
-        dq, dk, dv = (both[:, i * H:(i + 1) * H].unflatten(0, (B, S)) for i in range(3))
+    grads, pitch = _grad_rows(g, room)
     ws = torch.empty(2 * B * heads * S, dtype=torch.float32, device=g.device)
     check(_abi.load().hyc_attn_bwd(_p(g), pg, *ptrs, _p(lse), _p(cos), _p(sin), B, S, heads, H // heads, float(scale),
-                                   _p(dq), pitch, _p(dk), pitch, _p(dv), pitch, _p(ws), _stream()))
-    return (dq, dk, dv) if room is None else (dq, dk, dv, both)
+                                   _p(grads[0]), pitch, _p(grads[1]), pitch, _p(grads[2]), pitch, _p(ws), _stream()))
+    return grads
+
+
+def attn_kept_entries(budget, threshold, S, head_dim):
+    """slab entries per row with which attn_kept serves a site of this budget, or 0 where scores and probabilities as matrices
+    do: nothing seen yet, a threshold that keeps every positive probability, more than a sixteenth of the entries kept (the
+    entry-by-entry half of the backward grows with them: attention at 1 x 2048 x 32 heads x 128 in us, with matrices / here: 1 % kept
+    907 / 366, 3 % 898 / 499, 6 % 934 / 743), rows the softmax kernels refuse"""
+    if head_dim not in (64, 128) or S % 8 or not 0 < S <= 4096 or not 1e-30 < threshold < 1:
+        return 0
+    return _slab_entries(budget, S)
+
+
+def attn_kept(q, k, lse, heads, scale, threshold, budget, cap, first, matrices):
+    """the probabilities exp(bf16(scale q k^T) - lse) above the threshold of matrices [first, first + matrices) as SparseRows; lse:
+    attn_fwd's with round_scores; cap: attn_kept_entries"""
+    B, S, H, pq = _need_tokens(q, "q")
+    pk = _need_tokens(k, "k")[3]
+    if tuple(k.shape) != (B, S, H) or H % heads:
+        raise ValueError("q and k must be [B, S, heads*hd] alike, got %s, %s" % (tuple(q.shape), tuple(k.shape)))
+    _need_vec(lse, torch.float32, B * heads * S, "lse")
+    lib, rows, dev = _abi.load(), matrices * S, q.device
+    counts = torch.empty(rows, dtype=torch.int32, device=dev)
+    slab = torch.empty((rows, cap), dtype=torch.int32, device=dev)
+    args = (_p(q), pq, _p(k), pk, _p(lse), B, S, heads, H // heads, float(scale), float(threshold), first, matrices, _p(counts), _p(slab), cap)
+    check(lib.hyc_attn_kept(*args, _stream()))
+    row_ptr, nnz, total = _csr_offsets(lib, counts, rows, budget)
+    cols = torch.empty(nnz, dtype=torch.int32, device=dev)
+    vals = torch.empty(nnz, dtype=BF16, device=dev)
+    if nnz:
+        check(lib.hyc_attn_kept_fill(*args, _p(row_ptr), _p(cols), _p(vals), _stream()))
+    return SparseRows(row_ptr, cols, vals, (matrices, S, S), total)
+
+
+def attn_kept_bwd(g, q, k, v, kept, heads, scale, cos=None, sin=None, room=None):
+    """(dq, dk, dv) of causal attention at the given q, k, v with the probabilities in `kept` (SparseRows of consecutive ranges
+    of matrices, all of them together); cos / sin and room as in attn_bwd"""
+    B, S, H, pg = _need_tokens(g, "g")
+    ptrs = []
+    for name, t in (("q", q), ("k", k), ("v", v)):
+        if tuple(t.shape) != (B, S, H):
+            raise ValueError("%s is %s, the gradient is %s" % (name, tuple(t.shape), tuple(g.shape)))
+        ptrs += [_p(t), _need_tokens(t, name)[3]]
+    if H % heads or sum(sp.rows for sp in kept) != B * heads * S or any(sp.rows % S or sp.shape[-1] != S for sp in kept):
+        raise ValueError("the kept probabilities are %s, the gradient is %s" % ([tuple(sp.shape) for sp in kept], tuple(g.shape)))
+    _need_tables(cos, sin, S, H // heads)
+    grads, pitch = _grad_rows(g, room)
+    at, first = [_p(t) for t in grads], 0
+    for sp in kept:
+        matrices, n = sp.rows // S, sp.cols.numel()
+        _need_vec(sp.row_ptr, torch.int32, sp.rows + 1, "row_ptr")
+        _need_vec(sp.cols, torch.int32, n, "cols")
+        _need_vec(sp.vals, BF16, n, "vals")
+        records = torch.empty((max(n, 1), 2), dtype=torch.int32, device=g.device)
+        check(_abi.load().hyc_attn_kept_bwd(_p(g), pg, *ptrs, _p(sp.row_ptr), _p(sp.cols) or _p(records), _p(sp.vals) or _p(records), _p(cos),
+                                            _p(sin), B, S, heads, H // heads, float(scale), first, matrices, at[0], pitch, at[1], pitch,
+                                            at[2], pitch, _p(records), _stream()))
+        first += matrices
+    return grads
 
 
 # ----------------------------------------------------------------------------------------------------

@@ -372,6 +372,33 @@ int hyc_attn_bwd(const void* dout, int64_t ldg, const void* q, int64_t ldq, cons
                  int64_t heads, int64_t head_dim, float scale, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv,
                  int64_t lddv, float* workspace, void* stream);
 
+/* The attention that keeps its probabilities: scores are rounded to bf16, x = bf16(scale q.k), and of matrices
+ * [first, first + matrices) (matrix = b heads + h) the entries whose p = bf16(exp(x - lse)) exceeds bf16(threshold) are kept as
+ * CSR rows (row = position of the matrix in the range * S + query; columns = keys, ascending, at most the query itself).
+ * 1e-30 < threshold < 1, S at most 32768.
+ *   hyc_attn_kept_fwd   hyc_attn_fwd from such scores
+ *   hyc_attn_kept       counts int32 [matrices S] and the first `cap` entries of every row in slab [matrices S, cap], as
+ *                       hyc_softmax_fwd_slab leaves them
+ *   hyc_attn_kept_fill  the CSR arrays for the row_ptr hyc_csr_offsets made of the counts: from the slab, and for rows that kept more
+ *                       than cap from q and k
+ *   hyc_attn_kept_bwd   with Ph the kept entries (zero elsewhere): dp = dout v^T at them, dS = Ph (dp - sum_j Ph dp),
+ *                       dv = Ph^T dout, dq = scale dS k, dk = scale dS^T q, dq and dk through the transposed rotation if cos / sin
+ *                       are given; only the columns of those matrices' heads are written.  records: 8 bytes per entry that cols
+ *                       holds, 8-byte aligned.  fp32 up to Ph and dS as bf16 operands of dv and dk.
+ * No atomics: results repeat bit for bit. */
+int hyc_attn_kept_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, int64_t B, int64_t S,
+                      int64_t heads, int64_t head_dim, float scale, void* out, int64_t ldo, float* lse, void* stream);
+int hyc_attn_kept(const void* q, int64_t ldq, const void* k, int64_t ldk, const float* lse, int64_t B, int64_t S, int64_t heads,
+                  int64_t head_dim, float scale, float threshold, int64_t first, int64_t matrices, int32_t* counts, uint32_t* slab,
+                  int64_t cap, void* stream);
+int hyc_attn_kept_fill(const void* q, int64_t ldq, const void* k, int64_t ldk, const float* lse, int64_t B, int64_t S, int64_t heads,
+                       int64_t head_dim, float scale, float threshold, int64_t first, int64_t matrices, const int32_t* counts,
+                       const uint32_t* slab, int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals, void* stream);
+int hyc_attn_kept_bwd(const void* dout, int64_t ldg, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                      const int32_t* row_ptr, const int32_t* cols, const void* vals, const void* cosv, const void* sinv, int64_t B,
+                      int64_t S, int64_t heads, int64_t head_dim, float scale, int64_t first, int64_t matrices, void* dq, int64_t lddq,
+                      void* dk, int64_t lddk, void* dv, int64_t lddv, void* records, void* stream);
+
 /* ---- seeded dropout ----------------------------------------------------------------------------- */
 /* EfficientMemoryDropoutFunc, operators/efficient_dropout.py:56-79: the keep mask of element i is
  * tl.rand(seed, i) > p (Philox4x32-10, counter (i,0,0,0), key = the two words of seed), so nothing is saved.
