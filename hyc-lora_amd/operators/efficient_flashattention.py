@@ -11,7 +11,7 @@ activations plus one fp32 log-sum-exp per (head, token), and the backward kernel
 import torch
 
 from .. import kernels as K
-from ._calibration import CompressionSite, fold_statistics
+from ._calibration import CompressionSite, fold_statistics, only_result_has_gradient, result_gradient
 from .compress_function import compress_to_csr, get_statistics
 
 _CALIBRATION_CALLS = 5          # the reference averages the statistics of the first five calls here (:66, :197)
@@ -112,11 +112,12 @@ class EfficientFlashAttnVarlenQKVPackedFunc(torch.autograd.Function):
         ctx.saved, ctx.state, ctx.bounds = saved, state, bounds
         ctx.dropout_p, ctx.scale, ctx.causal, ctx.geom = dropout_p, scale, causal, (total, nh, hd)
         (qo, qL, qR, qs), (ko, kL, kR, ks), (vo, vL, vR, vs), (oo, oL, oR, os_) = stats
-        ctx.mark_non_differentiable(qo, ko, vo, oo, qs, ks, vs, os_, qL, qR, kL, kR, vL, vR, oL, oR)
+        only_result_has_gradient(ctx, out, qo, ko, vo, oo, qs, ks, vs, os_, qL, qR, kL, kR, vL, vR, oL, oR)
         return out, qo, ko, vo, oo, qs, ks, vs, os_, qL, qR, kL, kR, vL, vR, oL, oR
 
     @staticmethod
     def backward(ctx, dout, *args):
+        dout = result_gradient(ctx, dout)
         total, nh, hd = ctx.geom
         q, k, v, out = (K.decompress_threshold(c).view(total, nh, hd) for c in ctx.saved)
         ctx.saved = None

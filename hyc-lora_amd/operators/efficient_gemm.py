@@ -9,7 +9,7 @@ compress / decompress / sparsify work around them goes through the HIP kernels.
 import torch
 
 from .. import kernels as K
-from ._calibration import CompressionSite, fold_statistics, running_mean
+from ._calibration import CompressionSite, fold_statistics, running_mean, only_result_has_gradient, result_gradient
 from .compress_function import (compress_to_csr, get_statistics, get_statistics_softmax, head_to_hidden_shape,
                                 hidden_to_head_shape)
 
@@ -52,7 +52,7 @@ class EfficientMemoryGEMMFunc(torch.autograd.Function):
         c2, shape2 = compress_to_csr(x2t, o2, s2, sub_outlier_bit_2, sub_outlier_ratio_2,
                                      L2 if rank > 0 else None, R2 if rank > 0 else None)
         ctx.saved = (c1, shape1, c2, shape2)
-        ctx.mark_non_differentiable(o1, o2, L1, R1, s1, L2, R2, s2)
+        only_result_has_gradient(ctx, result, o1, o2, L1, R1, s1, L2, R2, s2)
         return result, o1, L1, R1, s1, o2, L2, R2, s2
 
     @staticmethod
@@ -60,7 +60,7 @@ class EfficientMemoryGEMMFunc(torch.autograd.Function):
         c1, shape1, c2, shape2 = ctx.saved
         x1 = _restore_heads(c1, shape1, ctx.num_heads)
         x2t = _restore_heads(c2, shape2, ctx.num_heads)              # [B,nh,S,hd] = x2 transposed
-        g = grad_output
+        g = result_gradient(ctx, grad_output)
         grad_input1 = g @ x2t.to(g.dtype)                            # g @ x2^T
         grad_input2 = x1.transpose(-2, -1).to(g.dtype) @ g
         return (grad_input1, grad_input2) + (None,) * 12
@@ -140,7 +140,7 @@ class EfficientMemoryGEMMWithSoftmaxFunc(torch.autograd.Function):
         c2, shape2 = compress_to_csr(x2, o2, s2, sub_outlier_bit_2, sub_outlier_ratio_2,
                                      L2 if rank > 0 else None, R2 if rank > 0 else None)
         ctx.saved = (c2, shape2)
-        ctx.mark_non_differentiable(o1, o2, L2, R2, s2)
+        only_result_has_gradient(ctx, result, o1, o2, L2, R2, s2)
         return result, o1, o2, L2, R2, s2
 
     @staticmethod
@@ -148,7 +148,7 @@ class EfficientMemoryGEMMWithSoftmaxFunc(torch.autograd.Function):
         c2, shape2 = ctx.saved
         x1 = K.softmax_dense(ctx.sparse)
         x2 = _restore_heads(c2, shape2, ctx.num_heads)
-        g = grad_output
+        g = result_gradient(ctx, grad_output)
         grad_input1 = g @ x2.transpose(-2, -1).to(g.dtype)
         grad_input2 = x1.transpose(-2, -1).to(g.dtype) @ g
         return (grad_input1, grad_input2) + (None,) * 9

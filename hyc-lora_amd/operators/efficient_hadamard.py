@@ -2,7 +2,7 @@
 import torch
 
 from .. import kernels as K
-from ._calibration import CompressionSite, as_rows, fold_statistics
+from ._calibration import CompressionSite, as_rows, fold_statistics, only_result_has_gradient, result_gradient
 from .compress_function import compress_to_csr, get_statistics
 
 
@@ -26,11 +26,12 @@ class EfficientMemoryHadamardFunc(torch.autograd.Function):
         ctx.shape = stats[0][5]
         o1, L1, R1, s1 = stats[0][:4]
         o2, L2, R2, s2 = stats[1][:4]
-        ctx.mark_non_differentiable(o1, o2, L1, R1, s1, L2, R2, s2)
+        only_result_has_gradient(ctx, result, o1, o2, L1, R1, s1, L2, R2, s2)
         return result, o1, L1, R1, s1, o2, L2, R2, s2
 
     @staticmethod
     def backward(ctx, grad_output, *unused):
+        grad_output = result_gradient(ctx, grad_output)
         g2, _ = as_rows(grad_output.to(torch.bfloat16))
         d1, d2 = K.hadamard_bwd(g2, ctx.saved[0], ctx.saved[1])
         return (d1.reshape(grad_output.shape), d2.reshape(grad_output.shape)) + (None,) * 12

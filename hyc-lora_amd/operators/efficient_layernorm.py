@@ -8,7 +8,7 @@ chunks per segment) take the framework's layer norm followed by the compress ker
 import torch
 
 from .. import kernels as K
-from ._calibration import CompressionSite, as_rows, fold_statistics
+from ._calibration import CompressionSite, as_rows, fold_statistics, only_result_has_gradient, result_gradient
 from .compress_function import compress_to_csr, get_statistics
 
 
@@ -67,12 +67,13 @@ class EfficientMemoryLayerNormFunc(torch.autograd.Function):
             c, _ = compress_to_csr(x, outlier, scale, sub_outlier_bit, sub_outlier_ratio, L if rank > 0 else None,
                                    R if rank > 0 else None)
         ctx.saved, ctx.mean, ctx.rstd, ctx.weight, ctx.bias = c, mean, rstd, weight, bias
-        ctx.mark_non_differentiable(outlier, L, R, scale)
-        return y.reshape(x.shape), outlier, L, R, scale
+        y = y.reshape(x.shape)
+        only_result_has_gradient(ctx, y, outlier, L, R, scale)
+        return y, outlier, L, R, scale
 
     @staticmethod
     def backward(ctx, dy, grad_outlier, grad_L, grad_R, grad_scale):
-        dx, dw, db = _backward(ctx, dy)
+        dx, dw, db = _backward(ctx, result_gradient(ctx, dy))
         return dx, None, None, None, None, None, None, dw, db, None, None, None
 
 

@@ -3,7 +3,7 @@ by the MFMA kernel.  Reference: operators/efficient_linear.py:11-149."""
 import torch
 
 from .. import kernels as K
-from ._calibration import CompressionSite, as_rows, fold_statistics
+from ._calibration import CompressionSite, as_rows, fold_statistics, only_result_has_gradient, result_gradient
 from .compress_function import compress_to_csr, get_statistics
 
 
@@ -44,12 +44,12 @@ class EfficientMemoryLinearFunc(torch.autograd.Function):
             ctx.saved, _ = compress_to_csr(x, outlier, scale, sub_outlier_bit, sub_outlier_ratio,
                                            L if rank > 0 else None, R if rank > 0 else None)
         ctx.w = w
-        ctx.mark_non_differentiable(outlier, L, R, scale)
+        only_result_has_gradient(ctx, output, outlier, L, R, scale)
         return output, outlier, L, R, scale
 
     @staticmethod
     def backward(ctx, grad_output, grad_outlier, grad_L, grad_R, grad_scale):
-        gi, gw, gb = _linear_backward(grad_output, ctx.w.detach(), ctx.saved, ctx.use_bias, ctx.needs_input_grad[:3])
+        gi, gw, gb = _linear_backward(result_gradient(ctx, grad_output), ctx.w.detach(), ctx.saved, ctx.use_bias, ctx.needs_input_grad[:3])
         return gi, gw, gb, None, None, None, None, None, None, None, None
 
 

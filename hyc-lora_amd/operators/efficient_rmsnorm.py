@@ -3,7 +3,7 @@ fused kernel (decompress + dx + dw partials) and a column reduce.  Reference: op
 import torch
 
 from .. import kernels as K
-from ._calibration import CompressionSite, as_rows, fold_statistics
+from ._calibration import CompressionSite, as_rows, fold_statistics, only_result_has_gradient, result_gradient
 from .compress_function import get_statistics
 
 
@@ -34,11 +34,13 @@ def _ref_forward(ctx, x, outlier_ratio, sub_outlier_ratio, sub_outlier_bit, sub_
     ctx.rstd = rstd
     ctx.weight = weight
     ctx.c2_quirk, ctx.weight_offset = c2_quirk, weight_offset
-    ctx.mark_non_differentiable(outlier, L, R, scale)
-    return y.reshape(x.shape), outlier, L, R, scale
+    y = y.reshape(x.shape)
+    only_result_has_gradient(ctx, y, outlier, L, R, scale)
+    return y, outlier, L, R, scale
 
 
 def _ref_backward(ctx, dy):
+    dy = result_gradient(ctx, dy)
     dy2, _ = as_rows(dy.to(torch.bfloat16))
     dx, dw = K.rmsnorm_bwd(dy2, ctx.saved, _effective_weight(ctx.weight, ctx.weight_offset), ctx.rstd, c2_quirk=ctx.c2_quirk)
     return dx.reshape(dy.shape), dw.to(ctx.weight.dtype)

@@ -4,7 +4,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import kernels as K
-from ._calibration import CompressionSite, as_rows, fold_statistics
+from ._calibration import CompressionSite, as_rows, fold_statistics, only_result_has_gradient, result_gradient
 from .compress_function import compress_to_csr, get_statistics, head_to_hidden_shape, hidden_to_head_shape
 
 
@@ -18,12 +18,12 @@ def _ref_forward(ctx, x, act_fwd, outlier_ratio, sub_outlier_ratio, sub_outlier_
                                                   L if rank > 0 else None, R if rank > 0 else None)
     ctx.is_head = x.dim() == 4
     ctx.num_heads = x.shape[1] if ctx.is_head else 1
-    ctx.mark_non_differentiable(outlier, L, R, scale)
+    only_result_has_gradient(ctx, result, outlier, L, R, scale)
     return result, outlier, L, R, scale
 
 
 def _ref_backward(ctx, act, grad_output):
-    g = grad_output.to(torch.bfloat16)
+    g = result_gradient(ctx, grad_output).to(torch.bfloat16)
     if ctx.is_head:
         g = head_to_hidden_shape(g)
     g2, _ = as_rows(g)

@@ -489,3 +489,26 @@ def test_forward_activation_tables_match_the_framework_for_every_bf16_value(K, a
     cf = [K.compress_channel(t[few].contiguous(), finp, 4, 128) for t in (a, ones, fin)]
     dg_few, _ = K.gated_act_bwd(act, g[few].contiguous(), *cf)
     assert same(dg_few, d_gate[few])
+
+
+@pytest.mark.parametrize("name", ["EfficientMemorySiLU", "EfficientMemorySoftmax"])
+def test_absent_gradient_stands_for_zeros(hyc, name):
+    """a result whose gradient is never computed (its consumer returns None) still gives its input a gradient of zeros, and the
+    statistics beside it none"""
+    class Drop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, y):
+            return y.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    mod = getattr(hyc.operators, name)(**({} if name.endswith("Softmax") else dict(rank=0, sub_outlier_ratio=1.0)))
+    x = torch.randn(2, 32, 64, device="cuda").bfloat16().requires_grad_(True)
+    for _ in range(3):
+        y = mod(x)
+    (dx,) = torch.autograd.grad(Drop.apply(y).sum(), x)
+    assert dx.shape == x.shape and dx.dtype == x.dtype and not bool(dx.any())
+    (dx,) = torch.autograd.grad(mod(x).float().pow(2).sum(), x)
+    assert bool(dx.any())
