@@ -564,7 +564,7 @@ def main():
 
     import torch
     pkg = importlib.import_module("hyc-lora_amd")
-    if not os.path.exists(pkg._abi.LIB_PATH):
+    if not pkg._abi.built():
         import __graft_entry__
         __graft_entry__.build()
     assert torch.cuda.is_available(), "bench.py needs a GPU"

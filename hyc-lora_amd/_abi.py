@@ -8,6 +8,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libhyc_gfx950.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_hyc_host.so")        # the native host path (_host.py), built with the library
 
 MODE_CHANNEL, MODE_THRESHOLD, MODE_DENSE = 0, 1, 2
 DTYPE_BF16, DTYPE_F32 = 0, 1
@@ -110,6 +111,10 @@ SIGNATURES = {
 }
 
 _lib = None
+
+
+def built():
+    return os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH)
 
 
 def load():

@@ -1,11 +1,13 @@
-"""Builds the gfx950 shared library from csrc/*.hip with hipcc (cross-compiles without a GPU).
+"""Builds the gfx950 shared library from csrc/*.hip with hipcc (cross-compiles without a GPU) and the native host path from
+csrc/host/host.cpp against it and torch.
 
-    python hyc-lora_amd/build.py            # -> hyc-lora_amd/lib/libhyc_gfx950.so
+    python hyc-lora_amd/build.py            # -> hyc-lora_amd/lib/libhyc_gfx950.so, hyc-lora_amd/lib/_hyc_host.so
 """
 import glob
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -26,6 +28,24 @@ FLAGS = [
 
 def lib_path():
     return os.path.join(LIBDIR, LIBNAME)
+
+
+def build_host(verbose=True):
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc, out = os.path.join(root, "include"), os.path.join(LIBDIR, "_hyc_host.so")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include",
+           "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "host", "host.cpp"), "-o", out,
+           "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-L" + LIBDIR, "-l:" + LIBNAME, "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on host.cpp:\n" + r.stderr)
+    if verbose and r.stderr.strip():
+        print(r.stderr, file=sys.stderr)
+    return out
 
 
 def build(verbose=True, jobs=4):
@@ -54,8 +74,9 @@ def build(verbose=True, jobs=4):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
+    host = build_host(verbose)
     if verbose:
-        print("built", out)
+        print("built", out, "and", os.path.basename(host))
     return out
 
 

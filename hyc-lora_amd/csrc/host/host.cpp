@@ -1,0 +1,965 @@
+// The host side of a calibrated operator's call in native code: checks, output allocation, descriptors and launches of one
+// step of kernels.py / operators / decoder_layer.py, without the interpreter in between.
+//
+// A short call is bound by its host work (rms norm of 45 x 4096, forward and backward: the kernels take 18 us of 70 to 150), and most
+// of that is a few dozen interpreted steps around each launch.  Every function here covers the plain case only - dense bf16
+// tensors on the GPU of the expected layout, a plan that matches - and returns None for everything else without having launched
+// or changed anything; the caller then goes through the interpreted form, which handles the rest and raises the errors.  What is
+// launched, and with what, is the same in both.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+
+#include "../../../include/hyc_abi.h"
+
+namespace {
+
+using at::Tensor;
+constexpr auto BF16 = at::kBFloat16;
+
+// torch.nn.Parameter, kernels.ChannelCompressed, ChannelPlan, ThresholdCompressed, SparseRows
+PyObject *t_parameter, *t_compressed, *t_plan, *t_threshold, *t_sparse;
+PyObject *s_H, *s_M, *s_S, *s_k, *s_idx, *s_plan, *s_scale_rule, *s_stored, *s_vals, *s_scales, *s_bits, *s_group, *s_row_ptr, *s_cols, *s_threshold,
+    *s_scale, *s_L, *s_R;
+
+struct Ref {                                                           // an owned reference
+  PyObject* p;
+  explicit Ref(PyObject* o) : p(o) {}
+  Ref(const Ref&) = delete;
+  ~Ref() { Py_XDECREF(p); }
+};
+
+void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// a dense GPU tensor of the exact type (a subclass may do anything on access, a functorch wrapper has no memory of its own)
+const Tensor* plain(PyObject* o) {
+  if (!THPVariable_CheckExact(o) && (PyObject*)Py_TYPE(o) != t_parameter) return nullptr;
+  const Tensor& t = THPVariable_Unpack(o);
+  if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.is_conj() || t.is_neg()) return nullptr;
+  return &t;
+}
+const Tensor* bf16(PyObject* o) {
+  const Tensor* t = plain(o);
+  return t && t->scalar_type() == BF16 ? t : nullptr;
+}
+bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+// [..., H] contiguous -> M rows
+bool rows_of(const Tensor& t, int64_t* M, int64_t* H) {
+  if (t.dim() < 1 || !t.is_contiguous()) return false;
+  *H = t.size(-1);
+  if (*H <= 0) return false;
+  *M = t.numel() / *H;
+  return true;
+}
+// [..., H] with contiguous, evenly spaced rows -> M rows `pitch` elements apart
+bool spaced_rows(const Tensor& t, int64_t* M, int64_t* H, int64_t* pitch) {
+  const int64_t d = t.dim();
+  if (d < 2 || t.size(-1) <= 0 || t.numel() == 0 || t.stride(-1) != 1) return false;
+  *H = t.size(-1);
+  *M = t.numel() / *H;
+  for (int64_t i = 0; i + 2 < d; ++i)
+    if (t.size(i) != 1 && t.stride(i) != t.stride(i + 1) * t.size(i + 1)) return false;
+  *pitch = *M > 1 ? t.stride(-2) : *H;
+  if (*M > 1 && t.size(-2) == 1) return false;                         // (the spacing is another dimension's: the general form finds it)
+  return true;
+}
+// the same as the fused kernels read it in place
+bool kernel_rows(const Tensor& t, int64_t* M, int64_t* H, int64_t* pitch) {
+  return spaced_rows(t, M, H, pitch) && aligned16(t.data_ptr()) && *pitch % 8 == 0 && *pitch >= *H;
+}
+
+int64_t attr_i64(PyObject* o, PyObject* name, bool* ok) {
+  Ref v(PyObject_GetAttr(o, name));
+  if (!v.p || !PyLong_CheckExact(v.p)) { PyErr_Clear(); *ok = false; return 0; }
+  return PyLong_AsLongLong(v.p);
+}
+
+struct Plan {
+  int64_t H = 0, k = 0;
+  void *idx = nullptr, *plan = nullptr;
+  int rule = 0;
+  void describe(int64_t bits, int64_t group, hyc_desc* d) const {
+    std::memset(d, 0, sizeof *d);
+    d->mode = HYC_MODE_CHANNEL;
+    d->bits = (int32_t)bits;
+    d->group = (int32_t)group;
+    d->k = (int32_t)k;
+    d->chan_plan = (decltype(d->chan_plan))plan;
+    d->chan_idx = k ? (decltype(d->chan_idx))idx : nullptr;
+    d->scale_rule = rule;
+  }
+};
+// what kernels._check_plan asks of a plan, for an activation of H channels on `device`
+bool get_plan(PyObject* o, int64_t H, c10::Device device, Plan* p) {
+  if ((PyObject*)Py_TYPE(o) != t_plan) return false;
+  bool ok = true;
+  p->H = attr_i64(o, s_H, &ok);
+  p->k = attr_i64(o, s_k, &ok);
+  if (!ok || p->H != H || p->k < 0) return false;
+  Ref idx(PyObject_GetAttr(o, s_idx)), plan(PyObject_GetAttr(o, s_plan)), rule(PyObject_GetAttr(o, s_scale_rule));
+  if (!idx.p || !plan.p || !rule.p) { PyErr_Clear(); return false; }
+  const Tensor *ti = plain(idx.p), *tp = plain(plan.p);
+  if (!ti || !tp || ti->scalar_type() != at::kInt || tp->scalar_type() != at::kInt || !ti->is_contiguous() || !tp->is_contiguous() ||
+      ti->numel() != p->k || tp->numel() != H / 8 || ti->device() != device || tp->device() != device || !PyUnicode_Check(rule.p))
+    return false;
+  if (PyUnicode_CompareWithASCIIString(rule.p, "absmax") == 0) p->rule = HYC_SCALE_ABSMAX;
+  else if (PyUnicode_CompareWithASCIIString(rule.p, "range") == 0) p->rule = HYC_SCALE_RANGE;
+  else return false;
+  p->idx = ti->data_ptr();
+  p->plan = tp->data_ptr();
+  return true;
+}
+
+// a compressed activation about to be written
+struct Out {
+  Tensor stored, vals, scales;
+  hyc_desc d;
+  PyObject *plan, *bits, *group;
+  int64_t M, H;
+  bool init(PyObject* plan_, PyObject* bits_, PyObject* group_, int64_t M_, int64_t H_, c10::Device device) {
+    plan = plan_; bits = bits_; group = group_; M = M_; H = H_;
+    if (!PyLong_CheckExact(bits) || !PyLong_CheckExact(group)) return false;
+    const int64_t b = PyLong_AsLongLong(bits), g = PyLong_AsLongLong(group);
+    Plan p;
+    if (hyc_check_shape(H, (int32_t)b, (int32_t)g, HYC_MODE_CHANNEL) != 0 || !get_plan(plan, H, device, &p)) return false;
+    p.describe(b, g, &d);
+    const auto opt = at::TensorOptions().device(device);
+    stored = at::empty({M, H * b / 8}, opt.dtype(b == 8 ? at::kChar : at::kByte));
+    vals = at::empty({M, p.k}, opt.dtype(BF16));
+    scales = at::empty({M, H / g}, opt.dtype(BF16));
+    return true;
+  }
+  PyObject* wrap() const {                                             // kernels.ChannelCompressed(stored, vals, scales, plan, bits, group, M, H)
+    Ref a(THPVariable_Wrap(stored)), b(THPVariable_Wrap(vals)), c(THPVariable_Wrap(scales)), m(PyLong_FromLongLong(M)), h(PyLong_FromLongLong(H));
+    if (!a.p || !b.p || !c.p || !m.p || !h.p) return nullptr;
+    PyObject* args[8] = {a.p, b.p, c.p, plan, bits, group, m.p, h.p};
+    return PyObject_Vectorcall(t_compressed, args, 8, nullptr);
+  }
+};
+// the threshold scheme's descriptor: a static scale read through two strides, a base of rank 0 or more
+struct Threshold {
+  hyc_desc d;
+  bool init(double threshold, PyObject* scale, int64_t bits, int64_t S, int64_t H, PyObject* L, PyObject* R) {
+    const Tensor* sc = bf16(scale);
+    if (!sc || !sc->is_contiguous()) return false;
+    std::memset(&d, 0, sizeof d);
+    d.mode = HYC_MODE_THRESHOLD;
+    d.bits = (int32_t)bits;
+    d.threshold = (float)threshold;
+    d.scale = (decltype(d.scale))sc->data_ptr();
+    const int64_t n = sc->numel();
+    if (n == 1) { d.scale_stride_token = 0; d.scale_stride_channel = 0; }
+    else if (sc->dim() >= 2 && sc->size(-1) == H && n == H) { d.scale_stride_token = 0; d.scale_stride_channel = 1; }
+    else if (sc->dim() >= 2 && sc->size(-1) == 1 && n == S) { d.scale_stride_token = 1; d.scale_stride_channel = 0; }
+    else return false;
+    d.S = S;
+    if (L != Py_None) {
+      const Tensor *l = bf16(L), *r = bf16(R);
+      if (!l || !r || !l->is_contiguous() || !r->is_contiguous() || l->dim() != 2 || r->dim() != 2 || l->size(0) < S || l->size(1) != r->size(0) || r->size(1) != H)
+        return false;                                                  // (fewer rows than S: padded by the general form)
+      d.rank = (int32_t)l->size(1);
+      if (d.rank) { d.L = (decltype(d.L))l->data_ptr(); d.R = (decltype(d.R))r->data_ptr(); }
+    }
+    return true;
+  }
+};
+const Tensor* attr_vec(const Ref& v, at::ScalarType type) {
+  const Tensor* t = v.p ? plain(v.p) : nullptr;
+  if (!v.p) PyErr_Clear();
+  return t && t->scalar_type() == type && t->is_contiguous() ? t : nullptr;
+}
+Tensor empty_like_on(const Tensor& t, at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, at::TensorOptions().device(t.device()).dtype(type)); }
+
+// a compressed activation about to be read: of the channel scheme as it is, of the threshold scheme restored (ready())
+struct In {
+  Tensor stored, vals, scales, row_ptr, cols;
+  Ref scale{nullptr}, L{nullptr}, R{nullptr};
+  hyc_desc d;
+  int64_t M, H;
+  bool restore_first = false;
+  const void* codes() const { return stored.data_ptr(); }
+  const void* values() const { return vals.defined() ? vals.data_ptr() : nullptr; }
+  const void* group_scales() const { return scales.defined() ? scales.data_ptr() : nullptr; }
+  bool init(PyObject* c) {
+    const bool thr = (PyObject*)Py_TYPE(c) == t_threshold;
+    if (!thr && (PyObject*)Py_TYPE(c) != t_compressed) return false;
+    bool ok = true;
+    M = attr_i64(c, s_M, &ok);
+    H = attr_i64(c, s_H, &ok);
+    const int64_t b = attr_i64(c, s_bits, &ok);
+    Ref st(PyObject_GetAttr(c, s_stored)), va(PyObject_GetAttr(c, s_vals));
+    const Tensor *ts = st.p ? plain(st.p) : nullptr, *tv = va.p ? plain(va.p) : nullptr;
+    if (!ok || !ts || !tv) { PyErr_Clear(); return false; }
+    stored = *ts; vals = *tv;
+    if (thr) {
+      const int64_t S = attr_i64(c, s_S, &ok);
+      Ref rp(PyObject_GetAttr(c, s_row_ptr)), co(PyObject_GetAttr(c, s_cols)), th(PyObject_GetAttr(c, s_threshold));
+      scale.p = PyObject_GetAttr(c, s_scale); L.p = PyObject_GetAttr(c, s_L); R.p = PyObject_GetAttr(c, s_R);
+      const Tensor *tr = attr_vec(rp, at::kInt), *tc = attr_vec(co, at::kInt);
+      Threshold t;
+      if (!ok || !tr || !tc || !th.p || !scale.p || !L.p || !R.p || !PyFloat_CheckExact(th.p) ||
+          !t.init(PyFloat_AS_DOUBLE(th.p), scale.p, b, S, H, L.p, R.p)) { PyErr_Clear(); return false; }
+      row_ptr = *tr; cols = *tc;
+      d = t.d;
+      d.csr_row_ptr = (decltype(d.csr_row_ptr))row_ptr.data_ptr();
+      d.csr_cols = cols.numel() ? (decltype(d.csr_cols))cols.data_ptr() : nullptr;
+      d.csr_vals = vals.numel() ? (decltype(d.csr_vals))vals.data_ptr() : nullptr;
+      restore_first = true;
+      return true;
+    }
+    const int64_t g = attr_i64(c, s_group, &ok);
+    Ref sc(PyObject_GetAttr(c, s_scales)), pl(PyObject_GetAttr(c, s_plan));
+    const Tensor* tc = sc.p ? plain(sc.p) : nullptr;
+    Plan p;
+    if (!ok || !tc || !pl.p || !get_plan(pl.p, H, ts->device(), &p)) { PyErr_Clear(); return false; }
+    scales = *tc;
+    p.describe(b, g, &d);
+    return true;
+  }
+  // the dense x_hat [M, H]
+  bool restore(Tensor* x) const {
+    *x = empty_like_on(stored, {M, H}, BF16);
+    const bool thr = restore_first;
+    return hyc_decompress(stored.data_ptr(), thr ? nullptr : values(), thr ? nullptr : group_scales(), M, H, &d, x->data_ptr(), stream()) == 0;
+  }
+  // from here on `stored` is the restored matrix itself
+  bool make_dense() {
+    Tensor x;
+    if (!restore(&x)) return false;
+    stored = x;
+    vals = Tensor();
+    scales = Tensor();
+    std::memset(&d, 0, sizeof d);
+    d.mode = HYC_MODE_DENSE;
+    d.bits = 4;
+    restore_first = false;
+    return true;
+  }
+  // what a consumer kernel reads: the last thing before its launch
+  bool ready() { return !restore_first || make_dense(); }
+};
+
+PyObject* none() { Py_RETURN_NONE; }
+PyObject* tuple2(PyObject* a, PyObject* b) {
+  if (!a || !b) { Py_XDECREF(a); Py_XDECREF(b); return nullptr; }
+  PyObject* t = PyTuple_New(2);
+  PyTuple_SET_ITEM(t, 0, a);
+  PyTuple_SET_ITEM(t, 1, b);
+  return t;
+}
+// the entry points' way out: a failed call goes through the interpreted form once more, which raises its error
+#define OR_NONE(call_) do { if ((call_) != 0) return none(); } while (0)
+#define ARGS(n_) do { if (nargs != (n_)) { PyErr_Format(PyExc_TypeError, "%s takes %d arguments", __func__, (n_)); return nullptr; } } while (0)
+
+// ---- compress / decompress -----------------------------------------------------------------------------------
+PyObject* compress_rows(const Tensor& x, PyObject* plan, PyObject* bits, PyObject* group) {    // nullptr without an error: not the plain case
+  int64_t M, H, pitch;
+  if (x.scalar_type() != BF16 || !spaced_rows(x, &M, &H, &pitch)) return nullptr;
+  Out o;
+  if (!o.init(plan, bits, group, M, H, x.device())) return nullptr;
+  if (hyc_compress_rows(x.data_ptr(), pitch, M, H, &o.d, o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(), nullptr, stream()) != 0) return nullptr;
+  return o.wrap();
+}
+PyObject* none_if_plain(PyObject* r) { return r || PyErr_Occurred() ? r : none(); }
+
+// compress(x [M, H], plan, bits, group) -> ChannelCompressed
+PyObject* compress(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(4);
+  const Tensor* x = bf16(a[0]);
+  return x && x->dim() == 2 ? none_if_plain(compress_rows(*x, a[1], a[2], a[3])) : none();
+  END_HANDLE_TH_ERRORS
+}
+bool restore(PyObject* c, Tensor* x) {
+  In in;
+  return in.init(c) && in.restore(x);
+}
+// decompress(c) -> bf16 [M, H]; c of either scheme
+PyObject* decompress(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(1);
+  Tensor x;
+  return restore(a[0], &x) ? THPVariable_Wrap(x) : none();
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- norms -----------------------------------------------------------------------------------------------------
+bool norm_weight(PyObject* o, int64_t H, const Tensor** w, int* dtype) {
+  *w = plain(o);
+  if (!*w || !(*w)->is_contiguous() || (*w)->numel() != H) return false;
+  if ((*w)->scalar_type() == at::kFloat) *dtype = HYC_DTYPE_F32;
+  else if ((*w)->scalar_type() == BF16) *dtype = HYC_DTYPE_BF16;
+  else return false;
+  return true;
+}
+// norm_fwd(x [..., H], w, bias or None, layer_norm, eps, plan, bits, group) -> (y like x, mean or None, rstd, ChannelCompressed)
+PyObject* norm_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(8);
+  const Tensor *x = bf16(a[0]), *w, *bias = nullptr;
+  int64_t M, H;
+  int dtype;
+  if (!x || !rows_of(*x, &M, &H) || !norm_weight(a[1], H, &w, &dtype)) return none();
+  if (a[2] != Py_None) {
+    bias = plain(a[2]);
+    if (!bias || !bias->is_contiguous() || bias->numel() != H || bias->scalar_type() != w->scalar_type()) return none();
+  }
+  const bool ln = a[3] == Py_True;
+  const double eps = PyFloat_AsDouble(a[4]);
+  if (PyErr_Occurred()) return nullptr;
+  Out o;
+  if (!o.init(a[5], a[6], a[7], M, H, x->device())) return none();
+  Tensor y = at::empty(x->sizes(), x->options()), rstd = empty_like_on(*x, {M}, at::kFloat), mean;
+  if (ln) {
+    mean = empty_like_on(*x, {M}, at::kFloat);
+    OR_NONE(hyc_layernorm_fwd_compress(x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, dtype, (float)eps, M, H, &o.d, y.data_ptr(),
+                                       (float*)mean.data_ptr(), (float*)rstd.data_ptr(), o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(),
+                                       nullptr, stream()));
+  } else {
+    OR_NONE(hyc_rmsnorm_fwd_compress(x->data_ptr(), w->data_ptr(), dtype, (float)eps, M, H, &o.d, y.data_ptr(), (float*)rstd.data_ptr(),
+                                     o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(), nullptr, stream()));
+  }
+  PyObject* c = o.wrap();
+  if (!c) return nullptr;
+  PyObject* t = PyTuple_New(4);
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(y));
+  PyTuple_SET_ITEM(t, 1, ln ? THPVariable_Wrap(mean) : none());
+  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(rstd));
+  PyTuple_SET_ITEM(t, 3, c);
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+// norm_bwd(dy [..., H], c, w, mean or None, rstd, quirk) -> (dx like dy, dw in w's dtype)
+PyObject* norm_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(6);
+  const Tensor *dy = bf16(a[0]), *w, *mean = nullptr, *rstd = plain(a[4]);
+  int64_t M, H;
+  int dtype;
+  In in;
+  if (!dy || !rows_of(*dy, &M, &H) || !norm_weight(a[2], H, &w, &dtype) || !in.init(a[1]) || in.M != M || in.H != H) return none();
+  auto stats = [&](const Tensor* t) { return t && t->scalar_type() == at::kFloat && t->is_contiguous() && t->numel() == M; };
+  if (!stats(rstd)) return none();
+  if (a[3] != Py_None) {
+    mean = plain(a[3]);
+    if (!stats(mean)) return none();
+  }
+  if (!in.ready()) return none();
+  const int64_t P = hyc_rmsnorm_bwd_partials(M, H);
+  Tensor partials = empty_like_on(*dy, {P > 1 ? P : 1, H}, at::kFloat), dx = at::empty(dy->sizes(), dy->options()),
+         dw = empty_like_on(*dy, {H}, w->scalar_type());
+  if (mean)
+    OR_NONE(hyc_layernorm_bwd(dy->data_ptr(), in.codes(), in.values(), in.group_scales(), w->data_ptr(), dtype,
+                              (const float*)mean->data_ptr(), (const float*)rstd->data_ptr(), M, H, &in.d, dx.data_ptr(), (float*)partials.data_ptr(),
+                              dw.data_ptr(), stream()));
+  else
+    OR_NONE(hyc_rmsnorm_bwd(dy->data_ptr(), in.codes(), in.values(), in.group_scales(), w->data_ptr(), dtype,
+                            (const float*)rstd->data_ptr(), M, H, &in.d, a[5] == Py_True, dx.data_ptr(), (float*)partials.data_ptr(), dw.data_ptr(),
+                            stream()));
+  return tuple2(THPVariable_Wrap(dx), THPVariable_Wrap(dw));
+  END_HANDLE_TH_ERRORS
+}
+// bias_grad(dy [..., H], fp32) -> db [H]
+PyObject* bias_grad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(2);
+  const Tensor* dy = bf16(a[0]);
+  int64_t M, H;
+  if (!dy || !rows_of(*dy, &M, &H)) return none();
+  const bool f32 = a[1] == Py_True;
+  const int64_t P = hyc_bias_grad_partials(M, H);
+  Tensor partials = empty_like_on(*dy, {P > 1 ? P : 1, H}, at::kFloat), db = empty_like_on(*dy, {H}, f32 ? at::kFloat : BF16);
+  OR_NONE(hyc_bias_grad(dy->data_ptr(), M, H, (float*)partials.data_ptr(), db.data_ptr(), f32 ? HYC_DTYPE_F32 : HYC_DTYPE_BF16, stream()));
+  return THPVariable_Wrap(db);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- the threshold scheme and kept probabilities: side data sized ahead of time ------------------------------------------
+struct Csr {
+  Tensor row_ptr, cols, vals, total;
+  // offsets of the counts, cut off at `cap` entries, and room for them
+  bool offsets(const Tensor& counts, int64_t rows, int64_t cap) {
+    row_ptr = empty_like_on(counts, {rows + 1}, at::kInt);
+    total = empty_like_on(counts, {}, at::kLong);
+    cols = empty_like_on(counts, {cap}, at::kInt);
+    vals = empty_like_on(counts, {cap}, BF16);
+    return hyc_csr_offsets((const int32_t*)counts.data_ptr(), rows, cap, (int32_t*)row_ptr.data_ptr(), (int64_t*)total.data_ptr(), stream()) == 0;
+  }
+  int32_t* rp() const { return (int32_t*)row_ptr.data_ptr(); }
+  int32_t* co() const { return (int32_t*)cols.data_ptr(); }
+};
+PyObject* wrap_all(std::initializer_list<Tensor> ts) {
+  PyObject* t = PyTuple_New((Py_ssize_t)ts.size());
+  Py_ssize_t i = 0;
+  for (const Tensor& x : ts) PyTuple_SET_ITEM(t, i++, x.defined() ? THPVariable_Wrap(x) : none());
+  return t;
+}
+// threshold_fwd(x [..., H], norm, w or None, bias or None, eps, S, threshold, scale, bits, L or None, R or None, cap)
+//   -> (y like x or None, mean or None, rstd or None, stored, row_ptr, cols, vals, total); norm: 0 compress only, 1 rms, 2 layer
+PyObject* threshold_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(12);
+  const Tensor *x = bf16(a[0]), *w = nullptr, *bias = nullptr;
+  const long norm = PyLong_AsLong(a[1]);
+  const double eps = PyFloat_AsDouble(a[4]), thr = PyFloat_AsDouble(a[6]);
+  const int64_t S = PyLong_AsLongLong(a[5]), bits = PyLong_AsLongLong(a[8]), cap = PyLong_AsLongLong(a[11]);
+  if (PyErr_Occurred()) return nullptr;
+  int64_t M, H;
+  int dtype = 0;
+  Threshold t;
+  if (!x || !rows_of(*x, &M, &H) || M == 0 || cap <= 0 || hyc_check_shape(H, (int32_t)bits, 0, HYC_MODE_THRESHOLD) != 0 ||
+      !t.init(thr, a[7], bits, S, H, a[9], a[10]) || (norm && !norm_weight(a[2], H, &w, &dtype)))
+    return none();
+  if (norm == 2 && a[3] != Py_None) {
+    bias = plain(a[3]);
+    if (!bias || !bias->is_contiguous() || bias->numel() != H || bias->scalar_type() != w->scalar_type()) return none();
+  }
+  Tensor y, mean, rstd, stored = empty_like_on(*x, {M, H * bits / 8}, bits == 8 ? at::kChar : at::kByte), counts = empty_like_on(*x, {M}, at::kInt);
+  if (norm) {
+    y = at::empty(x->sizes(), x->options());
+    rstd = empty_like_on(*x, {M}, at::kFloat);
+  }
+  if (norm == 2) mean = empty_like_on(*x, {M}, at::kFloat);
+  int32_t* n = (int32_t*)counts.data_ptr();
+  if (norm == 2)
+    OR_NONE(hyc_layernorm_fwd_compress(x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, dtype, (float)eps, M, H, &t.d, y.data_ptr(),
+                                       (float*)mean.data_ptr(), (float*)rstd.data_ptr(), stored.data_ptr(), nullptr, nullptr, n, stream()));
+  else if (norm)
+    OR_NONE(hyc_rmsnorm_fwd_compress(x->data_ptr(), w->data_ptr(), dtype, (float)eps, M, H, &t.d, y.data_ptr(), (float*)rstd.data_ptr(),
+                                     stored.data_ptr(), nullptr, nullptr, n, stream()));
+  else
+    OR_NONE(hyc_compress(x->data_ptr(), M, H, &t.d, stored.data_ptr(), nullptr, nullptr, n, stream()));
+  Csr csr;
+  if (!csr.offsets(counts, M, cap)) return none();
+  OR_NONE(hyc_ref_outlier_fill(x->data_ptr(), M, H, &t.d, csr.rp(), csr.co(), csr.vals.data_ptr(), stream()));
+  return wrap_all({y, mean, rstd, stored, csr.row_ptr, csr.cols, csr.vals, csr.total});
+  END_HANDLE_TH_ERRORS
+}
+// softmax_fwd(x [..., N], threshold, slab entries per row, cap) -> (y, row_ptr, cols, vals, total)
+PyObject* softmax_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(4);
+  const Tensor* x = bf16(a[0]);
+  const double thr = PyFloat_AsDouble(a[1]);
+  const int64_t slab_cap = PyLong_AsLongLong(a[2]), cap = PyLong_AsLongLong(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  int64_t M, N;
+  if (!x || !rows_of(*x, &M, &N) || M == 0 || slab_cap <= 0 || cap <= 0) return none();
+  Tensor y = at::empty(x->sizes(), x->options()), counts = empty_like_on(*x, {M}, at::kInt), slab = empty_like_on(*x, {M, slab_cap}, at::kInt);
+  OR_NONE(hyc_softmax_fwd_slab(x->data_ptr(), M, N, 0, (float)thr, y.data_ptr(), (int32_t*)counts.data_ptr(), (uint32_t*)slab.data_ptr(), slab_cap, stream()));
+  Csr csr;
+  if (!csr.offsets(counts, M, cap)) return none();
+  OR_NONE(hyc_softmax_fill_slab(y.data_ptr(), M, N, (float)thr, (const int32_t*)counts.data_ptr(), (const uint32_t*)slab.data_ptr(), slab_cap, csr.rp(),
+                                csr.co(), csr.vals.data_ptr(), stream()));
+  return wrap_all({y, csr.row_ptr, csr.cols, csr.vals, csr.total});
+  END_HANDLE_TH_ERRORS
+}
+struct Sparse {                                                        // kernels.SparseRows about to be read
+  Tensor row_ptr, cols, vals;
+  bool init(PyObject* o) {
+    if ((PyObject*)Py_TYPE(o) != t_sparse) return false;
+    Ref r(PyObject_GetAttr(o, s_row_ptr)), c(PyObject_GetAttr(o, s_cols)), v(PyObject_GetAttr(o, s_vals));
+    const Tensor *tr = attr_vec(r, at::kInt), *tc = attr_vec(c, at::kInt), *tv = attr_vec(v, BF16);
+    if (!tr || !tc || !tv || tc->numel() == 0 || tc->numel() != tv->numel()) return false;
+    row_ptr = *tr; cols = *tc; vals = *tv;
+    return true;
+  }
+  int64_t rows() const { return row_ptr.numel() - 1; }
+};
+// softmax_bwd(g [..., N], kept) -> dx like g; the kept entries' row length is the caller's to check
+PyObject* softmax_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(2);
+  const Tensor* g = bf16(a[0]);
+  int64_t M, N;
+  Sparse sp;
+  if (!g || !rows_of(*g, &M, &N) || M == 0 || !sp.init(a[1]) || sp.rows() != M) return none();
+  Tensor dx = at::empty(g->sizes(), g->options());
+  OR_NONE(hyc_softmax_bwd(g->data_ptr(), M, N, (const int32_t*)sp.row_ptr.data_ptr(), (const int32_t*)sp.cols.data_ptr(), sp.vals.data_ptr(),
+                          dx.data_ptr(), stream()));
+  return THPVariable_Wrap(dx);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- weight gradient, linear layer -------------------------------------------------------------------------------
+// dW [N, H] = dy^T x_hat from rows of dy `pitch` apart; staged: through a restored x_hat
+bool weight_grad(const void* dy, int64_t pitch, int64_t M, int64_t N, const Tensor& like, PyObject* c, bool f32, bool staged, Tensor* out) {
+  In in;
+  if (!in.init(c) || in.M != M || !(staged ? in.make_dense() : in.ready())) return false;
+  *out = empty_like_on(like, {N, in.H}, f32 ? at::kFloat : BF16);
+  const int64_t bytes = hyc_gradw_workspace_bytes(M, N, in.H);
+  Tensor ws;
+  if (bytes) ws = empty_like_on(like, {bytes / 4}, at::kFloat);
+  return hyc_gradw_gemm(dy, M > 1 ? pitch : N, in.codes(), in.values(), in.group_scales(), M, N, in.H, &in.d, 1.f, 0.f, out->data_ptr(),
+                        f32 ? HYC_DTYPE_F32 : HYC_DTYPE_BF16, bytes ? ws.data_ptr() : nullptr, stream()) == 0;
+}
+// gradw(dy [M, N], c, fp32, staged) -> dW [N, H]
+PyObject* gradw(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(4);
+  const Tensor* dy = bf16(a[0]);
+  int64_t M, N, pitch;
+  Tensor out;
+  if (!dy || dy->dim() != 2 || !spaced_rows(*dy, &M, &N, &pitch) ||
+      !weight_grad(dy->data_ptr(), pitch, M, N, *dy, a[1], a[2] == Py_True, a[3] == Py_True, &out)) return none();
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+// sizes of x with another last one
+std::vector<int64_t> with_last(const Tensor& x, int64_t n) {
+  std::vector<int64_t> s = x.sizes().vec();
+  s.back() = n;
+  return s;
+}
+// linear_fwd(x [..., K], w [N, K], plan or None, bits, group) -> (x w^T, ChannelCompressed or None)
+PyObject* linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(5);
+  const Tensor *x = bf16(a[0]), *w = bf16(a[1]);
+  int64_t M, K;
+  if (!x || !w || x->dim() < 2 || w->dim() != 2 || x->numel() == 0 || !rows_of(*x, &M, &K) || w->size(1) != K) return none();
+  PyObject* c = Py_None;
+  if (a[2] == Py_None) Py_INCREF(c);
+  else if (!(c = compress_rows(*x, a[2], a[3], a[4]))) return none_if_plain(nullptr);
+  Ref hold(c);
+  Tensor y = at::mm(x->view({M, K}), w->t()).view(with_last(*x, w->size(0)));
+  Py_INCREF(c);
+  return tuple2(THPVariable_Wrap(y), c);
+  END_HANDLE_TH_ERRORS
+}
+// linear_bwd(g [..., N], w [N, K], c or None, need_x, staged) -> (g w or None, dW bf16 or None)
+PyObject* linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(5);
+  const Tensor *g = bf16(a[0]), *w = bf16(a[1]);
+  int64_t M, N;
+  if (!g || !w || g->dim() < 2 || w->dim() != 2 || g->numel() == 0 || !rows_of(*g, &M, &N) || w->size(0) != N || c10::GradMode::is_enabled())
+    return none();
+  Tensor dw, dx;
+  if (a[2] != Py_None && !weight_grad(g->data_ptr(), N, M, N, *g, a[2], false, a[4] == Py_True, &dw)) return none();
+  if (a[3] == Py_True) dx = at::mm(g->view({M, N}), *w).view(with_last(*g, w->size(1)));
+  return tuple2(dx.defined() ? THPVariable_Wrap(dx) : none(), dw.defined() ? THPVariable_Wrap(dw) : none());
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- activations ---------------------------------------------------------------------------------------------------
+// act_fwd(code, x [..., H], plan, bits, group) -> (y like x, ChannelCompressed)
+PyObject* act_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(5);
+  const Tensor* x = bf16(a[1]);
+  int64_t M, H;
+  Out o;
+  if (!x || !rows_of(*x, &M, &H) || !o.init(a[2], a[3], a[4], M, H, x->device())) return none();
+  Tensor y = at::empty(x->sizes(), x->options());
+  OR_NONE(hyc_act_fwd_compress((int32_t)PyLong_AsLong(a[0]), x->data_ptr(), H, M, H, &o.d, y.data_ptr(), o.stored.data_ptr(), o.vals.data_ptr(),
+                               o.scales.data_ptr(), stream()));
+  return tuple2(THPVariable_Wrap(y), o.wrap());
+  END_HANDLE_TH_ERRORS
+}
+// act_bwd(code, g [..., H], c) -> dx like g
+PyObject* act_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(3);
+  const Tensor* g = bf16(a[1]);
+  int64_t M, H;
+  In in;
+  if (!g || !rows_of(*g, &M, &H) || !in.init(a[2]) || in.M != M || in.H != H || !in.ready()) return none();
+  Tensor dx = at::empty(g->sizes(), g->options());
+  OR_NONE(hyc_act_bwd((int32_t)PyLong_AsLong(a[0]), g->data_ptr(), in.codes(), in.values(), in.group_scales(), M, H, &in.d,
+                      dx.data_ptr(), stream()));
+  return THPVariable_Wrap(dx);
+  END_HANDLE_TH_ERRORS
+}
+// gated_fwd(code, gate [..., H], up, plan_act, plan_up, plan_gate, bits, group) -> (h [..., H], (c_act, c_up, c_gate))
+PyObject* gated_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(8);
+  const Tensor *gate = bf16(a[1]), *up = bf16(a[2]);
+  int64_t M, H, pg, M2, H2, pu;
+  if (!gate || !up || gate->sizes() != up->sizes() || !spaced_rows(*gate, &M, &H, &pg) || !spaced_rows(*up, &M2, &H2, &pu)) return none();
+  Out o[3];
+  for (int i = 0; i < 3; ++i)
+    if (!o[i].init(a[3 + i], a[6], a[7], M, H, gate->device())) return none();
+  Tensor h = at::empty(gate->sizes(), gate->options());
+  OR_NONE(hyc_gated_act_fwd((int32_t)PyLong_AsLong(a[0]), gate->data_ptr(), pg, up->data_ptr(), pu, M, H, &o[0].d, &o[1].d, &o[2].d, h.data_ptr(),
+                            o[0].stored.data_ptr(), o[0].vals.data_ptr(), o[0].scales.data_ptr(), o[1].stored.data_ptr(), o[1].vals.data_ptr(),
+                            o[1].scales.data_ptr(), o[2].stored.data_ptr(), o[2].vals.data_ptr(), o[2].scales.data_ptr(), stream()));
+  PyObject* cs = PyTuple_New(3);
+  for (int i = 0; i < 3; ++i) {
+    PyObject* c = o[i].wrap();
+    if (!c) { Py_DECREF(cs); return nullptr; }
+    PyTuple_SET_ITEM(cs, i, c);
+  }
+  return tuple2(THPVariable_Wrap(h), cs);
+  END_HANDLE_TH_ERRORS
+}
+// `n` matrices of [lead..., H] side by side in one [M, n H + room], or on their own (room < 0)
+void side_by_side(const Tensor& like, int64_t n, int64_t M, int64_t H, int64_t room, Tensor* both, std::vector<Tensor>* parts, int64_t* pitch) {
+  if (room < 0) {
+    for (int64_t i = 0; i < n; ++i) parts->push_back(at::empty(with_last(like, H), like.options()));
+    *pitch = H;
+    return;
+  }
+  *pitch = n * H + room;
+  *both = empty_like_on(like, {M, *pitch}, BF16);
+  const auto lead = like.sizes().slice(0, like.dim() - 1);
+  for (int64_t i = 0; i < n; ++i) parts->push_back(both->narrow(1, i * H, H).unflatten(0, lead));
+}
+PyObject* wrap_parts(const std::vector<Tensor>& parts, const Tensor& both) {
+  PyObject* t = PyTuple_New((Py_ssize_t)parts.size() + 1);
+  for (size_t i = 0; i < parts.size(); ++i) PyTuple_SET_ITEM(t, (Py_ssize_t)i, THPVariable_Wrap(parts[i]));
+  PyTuple_SET_ITEM(t, (Py_ssize_t)parts.size(), both.defined() ? THPVariable_Wrap(both) : none());
+  return t;
+}
+int64_t room_of(PyObject* o) { return o == Py_None ? -1 : PyLong_AsLongLong(o); }
+// gated_bwd(code, g [..., H], c_act, c_up, c_gate, room or None) -> (d_gate, d_up, their common matrix or None)
+PyObject* gated_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(6);
+  const Tensor* g = bf16(a[1]);
+  int64_t M, H, pitch;
+  In in[3];
+  if (!g || g->dim() < 2 || !rows_of(*g, &M, &H)) return none();
+  for (int i = 0; i < 3; ++i)
+    if (!in[i].init(a[2 + i]) || in[i].M != M || in[i].H != H || in[i].restore_first) return none();
+  Tensor both;
+  std::vector<Tensor> d;
+  side_by_side(*g, 2, M, H, room_of(a[5]), &both, &d, &pitch);
+  OR_NONE(hyc_gated_act_bwd_rows((int32_t)PyLong_AsLong(a[0]), g->data_ptr(), in[0].codes(), in[0].values(), in[0].group_scales(),
+                                 &in[0].d, in[1].codes(), in[1].values(), in[1].group_scales(), &in[1].d, in[2].codes(),
+                                 in[2].values(), in[2].group_scales(), &in[2].d, M, H, d[0].data_ptr(), pitch, d[1].data_ptr(), pitch, stream()));
+  return wrap_parts(d, both);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- LoRA groups -------------------------------------------------------------------------------------------------------
+struct Factors {                                                       // a group's A (or B): bf16 [rows_i, cols_i], as the kernels read them
+  int n = 0;
+  const void* p[4];
+  std::vector<const Tensor*> t;
+  bool init(PyObject* seq, const Tensor& like) {
+    if (!PyTuple_CheckExact(seq) || PyTuple_GET_SIZE(seq) < 1 || PyTuple_GET_SIZE(seq) > 4) return false;
+    n = (int)PyTuple_GET_SIZE(seq);
+    for (int i = 0; i < n; ++i) {
+      const Tensor* f = bf16(PyTuple_GET_ITEM(seq, i));
+      if (!f || f->dim() != 2 || !f->is_contiguous() || !aligned16(f->data_ptr()) || f->device() != like.device()) return false;
+      p[i] = f->data_ptr();
+      t.push_back(f);
+    }
+    return true;
+  }
+  bool shaped(int i, int64_t rows, int64_t cols) const { return t[i]->size(0) == rows && t[i]->size(1) == cols; }
+};
+bool widths(PyObject* seq, int n, int64_t* outs, int64_t* total) {
+  if (!PyTuple_CheckExact(seq) || PyTuple_GET_SIZE(seq) != n) return false;
+  *total = 0;
+  for (int i = 0; i < n; ++i) {
+    outs[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(seq, i));
+    if (outs[i] <= 0 || outs[i] % 8) return false;
+    *total += outs[i];
+  }
+  return true;
+}
+bool base_weight(PyObject* packed, PyObject* absmax, const Tensor& like, int64_t n, const Tensor** p, const Tensor** m) {
+  *p = plain(packed);
+  *m = plain(absmax);
+  return *p && *m && (*p)->scalar_type() == at::kByte && (*m)->scalar_type() == at::kFloat && (*p)->is_contiguous() && (*m)->is_contiguous() &&
+         (*p)->numel() * 2 == n && (*m)->numel() * 64 == n && (*p)->device() == like.device() && (*m)->device() == like.device();
+}
+// out [M, N] (+)= a b^T in one product, or in two at column `cut`
+void product(const Tensor& out, const Tensor& a, const Tensor& b, int64_t cut, bool accumulate) {
+  const int64_t N = out.size(1), lo[2] = {0, cut}, hi[2] = {cut ? cut : N, N};
+  for (int i = 0; i < (cut ? 2 : 1); ++i) {
+    Tensor part = out.narrow(1, lo[i], hi[i] - lo[i]), bt = b.narrow(0, lo[i], hi[i] - lo[i]).t();
+    if (accumulate) part.addmm_(a, bt);
+    else at::mm_out(part, a, bt);
+  }
+}
+// lora_forward(x [..., K], (A_i), (B_i), scale, (out_i), packed, absmax, cut, plan or None, bits, group)
+//   -> ((y_i [..., out_i]), h [M, n r], ChannelCompressed of x or None); the kernels' ranks and sizes are the caller's to check
+PyObject* lora_forward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(11);
+  const Tensor *x = bf16(a[0]), *packed, *absmax;
+  int64_t M, K, outs[4], total;
+  Factors A, B;
+  if (!x || x->dim() < 2 || x->numel() == 0 || !rows_of(*x, &M, &K) || !aligned16(x->data_ptr()) || !A.init(a[1], *x) || !B.init(a[2], *x) || A.n != B.n ||
+      !widths(a[4], A.n, outs, &total) || !base_weight(a[5], a[6], *x, total * K, &packed, &absmax) || c10::GradMode::is_enabled())
+    return none();
+  const int64_t r = A.t[0]->size(0);
+  for (int i = 0; i < A.n; ++i)
+    if (!A.shaped(i, r, K) || !B.shaped(i, outs[i], r)) return none();
+  const double scale = PyFloat_AsDouble(a[3]);
+  const int64_t cut = PyLong_AsLongLong(a[7]);
+  if (PyErr_Occurred()) return nullptr;
+  Tensor x2 = x->view({M, K}), h = empty_like_on(*x, {M, A.n * r}, BF16), y = empty_like_on(*x, {M, total}, BF16), w = empty_like_on(*x, {total, K}, BF16);
+  OR_NONE(hyc_lora_down(x->data_ptr(), K, M, K, A.p, A.n, (int32_t)r, h.data_ptr(), stream()));
+  OR_NONE(hyc_lora_up(h.data_ptr(), M, B.p, outs, B.n, (int32_t)r, (float)scale, y.data_ptr(), stream()));
+  OR_NONE(hyc_nf4_dequantize(packed->data_ptr(), (const float*)absmax->data_ptr(), total * K, w.data_ptr(), stream()));
+  product(y, x2, w, cut, true);
+  PyObject* c = Py_None;
+  if (a[8] == Py_None) Py_INCREF(c);
+  else if (!(c = compress_rows(x2, a[8], a[9], a[10]))) return none_if_plain(nullptr);
+  const auto lead = x->sizes().slice(0, x->dim() - 1);
+  PyObject* ys = PyTuple_New(A.n);
+  int64_t col = 0;
+  for (int i = 0; i < A.n; ++i) {
+    PyTuple_SET_ITEM(ys, i, THPVariable_Wrap(y.narrow(1, col, outs[i]).unflatten(0, lead)));
+    col += outs[i];
+  }
+  PyObject* t = PyTuple_New(3);
+  PyTuple_SET_ITEM(t, 0, ys);
+  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(h));
+  PyTuple_SET_ITEM(t, 2, c);
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+// lora_backward((g_i [..., out_i]), (A_i), (B_i), h, scale, (out_i), room, rows or None, packed, absmax, c, cut)
+//   -> (dx [..., K], dA_0, ..., dB_0, ...); rows: the [M, total + room] matrix whose first columns the g_i are
+PyObject* lora_backward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(12);
+  const Tensor *h = bf16(a[3]), *packed, *absmax;
+  Factors A, B;
+  int64_t outs[4], total, M = -1, pitches[4];
+  if (!h || !h->is_contiguous() || h->dim() != 2 || !A.init(a[1], *h) || !B.init(a[2], *h) || A.n != B.n || !widths(a[5], A.n, outs, &total) ||
+      !PyTuple_CheckExact(a[0]) || PyTuple_GET_SIZE(a[0]) != A.n || c10::GradMode::is_enabled())
+    return none();
+  const int n = A.n;
+  const int64_t r = A.t[0]->size(0), K = A.t[0]->size(1), room = PyLong_AsLongLong(a[6]), cut = PyLong_AsLongLong(a[11]);
+  const double scale = PyFloat_AsDouble(a[4]);
+  if (PyErr_Occurred()) return nullptr;
+  const void* dy[4];
+  const Tensor* g0 = nullptr;
+  for (int i = 0; i < n; ++i) {
+    const Tensor* g = bf16(PyTuple_GET_ITEM(a[0], i));
+    int64_t m, w;
+    if (!g || g->device() != h->device() || !kernel_rows(*g, &m, &w, &pitches[i]) || w != outs[i] || (M >= 0 && m != M) || !A.shaped(i, r, K) ||
+        !B.shaped(i, outs[i], r))
+      return none();
+    M = m;
+    dy[i] = g->data_ptr();
+    if (!i) g0 = g;
+    const int64_t range = (M < 32768 ? M : 32768) + 63;
+    if (range / 64 * 64 * pitches[i] >= ((int64_t)1 << 30)) return none();
+  }
+  if (h->size(0) != M || h->size(1) != n * r || room < n * r || !base_weight(a[8], a[9], *h, total * K, &packed, &absmax)) return none();
+  Tensor ext;
+  const bool copy = a[7] == Py_None;
+  if (copy) {
+    ext = empty_like_on(*h, {M, total + room}, BF16);
+  } else {
+    const Tensor* e = bf16(a[7]);
+    if (!e || !e->is_contiguous() || e->dim() != 2 || e->size(0) != M || e->size(1) != total + room || e->device() != h->device()) return none();
+    ext = *e;
+  }
+  In in;
+  if (!in.init(a[10]) || in.M != M || in.H != K || in.restore_first) return none();
+  Tensor dh = empty_like_on(*h, {M, n * r}, BF16), ws = empty_like_on(*h, {hyc_lora_up_bwd_workspace_bytes(M, outs, n, (int32_t)r) / 4}, at::kFloat);
+  std::vector<Tensor> dB;
+  void* pB[4];
+  for (int i = 0; i < n; ++i) {
+    dB.push_back(at::empty(B.t[i]->sizes(), B.t[i]->options()));
+    pB[i] = dB[i].data_ptr();
+  }
+  OR_NONE(hyc_lora_up_bwd(dy, pitches, M, outs, B.p, h->data_ptr(), n, (int32_t)r, (float)scale, dh.data_ptr(), ext.data_ptr(), total + room, room, copy ? 1 : 0, pB,
+                          ws.data_ptr(), stream()));
+  // the dh of a group go through the weight gradient side by side, 32 rows of dA a call
+  std::vector<Tensor> dA;
+  const int64_t per_call = (32 / r > 1 ? 32 / r : 1) * r;
+  for (int64_t c0 = 0; c0 < n * r; c0 += per_call) {
+    const int64_t cols = c0 + per_call <= n * r ? per_call : n * r - c0;
+    Tensor block;
+    if (!weight_grad((const char*)dh.data_ptr() + 2 * c0, n * r, M, cols, dh, a[10], false, false, &block)) return none();
+    for (int64_t j = 0; j < cols; j += r) dA.push_back(block.narrow(0, j, r));
+  }
+  Tensor wt = empty_like_on(*h, {K, total + room}, BF16), dx = empty_like_on(*h, {M, K}, BF16);
+  OR_NONE(hyc_lora_weight_t(packed->data_ptr(), (const float*)absmax->data_ptr(), K, A.p, outs, n, (int32_t)r, room, wt.data_ptr(), stream()));
+  product(dx, ext, wt, cut, false);
+  PyObject* t = PyTuple_New(1 + 2 * n);
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(dx.view(with_last(*g0, K))));
+  for (int i = 0; i < n; ++i) {
+    PyTuple_SET_ITEM(t, 1 + i, THPVariable_Wrap(dA[i]));
+    PyTuple_SET_ITEM(t, 1 + n + i, THPVariable_Wrap(dB[i]));
+  }
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- attention -----------------------------------------------------------------------------------------------------------
+struct Tokens {                                                        // bf16 [B, S, H], contiguous channels, evenly spaced tokens
+  const Tensor* t;
+  int64_t B, S, H, pitch;
+  bool init(PyObject* o) {
+    t = bf16(o);
+    if (!t || t->dim() != 3 || t->numel() == 0 || t->stride(2) != 1) return false;
+    B = t->size(0); S = t->size(1); H = t->size(2);
+    pitch = S > 1 ? t->stride(1) : (B > 1 ? t->stride(0) : H);
+    return B == 1 || t->stride(0) == S * pitch;
+  }
+  bool same(const Tokens& o) const { return B == o.B && S == o.S && H == o.H; }
+};
+bool tables(PyObject* cosv, PyObject* sinv, int64_t n, const Tensor** c, const Tensor** s) {
+  *c = bf16(cosv);
+  *s = bf16(sinv);
+  return *c && *s && (*c)->is_contiguous() && (*s)->is_contiguous() && (*c)->numel() == n && (*s)->numel() == n;
+}
+// rope_attn_fwd(q, k, v, heads, cos, sin, scale, round_scores) -> (q rows, k rows, out, lse): q and k rotated, and attention on them
+PyObject* rope_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(8);
+  Tokens q, k, v;
+  const Tensor *cosv, *sinv;
+  const int64_t heads = PyLong_AsLongLong(a[3]);
+  const double scale = PyFloat_AsDouble(a[6]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!q.init(a[0]) || !k.init(a[1]) || !v.init(a[2]) || !q.same(k) || !q.same(v) || heads <= 0 || q.H % heads ||
+      !tables(a[4], a[5], q.S * (q.H / heads), &cosv, &sinv))
+    return none();
+  const int64_t hd = q.H / heads;
+  const auto opt = q.t->options();
+  Tensor qr = at::empty({q.B, q.S, q.H}, opt), kr = at::empty({q.B, q.S, q.H}, opt), out = at::empty({q.B, q.S, q.H}, opt),
+         lse = empty_like_on(*q.t, {q.B, heads, q.S}, at::kFloat);
+  OR_NONE(hyc_rope_to_heads(q.t->data_ptr(), q.pitch, cosv->data_ptr(), sinv->data_ptr(), q.B, q.S, heads, hd, nullptr, qr.data_ptr(), stream()));
+  OR_NONE(hyc_rope_to_heads(k.t->data_ptr(), k.pitch, cosv->data_ptr(), sinv->data_ptr(), q.B, q.S, heads, hd, nullptr, kr.data_ptr(), stream()));
+  OR_NONE((a[7] == Py_True ? hyc_attn_kept_fwd : hyc_attn_fwd)(qr.data_ptr(), q.H, kr.data_ptr(), q.H, v.t->data_ptr(), v.pitch, q.B, q.S, heads, hd,
+                                                               (float)scale, out.data_ptr(), q.H, (float*)lse.data_ptr(), stream()));
+  PyObject* t = PyTuple_New(4);
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(qr));
+  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(kr));
+  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(out));
+  PyTuple_SET_ITEM(t, 3, THPVariable_Wrap(lse));
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+// attn_bwd(g [B, S, H], c_q, c_k, c_v, c_out, lse, heads, cos, sin, scale, room or None) -> (dq, dk, dv, their common matrix or None)
+PyObject* attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(11);
+  Tokens g;
+  const Tensor *cosv, *sinv, *lse = plain(a[5]);
+  const int64_t heads = PyLong_AsLongLong(a[6]);
+  const double scale = PyFloat_AsDouble(a[9]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!g.init(a[0]) || !g.t->is_contiguous() || heads <= 0 || g.H % heads || !tables(a[7], a[8], g.S * (g.H / heads), &cosv, &sinv) || !lse ||
+      lse->scalar_type() != at::kFloat || !lse->is_contiguous() || lse->numel() != g.B * heads * g.S)
+    return none();
+  Tensor x[4];
+  for (int i = 0; i < 4; ++i) {
+    if (!restore(a[1 + i], &x[i]) || x[i].size(0) != g.B * g.S || x[i].size(1) != g.H) return none();
+  }
+  int64_t pitch;
+  Tensor both, ws = empty_like_on(*g.t, {2 * g.B * heads * g.S}, at::kFloat);
+  std::vector<Tensor> d;
+  side_by_side(*g.t, 3, g.B * g.S, g.H, room_of(a[10]), &both, &d, &pitch);
+  OR_NONE(hyc_attn_bwd(g.t->data_ptr(), g.H, x[0].data_ptr(), g.H, x[1].data_ptr(), g.H, x[2].data_ptr(), g.H, x[3].data_ptr(), g.H,
+                       (const float*)lse->data_ptr(), cosv->data_ptr(), sinv->data_ptr(), g.B, g.S, heads, g.H / heads, (float)scale, d[0].data_ptr(),
+                       pitch, d[1].data_ptr(), pitch, d[2].data_ptr(), pitch, (float*)ws.data_ptr(), stream()));
+  return wrap_parts(d, both);
+  END_HANDLE_TH_ERRORS
+}
+
+// attn_kept(q rows [B, S, H], k rows, lse, heads, scale, threshold, slab entries per row, cap, first, matrices)
+//   -> (row_ptr, cols, vals, total) of kernels.attn_kept
+PyObject* attn_kept(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(10);
+  Tokens q, k;
+  const Tensor* lse = plain(a[2]);
+  const int64_t heads = PyLong_AsLongLong(a[3]), slab_cap = PyLong_AsLongLong(a[6]), cap = PyLong_AsLongLong(a[7]), first = PyLong_AsLongLong(a[8]),
+                matrices = PyLong_AsLongLong(a[9]);
+  const double scale = PyFloat_AsDouble(a[4]), thr = PyFloat_AsDouble(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!q.init(a[0]) || !k.init(a[1]) || !q.same(k) || heads <= 0 || q.H % heads || !lse || lse->scalar_type() != at::kFloat || !lse->is_contiguous() ||
+      lse->numel() != q.B * heads * q.S || cap <= 0 || slab_cap <= 0 || matrices <= 0)
+    return none();
+  const int64_t rows = matrices * q.S, hd = q.H / heads;
+  Tensor counts = empty_like_on(*q.t, {rows}, at::kInt), slab = empty_like_on(*q.t, {rows, slab_cap}, at::kInt);
+  int32_t* n = (int32_t*)counts.data_ptr();
+  uint32_t* sl = (uint32_t*)slab.data_ptr();
+  const float* ls = (const float*)lse->data_ptr();
+  OR_NONE(hyc_attn_kept(q.t->data_ptr(), q.pitch, k.t->data_ptr(), k.pitch, ls, q.B, q.S, heads, hd, (float)scale, (float)thr, first, matrices, n, sl, slab_cap,
+                        stream()));
+  Csr csr;
+  if (!csr.offsets(counts, rows, cap)) return none();
+  OR_NONE(hyc_attn_kept_fill(q.t->data_ptr(), q.pitch, k.t->data_ptr(), k.pitch, ls, q.B, q.S, heads, hd, (float)scale, (float)thr, first, matrices, n, sl,
+                             slab_cap, csr.rp(), csr.co(), csr.vals.data_ptr(), stream()));
+  return wrap_all({csr.row_ptr, csr.cols, csr.vals, csr.total});
+  END_HANDLE_TH_ERRORS
+}
+// attn_kept_bwd(g [B, S, H], c_q, c_k, c_v, [kept], heads, cos, sin, scale, room or None) -> (dq, dk, dv, their common matrix or None)
+PyObject* attn_kept_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(10);
+  Tokens g;
+  const Tensor *cosv, *sinv;
+  const int64_t heads = PyLong_AsLongLong(a[5]);
+  const double scale = PyFloat_AsDouble(a[8]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!g.init(a[0]) || !g.t->is_contiguous() || heads <= 0 || g.H % heads || !tables(a[6], a[7], g.S * (g.H / heads), &cosv, &sinv) || !PyList_CheckExact(a[4]))
+    return none();
+  std::vector<Sparse> kept((size_t)PyList_GET_SIZE(a[4]));
+  int64_t rows = 0;
+  for (size_t i = 0; i < kept.size(); ++i) {
+    if (!kept[i].init(PyList_GET_ITEM(a[4], (Py_ssize_t)i)) || kept[i].rows() % g.S) return none();
+    rows += kept[i].rows();
+  }
+  if (rows != g.B * heads * g.S) return none();
+  Tensor x[3];
+  for (int i = 0; i < 3; ++i)
+    if (!restore(a[1 + i], &x[i]) || x[i].size(0) != g.B * g.S || x[i].size(1) != g.H) return none();
+  int64_t pitch, first = 0;
+  Tensor both;
+  std::vector<Tensor> d;
+  side_by_side(*g.t, 3, g.B * g.S, g.H, room_of(a[9]), &both, &d, &pitch);
+  for (const Sparse& sp : kept) {
+    const int64_t matrices = sp.rows() / g.S;
+    Tensor records = empty_like_on(*g.t, {sp.cols.numel(), 2}, at::kInt);
+    OR_NONE(hyc_attn_kept_bwd(g.t->data_ptr(), g.H, x[0].data_ptr(), g.H, x[1].data_ptr(), g.H, x[2].data_ptr(), g.H, (const int32_t*)sp.row_ptr.data_ptr(),
+                              (const int32_t*)sp.cols.data_ptr(), sp.vals.data_ptr(), cosv->data_ptr(), sinv->data_ptr(), g.B, g.S, heads, g.H / heads,
+                              (float)scale, first, matrices, d[0].data_ptr(), pitch, d[1].data_ptr(), pitch, d[2].data_ptr(), pitch, records.data_ptr(),
+                              stream()));
+    first += matrices;
+  }
+  return wrap_parts(d, both);
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(Parameter, ChannelCompressed, ChannelPlan, ThresholdCompressed, SparseRows): the classes the functions above recognise
+PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  ARGS(5);
+  PyObject** to[5] = {&t_parameter, &t_compressed, &t_plan, &t_threshold, &t_sparse};
+  for (int i = 0; i < 5; ++i) {
+    Py_INCREF(a[i]);
+    Py_XDECREF(*to[i]);
+    *to[i] = a[i];
+  }
+  return none();
+}
+
+#define ENTRY(f_) {#f_, (PyCFunction)(void (*)(void))f_, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {ENTRY(bind), ENTRY(compress), ENTRY(decompress), ENTRY(norm_fwd), ENTRY(norm_bwd), ENTRY(bias_grad), ENTRY(gradw),
+                         ENTRY(linear_fwd), ENTRY(linear_bwd), ENTRY(act_fwd), ENTRY(act_bwd), ENTRY(gated_fwd), ENTRY(gated_bwd), ENTRY(lora_forward),
+                         ENTRY(lora_backward), ENTRY(rope_attn_fwd), ENTRY(attn_bwd), ENTRY(attn_kept), ENTRY(attn_kept_bwd),
+                         ENTRY(threshold_fwd), ENTRY(softmax_fwd), ENTRY(softmax_bwd), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hyc_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__hyc_host() {
+  struct { PyObject** to; const char* s; } names[] = {{&s_H, "H"}, {&s_M, "M"}, {&s_k, "k"}, {&s_idx, "idx"}, {&s_plan, "plan"},
+                                                      {&s_scale_rule, "scale_rule"}, {&s_stored, "stored"}, {&s_vals, "vals"},
+                                                      {&s_scales, "scales"}, {&s_bits, "bits"}, {&s_group, "group"},
+                                                      {&s_S, "S"}, {&s_row_ptr, "row_ptr"}, {&s_cols, "cols"}, {&s_threshold, "threshold"},
+                                                      {&s_scale, "scale"}, {&s_L, "L"}, {&s_R, "R"}};
+  for (auto& n : names) *n.to = PyUnicode_InternFromString(n.s);
+  return PyModule_Create(&module);
+}

@@ -16,6 +16,7 @@ Composite of one LoRA projection (peft `Linear.forward` around the swapped modul
     dB = s * dY^T @ h
     dA = (s * dY @ B)^T @ x_hat                 the only consumer of the compressed x (efficient_linear.py:56-67)
 """
+import functools
 import math
 from dataclasses import dataclass
 
@@ -102,6 +103,7 @@ class LoRAProjections(torch.nn.Module):
         return outs if len(self.out_features) > 1 else outs[0]
 
 
+@functools.lru_cache(maxsize=1024)
 def _cut_columns(M, N):
     """columns at which _product cuts an [M, N] result in two, 0 to leave it whole.  The library's kernels are chosen for
     256-wide tiles here, and where they do not come out even it takes ones that run at down to half the rate.  A cut behind the
@@ -172,8 +174,20 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, mod, plan, *ab):
-        n = len(mod.out_features)
+        n, cfg = len(mod.out_features), mod.cfg
         A, B = ab[:n], ab[n:]
+        if mod.record is None and (plan is not None) == cfg.compress:
+            outs, r, M = tuple(mod.out_features), A[0].shape[0], x.numel() // mod.in_features
+            if K._lora_kernels_cover(M, n, r, mod.in_features, outs):
+                done = K.native.lora_forward(x, A, B, mod.scaling, outs, mod.base_all.packed, mod.base_all.absmax,
+                                             _cut_columns(M, sum(outs)), plan, cfg.linear_bits, cfg.linear_group)
+                if done is not None:
+                    ys, ctx.h, ctx.saved_x = done
+                    if not cfg.compress:
+                        ctx.saved_x = _kernel_rows(x).contiguous()
+                    ctx.mod = mod
+                    ctx.save_for_backward(*ab)
+                    return ys
         x2 = _kernel_rows(x)
         h = K.lora_down(x2, A)
         y_all = K.lora_up(h, B, mod.scaling, mod.out_features)
@@ -182,7 +196,6 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
         for out in mod.out_features:                            # column slices: no copies, consumers take the pitch
             outs.append(y_all[:, row:row + out].unflatten(0, x.shape[:-1]))
             row += out
-        cfg = mod.cfg
         ctx.saved_x = K.compress_channel(x2, plan, cfg.linear_bits, cfg.linear_group) if cfg.compress else x2.contiguous()
         if mod.record is not None:
             mod.record["x"], mod.record["saved"] = x2.detach().clone(), ctx.saved_x
@@ -200,6 +213,14 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
             return _LoRAProjectionsFunc._backward_with_graph(ctx, A, B, gs)
         room = K.lora_room(n, r)
         rows = _room_behind(getattr(gs[0], "_hyc_rows", None), gs, total, room)
+        if not K.gradw_staged_by_default(32, mod.in_features):
+            M, outs = ctx.h.shape[0], tuple(mod.out_features)
+            if K._lora_kernels_cover(M, n, r, mod.in_features, outs):
+                done = K.native.lora_backward(gs, A, B, ctx.h, mod.scaling, outs, room, rows, mod.base_all.packed, mod.base_all.absmax,
+                                              ctx.saved_x, _cut_columns(M, mod.in_features))
+                if done is not None:
+                    ctx.h = ctx.saved_x = None
+                    return done[:1] + (None, None) + done[1:]
         ext, dh, dB = K.lora_up_bwd([_kernel_rows(g.to(BF16)) for g in gs], B, ctx.h, mod.scaling, room, rows)
         dA = _LoRAProjectionsFunc._grad_A(ctx, dh, A)
         dx = torch.empty((ext.shape[0], mod.in_features), dtype=BF16, device=ext.device)
@@ -365,8 +386,11 @@ class _AttentionFunc(torch.autograd.Function):
         b, s, H = q.shape
         nh = cfg.heads
         scale = 1.0 / math.sqrt(cfg.head_dim)
-        q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
-        out, lse = K.attn_fwd(q_rows, k_rows, v, nh, scale, round_scores=True)
+        done = K.native.rope_attn_fwd(q, k, v, nh, cos, sin, scale, True)
+        if done is None:
+            q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
+            done = (q_rows, k_rows) + K.attn_fwd(q_rows, k_rows, v, nh, scale, round_scores=True)
+        q_rows, k_rows, out, lse = done
         thr, budget = K.threshold_value(mod.static_value), K.kept_budget(mod.static_value)
         # (the slab of kept entries is what grows with the number of matrices here)
         group = max(1, min(b * nh, cfg.attn_group_bytes // (4 * s * cap)))
@@ -386,8 +410,10 @@ class _AttentionFunc(torch.autograd.Function):
         b, nh, s, hd = ctx.geom
         cos, sin = ctx.saved_tensors
         if ctx.rows:
-            qq, kk, vv = (K.decompress_channel(c).view(b, s, nh * hd) for c in ctx.saved)
-            grads = K.attn_kept_bwd(g.to(BF16).contiguous(), qq, kk, vv, ctx.kept, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
+            grads = K.native.attn_kept_bwd(g, *ctx.saved, ctx.kept, nh, cos, sin, 1.0 / math.sqrt(hd), ctx.grad_room)
+            if grads is None:
+                qq, kk, vv = (K.decompress_channel(c).view(b, s, nh * hd) for c in ctx.saved)
+                grads = K.attn_kept_bwd(g.to(BF16).contiguous(), qq, kk, vv, ctx.kept, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
             ctx.saved = ctx.kept = None
             if ctx.grad_room is not None:
                 for t in grads[:3]:
@@ -444,8 +470,11 @@ class _FlashAttentionFunc(torch.autograd.Function):
         ctx.rows = K.attn_supported(hd, s, max(v.stride(1), pitch), b * nh)
         seed = offset = None
         if ctx.rows:                                                # the kernels read and write the rows as they are
-            q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
-            out, lse = K.attn_fwd(q_rows, k_rows, v, nh, scale)
+            done = K.native.rope_attn_fwd(q, k, v, nh, cos, sin, scale, False)
+            if done is None:
+                q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
+                done = (q_rows, k_rows) + K.attn_fwd(q_rows, k_rows, v, nh, scale)
+            q_rows, k_rows, out, lse = done
             ctx.grad_room = grad_room
         else:
             qh, q_rows = K.rope_to_heads(q, nh, cos, sin, want_rows=True)
@@ -478,9 +507,11 @@ class _FlashAttentionFunc(torch.autograd.Function):
         cos, sin, lse = ctx.saved_tensors
         restore = (lambda c: K.decompress_channel(c)) if ctx.compress else (lambda c: c)
         if ctx.rows:
-            qq, kk, vv, oo = (restore(c).view(b, s, nh * hd) for c in ctx.saved)
+            grads = K.native.attn_bwd(g, *ctx.saved, lse, nh, cos, sin, 1.0 / math.sqrt(hd), ctx.grad_room) if ctx.compress else None
+            if grads is None:
+                qq, kk, vv, oo = (restore(c).view(b, s, nh * hd) for c in ctx.saved)
+                grads = K.attn_bwd(g.to(BF16).contiguous(), qq, kk, vv, oo, lse, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
             ctx.saved = None
-            grads = K.attn_bwd(g.to(BF16).contiguous(), qq, kk, vv, oo, lse, nh, 1.0 / math.sqrt(hd), cos, sin, room=ctx.grad_room)
             if ctx.grad_room is not None:
                 for t in grads[:3]:
                     t._hyc_rows = grads[3]

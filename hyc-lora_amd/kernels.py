@@ -10,7 +10,7 @@ from typing import Optional
 
 import torch
 
-from . import _abi
+from . import _abi, _host
 from ._abi import HycDesc, check
 
 BF16 = torch.bfloat16
@@ -300,6 +300,19 @@ class ChannelCompressed:
         return self.stored.numel() * self.stored.element_size() + 2 * self.vals.numel() + 2 * self.scales.numel()
 
 
+class _Native:
+    """the functions of csrc/host/host.cpp, loaded with the first one asked for (a package whose libraries are not built can be
+    imported).  Each returns None for what it does not cover, and the caller goes on with the form written out here."""
+
+    def __getattr__(self, name):
+        module = _host.load(torch.nn.Parameter, ChannelCompressed, ChannelPlan, ThresholdCompressed, SparseRows)
+        self.__dict__.update((n, f) for n, f in vars(module).items() if not n.startswith("_"))
+        return self.__dict__[name]
+
+
+native = _Native()
+
+
 def alloc_channel(M, H, plan, bits, group, device):
     if plan.H != H:
         raise ValueError("the outlier-channel plan was made for %d channels, the activation has %d" % (plan.H, H))
@@ -320,6 +333,9 @@ def _need_rows(t, name):
 
 
 def compress_channel(x2d, plan, bits, group):
+    out = native.compress(x2d, plan, bits, group)
+    if out is not None:
+        return out
     _need_rows(x2d, "x")
     M, H = x2d.shape
     lib = _abi.load()
@@ -333,6 +349,9 @@ def compress_channel(x2d, plan, bits, group):
 
 
 def decompress_channel(c: ChannelCompressed):
+    xhat = native.decompress(c)
+    if xhat is not None:
+        return xhat
     xhat = torch.empty((c.M, c.H), dtype=BF16, device=c.stored.device)
     d = c.desc()
     check(_abi.load().hyc_decompress(_p(c.stored), _p(c.vals), _p(c.scales), c.M, c.H, ctypes.byref(d), _p(xhat), _stream()))
@@ -405,10 +424,30 @@ def fit_rows(L, S):
     return out
 
 
+def threshold_native(x, norm, w, bias, eps, S, threshold, scale, bits, L, R, budget):
+    """(y, mean, rstd, ThresholdCompressed) of x [..., H] in native code (norm: 0 compress only, 1 rms norm, 2 layer norm), or None:
+    a budget that has seen nothing yet, or what the native form does not cover"""
+    if budget is None or not budget.ready or not isinstance(x, torch.Tensor) or not x.numel():
+        return None
+    H = x.shape[-1]
+    M = x.numel() // H
+    budget.poll()
+    cap = budget.capacity(M)
+    done = native.threshold_fwd(x, norm, w, bias, eps, S, threshold, scale, bits, L, R, cap)
+    if done is None:
+        return None
+    y, mean, rstd, stored, row_ptr, cols, vals, total = done
+    budget.watch(total, cap, M)
+    return y, mean, rstd, ThresholdCompressed(stored, row_ptr, cols, vals, float(threshold), scale, L, R, bits, M, H, S)
+
+
 def compress_threshold(x2d, S, threshold, scale, bits, L=None, R=None, budget=None):
     """codes + CSR outliers of x [M,H] (row m is sequence position m mod S).  One host read-back
     (the outlier total) sizes the CSR arrays, as `.to_sparse()` does in the reference; with a KeptBudget that has seen
     a call they are sized ahead of time and nothing waits."""
+    done = threshold_native(x2d, 0, None, None, 0.0, S, threshold, scale, bits, L, R, budget) if x2d.dim() == 2 else None
+    if done is not None:
+        return done[3]
     _need(x2d, BF16, "x")
     _need(scale, BF16, "scale")
     M, H = x2d.shape
@@ -443,6 +482,9 @@ def outlier_counts(x2d, S, threshold, bits=8, L=None, R=None):
 
 
 def decompress_threshold(c: ThresholdCompressed):
+    xhat = native.decompress(c)
+    if xhat is not None:
+        return xhat
     xhat = torch.empty((c.M, c.H), dtype=BF16, device=c.stored.device)
     d = c.desc()
     check(_abi.load().hyc_decompress(_p(c.stored), None, None, c.M, c.H, ctypes.byref(d), _p(xhat), _stream()))
@@ -452,6 +494,9 @@ def decompress_threshold(c: ThresholdCompressed):
 # ----------------------------------------------------------------------------------------------------
 # fused operators
 # ----------------------------------------------------------------------------------------------------
+ACT_CODES = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}
+
+
 def _wdtype(w):
     if w.dtype == torch.float32:
         return _abi.DTYPE_F32
@@ -643,7 +688,7 @@ def act_bwd(act, g2d, src):
     M, H = g2d.shape
     stored, vals, scales, d = _source(src, M, H)
     dx = torch.empty_like(g2d)
-    code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
+    code = ACT_CODES[act]
     check(_abi.load().hyc_act_bwd(code, _p(g2d), _p(stored), _p(vals), _p(scales), M, H, ctypes.byref(d), _p(dx), _stream()))
     return dx
 
@@ -674,7 +719,7 @@ def gated_act_bwd(act, g2d, src_act, src_up, src_gate, room=None):
     else:
         both = torch.empty((M, 2 * H + room), dtype=BF16, device=g2d.device)
         d_gate, d_up, pitch = both[:, :H], both[:, H:2 * H], 2 * H + room
-    code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
+    code = ACT_CODES[act]
     check(_abi.load().hyc_gated_act_bwd_rows(code, _p(g2d), _p(sa), _p(va), _p(ca), ctypes.byref(da), _p(su), _p(vu), _p(cu),
                                              ctypes.byref(du), _p(sg), _p(vg), _p(cg), ctypes.byref(dg), M, H, _p(d_gate), pitch,
                                              _p(d_up), pitch, _stream()))
@@ -703,7 +748,7 @@ def act_fwd_compress(act, x2d, plan, bits, group):
     c = alloc_channel(M, H, plan, bits, group, x2d.device)
     d = _checked_desc(plan, bits, group)
     y = torch.empty((M, H), dtype=BF16, device=x2d.device)
-    code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
+    code = ACT_CODES[act]
     check(_abi.load().hyc_act_fwd_compress(code, _p(x2d), x2d.stride(0) if M > 1 else H, M, H, ctypes.byref(d), _p(y),
                                            _p(c.stored), _p(c.vals), _p(c.scales), _stream()))
     return y, c
@@ -749,7 +794,7 @@ def gated_act_fwd(act, gate2d, up2d, plan_act, plan_up, plan_gate, bits, group):
     outs = [alloc_channel(M, H, p, bits, group, dev) for p in (plan_act, plan_up, plan_gate)]
     descs = [_checked_desc(p, bits, group) for p in (plan_act, plan_up, plan_gate)]
     h = torch.empty((M, H), dtype=BF16, device=dev)
-    code = {"silu": _abi.ACT_SILU, "gelu": _abi.ACT_GELU_TANH}[act]
+    code = ACT_CODES[act]
     flat = []
     for o in outs:
         flat += [_p(o.stored), _p(o.vals), _p(o.scales)]
@@ -848,6 +893,15 @@ def softmax_fwd(x, threshold=None, causal_period=None, inplace=False, budget=Non
     call returns without waiting for the GPU.
     causal_period = S applies the causal mask of S query positions inside the kernel (row r is position r % S).
     inplace: y overwrites x (rows of at most 4096 entries: a row is held in registers before anything is written)."""
+    if threshold is not None and causal_period is None and not inplace and budget is not None and budget.ready:
+        N, cap = x.shape[-1], _slab_entries(budget, x.shape[-1])
+        if cap and x.numel():
+            budget.poll()
+            room = budget.capacity(x.numel() // N)
+            done = native.softmax_fwd(x, float(threshold), cap, room)
+            if done is not None:
+                budget.watch(done[4], room, x.numel() // N)
+                return done[0], SparseRows(done[1], done[2], done[3], tuple(x.shape), done[4])
     _need(x, BF16, "x")
     N = x.shape[-1]
     x2 = x.reshape(-1, N)
@@ -886,6 +940,10 @@ def softmax_sparsify(y, threshold, budget=None):
 
 def softmax_bwd(g, sp: SparseRows, inplace=False):
     """dx = (g - sum(g * p_hat)) * p_hat; with inplace, dx overwrites g"""
+    if not inplace and g.dim() and sp.shape[-1] == g.shape[-1]:
+        dx = native.softmax_bwd(g, sp)
+        if dx is not None:
+            return dx
     _need(g, BF16, "grad_output")
     N = g.shape[-1]
     g2 = g.reshape(-1, N)
@@ -1277,6 +1335,14 @@ def attn_kept_entries(budget, threshold, S, head_dim):
 def attn_kept(q, k, lse, heads, scale, threshold, budget, cap, first, matrices):
     """the probabilities exp(bf16(scale q k^T) - lse) above the threshold of matrices [first, first + matrices) as SparseRows; lse:
     attn_fwd's with round_scores; cap: attn_kept_entries"""
+    if budget is not None and budget.ready and q.dim() == 3:
+        rows = matrices * q.shape[1]
+        budget.poll()
+        room = budget.capacity(rows)
+        done = native.attn_kept(q, k, lse, heads, scale, threshold, cap, room, first, matrices)
+        if done is not None:
+            budget.watch(done[3], room, rows)
+            return SparseRows(done[0], done[1], done[2], (matrices, q.shape[1], q.shape[1]), done[3])
     B, S, H, pq = _need_tokens(q, "q")
     pk = _need_tokens(k, "k")[3]
     if tuple(k.shape) != (B, S, H) or H % heads:

@@ -118,6 +118,10 @@ class _ChannelGatedActFunc(torch.autograd.Function):
         if calibrated and K.gated_act_fwd_supported(gate.shape[-1], bits, group):
             # steady state: one pass over gate and up writes the product and the three compressed activations;
             # act(gate) is never held in memory
+            done = K.native.gated_fwd(K.ACT_CODES[act], gate, up, sites[0].plan, sites[1].plan, sites[2].plan, bits, group)
+            if done is not None:
+                h, ctx.saved = done
+                return h
             h, c_act, c_up, c_gate = K.gated_act_fwd(act, _row_view(gate), _row_view(up), sites[0].plan, sites[1].plan,
                                                      sites[2].plan, bits, group)
             ctx.saved = (c_act, c_up, c_gate)
@@ -131,9 +135,13 @@ class _ChannelGatedActFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        g2, _ = as_rows(grad_output.to(torch.bfloat16))
-        grads = K.gated_act_bwd(ctx.act, g2, *ctx.saved, room=ctx.grad_room)
-        d_gate, d_up = (t.reshape(grad_output.shape) for t in grads[:2])
+        grads = K.native.gated_bwd(K.ACT_CODES[ctx.act], grad_output, *ctx.saved, ctx.grad_room)
+        if grads is not None:
+            d_gate, d_up = grads[:2]
+        else:
+            g2, _ = as_rows(grad_output.to(torch.bfloat16))
+            grads = K.gated_act_bwd(ctx.act, g2, *ctx.saved, room=ctx.grad_room)
+            d_gate, d_up = (t.reshape(grad_output.shape) for t in grads[:2])
         if ctx.grad_room is not None:
             d_gate._hyc_rows = d_up._hyc_rows = grads[2]
         return d_gate, d_up, None, None, None, None, None, None

@@ -30,6 +30,14 @@ def _affine(weight, bias):
 
 
 def _backward(ctx, dy):
+    done = K.native.norm_bwd(dy, ctx.saved, ctx.weight, ctx.mean, ctx.rstd, False)
+    if done is not None:
+        if ctx.bias is None:
+            return done + (None,)
+        if not torch.is_grad_enabled():
+            db = K.native.bias_grad(dy, ctx.bias.dtype != torch.bfloat16)
+            if db is not None:
+                return done + (db if db.dtype == ctx.bias.dtype else db.to(ctx.bias.dtype),)
     dy2, _ = as_rows(dy.to(torch.bfloat16))
     dx, dw = K.layernorm_bwd(dy2, ctx.saved, ctx.weight.detach().contiguous(), ctx.mean, ctx.rstd)
     db = None
@@ -58,10 +66,15 @@ class EfficientMemoryLayerNormFunc(torch.autograd.Function):
             outlier, L, scale, R = static_value[0], static_value[1], static_value[2], static_value[3]
         if (sub_outlier_ratio > 0. and sub_outlier_bit != 16 and x.dim() == 3
                 and K.layernorm_fwd_supported(x2.shape[-1], sub_outlier_bit)):
-            w, b = _affine(weight, bias)
-            y, mean, rstd, c = K.layernorm_fwd_compress_threshold(
-                x2, w, b, eps, x.shape[-2], K.threshold_value(outlier), scale.contiguous(), sub_outlier_bit,
-                L.contiguous() if rank > 0 else None, R.contiguous() if rank > 0 else None, budget=K.kept_budget(outlier))
+            threshold, budget = K.threshold_value(outlier), K.kept_budget(outlier)
+            done = K.threshold_native(x, 2, weight, bias, eps, x.shape[-2], threshold, scale, sub_outlier_bit,
+                                      L if rank > 0 else None, R if rank > 0 else None, budget)
+            if done is None:
+                w, b = _affine(weight, bias)
+                done = K.layernorm_fwd_compress_threshold(
+                    x2, w, b, eps, x.shape[-2], threshold, scale.contiguous(), sub_outlier_bit,
+                    L.contiguous() if rank > 0 else None, R.contiguous() if rank > 0 else None, budget=budget)
+            y, mean, rstd, c = done
         else:
             y, mean, rstd = _forward_stats(x2, weight, bias, eps)
             c, _ = compress_to_csr(x, outlier, scale, sub_outlier_bit, sub_outlier_ratio, L if rank > 0 else None,
@@ -80,6 +93,12 @@ class EfficientMemoryLayerNormFunc(torch.autograd.Function):
 class _ChannelLayerNormFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, eps, plan, bits, group):
+        if K.layernorm_fwd_supported(x.shape[-1], bits):
+            done = K.native.norm_fwd(x, weight, bias, True, eps, plan, bits, group)
+            if done is not None:
+                y, ctx.mean, ctx.rstd, ctx.saved = done
+                ctx.weight, ctx.bias = weight, bias
+                return y
         x2, _ = as_rows(x)
         if K.layernorm_fwd_supported(x2.shape[-1], bits):
             w, b = _affine(weight, bias)

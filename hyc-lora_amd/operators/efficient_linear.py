@@ -56,18 +56,29 @@ class EfficientMemoryLinearFunc(torch.autograd.Function):
 class _ChannelLinearFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b, plan, bits, group):
+        ctx.w, ctx.use_bias = w, b is not None
+        keep = ctx.needs_input_grad[1]               # x is kept for dW only
+        if b is None:
+            done = K.native.linear_fwd(x, w, plan if keep else None, bits, group)
+            if done is not None:
+                output, ctx.saved = done
+                return output
         output = x @ w.transpose(0, 1)
         if b is not None:
             output = output + b[None, ...]
         ctx.saved = None
-        if ctx.needs_input_grad[1]:                  # x is kept for dW only
+        if keep:
             x2, _ = as_rows(x)
             ctx.saved = K.compress_channel(x2, plan, bits, group)
-        ctx.w, ctx.use_bias = w, b is not None
         return output
 
     @staticmethod
     def backward(ctx, grad_output):
+        if not ctx.use_bias:
+            needs, w = ctx.needs_input_grad, ctx.w
+            done = K.native.linear_bwd(grad_output, w, ctx.saved if needs[1] else None, needs[0], K.gradw_staged_by_default(*w.shape))
+            if done is not None:
+                return done[0], done[1], None, None, None, None
         gi, gw, gb = _linear_backward(grad_output, ctx.w.detach(), ctx.saved, ctx.use_bias, ctx.needs_input_grad[:3])
         return gi, gw, gb, None, None, None
 

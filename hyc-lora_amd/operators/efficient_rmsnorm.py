@@ -26,12 +26,16 @@ def _ref_forward(ctx, x, outlier_ratio, sub_outlier_ratio, sub_outlier_bit, sub_
         outlier, L, scale, R = static_value[0], static_value[1], static_value[2], static_value[3]
     if sub_outlier_ratio == 0. or sub_outlier_bit == 16:
         raise NotImplementedError("the branches without a quantised part are outside the accelerated path")
-    y, rstd, c = K.rmsnorm_fwd_compress_threshold(x2, _effective_weight(weight, weight_offset), eps, S, K.threshold_value(outlier),
-                                                  scale.contiguous(), sub_outlier_bit,
-                                                  L.contiguous() if rank > 0 else None,
-                                                  R.contiguous() if rank > 0 else None, budget=K.kept_budget(outlier))
-    ctx.saved = c
-    ctx.rstd = rstd
+    threshold, budget = K.threshold_value(outlier), K.kept_budget(outlier)
+    done = None if weight_offset else K.threshold_native(x, 1, weight, None, eps, S, threshold, scale, sub_outlier_bit,
+                                                         L if rank > 0 else None, R if rank > 0 else None, budget)
+    if done is not None:
+        y, _, ctx.rstd, ctx.saved = done
+    else:
+        y, ctx.rstd, ctx.saved = K.rmsnorm_fwd_compress_threshold(x2, _effective_weight(weight, weight_offset), eps, S, threshold,
+                                                                  scale.contiguous(), sub_outlier_bit,
+                                                                  L.contiguous() if rank > 0 else None,
+                                                                  R.contiguous() if rank > 0 else None, budget=budget)
     ctx.weight = weight
     ctx.c2_quirk, ctx.weight_offset = c2_quirk, weight_offset
     y = y.reshape(x.shape)
@@ -41,6 +45,10 @@ def _ref_forward(ctx, x, outlier_ratio, sub_outlier_ratio, sub_outlier_bit, sub_
 
 def _ref_backward(ctx, dy):
     dy = result_gradient(ctx, dy)
+    if not ctx.weight_offset:
+        done = K.native.norm_bwd(dy, ctx.saved, ctx.weight, None, ctx.rstd, bool(ctx.c2_quirk))
+        if done is not None:
+            return done
     dy2, _ = as_rows(dy.to(torch.bfloat16))
     dx, dw = K.rmsnorm_bwd(dy2, ctx.saved, _effective_weight(ctx.weight, ctx.weight_offset), ctx.rstd, c2_quirk=ctx.c2_quirk)
     return dx.reshape(dy.shape), dw.to(ctx.weight.dtype)
@@ -85,6 +93,12 @@ class _RMSNormFunc(torch.autograd.Function):
 class _ChannelRMSNormFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, eps, plan, bits, group, c2_quirk, weight_offset=0.0):
+        if not weight_offset:
+            done = K.native.norm_fwd(x, weight, None, False, eps, plan, bits, group)
+            if done is not None:
+                y, _, ctx.rstd, ctx.saved = done
+                ctx.weight, ctx.c2_quirk, ctx.weight_offset = weight, c2_quirk, weight_offset
+                return y
         x2, _ = as_rows(x)
         y, rstd, c = K.rmsnorm_fwd_compress_channel(x2, _effective_weight(weight, weight_offset), eps, plan, bits, group)
         ctx.saved, ctx.rstd, ctx.weight, ctx.c2_quirk, ctx.weight_offset = c, rstd, weight, c2_quirk, weight_offset
@@ -92,6 +106,10 @@ class _ChannelRMSNormFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
+        if not ctx.weight_offset:
+            done = K.native.norm_bwd(dy, ctx.saved, ctx.weight, None, ctx.rstd, bool(ctx.c2_quirk))
+            if done is not None:
+                return done[0], done[1], None, None, None, None, None, None
         dy2, _ = as_rows(dy.to(torch.bfloat16))
         dx, dw = K.rmsnorm_bwd(dy2, ctx.saved, _effective_weight(ctx.weight, ctx.weight_offset), ctx.rstd,
                                c2_quirk=ctx.c2_quirk)

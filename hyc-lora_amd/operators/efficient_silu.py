@@ -26,8 +26,11 @@ def _ref_backward(ctx, act, grad_output):
     g = result_gradient(ctx, grad_output).to(torch.bfloat16)
     if ctx.is_head:
         g = head_to_hidden_shape(g)
-    g2, _ = as_rows(g)
-    dx = K.act_bwd(act, g2, ctx.saved).reshape(ctx.hidden_shape)
+    dx = K.native.act_bwd(K.ACT_CODES[act], g, ctx.saved)
+    if dx is None:
+        g2, _ = as_rows(g)
+        dx = K.act_bwd(act, g2, ctx.saved)
+    dx = dx.reshape(ctx.hidden_shape)
     if ctx.is_head:
         dx = hidden_to_head_shape(dx, ctx.num_heads)
     return dx
@@ -53,8 +56,13 @@ class _ChannelActFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, act, plan, bits, group):
-        x2, _ = as_rows(x)
         ctx.act = act
+        if K.act_fwd_compress_supported(x.shape[-1], bits, group):
+            done = K.native.act_fwd(K.ACT_CODES[act], x, plan, bits, group)
+            if done is not None:
+                y, ctx.saved = done
+                return y
+        x2, _ = as_rows(x)
         if K.act_fwd_compress_supported(x2.shape[-1], bits, group):
             y, ctx.saved = K.act_fwd_compress(act, x2, plan, bits, group)      # one read of x
             return y.view(x.shape)
@@ -63,6 +71,9 @@ class _ChannelActFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
+        dx = K.native.act_bwd(K.ACT_CODES[ctx.act], grad_output, ctx.saved)
+        if dx is not None:
+            return dx, None, None, None, None
         g2, _ = as_rows(grad_output.to(torch.bfloat16))
         return K.act_bwd(ctx.act, g2, ctx.saved).reshape(grad_output.shape), None, None, None, None
 
