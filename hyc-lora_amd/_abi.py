@@ -51,6 +51,8 @@ SIGNATURES = {
     "hyc_decompress": (c_i32, [c_ptr, c_ptr, c_ptr, c_i64, c_i64, ctypes.POINTER(HycDesc), c_ptr, c_ptr]),
     "hyc_ref_outlier_count": (c_i32, [c_ptr, c_i64, c_i64, ctypes.POINTER(HycDesc), c_ptr, c_ptr]),
     "hyc_ref_outlier_fill": (c_i32, [c_ptr, c_i64, c_i64, ctypes.POINTER(HycDesc), c_ptr, c_ptr, c_ptr, c_ptr]),
+    "hyc_ref_outlier_fill_slab": (c_i32, [c_ptr, c_i64, c_i64, ctypes.POINTER(HycDesc), c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_ptr]),
+    "hyc_threshold_fwd": (c_i32, [c_i32, c_ptr, c_ptr, c_ptr, c_i32, c_f32, c_i64, c_i64, ctypes.POINTER(HycDesc)] + [c_ptr] * 6 + [c_i64, c_ptr]),
     "hyc_rmsnorm_fwd_compress": (c_i32, [c_ptr, c_ptr, c_i32, c_f32, c_i64, c_i64, ctypes.POINTER(HycDesc),
                                          c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),
     "hyc_layernorm_fwd_compress": (c_i32, [c_ptr, c_ptr, c_ptr, c_i32, c_f32, c_i64, c_i64, ctypes.POINTER(HycDesc),

@@ -4,6 +4,7 @@
 
 #include "abi_util.hpp"
 #include "row_kernels.hpp"
+#include "threshold.hpp"
 #include "wave_scan.hpp"
 
 namespace hyc {
@@ -316,9 +317,11 @@ k_outlier_count(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a,
   if (lane == 0) counts[row] = (int32_t)total;
 }
 
+// slab (may be null): rows of at most `cap` kept elements are copied from there (threshold.hip), x is read for the others only
 __global__ void __launch_bounds__(256)
 k_outlier_fill(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a, const int32_t* __restrict__ row_ptr,
-               int32_t* __restrict__ cols, uint16_t* __restrict__ vals) {
+               int32_t* __restrict__ cols, uint16_t* __restrict__ vals, const int32_t* __restrict__ counts,
+               const uint32_t* __restrict__ slab, int cap) {
   __shared__ uint32_t stage_all[4][STAGE_CAP];
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -331,6 +334,18 @@ k_outlier_fill(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a, 
   const int limit = (int)(row_ptr[row + 1] - base);        // the row's room in cols / vals
   int32_t* cols_row = cols + base;
   uint16_t* vals_row = vals + base;
+  if (slab) {
+    const int n = counts[row];
+    if (n <= cap) {
+      const int m = n < limit ? n : limit;
+      for (int e = lane; e < m; e += 64) {
+        const uint32_t w = slab[row * cap + e];
+        cols_row[e] = (int32_t)(w & 0xFFFFu);
+        vals_row[e] = (uint16_t)(w >> 16);
+      }
+      return;
+    }
+  }
   int running = 0;
   uint4 next = lane < nch ? *reinterpret_cast<const uint4*>(xr + 8 * lane) : make_uint4(0, 0, 0, 0);
   for (int64_t c0 = 0; c0 < nch; c0 += 64) {
@@ -512,6 +527,7 @@ int hyc_decompress(const void* stored, const void* vals, const void* scales, int
     if (!stored || !xhat) return fail(HYC_EFAULT, "hyc_decompress: null buffer");
     if (!a.row_ptr) return fail(HYC_EFAULT, "hyc_decompress: threshold mode needs csr_row_ptr");
     if (!aligned16(xhat) || !aligned8(stored)) return fail(HYC_EINVAL, "hyc_decompress: xhat must be 16-byte and stored 8-byte aligned");
+    if (launch_thr_restore(stored, M, H, g, a, perchan, xhat, st)) return check_launch("hyc_decompress");
     const int grid = long_input_grid(M, row_grid(M, g.threads));
     const size_t lds = (size_t)H * 2;
     HYC_DISPATCH_BITS(d->bits,
@@ -550,17 +566,29 @@ int hyc_ref_outlier_count(const void* x, int64_t M, int64_t H, const hyc_desc* d
   return check_launch("hyc_ref_outlier_count");
 }
 
-int hyc_ref_outlier_fill(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* row_ptr, int32_t* cols,
-                         void* vals, void* stream) {
+static int outlier_fill(const char* who, const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* counts, const uint32_t* slab,
+                        int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals, void* stream) {
   ThrArgs a;
-  int rc = outlier_args("hyc_ref_outlier_fill", x, M, H, d, &a);
+  int rc = outlier_args(who, x, M, H, d, &a);
   if (rc) return rc;
   if (M == 0) return HYC_OK;
-  if (!x || !row_ptr) return fail(HYC_EFAULT, "hyc_ref_outlier_fill: null buffer");
-  if (!aligned16(x)) return fail(HYC_EINVAL, "hyc_ref_outlier_fill: x must be 16-byte aligned");
+  if (!x || !row_ptr) return fail(HYC_EFAULT, "%s: null buffer", who);
+  if (!aligned16(x)) return fail(HYC_EINVAL, "%s: x must be 16-byte aligned", who);
   hipLaunchKernelGGL(k_outlier_fill, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, begin_launch(stream),
-                     static_cast<const uint16_t*>(x), M, H, a, row_ptr, cols, static_cast<uint16_t*>(vals));
-  return check_launch("hyc_ref_outlier_fill");
+                     static_cast<const uint16_t*>(x), M, H, a, row_ptr, cols, static_cast<uint16_t*>(vals), counts, slab, (int)cap);
+  return check_launch(who);
+}
+
+int hyc_ref_outlier_fill(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* row_ptr, int32_t* cols,
+                         void* vals, void* stream) {
+  return outlier_fill("hyc_ref_outlier_fill", x, M, H, d, nullptr, nullptr, 0, row_ptr, cols, vals, stream);
+}
+
+int hyc_ref_outlier_fill_slab(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* counts, const uint32_t* slab, int64_t cap,
+                              const int32_t* row_ptr, int32_t* cols, void* vals, void* stream) {
+  if (cap <= 0 || cap > H) return fail(HYC_EINVAL, "hyc_ref_outlier_fill_slab: cap=%lld must be in 1..H=%lld", (long long)cap, (long long)H);
+  if (M > 0 && (!counts || !slab)) return fail(HYC_EFAULT, "hyc_ref_outlier_fill_slab: null buffer");
+  return outlier_fill("hyc_ref_outlier_fill_slab", x, M, H, d, counts, slab, cap, row_ptr, cols, vals, stream);
 }
 
 }  // extern "C"

@@ -401,15 +401,16 @@ PyObject* wrap_all(std::initializer_list<Tensor> ts) {
   for (const Tensor& x : ts) PyTuple_SET_ITEM(t, i++, x.defined() ? THPVariable_Wrap(x) : none());
   return t;
 }
-// threshold_fwd(x [..., H], norm, w or None, bias or None, eps, S, threshold, scale, bits, L or None, R or None, cap)
+// threshold_fwd(x [..., H], norm, w or None, bias or None, eps, S, threshold, scale, bits, L or None, R or None, cap, slab entries per row)
 //   -> (y like x or None, mean or None, rstd or None, stored, row_ptr, cols, vals, total); norm: 0 compress only, 1 rms, 2 layer
 PyObject* threshold_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  ARGS(12);
+  ARGS(13);
   const Tensor *x = bf16(a[0]), *w = nullptr, *bias = nullptr;
   const long norm = PyLong_AsLong(a[1]);
   const double eps = PyFloat_AsDouble(a[4]), thr = PyFloat_AsDouble(a[6]);
-  const int64_t S = PyLong_AsLongLong(a[5]), bits = PyLong_AsLongLong(a[8]), cap = PyLong_AsLongLong(a[11]);
+  const int64_t S = PyLong_AsLongLong(a[5]), bits = PyLong_AsLongLong(a[8]), cap = PyLong_AsLongLong(a[11]),
+                slab_cap = PyLong_AsLongLong(a[12]);
   if (PyErr_Occurred()) return nullptr;
   int64_t M, H;
   int dtype = 0;
@@ -428,17 +429,31 @@ PyObject* threshold_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   }
   if (norm == 2) mean = empty_like_on(*x, {M}, at::kFloat);
   int32_t* n = (int32_t*)counts.data_ptr();
-  if (norm == 2)
+  Tensor slab;
+  if (slab_cap > 0) {
+    slab = empty_like_on(*x, {M, slab_cap}, at::kInt);
+    const int rc = hyc_threshold_fwd((int32_t)norm, x->data_ptr(), norm ? w->data_ptr() : nullptr, bias ? bias->data_ptr() : nullptr, dtype, (float)eps, M, H,
+                                     &t.d, norm ? y.data_ptr() : nullptr, norm == 2 ? (float*)mean.data_ptr() : nullptr,
+                                     norm ? (float*)rstd.data_ptr() : nullptr, stored.data_ptr(), n, (uint32_t*)slab.data_ptr(), slab_cap, stream());
+    if (rc == HYC_ENOTSUP) slab = Tensor();
+    else if (rc != 0) return none();
+  }
+  const bool general = !slab.defined();
+  if (general && norm == 2)
     OR_NONE(hyc_layernorm_fwd_compress(x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, dtype, (float)eps, M, H, &t.d, y.data_ptr(),
                                        (float*)mean.data_ptr(), (float*)rstd.data_ptr(), stored.data_ptr(), nullptr, nullptr, n, stream()));
-  else if (norm)
+  else if (general && norm)
     OR_NONE(hyc_rmsnorm_fwd_compress(x->data_ptr(), w->data_ptr(), dtype, (float)eps, M, H, &t.d, y.data_ptr(), (float*)rstd.data_ptr(),
                                      stored.data_ptr(), nullptr, nullptr, n, stream()));
-  else
+  else if (general)
     OR_NONE(hyc_compress(x->data_ptr(), M, H, &t.d, stored.data_ptr(), nullptr, nullptr, n, stream()));
   Csr csr;
   if (!csr.offsets(counts, M, cap)) return none();
-  OR_NONE(hyc_ref_outlier_fill(x->data_ptr(), M, H, &t.d, csr.rp(), csr.co(), csr.vals.data_ptr(), stream()));
+  if (!general)
+    OR_NONE(hyc_ref_outlier_fill_slab(x->data_ptr(), M, H, &t.d, n, (const uint32_t*)slab.data_ptr(), slab_cap, csr.rp(), csr.co(), csr.vals.data_ptr(),
+                                      stream()));
+  else
+    OR_NONE(hyc_ref_outlier_fill(x->data_ptr(), M, H, &t.d, csr.rp(), csr.co(), csr.vals.data_ptr(), stream()));
   return wrap_all({y, mean, rstd, stored, csr.row_ptr, csr.cols, csr.vals, csr.total});
   END_HANDLE_TH_ERRORS
 }

@@ -433,7 +433,7 @@ def threshold_native(x, norm, w, bias, eps, S, threshold, scale, bits, L, R, bud
     M = x.numel() // H
     budget.poll()
     cap = budget.capacity(M)
-    done = native.threshold_fwd(x, norm, w, bias, eps, S, threshold, scale, bits, L, R, cap)
+    done = native.threshold_fwd(x, norm, w, bias, eps, S, threshold, scale, bits, L, R, cap, _slab_entries(budget, H, 16384))
     if done is None:
         return None
     y, mean, rstd, stored, row_ptr, cols, vals, total = done
@@ -862,11 +862,11 @@ class SparseRows:
         return self.row_ptr.numel() - 1
 
 
-def _slab_entries(budget, N):
+def _slab_entries(budget, N, longest=4096):
     """entries per row of the forward's slab of kept probabilities, or 0 to read y a second time instead.  A slab entry is
     written and read (8 bytes) where the second read of y costs 2 N bytes a row: worth it while twice the share seen before
     fits an eighth of the row (N / 2 bytes of traffic for the average row)."""
-    if budget is None or not budget.ready or N > 4096:
+    if budget is None or not budget.ready or N > longest:
         return 0
     cap = max(32, (int(2 * budget.per_row) + 31) // 32 * 32)
     return cap if cap <= max(32, N // 8) and cap <= N else 0

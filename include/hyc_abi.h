@@ -165,6 +165,15 @@ int hyc_ref_outlier_count(const void* x, int64_t M, int64_t H, const hyc_desc* d
  * first row_ptr[m+1] - row_ptr[m] outliers); fills cols / vals in ascending column order */
 int hyc_ref_outlier_fill(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* row_ptr,
                          int32_t* cols, void* vals, void* stream);
+/* Codes (hyc_compress), counts and the first `cap` outliers of every row in slab [M, cap] (column in the low half of a word, bf16 bits
+ * of x - base in the high half, ascending) from one read of x; norm 1: with hyc_rmsnorm_fwd_compress's y and rstd, norm 2: with
+ * hyc_layernorm_fwd_compress's y, mean and rstd.  4- and 8-bit codes, H bits / 64 <= 1024, rank at most 2, a scale per tensor, token
+ * or channel; HYC_ENOTSUP for others.  hyc_ref_outlier_fill_slab: hyc_ref_outlier_fill, reading x only for rows of more than cap. */
+int hyc_threshold_fwd(int32_t norm, const void* x, const void* w, const void* bias, int32_t w_dtype, float eps, int64_t M, int64_t H,
+                      const hyc_desc* d, void* y, float* mean, float* rstd, void* stored, int32_t* counts, uint32_t* slab, int64_t cap,
+                      void* stream);
+int hyc_ref_outlier_fill_slab(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* counts, const uint32_t* slab,
+                              int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals, void* stream);
 
 /* ---- RMSNorm ----------------------------------------------------------------------------------- */
 /* y = bf16((x*rstd)*w), rstd = 1/sqrt(mean(x^2)+eps) [M] fp32, and x compressed as hyc_compress does. */
