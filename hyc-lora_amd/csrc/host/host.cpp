@@ -533,6 +533,11 @@ std::vector<int64_t> with_last(const Tensor& x, int64_t n) {
   s.back() = n;
   return s;
 }
+// a weight and rows that the kernels for few output features read as they lie
+bool thin(const Tensor& rows, const Tensor& w, int64_t M, bool input_grad) {
+  return hyc_thin_covers(M, w.size(1), w.size(0), input_grad) && aligned16(rows.data_ptr()) && aligned16(w.data_ptr()) && w.is_contiguous() &&
+         rows.device() == w.device() && rows.device().index() == c10::hip::current_device();
+}
 // linear_fwd(x [..., K], w [N, K], plan or None, bits, group) -> (x w^T, ChannelCompressed or None)
 PyObject* linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -544,7 +549,14 @@ PyObject* linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (a[2] == Py_None) Py_INCREF(c);
   else if (!(c = compress_rows(*x, a[2], a[3], a[4]))) return none_if_plain(nullptr);
   Ref hold(c);
-  Tensor y = at::mm(x->view({M, K}), w->t()).view(with_last(*x, w->size(0)));
+  Tensor y;
+  if (thin(*x, *w, M, false)) {
+    y = at::empty(with_last(*x, w->size(0)), x->options());
+    const void* factor = w->data_ptr();
+    OR_NONE(hyc_lora_down(x->data_ptr(), K, M, K, &factor, 1, (int32_t)w->size(0), y.data_ptr(), stream()));
+  } else {
+    y = at::mm(x->view({M, K}), w->t()).view(with_last(*x, w->size(0)));
+  }
   Py_INCREF(c);
   return tuple2(THPVariable_Wrap(y), c);
   END_HANDLE_TH_ERRORS
@@ -559,7 +571,12 @@ PyObject* linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     return none();
   Tensor dw, dx;
   if (a[2] != Py_None && !weight_grad(g->data_ptr(), N, M, N, *g, a[2], false, a[4] == Py_True, &dw)) return none();
-  if (a[3] == Py_True) dx = at::mm(g->view({M, N}), *w).view(with_last(*g, w->size(1)));
+  if (a[3] == Py_True && thin(*g, *w, M, true)) {
+    dx = at::empty(with_last(*g, w->size(1)), g->options());
+    OR_NONE(hyc_thin_dx(g->data_ptr(), N, M, w->data_ptr(), (int32_t)N, w->size(1), dx.data_ptr(), stream()));
+  } else if (a[3] == Py_True) {
+    dx = at::mm(g->view({M, N}), *w).view(with_last(*g, w->size(1)));
+  }
   return tuple2(dx.defined() ? THPVariable_Wrap(dx) : none(), dw.defined() ? THPVariable_Wrap(dw) : none());
   END_HANDLE_TH_ERRORS
 }

@@ -246,6 +246,41 @@ k_lora_up(const uint16_t* __restrict__ h, int64_t M, LoraOut a, float scale, uin
   }
 }
 
+// ---- dx = g w for a weight of few rows -------------------------------------------------------------------------------------
+// dx[m, k] = sum_j g[m, j] w[j, k], j < N <= 32.  A pure write like k_lora_up, and laid out like it; what differs is the weight, whose
+// columns are the features here: a lane gathers the 8 rows of its feature (2 bytes each, 64-byte runs over the lanes, once per
+// 128 tokens, from L2).
+__global__ void __launch_bounds__(256)
+k_thin_dx(const uint16_t* __restrict__ g, int64_t ldg, int64_t M, const uint16_t* __restrict__ w, int N, int K, uint16_t* __restrict__ dx) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, lq = lane >> 4;
+  const int f0 = (int)blockIdx.x * LO_F + 64 * wave;
+  const int64_t m_begin = (int64_t)blockIdx.y * LO_M;
+  const bool on = 8 * lq < N;                            // (N is a multiple of 8)
+  bf16x8_t wf[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int f = f0 + 32 * (q >> 1) + 8 * (l15 >> 2) + 4 * (q & 1) + (l15 & 3);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) wf[q][j] = __builtin_bit_cast(__bf16, on && f < K ? w[(int64_t)(8 * lq + j) * K + f] : (uint16_t)0);
+  }
+#pragma unroll 4
+  for (int t = 0; t < LO_M; t += 16) {
+    const int64_t m = m_begin + t + l15;
+    const uint4 v = on && m < M ? *reinterpret_cast<const uint4*>(g + m * ldg + 8 * lq) : make_uint4(0, 0, 0, 0);
+    const bf16x8_t gf = __builtin_bit_cast(bf16x8_t, v);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const floatx4_t z = {0.f, 0.f, 0.f, 0.f};
+      const floatx4_t d0 = HYC_MFMA16(wf[2 * c], gf, z), d1 = HYC_MFMA16(wf[2 * c + 1], gf, z);
+      const int f = f0 + 32 * c + 8 * lq;
+      if (m < M && f < K) {
+        const float o[8] = {d0[0], d0[1], d0[2], d0[3], d1[0], d1[1], d1[2], d1[3]};
+        *reinterpret_cast<uint4*>(dx + m * K + f) = pack8(o);
+      }
+    }
+  }
+}
+
 // ---- dh = s dY B and dB = s dY^T h from one read of dY -----------------------------------------------------------------
 struct LoraUp {
   const uint16_t* g[LORA_MAX];                           // dY_i [M, n_out_i], rows ldg_i apart
@@ -564,6 +599,33 @@ int hyc_lora_up(const void* h, int64_t M, const void* const* B, const int64_t* n
   hipLaunchKernelGGL(k_lora_up, dim3((unsigned)a.fb0[n], (unsigned)((M + LO_M - 1) / LO_M)), dim3(256), 0, begin_launch(stream),
                      static_cast<const uint16_t*>(h), M, a, scale, static_cast<uint16_t*>(y));
   return check_launch("hyc_lora_up");
+}
+
+// Where a linear layer of few output features takes k_lora_down and k_thin_dx instead of library products (us, library -> these):
+//   x w^T   4096 x 4096 with 8 / 16 / 32 features 11.6 / 12.1 / 9.8 -> 5.7 / 6.0 / 8.6, 4096 x 11008 26.4 / 27.1 / 22.4 -> 17.0 / 17.5 / 20.6,
+//           157 x 4096 7.9 / 7.9 / 7.4 -> 4.9 / 5.0 / 7.1; where x no longer stays in the last-level cache the waves' 128-byte rows fall
+//           behind: 16384 x 4096 21.8 / 22.0 / 22.6 -> 22.6 / 23.0 / 30.4, 9000 x 13824 37.9 / 39.0 / 41.2 -> 43.6 / 46.0 / 56.8;
+//           64 features 157 x 4096 8.0 -> 10.2, 4096 x 4096 16.2 -> 13.1, 16384 x 4096 23.6 -> 43.7
+//   g w     4096 x 4096 with 8 / 16 / 32 15.0 / 15.4 / 11.4 -> 10.9 / 11.0 / 10.9, 4096 x 11008 42.9 / 44.2 / 30.7 -> 20.2 / 20.6 / 22.5, 65536 x 2048
+//           81.7 / 84.0 / 57.9 -> 52.1 / 58.5 / 68.8, 157 x 4096 5.2 / 5.2 / 4.3 -> 5.8 / 5.8 / 6.1 (the library's call costs the host 20 us more)
+int32_t hyc_thin_covers(int64_t M, int64_t K, int64_t N, int32_t input_grad) {
+  if (M <= 0 || K <= 0 || N < 8 || N > 32 || N % 8 != 0 || K % 64 != 0 || K > (1 << 24) || M > (int64_t)65535 * LO_M) return 0;
+  if (input_grad && N <= 16) return 1;
+  return M * K <= (input_grad ? (int64_t)1 << 26 : (int64_t)3 << 24) ? 1 : 0;
+}
+
+int hyc_thin_dx(const void* g, int64_t ldg, int64_t M, const void* w, int32_t N, int64_t K, void* dx, void* stream) {
+  if (N < 8 || N > 32 || N % 8 != 0) return fail(HYC_ENOTSUP, "hyc_thin_dx: a weight of %d rows (8 to 32, a multiple of 8)", N);
+  if (K <= 0 || K % 8 != 0 || K > (1 << 24)) return fail(HYC_ENOTSUP, "hyc_thin_dx: rows of %lld (a multiple of 8)", (long long)K);
+  if (M < 0 || ldg < N || ldg % 8 != 0) return fail(HYC_EINVAL, "hyc_thin_dx: M=%lld, row pitch %lld", (long long)M, (long long)ldg);
+  if (M == 0) return HYC_OK;
+  if (!g || !w || !dx) return fail(HYC_EFAULT, "hyc_thin_dx: null buffer");
+  if (!aligned16(g) || !aligned16(dx)) return fail(HYC_EINVAL, "hyc_thin_dx: g and dx must be 16-byte aligned");
+  if ((M + LO_M - 1) / LO_M > 65535) return fail(HYC_ENOTSUP, "hyc_thin_dx: too many tokens");
+  const dim3 grid((unsigned)((K + LO_F - 1) / LO_F), (unsigned)((M + LO_M - 1) / LO_M));
+  hipLaunchKernelGGL(k_thin_dx, grid, dim3(256), 0, begin_launch(stream), static_cast<const uint16_t*>(g), ldg, M,
+                     static_cast<const uint16_t*>(w), N, (int)K, static_cast<uint16_t*>(dx));
+  return check_launch("hyc_thin_dx");
 }
 
 int64_t hyc_lora_up_bwd_workspace_bytes(int64_t M, const int64_t* n_out, int32_t n, int32_t r) {

@@ -1116,6 +1116,35 @@ def lora_down(x2d, A):
     return h
 
 
+def _thin(rows, w, input_grad):
+    """whether `rows` (x or dY of a linear layer with weight w) and w are what the kernels for few output features take and read as they lie"""
+    plain = (torch.Tensor, torch.nn.Parameter)
+    return (type(rows) in plain and type(w) in plain and rows.dtype is BF16 and w.dtype is BF16 and rows.is_cuda and rows.device == w.device
+            and rows.dim() >= 2 and w.dim() == 2 and not torch.is_grad_enabled() and rows.shape[-1] == w.shape[0 if input_grad else 1]
+            and rows.is_contiguous() and w.is_contiguous() and rows.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and rows.device.index == torch.cuda.current_device()
+            and bool(_abi.load().hyc_thin_covers(rows.numel() // rows.shape[-1], w.shape[1], w.shape[0], input_grad)))
+
+
+def linear_fwd(x, w):
+    """x w^T"""
+    if not _thin(x, w, False):
+        return x @ w.transpose(0, 1)
+    y = torch.empty((*x.shape[:-1], w.shape[0]), dtype=BF16, device=x.device)
+    M, Kf = x.numel() // w.shape[1], w.shape[1]
+    check(_abi.load().hyc_lora_down(_p(x), Kf, M, Kf, _ptrs([w]), 1, w.shape[0], _p(y), _stream()))
+    return y
+
+
+def linear_dx(g, w):
+    """g w"""
+    if not _thin(g, w, True):
+        return g @ w
+    dx = torch.empty((*g.shape[:-1], w.shape[1]), dtype=BF16, device=g.device)
+    check(_abi.load().hyc_thin_dx(_p(g), w.shape[0], g.numel() // w.shape[0], _p(w), w.shape[0], w.shape[1], _p(dx), _stream()))
+    return dx
+
+
 def _need_h(h, M, width):
     _need(h, BF16, "h")
     if h.shape != (M, width):

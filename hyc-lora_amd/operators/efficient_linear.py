@@ -11,7 +11,7 @@ def _linear_backward(grad_output, w, saved, use_bias, needs):
     """(dX, dW, db); `needs` = ctx.needs_input_grad[:3]: a gradient nobody asked for is not computed (a frozen weight
     has no dW, and its input was not saved)"""
     g = grad_output.to(w.dtype)
-    grad_input = g @ w if needs[0] else None
+    grad_input = K.linear_dx(g, w) if needs[0] else None
     g2, _ = as_rows(g.to(torch.bfloat16))
     grad_weight = None
     if needs[1]:
@@ -63,7 +63,7 @@ class _ChannelLinearFunc(torch.autograd.Function):
             if done is not None:
                 output, ctx.saved = done
                 return output
-        output = x @ w.transpose(0, 1)
+        output = K.linear_fwd(x, w)
         if b is not None:
             output = output + b[None, ...]
         ctx.saved = None

@@ -346,6 +346,9 @@ int hyc_rope_from_heads(const void* g, const void* cosv, const void* sinv, int64
  * n_out[i] output features (multiples of 8); A_i bf16 [r, K], B_i bf16 [n_out_i, r]; `packed` / `absmax` hold the stacked
  * base [sum n_out, K] as hyc_nf4_quantize writes it.  What stands beside the products with the base weight:
  *   hyc_lora_down      h bf16 [M, n r] = x A_i^T side by side
+ *   hyc_thin_dx        dx bf16 [M, K] = g w for g bf16 [M, N] (rows ldg apart) and a weight w [N, K] of 8 to 32 rows
+ *   hyc_thin_covers    1 where x w^T (hyc_lora_down with w as its one factor) or, with input_grad, g w (hyc_thin_dx) of a
+ *                      linear layer with N output features is better taken by these kernels than by a library product
  *   hyc_lora_up        y bf16 [M, sum n_out] = scale * h_i B_i^T side by side (the base product accumulates onto it)
  *   hyc_lora_up_bwd    from one read of dY_i [M, n_out_i] (rows ldg[i] apart): dh = bf16(scale * dY_i B_i) to dh [M, n r] and,
  *                      with zeros behind them, to the `room` columns [sum n_out, + room) of ext (rows ld_ext apart);
@@ -356,6 +359,8 @@ int hyc_rope_from_heads(const void* g, const void* cosv, const void* sinv, int64
  * fp32 accumulation in a fixed order throughout; room >= n r, a multiple of 8.
  * (peft's Linear.forward around bitsandbytes_fix/_function.py:509-540 computes the same per projection.) */
 int hyc_lora_down(const void* x, int64_t ldx, int64_t M, int64_t K, const void* const* A, int32_t n, int32_t r, void* h, void* stream);
+int32_t hyc_thin_covers(int64_t M, int64_t K, int64_t N, int32_t input_grad);
+int hyc_thin_dx(const void* g, int64_t ldg, int64_t M, const void* w, int32_t N, int64_t K, void* dx, void* stream);
 int hyc_lora_up(const void* h, int64_t M, const void* const* B, const int64_t* n_out, int32_t n, int32_t r, float scale, void* y,
                 void* stream);
 int64_t hyc_lora_up_bwd_workspace_bytes(int64_t M, const int64_t* n_out, int32_t n, int32_t r);
