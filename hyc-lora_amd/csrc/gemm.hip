@@ -600,7 +600,7 @@ constexpr int WPAD = 32;    // row padding of the wide kernel's LDS tiles, in el
 template <int NSEG, int A_PER, int B_PER>
 struct WideRegs {            // one stage of global data per thread
   uint4 a[A_PER];            // dY chunks
-  uint4 b[B_PER];            // channel scheme: .x/.y = packed word; dense: 8 bf16
+  uint4 b[B_PER];            // k_gradw_big: .x/.y = packed word; k_gradw_wide: 8 bf16
   uint32_t s[B_PER][NSEG];   // channel scheme: the group scale of each segment's chunk
   uint32_t o0[B_PER][NSEG], o1[B_PER][NSEG];   // ... and the first two outlier values of the chunk
 };
@@ -765,16 +765,87 @@ template <int V> struct StageNo { static constexpr int value = V; };
 template <class F, int... T>
 __device__ __forceinline__ void for_each_slot(F&& f, std::integer_sequence<int, T...>) { (f(StageNo<T>{}), ...); }
 
-template <int BITS, int SRC>
+// Which tile: workgroups are dealt to the 8 XCDs in turn (workgroup L of a launch runs on XCD L mod 8) and every XCD
+// has an L2 of its own, so XCD q takes a contiguous run of tiles in an order that walks 4 feature tiles by all
+// channel tiles: its workgroups then share 4 dY panels and a short run of x_hat panels instead of 2 and all of them
+// (1-4 % on real operands: 4096 x 4096 x 11008 dense 328 -> 320 us, INT2 4096^3 138 -> 132 us).
+__device__ __forceinline__ void big_tile(int* tile_n, int* tile_h) {
+  const int gx = (int)gridDim.x, gy = (int)gridDim.y, T = gx * gy;
+  *tile_n = (int)blockIdx.x;
+  *tile_h = (int)blockIdx.y;
+  if (T % 8 == 0 && gx % 4 == 0) {
+    const int L = *tile_n + gx * *tile_h;
+    const int t = (L % 8) * (T / 8) + L / 8;
+    const int band = t / (4 * gy), r = t - band * (4 * gy);
+    *tile_n = band * 4 + r % 4;
+    *tile_h = r / 4;
+  }
+}
+
+// The tile of a workgroup leaves the accumulators of its four waves; `lds`: BIG_EPILOGUE_LDS bytes that nobody reads any more.
+constexpr int BIG_EPP = 128 + 4;                             // floats per staged row
+constexpr int BIG_EPILOGUE_LDS = 4 * 32 * BIG_EPP * 4;
+template <int NSEG>
+__device__ __forceinline__ void store_big_tile(floatx16_t (&acc)[4][4], uint16_t* lds, int wave, int64_t n0, int wn, int wh, int64_t j0, int64_t SEG,
+                                               int64_t N_out, int64_t H, float alpha, float beta, void* __restrict__ out, int out_f32,
+                                               float* __restrict__ partial) {
+  constexpr int HS = WH / NSEG;
+  const int lane = threadIdx.x & 63;
+  // ---- epilogue.  A lane holds column (lane mod 32), rows 8*(v/4) + 4*(lane/32) + (v mod 4) of each 32x32 tile.  The
+  // wave turns 32 rows x 128 columns at a time around in a private piece of LDS so that every lane stores eight
+  // neighbouring columns (16 bytes of bf16, 32 of fp32) and a row leaves as one contiguous run. ----
+  float* ep = reinterpret_cast<float*>(lds) + wave * (32 * BIG_EPP);
+  const int er = lane >> 4, ec = 8 * (lane & 15);
+  const int hl = wh + ec;                                    // first of the lane's columns inside the tile
+  const int64_t h = (int64_t)(hl / HS) * SEG + j0 + (hl % HS);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) ep[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * BIG_EPP + 32 * b + (lane & 31)] = acc[a][b][v];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (one wave: LDS keeps its order, the compiler must too)
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      const int r = 4 * p + er;
+      const int64_t n = n0 + wn + 32 * a + r;
+      float4 lo = *reinterpret_cast<const float4*>(&ep[r * BIG_EPP + ec]);
+      float4 hi = *reinterpret_cast<const float4*>(&ep[r * BIG_EPP + ec + 4]);
+      if (n < N_out) {
+        if (partial != nullptr) {
+          float4* o = reinterpret_cast<float4*>(partial + ((int64_t)blockIdx.z * N_out + n) * H + h);
+          o[0] = lo; o[1] = hi;
+        } else if (out_f32) {
+          float4* o = reinterpret_cast<float4*>(static_cast<float*>(out) + n * H + h);
+          float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0;
+          if (beta != 0.f) { p0 = o[0]; p1 = o[1]; }
+          o[0] = make_float4(alpha * lo.x + beta * p0.x, alpha * lo.y + beta * p0.y, alpha * lo.z + beta * p0.z, alpha * lo.w + beta * p0.w);
+          o[1] = make_float4(alpha * hi.x + beta * p1.x, alpha * hi.y + beta * p1.y, alpha * hi.z + beta * p1.z, alpha * hi.w + beta * p1.w);
+        } else {
+          uint4* o = reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + n * H + h);
+          uint4 q = make_uint4(0, 0, 0, 0);
+          if (beta != 0.f) q = *o;
+          auto mix = [&](float x0, float x1, uint32_t old) __attribute__((always_inline)) {
+            return pack_bf16(alpha * x0 + beta * bf_to_f((uint16_t)(old & 0xFFFFu)), alpha * x1 + beta * bf_to_f((uint16_t)(old >> 16)));
+          };
+          *o = make_uint4(mix(lo.x, lo.y, q.x), mix(lo.z, lo.w, q.y), mix(hi.x, hi.y, q.z), mix(hi.z, hi.w, q.w));
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
+template <int BITS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_out, int64_t H,
             const uint8_t* __restrict__ stored, const uint16_t* __restrict__ vals, const uint16_t* __restrict__ scales,
             ChanArgs ca, int CPS, int64_t tokens_per_split, float alpha, float beta,
             void* __restrict__ out, int out_f32, float* __restrict__ partial) {
-  constexpr int NSEG = (SRC == 0) ? Q<BITS>::NSEG : 1;
+  constexpr int NSEG = Q<BITS>::NSEG;
   constexpr int TN = 256;                     // dY features per workgroup
   constexpr int HS = WH / NSEG;               // columns of the tile that come from one segment
-  constexpr int CPR = HS / 8;                 // packed 8-byte chunks (channel scheme) / 16-byte chunks (dense) per token row and segment
+  constexpr int CPR = HS / 8;                 // packed 8-byte chunks per token row and segment
   constexpr int THREADS = 256;
   constexpr int AP = TN + WPAD, BP = WH + WPAD;
   constexpr int NBUF = 3;
@@ -782,25 +853,12 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
 #define HYC_AS(b_) (lds + (b_) * (WK * AP))
 #define HYC_BS(b_) (lds + NBUF * (WK * AP) + (b_) * (WK * BP))
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Which tile: workgroups are dealt to the 8 XCDs in turn (workgroup L of a launch runs on XCD L mod 8) and every XCD
-  // has an L2 of its own, so XCD q takes a contiguous run of tiles in an order that walks 4 feature tiles by all
-  // channel tiles: its workgroups then share 4 dY panels and a short run of x_hat panels instead of 2 and all of them
-  // (1-4 % on real operands: 4096 x 4096 x 11008 dense 328 -> 320 us, INT2 4096^3 138 -> 132 us).
-  int tile_n = (int)blockIdx.x, tile_h = (int)blockIdx.y;
-  {
-    const int gx = (int)gridDim.x, gy = (int)gridDim.y, T = gx * gy;
-    if (T % 8 == 0 && gx % 4 == 0) {
-      const int L = tile_n + gx * tile_h;
-      const int t = (L % 8) * (T / 8) + L / 8;
-      const int band = t / (4 * gy), r = t - band * (4 * gy);
-      tile_n = band * 4 + r % 4;
-      tile_h = r / 4;
-    }
-  }
+  int tile_n, tile_h;
+  big_tile(&tile_n, &tile_h);
   const int64_t n0 = (int64_t)tile_n * TN;
-  const int64_t SEG = (SRC == 0) ? (int64_t)CPS * 8 : H;
+  const int64_t SEG = (int64_t)CPS * 8;
   const int64_t j0 = (int64_t)tile_h * HS;              // first column of the tile inside each segment
   const int64_t m_begin = (int64_t)blockIdx.z * tokens_per_split;
   const int64_t m_end = m_begin + tokens_per_split < M ? m_begin + tokens_per_split : M;
@@ -819,7 +877,7 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
   constexpr int B_PER = (B_ITEMS + THREADS - 1) / THREADS;
   static_assert(B_ITEMS % THREADS == 0 || B_ITEMS < THREADS, "items per stage");
   // Narrow codes give fewer packed words per stage than threads: PARTS threads then share a word, NST segments each.
-  constexpr int PARTS = (SRC == 0 && B_ITEMS < THREADS) ? THREADS / B_ITEMS : 1;
+  constexpr int PARTS = B_ITEMS < THREADS ? THREADS / B_ITEMS : 1;
   constexpr int NST = NSEG / PARTS;                       // segments a thread decodes
   static_assert(NSEG % PARTS == 0 && (PARTS == 1 || PARTS * B_ITEMS == THREADS), "threads per packed word");
   constexpr int NCH = B_PER * NST;                        // 16-byte chunks of the x stage per thread
@@ -832,7 +890,7 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
     uint32_t pw[NST];
 #pragma unroll
     for (int i = 0; i < NST; ++i)
-      pw[i] = (SRC == 0) ? ca.plan[(seg0 + i) * CPS + (int)(j0 / 8) + item0 % CPR] : 0u;
+      pw[i] = ca.plan[(seg0 + i) * CPS + (int)(j0 / 8) + item0 % CPR];
     co.init(pw);
   }
 
@@ -841,7 +899,7 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
   // reads zeros, and the addresses are per-thread constants.
   const uint32_t gpr = (uint32_t)ca.groups_per_row, kk2 = 2u * (uint32_t)ca.k;
   const uint32_t a_pitch = 2u * (uint32_t)ldy;
-  const uint32_t b_pitch = (SRC == 0) ? (uint32_t)SEG : 2u * (uint32_t)H;          // bytes per token of the x operand
+  const uint32_t b_pitch = (uint32_t)SEG;                                   // bytes per token of the x operand
   uint32_t va[A_PER], vb[B_PER], vs[B_PER][NST], vo0[B_PER][NST], vo1[B_PER][NST];
   int a_at[A_PER], b_at[NCH];                                                       // element offsets inside an LDS buffer
 #pragma unroll
@@ -855,19 +913,14 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
   for (int u = 0; u < B_PER; ++u) {
     const int idx = item0 + u * THREADS;
     const int row = idx / CPR, cc = idx % CPR;
-    if (SRC == 0) {
-      const int c = (int)(j0 / 8) + cc;
-      vb[u] = (uint32_t)row * b_pitch + 8u * c;
+    const int c = (int)(j0 / 8) + cc;
+    vb[u] = (uint32_t)row * b_pitch + 8u * c;
 #pragma unroll
-      for (int i = 0; i < NST; ++i) {
-        vs[u][i] = 2u * ((uint32_t)row * gpr + (uint32_t)(((seg0 + i) * CPS + c) >> ca.chunk_to_group_shift));
-        vo0[u][i] = co.has0[i] ? (uint32_t)row * kk2 + co.vb[i] : NOWHERE;
-        vo1[u][i] = co.has1[i] ? (uint32_t)row * kk2 + co.vb[i] + 2u : NOWHERE;
-        b_at[u * NST + i] = row * BP + (seg0 + i) * HS + 8 * cc;
-      }
-    } else {
-      vb[u] = (uint32_t)row * b_pitch + 2u * ((uint32_t)j0 + 8u * cc);
-      b_at[u] = row * BP + 8 * cc;
+    for (int i = 0; i < NST; ++i) {
+      vs[u][i] = 2u * ((uint32_t)row * gpr + (uint32_t)(((seg0 + i) * CPS + c) >> ca.chunk_to_group_shift));
+      vo0[u][i] = co.has0[i] ? (uint32_t)row * kk2 + co.vb[i] : NOWHERE;
+      vo1[u][i] = co.has1[i] ? (uint32_t)row * kk2 + co.vb[i] + 2u : NOWHERE;
+      b_at[u * NST + i] = row * BP + (seg0 + i) * HS + 8 * cc;
     }
   }
   // Chunks with more than two outlier channels are rare, but one of them must not slow the launch down: the third
@@ -875,34 +928,32 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
   // they are needed; their cache line arrived with the first two) and written over the decoded chunk in LDS.  What
   // that does not cover (a fifth value, a second such chunk in a thread, 8-bit codes, whose register budget is
   // spent) takes patch_more() below; both conditions are wave-uniform.
-  constexpr bool FASTX = SRC == 0 && BITS != 8;
+  constexpr bool FASTX = BITS != 8;
   constexpr int UROW = (THREADS / CPR) * BP;               // elements between a thread's chunks u and u + 1 in an LDS buffer
   bool hasx = false, has4 = false, slow = false;
   int xat2 = 0, xat3 = 0;                                  // LDS element offsets (chunk u = 0) of the two values
   uint32_t vx2 = NOWHERE, vx3 = NOWHERE;                   // their byte offsets in vals, token row 0 of the stage
-  if (SRC == 0) {
 #pragma unroll
-    for (int i = 0; i < NST; ++i) {
-      const int n = __popc(co.m8[i]);
-      if (n > 2) {
-        if (FASTX && !hasx) {
-          hasx = true;
-          uint32_t m = co.m8[i];
-          m &= m - 1; m &= m - 1;
-          xat2 = b_at[i] + (__ffs(m) - 1);
-          vx2 = (uint32_t)((item0 / CPR) * kk2) + co.vb[i] + 4u;
-          m &= m - 1;
-          has4 = m != 0;
-          if (has4) { xat3 = b_at[i] + (__ffs(m) - 1); vx3 = vx2 + 2u; }
-          slow = slow || n > 4;
-        } else {
-          slow = true;
-        }
+  for (int i = 0; i < NST; ++i) {
+    const int n = __popc(co.m8[i]);
+    if (n > 2) {
+      if (FASTX && !hasx) {
+        hasx = true;
+        uint32_t m = co.m8[i];
+        m &= m - 1; m &= m - 1;
+        xat2 = b_at[i] + (__ffs(m) - 1);
+        vx2 = (uint32_t)((item0 / CPR) * kk2) + co.vb[i] + 4u;
+        m &= m - 1;
+        has4 = m != 0;
+        if (has4) { xat3 = b_at[i] + (__ffs(m) - 1); vx3 = vx2 + 2u; }
+        slow = slow || n > 4;
+      } else {
+        slow = true;
       }
     }
   }
   const bool slow_any = __ballot(slow) != 0;
-  const BufferRsrc rs_x = make_rsrc(SRC == 0 && ca.k ? vals + m_begin * (int64_t)ca.k : nullptr,
+  const BufferRsrc rs_x = make_rsrc(ca.k ? vals + m_begin * (int64_t)ca.k : nullptr,
                                     __builtin_amdgcn_readfirstlane((uint32_t)(m_end - m_begin) * kk2));
   // One resource per operand, from the workgroup's first token to the end of its token range; the stage being
   // requested is selected through the scalar offset of the load (the hardware checks the sum of the lane's offset and
@@ -913,24 +964,21 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
   const BufferRsrc rs_a = make_rsrc(dy + m_begin * ldy, (uint32_t)left0 * a_pitch);
   const BufferRsrc rs_b = make_rsrc(reinterpret_cast<const char*>(stored) + m_begin * (int64_t)b_pitch,
                                     __builtin_amdgcn_readfirstlane((uint32_t)left0 * b_pitch));
-  const BufferRsrc rs_s = make_rsrc(SRC == 0 ? scales + m_begin * (int64_t)gpr : nullptr, SRC == 0 ? (uint32_t)left0 * 2u * gpr : 0u);
-  const BufferRsrc rs_o = make_rsrc(SRC == 0 && ca.k ? vals + m_begin * (int64_t)ca.k : nullptr,
+  const BufferRsrc rs_s = make_rsrc(scales + m_begin * (int64_t)gpr, (uint32_t)left0 * 2u * gpr);
+  const BufferRsrc rs_o = make_rsrc(ca.k ? vals + m_begin * (int64_t)ca.k : nullptr,
                                     __builtin_amdgcn_readfirstlane((uint32_t)left0 * kk2));
   uint32_t so_a = 0, so_b = 0, so_s = 0, so_o = 0;                                  // byte offsets of the stage to request next
   auto advance = [&](int part) __attribute__((always_inline)) {                     // four parts, one operand each
     if (part == 0) so_a += WK * a_pitch;
     else if (part == 1) so_b += WK * b_pitch;
-    else if (part == 2 && SRC == 0) so_s += WK * 2u * gpr;
-    else if (part == 3 && SRC == 0) so_o += WK * kk2;
+    else if (part == 2) so_s += WK * 2u * gpr;
+    else so_o += WK * kk2;
     asm volatile("" : "+s"(so_a), "+s"(so_b), "+s"(so_s), "+s"(so_o));              // (in the slot it is written in, in scalar registers)
   };
   // The requests of a stage, numbered: codes and scales (decoded first) before dY and the outlier values.
-  constexpr int NLOAD = A_PER + (SRC == 0 ? B_PER * (1 + 3 * NST) : B_PER);
+  constexpr int NLOAD = A_PER + B_PER * (1 + 3 * NST);
   auto request = [&](Regs& R, int j) __attribute__((always_inline)) {
-    if (SRC != 0) {
-      if (j < B_PER) R.b[j] = load_b128(rs_b, vb[j], so_b);
-      else R.a[j - B_PER] = load_b128(rs_a, va[j - B_PER], so_a);
-    } else if (j < B_PER) {
+    if (j < B_PER) {
       const uint2 pk = load_b64(rs_b, vb[j], so_b);
       R.b[j] = make_uint4(pk.x, pk.y, 0, 0);
     } else if (j < B_PER + NCH) {
@@ -980,16 +1028,12 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
     for (int u = 0; u < A_PER; ++u) *reinterpret_cast<uint4*>(&Ab[a_at[u]]) = R.a[u];
 #pragma unroll
     for (int u = 0; u < B_PER; ++u) {
-      if (SRC == 0) {
 #pragma unroll
-        for (int i = 0; i < NST; ++i)
-          *reinterpret_cast<uint4*>(&Bb[b_at[u * NST + i]]) =
-              co.splice_value(i, dequant8_fast<BITS>(R.b[u].x, R.b[u].y, seg0 + i, bf_to_f((uint16_t)R.s[u][i])), R.o0[u][i], R.o1[u][i]);
-      } else {
-        *reinterpret_cast<uint4*>(&Bb[b_at[u]]) = R.b[u];
-      }
+      for (int i = 0; i < NST; ++i)
+        *reinterpret_cast<uint4*>(&Bb[b_at[u * NST + i]]) =
+            co.splice_value(i, dequant8_fast<BITS>(R.b[u].x, R.b[u].y, seg0 + i, bf_to_f((uint16_t)R.s[u][i])), R.o0[u][i], R.o1[u][i]);
     }
-    if (SRC == 0 && co.more_pairs) patch_more(Bb, mb);
+    if (co.more_pairs) patch_more(Bb, mb);
   };
   bf16x8_t fa0[4], fb0[4], fa1[4], fb1[4];                    // operand fragments of the stage's first / second 16 tokens
   // fragment q of 8 of a 16-token half: the x fragment of the first MFMAs, the four dY fragments, the other three of x
@@ -1048,7 +1092,7 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
         acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t < 16 ? fa0[a] : fa1[a], t < 16 ? fb0[b] : fb1[b], acc[a][b], 0, 0, 0);
       }
       if constexpr (t < 8) read_frag(HYC_AS(B), HYC_BS(B), 16, t, fa1, fb1);
-      if constexpr (SRC == 0 && t < 16) {                               // two elements of chunk c of stage s+1
+      if constexpr (t < 16) {                               // two elements of chunk c of stage s+1
         constexpr int c = t >> 2, w = t & 3;
         const uint32_t src = cw[c][w >> 1];
         float c0, c1;
@@ -1075,12 +1119,9 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
       }
       if constexpr (t >= 20 && t < 24) {
         constexpr int c = t - 20, u = c / NST, i = c % NST;
-        if constexpr (SRC == 0)
-          *reinterpret_cast<uint4*>(&HYC_BS(NB)[b_at[c]]) =
-              co.splice_value(i, make_uint4(res[c][0], res[c][1], res[c][2], res[c][3]), Rd.o0[u][i], Rd.o1[u][i]);
-        else
-          *reinterpret_cast<uint4*>(&HYC_BS(NB)[b_at[c]]) = Rd.b[c];
-        if constexpr (t == 23 && SRC == 0) {
+        *reinterpret_cast<uint4*>(&HYC_BS(NB)[b_at[c]]) =
+            co.splice_value(i, make_uint4(res[c][0], res[c][1], res[c][2], res[c][3]), Rd.o0[u][i], Rd.o1[u][i]);
+        if constexpr (t == 23) {
           if (co.more_pairs) {
             if (FASTX && hasx) {
 #pragma unroll
@@ -1095,7 +1136,7 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
       }
       if constexpr (t == 24) __syncthreads();                           // buffer NB is complete, buffer B read for the last time
       if constexpr (t >= 24) read_frag(HYC_AS(NB), HYC_BS(NB), 0, t - 24, fa0, fb0);
-      if constexpr (SRC == 0 && t >= 24) {                              // for the next stage's decode
+      if constexpr (t >= 24) {                              // for the next stage's decode
         if constexpr ((t & 1) == 0) prepare_codes(Rn, (t - 24) >> 1); else prepare_scale(Rn, (t - 24) >> 1);
         if constexpr (FASTX && (t == 26 || t == 27)) request_extras(m1 + WK, t - 26);
       }
@@ -1104,6 +1145,7 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  static_assert(BIG_EPILOGUE_LDS <= (int)sizeof(lds), "epilogue staging");
   if (m_begin < m_end) {
     Regs R0, R1, R2;
     const int64_t nstages = (m_end - m_begin + WK - 1) / WK;
@@ -1115,11 +1157,9 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
 #pragma unroll
     for (int q = 0; q < 8; ++q) read_frag(HYC_AS(0), HYC_BS(0), 0, q, fa0, fb0);
     int64_t m1 = m_begin + WK;
-    if (SRC == 0) {
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) { prepare_codes(R1, c); prepare_scale(R1, c); }
-      if (FASTX) { request_extras(m1, 0); request_extras(m1, 1); }
-    }
+    for (int c = 0; c < NCH; ++c) { prepare_codes(R1, c); prepare_scale(R1, c); }
+    if (FASTX) { request_extras(m1, 0); request_extras(m1, 1); }
     for (int64_t s = 0; s < nstages; s += 3) {                         // a stage past the end holds zeros
       stage(StageNo<0>{}, R1, R0, R2, m1);
       stage(StageNo<1>{}, R2, R1, R0, m1 + WK);
@@ -1130,52 +1170,135 @@ k_gradw_big(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_o
 #undef HYC_AS
 #undef HYC_BS
 
-  // ---- epilogue.  A lane holds column (lane mod 32), rows 8*(v/4) + 4*(lane/32) + (v mod 4) of each 32x32 tile.  The
-  // wave turns 32 rows x 128 columns at a time around in a private piece of LDS so that every lane stores eight
-  // neighbouring columns (16 bytes of bf16, 32 of fp32) and a row leaves as one contiguous run. ----
-  constexpr int EPP = 128 + 4;                               // floats per staged row
-  static_assert(4 * 32 * EPP * 4 <= (int)sizeof(lds), "epilogue staging");
   __syncthreads();                                           // the last fragments have been read
-  float* ep = reinterpret_cast<float*>(lds) + wave * (32 * EPP);
-  const int er = lane >> 4, ec = 8 * (lane & 15);
-  const int hl = wh + ec;                                    // first of the lane's columns inside the tile
-  const int64_t h = (int64_t)(hl / HS) * SEG + j0 + (hl % HS);
+  store_big_tile<NSEG>(acc, lds, wave, n0, wn, wh, j0, SEG, N_out, H, alpha, beta, out, out_f32, partial);
+}
+
+// dma_b128 at a scalar offset further on in memory
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma_b128_at(u32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
+}
+#pragma clang diagnostic pop
+
+// The same tile for a dense activation (bf16 [M, H]), where nothing has to be decoded on the way: both operands go from
+// memory straight to LDS (8 requests of 1 KB a wave and stage, no registers, no writes to LDS), four buffers of 32 KB, a
+// stage requested three stages ahead.  A slot is one MFMA and one transposing read, the second half of a stage's slots a
+// request every other time; the one barrier waits for nothing young: the next stage was requested two stages ago.  Rows lie
+// unpadded (a request fills two of them); the 64-byte groups of row r are exchanged by r mod 4, so that the four rows of a
+// transposing read lie on different banks.  Same products in the same order as with the operands through registers, whose
+// waits for the writes to LDS left the matrix cores busy for 66 % of the cycles (us, alone): 4096^3 133 -> 124, 8192 x 4096 x 4096
+// 234 -> 220, 4096 x 11008 x 4096 351 -> 327, 3627 x 1024 x 3072 51.7 -> 48.4, 8192 x 256 x 11008 77.7 -> 70.5, 777 x 4096 x 2048
+// 32.9 -> 29.5.  With two reads a slot in half of the slots the small ones gained nothing.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+k_gradw_dense(const uint16_t* __restrict__ dy, int64_t ldy, int64_t M, int64_t N_out, int64_t H, const uint16_t* __restrict__ x,
+              int64_t tokens_per_split, float alpha, float beta, void* __restrict__ out, int out_f32, float* __restrict__ partial) {
+  constexpr int TN = 256, NBUF = 4, TILE = WK * 256;         // elements of one operand's tile
+  __shared__ __align__(1024) uint16_t lds[2 * NBUF * TILE];  // the four of dY, the four of x
+  static_assert(BIG_EPILOGUE_LDS <= (int)sizeof(lds), "epilogue staging");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tile_n, tile_h;
+  big_tile(&tile_n, &tile_h);
+  const int64_t n0 = (int64_t)tile_n * TN, j0 = (int64_t)tile_h * WH;
+  const int64_t m_begin = (int64_t)blockIdx.z * tokens_per_split;
+  const int64_t m_end = m_begin + tokens_per_split < M ? m_begin + tokens_per_split : M;
+  const int wn = (wave >> 1) * 128, wh = (wave & 1) * 128;
+
+  floatx16_t acc[4][4];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+  for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) ep[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * EPP + 32 * b + (lane & 31)] = acc[a][b][v];
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (one wave: LDS keeps its order, the compiler must too)
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
+
+  if (m_begin < m_end) {
+    // One resource per operand, from the workgroup's first token to the end of its range: stages past it arrive as zeros.
+    const int left = (int)(m_end - m_begin);
+    const uint32_t a_pitch = 2u * (uint32_t)ldy, b_pitch = 2u * (uint32_t)H;
+    const u32x4_t rs_a = uniform_rsrc(dy + m_begin * ldy, (uint32_t)left * a_pitch), rs_b = uniform_rsrc(x + m_begin * H, (uint32_t)left * b_pitch);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)&lds[0];
+    uint32_t va[4], vb[4];
+    {
+      const int row = 2 * wave + (lane >> 5), c = (lane & 31) ^ ((row & 3) << 2);
+      const int ca = n0 + 8 * c < N_out ? c : 0;               // features past the end: any others (their rows are not stored)
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-      const int r = 4 * p + er;
-      const int64_t n = n0 + wn + 32 * a + r;
-      float4 lo = *reinterpret_cast<const float4*>(&ep[r * EPP + ec]);
-      float4 hi = *reinterpret_cast<const float4*>(&ep[r * EPP + ec + 4]);
-      if (n < N_out) {
-        if (partial != nullptr) {
-          float4* o = reinterpret_cast<float4*>(partial + ((int64_t)blockIdx.z * N_out + n) * H + h);
-          o[0] = lo; o[1] = hi;
-        } else if (out_f32) {
-          float4* o = reinterpret_cast<float4*>(static_cast<float*>(out) + n * H + h);
-          float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0;
-          if (beta != 0.f) { p0 = o[0]; p1 = o[1]; }
-          o[0] = make_float4(alpha * lo.x + beta * p0.x, alpha * lo.y + beta * p0.y, alpha * lo.z + beta * p0.z, alpha * lo.w + beta * p0.w);
-          o[1] = make_float4(alpha * hi.x + beta * p1.x, alpha * hi.y + beta * p1.y, alpha * hi.z + beta * p1.z, alpha * hi.w + beta * p1.w);
-        } else {
-          uint4* o = reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + n * H + h);
-          uint4 q = make_uint4(0, 0, 0, 0);
-          if (beta != 0.f) q = *o;
-          auto mix = [&](float x0, float x1, uint32_t old) __attribute__((always_inline)) {
-            return pack_bf16(alpha * x0 + beta * bf_to_f((uint16_t)(old & 0xFFFFu)), alpha * x1 + beta * bf_to_f((uint16_t)(old >> 16)));
-          };
-          *o = make_uint4(mix(lo.x, lo.y, q.x), mix(lo.z, lo.w, q.y), mix(hi.x, hi.y, q.z), mix(hi.z, hi.w, q.w));
-        }
+      for (int u = 0; u < 4; ++u) {
+        va[u] = (uint32_t)(row + 8 * u) * a_pitch + 2u * (uint32_t)n0 + 16u * (uint32_t)ca;
+        vb[u] = (uint32_t)(row + 8 * u) * b_pitch + 2u * (uint32_t)j0 + 16u * (uint32_t)c;
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    uint32_t so_a = 0, so_b = 0;                              // byte offsets of the stage to request next
+    const uint32_t lds_wave = lds0 + 1024u * (uint32_t)wave;
+    auto request = [&](uint32_t buf, int j) __attribute__((always_inline)) {      // buf: a buffer's offset in bytes
+      const uint32_t to = lds_wave + buf + 4096u * (uint32_t)(j & 3);
+      if (j < 4) dma_b128_at(rs_a, va[j], so_a, to);
+      else dma_b128_at(rs_b, vb[j - 4], so_b, to + NBUF * 2 * TILE);
+    };
+    auto advance = [&]() __attribute__((always_inline)) { so_a += WK * a_pitch; so_b += WK * b_pitch; };
+    // The eight fragments of a half stage (16 tokens) in the order they are needed in: the first of x, the four of dY, the other
+    // three of x; `at`: the lane's places in the tiles being read (elements).
+    constexpr int FX[4] = {0, 5, 6, 7}, FY = 1;
+    int at[8];
+    {
+      const int g = lane >> 4, s = lane & 15;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int place = (8 * (g >> 1) + (s >> 2)) * 256 + 32 * (q ^ (s >> 2)) + 16 * (g & 1) + 4 * (s & 3);
+        at[FY + q] = place + wn;
+        at[FX[q]] = place + wh + NBUF * TILE;
+      }
+    }
+    bf16x8_t f0[8], f1[8];                                    // of the stage's first / second 16 tokens
+    auto read = [&](int kk, int i, bf16x8_t (&f)[8]) __attribute__((always_inline)) {      // read i of 16: four tokens of fragment i / 2
+      const bf16x4_t v = tr_read(lds + at[i >> 1] + (kk + 4 * (i & 1)) * 256);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[i >> 1][4 * (i & 1) + e] = v[e];
+    };
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) request((uint32_t)s * (2 * TILE), j);
+      advance();
+    }
+    asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 16; ++i) read(0, i, f0);
+    const int stages = (left + WK - 1) / WK;
+    uint32_t rb = 3 * 2 * TILE;                               // the buffer to request into
+    for (int st = 0; st < stages; ++st) {
+      const int step = (st & 3) == 3 ? -3 * TILE : TILE;      // from this buffer to the next
+      auto slot = [&](auto tno) __attribute__((always_inline)) {
+        constexpr int t = decltype(tno)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        {
+          constexpr int a = t & 3, b = (t >> 2) & 3;
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t < 16 ? f0[FY + a] : f1[FY + a], t < 16 ? f0[FX[b]] : f1[FX[b]], acc[a][b], 0, 0, 0);
+        }
+        if constexpr (t < 16) read(16, t, f1);
+        // a place that has been read for the last time moves to the next buffer
+        if constexpr (t >= 2 && t <= 16 && t % 2 == 0) {
+          at[t / 2 - 1] += step;
+          asm volatile("" : "+v"(at[t / 2 - 1]));
+        }
+        // The wave's requests but for the youngest stage's are there; behind the barrier everybody's are, and the buffer of the stage
+        // before this one, which is requested into next, has been read (its fragments were in use by slot 31 of that stage).
+        if constexpr (t == 16) asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+        if constexpr (t >= 16) read(0, t - 16, f0);
+        if constexpr (t > 16 && t % 2 == 1) request(rb, (t - 17) / 2);
+      };
+      for_each_slot(slot, std::make_integer_sequence<int, 32>{});
+      advance();
+      rb = rb == 3 * 2 * TILE ? 0u : rb + 2 * TILE;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // requests past the range still fill buffers
   }
+  __syncthreads();
+  store_big_tile<1>(acc, lds, wave, n0, wn, wh, j0, H, N_out, H, alpha, beta, out, out_f32, partial);
 }
 
 // out = alpha * sum_z partial[z] + beta * out, splits added in increasing z
@@ -1351,21 +1474,22 @@ int hyc_gradw_gemm(const void* dy, int64_t ldy, const void* stored, const void* 
 #define HYC_WIDE()                                                                                               \
   hipLaunchKernelGGL(k_gradw_wide, wgrid, dim3(2 * WN), 0, st, static_cast<const uint16_t*>(dy), ldy, M, N_out, H, \
                      static_cast<const uint16_t*>(stored), tps, alpha, beta, out, of32, partial)
-#define HYC_BIG(B_, S_)                                                                                            \
-  hipLaunchKernelGGL((k_gradw_big<B_, S_>), wgrid, dim3(256), 0, st, static_cast<const uint16_t*>(dy), ldy, M,     \
+#define HYC_BIG(B_)                                                                                                \
+  hipLaunchKernelGGL((k_gradw_big<B_>)    , wgrid, dim3(256), 0, st, static_cast<const uint16_t*>(dy), ldy, M,     \
                      N_out, H, static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),          \
                      static_cast<const uint16_t*>(scales), ca, g.cps, tps, alpha, beta, out, of32, partial)
     if (wnt == WN) {
       HYC_WIDE();
     } else if (chan) {
       switch (d->bits) {
-        case 1: HYC_BIG(1, 0); break;
-        case 2: HYC_BIG(2, 0); break;
-        case 4: HYC_BIG(4, 0); break;
-        default: HYC_BIG(8, 0); break;
+        case 1: HYC_BIG(1); break;
+        case 2: HYC_BIG(2); break;
+        case 4: HYC_BIG(4); break;
+        default: HYC_BIG(8); break;
       }
     } else {
-      HYC_BIG(4, 2);
+      hipLaunchKernelGGL(k_gradw_dense, wgrid, dim3(256), 0, st, static_cast<const uint16_t*>(dy), ldy, M, N_out, H,
+                         static_cast<const uint16_t*>(stored), tps, alpha, beta, out, of32, partial);
     }
 #undef HYC_BIG
 #undef HYC_WIDE
