@@ -1001,7 +1001,15 @@ int hyc_gated_act_bwd_rows(int32_t act, const void* g, const void* stored_a, con
   // Rows of eight waves or more: a CU holds one such workgroup at a time, so one per CU (and row part) with all its
   // rows beats three or four that each fill a table and start from an empty pipeline (4096 x 11008: 64.6 -> 60.1 us,
   // 2048 rows: 39.5 -> 32.8; the same at 16 384 rows; a grid that is not a multiple of the 256 CUs loses up to 15 %).
-  const int64_t cap = threads * parts >= 512 ? 256 : M >= 32768 ? 2048 : threads <= 128 ? 1024 : threads <= 256 ? 768 : 512;
+  // Rows of five to seven waves likewise (4-bit, 2048 x 5632: 512 -> 256 workgroups 28.6 -> 25.9 us); at many rows two of up to six
+  // waves on a CU are ahead again (12 000 x 5120: 256 / 512 workgroups 127 / 117 us, 33 000: 349 / 337, 2048: 350).
+  // 2-bit codes of three or four waves: 512 instead of 768 (4096 x 8192 57.1 -> 50.0 us, 12 000 x 5120 144 -> 123).
+  const int64_t cap = threads * parts >= 512 ? 256
+                      : threads > 256        ? (M > 8192 && threads <= 384 ? 512 : 256)
+                      : M >= 32768           ? 2048
+                      : threads <= 128       ? 1024
+                      : d_a->bits == 2       ? 512
+                                             : 768;
   const int gx = (int)(M < cap ? M : cap);
   const dim3 grid((unsigned)gx, (unsigned)(parts > 1 ? parts : 1));
   hipStream_t st = begin_launch(stream);
@@ -1022,7 +1030,9 @@ int hyc_gated_act_bwd_rows(int32_t act, const void* g, const void* stored_a, con
   } while (0)
 #define HYC_GATED_B(A_)                                                           \
   do {                                                                            \
-    if (d_a->bits == 2) HYC_GATED_T(2, A_); else if (d_a->bits == 4) HYC_GATED_T(4, A_); else HYC_GATED_T(8, A_); \
+    /* (2-bit codes need 233 registers a thread: spilled with 768 threads' share, 2048 x 11008 98 -> 51 us, 4096 x 13824 236 -> 90) */ \
+    if (d_a->bits == 2 && threads > 256 && threads <= 512) HYC_GATED(2, A_, 512);                                  \
+    else if (d_a->bits == 2) HYC_GATED_T(2, A_); else if (d_a->bits == 4) HYC_GATED_T(4, A_); else HYC_GATED_T(8, A_); \
   } while (0)
   if (act == HYC_ACT_SILU) HYC_GATED_B(HYC_ACT_SILU); else HYC_GATED_B(HYC_ACT_GELU_TANH);
 #undef HYC_GATED_B
@@ -1072,10 +1082,15 @@ int hyc_gated_act_fwd(int32_t act, const void* gate, int64_t ld_gate, const void
   const GatedFwdSite sa = {c_a, static_cast<uint8_t*>(stored_a), static_cast<uint16_t*>(vals_a), static_cast<uint16_t*>(scales_a)};
   const GatedFwdSite su = {c_u, static_cast<uint8_t*>(stored_u), static_cast<uint16_t*>(vals_u), static_cast<uint16_t*>(scales_u)};
   const GatedFwdSite sg = {c_g, static_cast<uint8_t*>(stored_g), static_cast<uint16_t*>(vals_g), static_cast<uint16_t*>(scales_g)};
-  const int64_t cap = 256 * (threads * parts >= 512 ? 3 : 8) / parts;
-  // (rows of eight waves or more: one workgroup per CU and row part, as in the gated backward - 4096 x 11008:
-  // 85.7 -> 79.1 us, 4096 x 14336: 124.9 -> 107.5, 2048 x 11008: 48.3 -> 40.0, 16 384 x 11008: 339 -> 321)
-  const int gx = threads * parts >= 512 ? (int)(M < 256 ? M : 256) : (int)(M < cap ? M : cap);
+  // (rows of more than four waves: one workgroup per CU and row part, as in the gated backward - 4096 x 11008: 85.7 -> 79.1
+  // us, 4096 x 14336: 124.9 -> 107.5, 2048 x 11008: 48.3 -> 40.0, 16 384 x 11008: 339 -> 321.  Rows of five to seven waves, 2048 ->
+  // 256 workgroups: 4096 x 5632 65.6 -> 52.1, 2048 x 7168 43.9 -> 31.2, 2-bit 2048 x 11008 95 -> 67; at many rows up to six waves take
+  // two per CU, 12 000 x 5120 146 -> 127, 33 000 352 -> 337.  2-bit codes hold twice the state: 4096 x 8192 in four waves 111 -> 73,
+  // 12 000 x 5120 in three 227 -> 194; in two, 512 workgroups: 4096 x 4096 57.8 -> 45.6, 33 000 rows 290 -> 266)
+  const int64_t cap = threads * parts > 256 ? (M > 8192 && threads * parts <= 384 ? 512 : 256)
+                      : d_a->bits == 2      ? (threads > 128 ? 256 : threads > 64 ? 512 : 2048)
+                                            : 2048;
+  const int gx = (int)(M < cap ? M : cap);
   const dim3 grid((unsigned)gx, (unsigned)parts);
   hipStream_t st = begin_launch(stream);
   const int use_lut = lut_pays(M, gx, threads, LUT_PAYS_OTHER);
