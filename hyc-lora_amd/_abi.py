@@ -104,6 +104,9 @@ SIGNATURES = {
     "hyc_attn_fwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_ptr, c_i64, c_ptr, c_ptr]),
     "hyc_attn_bwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64,
                              c_i64, c_f32, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_ptr]),
+    "hyc_attn_bwd_terms": (c_i32, [c_ptr, c_i64] * 4 + [c_ptr] * 2 + [c_i64] * 4 + [c_f32] + [c_ptr, c_i64] * 3 + [c_ptr, c_ptr]),
+    "hyc_attn_sites_fwd": (c_i32, [c_ptr] * 4 + [c_i64] * 4 + [ctypes.POINTER(HycDesc)] + [c_ptr] * 5),
+    "hyc_attn_sites_bwd": (c_i32, [c_ptr] * 3 + [ctypes.POINTER(HycDesc), c_i32] + [c_i64] * 4 + [c_ptr, c_ptr, c_i64, c_ptr, c_f32, c_ptr, c_ptr]),
     "hyc_attn_kept_fwd": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_ptr, c_i64, c_ptr, c_ptr]),
     "hyc_attn_kept": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_f32, c_f32, c_i64, c_i64, c_ptr, c_ptr, c_i64, c_ptr]),
     "hyc_attn_kept_fill": (c_i32, [c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64, c_i64, c_i64, c_f32, c_f32, c_i64, c_i64, c_ptr, c_ptr, c_i64,

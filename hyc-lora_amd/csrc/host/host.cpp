@@ -959,41 +959,93 @@ bool tables(PyObject* cosv, PyObject* sinv, int64_t n, const Tensor** c, const T
   *s = bf16(sinv);
   return *c && *s && (*c)->is_contiguous() && (*s)->is_contiguous() && (*c)->numel() == n && (*s)->numel() == n;
 }
-// rope_attn_fwd(q, k, v, heads, cos, sin, scale, round_scores) -> (q rows, k rows, out, lse): q and k rotated, and attention on them
+// rope_attn_fwd(q, k, v, heads, cos, sin, scale, round_scores, plans of q, k, v (and out) or None, bits, group)
+//   -> (q rows, k rows, out, lse, their ChannelCompressed or None): q and k rotated, attention on them, and with plans the codes
 PyObject* rope_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  ARGS(8);
-  Tokens q, k, v;
+  ARGS(11);
+  Tokens t[3], &q = t[0], &v = t[2];
   const Tensor *cosv, *sinv;
   const int64_t heads = PyLong_AsLongLong(a[3]);
   const double scale = PyFloat_AsDouble(a[6]);
   if (PyErr_Occurred()) return nullptr;
-  if (!q.init(a[0]) || !k.init(a[1]) || !v.init(a[2]) || !q.same(k) || !q.same(v) || heads <= 0 || q.H % heads ||
-      !tables(a[4], a[5], q.S * (q.H / heads), &cosv, &sinv))
-    return none();
-  const int64_t hd = q.H / heads;
+  for (int i = 0; i < 3; ++i)
+    if (!t[i].init(a[i]) || !q.same(t[i])) return none();
+  if (heads <= 0 || q.H % heads || !tables(a[4], a[5], q.S * (q.H / heads), &cosv, &sinv)) return none();
+  const int64_t hd = q.H / heads, M = q.B * q.S;
   const bool round_scores = a[7] == Py_True;
-  Tensor qr, kr, out, lse;
+  Out o[4];
+  const int sites = a[8] != Py_None && PyTuple_CheckExact(a[8]) ? (int)PyTuple_GET_SIZE(a[8]) : 0;
+  if (a[8] != Py_None && sites != 3 && sites != 4) return none();
+  for (int i = 0; i < sites; ++i)
+    if (!o[i].init(PyTuple_GET_ITEM(a[8], i), a[9], a[10], M, q.H, q.t->device())) return none();
+  Tensor rows[2], out, lse;
   OR_NONE(unlocked([&] {
     const auto opt = q.t->options();
-    qr = at::empty({q.B, q.S, q.H}, opt);
-    kr = at::empty({q.B, q.S, q.H}, opt);
+    for (Tensor& r : rows) r = at::empty({q.B, q.S, q.H}, opt);
+    const void* x[3] = {q.t->data_ptr(), t[1].t->data_ptr(), v.t->data_ptr()};
+    const int64_t ldx[3] = {q.pitch, t[1].pitch, v.pitch};
+    int rc = HYC_ENOTSUP;
+    if (sites) {
+      void *rp[3] = {rows[0].data_ptr(), rows[1].data_ptr(), nullptr}, *st[3], *va[3], *sc[3];
+      hyc_desc d[3];
+      for (int i = 0; i < 3; ++i) {
+        o[i].alloc();
+        st[i] = o[i].stored.data_ptr(); va[i] = o[i].vals.data_ptr(); sc[i] = o[i].scales.data_ptr(); d[i] = o[i].d;
+      }
+      rc = hyc_attn_sites_fwd(x, ldx, cosv->data_ptr(), sinv->data_ptr(), q.B, q.S, heads, hd, d, rp, st, va, sc, stream());
+    }
+    const bool one_by_one = rc == HYC_ENOTSUP;
+    auto compress_site = [&](int i, const void* xi, int64_t ld) {
+      return hyc_compress_rows(xi, ld, M, q.H, &o[i].d, o[i].stored.data_ptr(), o[i].vals.data_ptr(), o[i].scales.data_ptr(), nullptr, stream());
+    };
+    if (one_by_one) {
+      rc = 0;
+      for (int i = 0; i < 2 && !rc; ++i)
+        rc = hyc_rope_to_heads(x[i], ldx[i], cosv->data_ptr(), sinv->data_ptr(), q.B, q.S, heads, hd, nullptr, rows[i].data_ptr(), stream());
+      for (int i = 0; i < 3 && sites && !rc; ++i) rc = i < 2 ? compress_site(i, rows[i].data_ptr(), q.H) : compress_site(i, x[2], ldx[2]);
+    }
+    if (rc) return rc;
     out = at::empty({q.B, q.S, q.H}, opt);
     lse = empty_like_on(*q.t, {q.B, heads, q.S}, at::kFloat);
-    int rc = hyc_rope_to_heads(q.t->data_ptr(), q.pitch, cosv->data_ptr(), sinv->data_ptr(), q.B, q.S, heads, hd, nullptr, qr.data_ptr(), stream());
-    if (!rc) rc = hyc_rope_to_heads(k.t->data_ptr(), k.pitch, cosv->data_ptr(), sinv->data_ptr(), q.B, q.S, heads, hd, nullptr, kr.data_ptr(), stream());
-    if (!rc)
-      rc = (round_scores ? hyc_attn_kept_fwd : hyc_attn_fwd)(qr.data_ptr(), q.H, kr.data_ptr(), q.H, v.t->data_ptr(), v.pitch, q.B, q.S, heads, hd,
-                                                             (float)scale, out.data_ptr(), q.H, (float*)lse.data_ptr(), stream());
-    return rc;
+    rc = (round_scores ? hyc_attn_kept_fwd : hyc_attn_fwd)(rows[0].data_ptr(), q.H, rows[1].data_ptr(), q.H, v.t->data_ptr(), v.pitch, q.B, q.S, heads, hd,
+                                                           (float)scale, out.data_ptr(), q.H, (float*)lse.data_ptr(), stream());
+    if (rc || sites < 4) return rc;
+    o[3].alloc();
+    return compress_site(3, out.data_ptr(), q.H);
   }));
-  PyObject* t = PyTuple_New(4);
-  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(qr));
-  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(kr));
-  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(out));
-  PyTuple_SET_ITEM(t, 3, THPVariable_Wrap(lse));
-  return t;
+  PyObject* saved = sites ? PyTuple_New(sites) : none();
+  for (int i = 0; i < sites; ++i) {
+    PyObject* c = o[i].wrap();
+    if (!c) { Py_DECREF(saved); return nullptr; }
+    PyTuple_SET_ITEM(saved, i, c);
+  }
+  PyObject* r = PyTuple_New(5);
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(rows[0]));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(rows[1]));
+  PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(out));
+  PyTuple_SET_ITEM(r, 3, THPVariable_Wrap(lse));
+  PyTuple_SET_ITEM(r, 4, saved);
+  return r;
   END_HANDLE_TH_ERRORS
+}
+// q, k and v (and the row terms of the backward from the output's codes, with n = 4) out of their codes, in one launch where
+// hyc_attn_sites_bwd covers them: HYC_ENOTSUP where not, before anything is launched
+int restore_sites(In* in, int n, const Tokens& g, int64_t heads, const Tensor* lse, double scale, Tensor* x, Tensor* ws) {
+  for (int i = 0; i < n; ++i)
+    if (in[i].restore_first) return HYC_ENOTSUP;
+  const void *st[4], *va[4], *sc[4];
+  void* to[4] = {};
+  hyc_desc d[4];
+  for (int i = 0; i < n; ++i) {
+    st[i] = in[i].codes(); va[i] = in[i].values(); sc[i] = in[i].group_scales(); d[i] = in[i].d;
+    if (i >= 3) continue;
+    x[i] = empty_like_on(in[i].stored, {in[i].M, in[i].H}, BF16);
+    to[i] = x[i].data_ptr();
+  }
+  if (n == 4) *ws = empty_like_on(*g.t, {2 * g.B * heads * g.S}, at::kFloat);
+  return hyc_attn_sites_bwd(st, va, sc, d, n, g.B, g.S, heads, g.H / heads, to, n == 4 ? g.t->data_ptr() : nullptr, g.H,
+                            n == 4 ? (const float*)lse->data_ptr() : nullptr, (float)scale, n == 4 ? (float*)ws->data_ptr() : nullptr, stream());
 }
 // attn_bwd(g [B, S, H], [c_q, c_k, c_v, c_out], lse, heads, cos, sin, scale, room or None) -> (dq, dk, dv, their common matrix or None).
 // The list is the call's to empty: once the four are restored their codes go, and the gradients take that room.
@@ -1011,12 +1063,16 @@ PyObject* attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
       PyList_GET_SIZE(a[1]) != 4)
     return none();
   const int64_t room = room_of(a[7]);
-  Tensor x[4];
+  Tensor x[4], ws;
+  bool terms = false;                                                  // the output went into the row terms, not into x[3]
   {
     In in[4];
     for (int i = 0; i < 4; ++i)
       if (!in[i].init(PyList_GET_ITEM(a[1], i)) || in[i].M != g.B * g.S || in[i].H != g.H) return none();
     if (!unlocked([&] {
+          const int rc = restore_sites(in, 4, g, heads, lse, scale, x, &ws);
+          terms = rc == 0;
+          if (rc != HYC_ENOTSUP) return terms;
           for (int i = 0; i < 4; ++i)
             if (!in[i].restore(&x[i])) return false;
           return true;
@@ -1028,8 +1084,12 @@ PyObject* attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   std::vector<Tensor> d;
   const int rc = unlocked([&] {
     int64_t pitch;
-    const Tensor ws = empty_like_on(*g.t, {2 * g.B * heads * g.S}, at::kFloat);
+    if (!terms) ws = empty_like_on(*g.t, {2 * g.B * heads * g.S}, at::kFloat);
     side_by_side(*g.t, 3, g.B * g.S, g.H, room, &both, &d, &pitch);
+    if (terms)
+      return hyc_attn_bwd_terms(g.t->data_ptr(), g.H, x[0].data_ptr(), g.H, x[1].data_ptr(), g.H, x[2].data_ptr(), g.H, cosv->data_ptr(),
+                                sinv->data_ptr(), g.B, g.S, heads, g.H / heads, (float)scale, d[0].data_ptr(), pitch, d[1].data_ptr(), pitch,
+                                d[2].data_ptr(), pitch, (float*)ws.data_ptr(), stream());
     return hyc_attn_bwd(g.t->data_ptr(), g.H, x[0].data_ptr(), g.H, x[1].data_ptr(), g.H, x[2].data_ptr(), g.H, x[3].data_ptr(), g.H,
                         (const float*)lse->data_ptr(), cosv->data_ptr(), sinv->data_ptr(), g.B, g.S, heads, g.H / heads, (float)scale, d[0].data_ptr(),
                         pitch, d[1].data_ptr(), pitch, d[2].data_ptr(), pitch, (float*)ws.data_ptr(), stream());
@@ -1095,17 +1155,22 @@ PyObject* attn_kept_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   std::vector<Tensor> d;
   OR_NONE(unlocked([&] {
     Tensor x[3];
-    for (int i = 0; i < 3; ++i)
-      if (!in[i].restore(&x[i])) return -1;
+    int rc = restore_sites(in, 3, g, heads, nullptr, 0.0, x, nullptr);
+    if (rc == HYC_ENOTSUP) {
+      rc = 0;
+      for (int i = 0; i < 3; ++i)
+        if (!in[i].restore(&x[i])) rc = -1;
+    }
+    if (rc) return rc;
     int64_t pitch, first = 0;
     side_by_side(*g.t, 3, g.B * g.S, g.H, room, &both, &d, &pitch);
     for (const Sparse& sp : kept) {
       const int64_t matrices = sp.rows() / g.S;
       const Tensor records = empty_like_on(*g.t, {sp.cols.numel(), 2}, at::kInt);
-      const int rc = hyc_attn_kept_bwd(g.t->data_ptr(), g.H, x[0].data_ptr(), g.H, x[1].data_ptr(), g.H, x[2].data_ptr(), g.H,
-                                       (const int32_t*)sp.row_ptr.data_ptr(), (const int32_t*)sp.cols.data_ptr(), sp.vals.data_ptr(), cosv->data_ptr(),
-                                       sinv->data_ptr(), g.B, g.S, heads, g.H / heads, (float)scale, first, matrices, d[0].data_ptr(), pitch,
-                                       d[1].data_ptr(), pitch, d[2].data_ptr(), pitch, records.data_ptr(), stream());
+      rc = hyc_attn_kept_bwd(g.t->data_ptr(), g.H, x[0].data_ptr(), g.H, x[1].data_ptr(), g.H, x[2].data_ptr(), g.H,
+                             (const int32_t*)sp.row_ptr.data_ptr(), (const int32_t*)sp.cols.data_ptr(), sp.vals.data_ptr(), cosv->data_ptr(),
+                             sinv->data_ptr(), g.B, g.S, heads, g.H / heads, (float)scale, first, matrices, d[0].data_ptr(), pitch,
+                             d[1].data_ptr(), pitch, d[2].data_ptr(), pitch, records.data_ptr(), stream());
       if (rc) return rc;
       first += matrices;
     }

@@ -317,6 +317,21 @@ class CompressedAttention(torch.nn.Module):
         return func.apply(q, k, v, cos, sin, self, grad_room)
 
 
+def _frozen_plans(sites, iteration):
+    """the plans of calibrated sites, None while one of them still looks at what it is given"""
+    if iteration < 2 or any(site.plan is None for site in sites):
+        return None
+    return tuple(site.plan for site in sites)
+
+
+def _compress_sites(sites, tensors, iteration, cfg):
+    out = []
+    for site, t in zip(sites, tensors):
+        t = t.reshape(-1, t.shape[-1])
+        out.append(K.compress_channel(t, site.channel_plan(t, iteration), cfg.act_bits, cfg.act_group))
+    return out
+
+
 def _matrices_per_group(total, s, budget_bytes):
     """[S, S] bf16 score matrices per group: within the budget, and the groups of equal size"""
     most = max(1, min(total, budget_bytes // (2 * s * s)))
@@ -411,21 +426,19 @@ class _AttentionFunc(torch.autograd.Function):
         b, s, H = q.shape
         nh = cfg.heads
         scale = 1.0 / math.sqrt(cfg.head_dim)
-        done = K.native.rope_attn_fwd(q, k, v, nh, cos, sin, scale, True)
+        sites = (mod.site_q, mod.site_k, mod.site_v)
+        done = K.native.rope_attn_fwd(q, k, v, nh, cos, sin, scale, True, _frozen_plans(sites, mod.iteration), cfg.act_bits, cfg.act_group)
         if done is None:
             q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
-            done = (q_rows, k_rows) + K.attn_fwd(q_rows, k_rows, v, nh, scale, round_scores=True)
-        q_rows, k_rows, out, lse = done
+            done = (q_rows, k_rows) + K.attn_fwd(q_rows, k_rows, v, nh, scale, round_scores=True) + (None,)
+        q_rows, k_rows, out, lse, saved = done
         thr, budget = K.threshold_value(mod.static_value), K.kept_budget(mod.static_value)
         cap = K.attn_kept_entries(budget, thr, s, cfg.head_dim) or K.slab_room(cfg.softmax_ratio * s, s)
         # (the slab of kept entries is what grows with the number of matrices here)
         group = max(1, min(b * nh, cfg.attn_group_bytes // (4 * s * cap)))
         ctx.kept = [K.attn_kept(q_rows, k_rows, lse, nh, scale, thr, budget, cap, c0, min(group, b * nh - c0))
                     for c0 in range(0, b * nh, group)]
-        ctx.saved = []
-        for site, r in zip((mod.site_q, mod.site_k, mod.site_v), (q_rows, k_rows, v)):
-            r = r.reshape(b * s, H)
-            ctx.saved.append(K.compress_channel(r, site.channel_plan(r, mod.iteration), cfg.act_bits, cfg.act_group))
+        ctx.saved = saved or _compress_sites(sites, (q_rows, k_rows, v), mod.iteration, cfg)
         mod.iteration += 1
         ctx.geom, ctx.grad_room = (b, nh, s, cfg.head_dim), grad_room
         ctx.save_for_backward(cos, sin)
@@ -494,13 +507,15 @@ class _FlashAttentionFunc(torch.autograd.Function):
         scale = 1.0 / math.sqrt(hd)
         pitch = H if grad_room is None else 3 * H + grad_room       # of the gradients
         ctx.rows = K.attn_supported(hd, s, max(v.stride(1), pitch), b * nh)
-        seed = offset = None
+        sites, it = (mod.site_q, mod.site_k, mod.site_v, mod.site_o), mod.iteration
+        seed = offset = saved = None
         if ctx.rows:                                                # the kernels read and write the rows as they are
-            done = K.native.rope_attn_fwd(q, k, v, nh, cos, sin, scale, False)
+            plans = _frozen_plans(sites, it) if cfg.compress else None
+            done = K.native.rope_attn_fwd(q, k, v, nh, cos, sin, scale, False, plans, cfg.act_bits, cfg.act_group)
             if done is None:
                 q_rows, k_rows = K.rope_rows(q, nh, cos, sin), K.rope_rows(k, nh, cos, sin)
-                done = (q_rows, k_rows) + K.attn_fwd(q_rows, k_rows, v, nh, scale)
-            q_rows, k_rows, out, lse = done
+                done = (q_rows, k_rows) + K.attn_fwd(q_rows, k_rows, v, nh, scale) + (None,)
+            q_rows, k_rows, out, lse, saved = done
             ctx.grad_room = grad_room
         else:
             qh, q_rows = K.rope_to_heads(q, nh, cos, sin, want_rows=True)
@@ -512,11 +527,8 @@ class _FlashAttentionFunc(torch.autograd.Function):
             out = K.rope_from_heads(out_h)                          # [B, S, H]
             del out_h
         rows = [t.reshape(b * s, H) for t in (q_rows, k_rows, v, out)]
-        it = mod.iteration
         if cfg.compress:
-            saved = []
-            for site, r in zip((mod.site_q, mod.site_k, mod.site_v, mod.site_o), rows):
-                saved.append(K.compress_channel(r, site.channel_plan(r, it), cfg.act_bits, cfg.act_group))
+            saved = saved or _compress_sites(sites, rows, it, cfg)
         else:
             saved = [r.contiguous() for r in rows]
         mod.iteration += 1

@@ -385,6 +385,23 @@ int hyc_attn_bwd(const void* dout, int64_t ldg, const void* q, int64_t ldq, cons
                  const void* out, int64_t ldo, const float* lse, const void* cosv, const void* sinv, int64_t B, int64_t S,
                  int64_t heads, int64_t head_dim, float scale, void* dq, int64_t lddq, void* dk, int64_t lddk, void* dv,
                  int64_t lddv, float* workspace, void* stream);
+int hyc_attn_bwd_terms(const void* dout, int64_t ldg, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv,
+                       const void* cosv, const void* sinv, int64_t B, int64_t S, int64_t heads, int64_t head_dim, float scale, void* dq,
+                       int64_t lddq, void* dk, int64_t lddk, void* dv, int64_t lddv, float* workspace, void* stream);
+
+/* The saved activations around it in one launch each way, for channel codes of 4 or 8 bits in groups of 64 or 128 (the same for all)
+ * where a row fits one workgroup and the segments of a packed row hold whole heads; HYC_ENOTSUP for the rest.
+ *   hyc_attn_sites_fwd  x = {q, k, v} [B S, heads head_dim] (rows ldx apart): rows[0] and rows[1] = q and k through
+ *                       hyc_rope_to_heads' rotation (rows[2] is not used), and the codes hyc_compress makes of those and of v
+ *   hyc_attn_sites_bwd  n = 3: xhat[0 .. 2] = what hyc_decompress restores.  n = 4: also the row terms of the backward from the
+ *                       fourth tensor's codes (the attention's output), dout and lse, where hyc_attn_bwd_terms (hyc_attn_bwd
+ *                       without its out and lse) finds them: workspace, 2 * B * heads * S floats */
+int hyc_attn_sites_fwd(const void* const* x, const int64_t* ldx, const void* cosv, const void* sinv, int64_t B, int64_t S, int64_t heads,
+                       int64_t head_dim, const hyc_desc* d, void* const* rows, void* const* stored, void* const* vals, void* const* scales,
+                       void* stream);
+int hyc_attn_sites_bwd(const void* const* stored, const void* const* vals, const void* const* scales, const hyc_desc* d, int32_t n, int64_t B,
+                       int64_t S, int64_t heads, int64_t head_dim, void* const* xhat, const void* dout, int64_t ldg, const float* lse, float scale,
+                       float* workspace, void* stream);
 
 /* The attention that keeps its probabilities: scores are rounded to bf16, x = bf16(scale q.k), and of matrices
  * [first, first + matrices) (matrix = b heads + h) the entries whose p = bf16(exp(x - lse)) exceeds bf16(threshold) are kept as
