@@ -290,24 +290,30 @@ struct LoraUp {
   int n_out[LORA_MAX], fb0[LORA_MAX + 1], row0[LORA_MAX + 1];   // first feature block / first stacked row of projection i
   int n, r;
 };
-constexpr int LU_F = 256, LU_M = 64;                     // features of a workgroup, tokens of a tile
+constexpr int LU_F = 256, LU_M = 32;                     // features of a workgroup, tokens of a tile
 
 __device__ __forceinline__ int lu_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
-// A workgroup owns 256 features and a range of tokens, walked in tiles of 64 that go from memory straight to LDS (two
-// buffers of 32 KB, two workgroups per CU).  From a tile, wave w takes the 16 tokens 16 w .. for dh (all 256 features, the
-// B factors in registers) and the 64 features 64 w .. for dB (all 64 tokens): dY rows as stored are the operand of the
-// first, the transposing read gives that of the second, and no sum crosses a wave.  dh leaves as one fp32 partial per
-// feature block, dB as one per token range; k_lora_up_finish adds them in a fixed order.  The read of dY should bound it; 4096
-// tokens x 4096 / 3 x 4096 / 2 x 11008 features take 14 / 34 / 68 us, 2.3 to 3.0 TB/s of dY (3.2 with the partial results; LDS
-// busy for a tenth of the cycles, matrix cores for 4 %): the wait for the next tile also waits for the stores of this one.
-template <int RT>
+// A workgroup owns 256 features and a range of tokens, walked in tiles of 32 that go from memory straight to LDS, NB of them
+// under way (two workgroups per CU).  From a tile, wave w takes the 64 features 64 w .. for both products: dY rows as stored
+// are the operand of dh (the wave's part of B in registers), the transposing read gives that of dB.  The waves' sums for dh meet in
+// LDS.  dh leaves as one fp32 partial per feature block, dB as one per token range; k_lora_up_finish adds them in a fixed order.
+//
+// The read of dY bounds it, so nothing may empty the queue of loads: every memory operation of the walk is unconditional (what
+// lies outside its resource is dropped, or reads zeros) and a wave waits for its oldest tile by count, over the stores behind it.
+// Both launches at 4096 tokens x 4096 with the copy / 3 x 4096 / 2 x 11008 features: 25.9 / 33.8 / 49.4 -> 21.8 / 26.6 / 40.5 us against two
+// buffers of 64 tokens, waited for with the stores, and a grid that was a little more than resident (2048 tokens: 16.9 / 25.8 / 31.3 -> 14.3 /
+// 18.7 / 27.9; 157 tokens x 2048 / 3 x 2048 / 2 x 5632: 10.8 / 10.9 / 11.7 -> 8.3 / 9.2 / 8.8).  dY then arrives at up to 4.9 TB/s.
+template <int RT, bool COPY>
 __global__ void __launch_bounds__(256, 2)
 k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, float* __restrict__ dhp, float* __restrict__ dbp,
               uint16_t* __restrict__ copy, int64_t ld_copy) {
   constexpr int RC = 16 * RT;                            // columns of the factor, padded
-  __shared__ __align__(1024) uint16_t tile[2][LU_M * LU_F];
-  __shared__ __align__(1024) uint16_t ht[2][LU_M * RC];
+  constexpr int NB = RT == 1 ? 4 : 3;                    // (76 and 70 KB of LDS)
+  constexpr int S = COPY ? 5 : 1;                        // stores of a wave per tile
+  __shared__ __align__(1024) uint16_t tile[NB][LU_M * LU_F];
+  __shared__ __align__(1024) uint16_t ht[NB][LU_M * RC];
+  __shared__ __align__(16) float red[4][LU_M * RC];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, lq = lane >> 4;
   const int fb = blockIdx.x;
   int p = 0;
@@ -317,49 +323,62 @@ k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, f
   const int count = (int)(m_end - m_begin), tiles = (count + LU_M - 1) / LU_M;
   const uint32_t pitch = (uint32_t)a.ldg[p] * 2u;
   const uint16_t* base = a.g[p] + m_begin * a.ldg[p] + f0;
-  // (the resource ends with the last row's last feature of this block)
+  // (the resources end with the last row's last feature of this block: tokens past the range and features past the end are zeros)
   const int fl = n_out - f0 < LU_F ? n_out - f0 : LU_F;  // features this block really has, a multiple of 8
   const u32x4_t rs = uniform_rsrc(base, (uint32_t)(count - 1) * pitch + 2u * (uint32_t)fl);
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)&tile[0][0];
+  const u32x4_t rs_h = uniform_rsrc(h + m_begin * nr + p * r, 2u * ((uint32_t)(count - 1) * (uint32_t)nr + (uint32_t)r));
+  const uint32_t lds_t = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)&tile[0][0];
+  const uint32_t lds_h = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)&ht[0][0];
   const int ir = lane >> 5, ic = lane & 31;              // an instruction brings two rows of 32 chunks
+  // (the chunk at position ic of row 2 (wave + 4 u) + ir is ic ^ swz(row); swz has a period of 16 rows: that of u + 2)
+  uint32_t vt[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int row = 2 * (wave + 4 * u) + ir, c = ic ^ lu_swz(row & 15);
+    vt[u] = 8 * c < fl ? (uint32_t)row * pitch + 16u * (uint32_t)c : NOWHERE;
+  }
+  const int hrow = (wave * 64 + lane) / (RC / 8), hcol = 8 * ((wave * 64 + lane) % (RC / 8));   // (the first RT waves bring the rows of h)
+  const uint32_t vh = hcol < r ? 2u * ((uint32_t)hrow * (uint32_t)nr + (uint32_t)hcol) : NOWHERE;
   auto issue = [&](int t, int buf) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)(t * LU_M) * pitch;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int row = 2 * (wave + 4 * u) + ir;           // row of the tile; its chunk c lies at position c ^ swz(row)
-      int c = ic ^ lu_swz(row & 15);
-      c = 8 * c < fl ? c : 0;                            // features past the end: any finite values (their factors are zero)
-      const int m = t * LU_M + row < count ? t * LU_M + row : count - 1;
-      const uint32_t dst = lds0 + (uint32_t)(buf * LU_M * LU_F * 2 + (wave + 4 * u) * 1024);
-      dma_b128(rs, (uint32_t)m * pitch + 16u * c, dst);
-    }
+    for (int u = 0; u < 4; ++u) dma_b128(rs, vt[u] == NOWHERE ? NOWHERE : vt[u] + at, lds_t + (uint32_t)(buf * LU_M * LU_F * 2 + (wave + 4 * u) * 1024));
+    if (wave < RT)
+      dma_b128(rs_h, vh == NOWHERE ? NOWHERE : vh + (uint32_t)(t * LU_M) * 2u * (uint32_t)nr, lds_h + (uint32_t)(buf * LU_M * RC * 2 + wave * 1024));
   };
-  // the tile's rows of h (this projection's r columns, zeros behind them and past the range): registers, then LDS
-  constexpr int HC = LU_M * RC / 8;                      // 16-byte chunks: one per thread at RT = 2, half the threads at 1
-  const int hrow = threadIdx.x / (RC / 8), hcol = 8 * (threadIdx.x % (RC / 8));
-  auto load_h = [&](int t) __attribute__((always_inline)) {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    const int m = t * LU_M + hrow;
-    if (threadIdx.x < HC && m < count && hcol < r) v = *reinterpret_cast<const uint4*>(h + (m_begin + m) * nr + p * r + hcol);
-    return v;
+  // tile t has landed.  Behind its loads in the queue are those of up to NB - 1 further tiles and the stores of as many steps (at the
+  // start and the end of the walk the loads alone are counted: the stores then only make the wait longer than it need be)
+  auto landed = [&](int t) __attribute__((always_inline)) {
+    const int ahead = tiles - 1 - t < NB - 1 ? tiles - 1 - t : NB - 1;
+#define HYC_WAIT(L_)                                                                                                         \
+    do {                                                                                                                     \
+      if (ahead == NB - 1 && t >= NB - 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NB - 1) * (L_ + S)) : "memory");         \
+      else if (ahead == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(3 * L_) : "memory");                                    \
+      else if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * L_) : "memory");                                    \
+      else if (ahead == 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(L_) : "memory");                                        \
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                                                  \
+    } while (0)
+    if (wave < RT) HYC_WAIT(5);
+    else HYC_WAIT(4);
+#undef HYC_WAIT
   };
-  auto store_h = [&](int buf, const uint4& v) __attribute__((always_inline)) {
-    if (threadIdx.x < HC) *reinterpret_cast<uint4*>(&ht[buf][hrow * RC + hcol]) = v;
-  };
-  issue(0, 0);
-  uint4 hv = load_h(0);
-  // B as the second operand of dh: lane = column l % 16, 8 consecutive features per reduction step
-  bf16x8_t bf[8][RT];
+  // (LDS operations only: __syncthreads may wait for the loads and stores under way)
+  auto meet = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks)
+  for (int t = 0; t < NB; ++t)
+    if (t < tiles) issue(t, t);
+  // B as the first operand of dh^T: lane = column l % 16, 8 consecutive features per reduction step
+  bf16x8_t bf[2][RT];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int f = f0 + 32 * ks + 8 * lq + j, c = 16 * rt + l15;
+        const int f = f0 + 64 * wave + 32 * ks + 8 * lq + j, c = 16 * rt + l15;
         const uint16_t v = f < n_out && c < r ? a.B[p][(int64_t)f * r + c] : (uint16_t)0;
         bf[ks][rt][j] = __builtin_bit_cast(__bf16, v);
       }
-  store_h(0, hv);
   floatx4_t db[4][RT];
 #pragma unroll
   for (int ft = 0; ft < 4; ++ft)
@@ -373,43 +392,39 @@ k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, f
     f[0] = x[0]; f[1] = x[1]; f[2] = x[2]; f[3] = x[3]; f[4] = y[0]; f[5] = y[1]; f[6] = y[2]; f[7] = y[3];
     return f;
   };
+  const BufferRsrc rs_dh = make_rsrc(dhp + ((int64_t)fb * M + m_begin) * RC, (uint32_t)count * RC * 4u);
+  int buf = 0;
   for (int t = 0; t < tiles; ++t) {
-    const int buf = t & 1;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const bool more = t + 1 < tiles;
-    if (more) { issue(t + 1, buf ^ 1); hv = load_h(t + 1); }
+    landed(t);
+    meet();
     const uint16_t* T = tile[buf];
-    if (copy) {
+    if constexpr (COPY) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int at = threadIdx.x + 256 * u, row = at / 32, c = at % 32;
-        if (t * LU_M + row < count && 8 * c < fl)
-          *reinterpret_cast<uint4*>(copy + (m_begin + t * LU_M + row) * ld_copy + a.row0[p] + f0 + 8 * c) =
-              *reinterpret_cast<const uint4*>(T + row * LU_F + 8 * (c ^ lu_swz(row & 15)));
-      }
-    }
-    floatx4_t dh[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) dh[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    const uint16_t* arow = T + (16 * wave + l15) * LU_F;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      const bf16x8_t x = *reinterpret_cast<const bf16x8_t*>(arow + 8 * ((4 * ks + lq) ^ lu_swz(l15)));
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) dh[rt] = HYC_MFMA16(x, bf[ks][rt], dh[rt]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = t * LU_M + 16 * wave + 4 * lq + i;
-      if (m < count) {
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) dhp[((int64_t)fb * M + m_begin + m) * RC + 16 * rt + l15] = dh[rt][i];
+      for (int u = 0; u < 4; ++u) {
+        const int row0 = 2 * wave + 8 * u, left = count - t * LU_M - row0, c = ic ^ lu_swz((row0 + ir) & 15);
+        const BufferRsrc rs_c = make_rsrc(copy + (m_begin + t * LU_M + row0) * ld_copy + a.row0[p] + f0,
+                                          left > 0 ? 2u * ((left > 1 ? (uint32_t)ld_copy : 0u) + (uint32_t)fl) : 0u);
+        const uint4 v = *reinterpret_cast<const uint4*>(T + (row0 + ir) * LU_F + 8 * ic);
+        const u32x4_t w = {v.x, v.y, v.z, v.w};
+        __builtin_amdgcn_raw_buffer_store_b128(w, rs_c, (int)(8 * c < fl ? (ir ? 2u * (uint32_t)ld_copy : 0u) + 16u * (uint32_t)c : NOWHERE), 0, 0);
       }
     }
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int r0 = 32 * kk + 8 * lq + (l15 >> 2), r1 = r0 + 4;
+    for (int tg = 0; tg < 2; ++tg) {
+      floatx4_t dh[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) dh[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const bf16x8_t x = *reinterpret_cast<const bf16x8_t*>(T + (16 * tg + l15) * LU_F + 8 * ((8 * wave + 4 * ks + lq) ^ lu_swz(l15)));
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) dh[rt] = HYC_MFMA16(bf[ks][rt], x, dh[rt]);
+      }
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<floatx4_t*>(&red[wave][(16 * tg + l15) * RC + 16 * rt + 4 * lq]) = dh[rt];
+    }
+    {
+      const int r0 = 8 * lq + (l15 >> 2), r1 = r0 + 4;
       bf16x8_t hb[RT];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
@@ -425,7 +440,24 @@ k_lora_up_bwd(LoraUp a, int64_t M, const uint16_t* __restrict__ h, int tokens, f
         for (int rt = 0; rt < RT; ++rt) db[ft][rt] = HYC_MFMA16(x, hb[rt], db[ft][rt]);
       }
     }
-    if (more) store_h(buf ^ 1, hv);
+    meet();
+    if (t + NB < tiles) issue(t + NB, buf);
+    {
+      typedef float sum_t __attribute__((ext_vector_type(2 * RT)));
+      const int e = 2 * RT * threadIdx.x;
+      sum_t s = *reinterpret_cast<const sum_t*>(&red[0][e]);
+#pragma unroll
+      for (int w = 1; w < 4; ++w) s += *reinterpret_cast<const sum_t*>(&red[w][e]);
+      const uint32_t off = 4u * (uint32_t)(t * LU_M * RC + e);
+      if constexpr (RT == 1) {
+        const u32x2_t w = __builtin_bit_cast(u32x2_t, s);    // (the whole vector: a bit cast of one element reads the first)
+        store_b64(rs_dh, off, w.x, w.y);
+      } else {
+        const u32x4_t w = __builtin_bit_cast(u32x4_t, s);
+        __builtin_amdgcn_raw_buffer_store_b128(w, rs_dh, (int)off, 0, 0);
+      }
+    }
+    buf = buf + 1 < NB ? buf + 1 : 0;
   }
   float* o = dbp + ((int64_t)blockIdx.y * a.row0[a.n] + a.row0[p] + f0) * RC;
 #pragma unroll
@@ -508,14 +540,25 @@ static int lora_group(const char* who, const void* const* factors, const int64_t
   return HYC_OK;
 }
 
-// token ranges of k_lora_up_bwd: enough workgroups for two per CU, whole tiles each, at most 32 (the partial dB) unless that
-// leaves a range more than 32768 tokens (its offsets into dY are 31-bit numbers of bytes up to row pitches of 32760)
+// Token ranges of k_lora_up_bwd, whole tiles each.  512 workgroups are resident at once, two per CU: of the ranges that make a
+// workgroup's share of the walk shortest, rounds included, the fewest (each is one more partial dB).  A workgroup's start and end
+// count as LU_FIXED tiles.  One workgroup too many is a round of its own: us with 10 / 12 ranges of 4096 x 3 x 4096 26.8 / 31.2, with
+// 5 / 6 of 4096 x 2 x 11008 40.6 / 47.4.  At most 32, unless that leaves a range more than 32768 tokens (its offsets into dY are
+// 31-bit numbers of bytes up to row pitches of 32760).
+constexpr int64_t LU_FIXED = 3;
+static int64_t lora_up_tokens(int64_t M, int64_t fblocks) {
+  const int64_t tiles = (M + LU_M - 1) / LU_M, least = (M + 32767) / 32768;
+  int64_t best = 0, best_cost = 0;
+  for (int64_t n = 1; n <= 32 && n <= tiles; ++n) {
+    const int64_t each = (tiles + n - 1) / n, used = (tiles + each - 1) / each, cost = (fblocks * used + 511) / 512 * (each + LU_FIXED);
+    if (!best || cost < best_cost) { best = each; best_cost = cost; }
+  }
+  const int64_t most = least > 0 ? (tiles + least - 1) / least : 1;
+  return LU_M * (best < most ? (best > 0 ? best : 1) : most);
+}
 static int lora_up_ranges(int64_t M, int fblocks) {
-  int64_t want = (512 + fblocks - 1) / fblocks, most = (M + LU_M - 1) / LU_M;
-  if (want > most) want = most;
-  if (want > 32) want = 32;
-  if (want < (M + 32767) / 32768) want = (M + 32767) / 32768;
-  return (int)(want < 1 ? 1 : want);
+  const int64_t tokens = lora_up_tokens(M, fblocks);
+  return M > 0 ? (int)((M + tokens - 1) / tokens) : 1;
 }
 static int lora_up_blocks(const int64_t* n_out, int n) {
   int64_t b = 0;
@@ -664,20 +707,24 @@ int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const 
     a.fb0[i + 1] = a.fb0[i] + (int)((n_out[i] + LU_F - 1) / LU_F);
     a.row0[i + 1] = a.row0[i] + (int)n_out[i];
   }
-  const int fblocks = a.fb0[n], ranges = lora_up_ranges(M, fblocks);
-  int64_t tokens = (M + ranges - 1) / ranges;
-  tokens = (tokens + LU_M - 1) / LU_M * LU_M;
+  const int fblocks = a.fb0[n];
+  const int64_t tokens = lora_up_tokens(M, fblocks);
   for (int i = 0; i < n; ++i)
     if (tokens * ldg[i] >= ((int64_t)1 << 30)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: a token range of dy must stay below 2 GiB");
+  if (copy_dy && ld_ext >= ((int64_t)1 << 29)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: rows %lld apart", (long long)ld_ext);
   const int used = M ? (int)((M + tokens - 1) / tokens) : 0;   // (no tokens: the sums below are empty and dB is zero)
   const int RC = r <= 16 ? 16 : 32;
   float *dhp = static_cast<float*>(workspace), *dbp = dhp + (int64_t)fblocks * M * RC;
   uint16_t* cp = copy_dy ? static_cast<uint16_t*>(ext) : nullptr;
   hipStream_t st = begin_launch(stream);
   const dim3 grid((unsigned)fblocks, (unsigned)used);
-  if (M == 0) {}
-  else if (RC == 16) hipLaunchKernelGGL((k_lora_up_bwd<1>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
-  else hipLaunchKernelGGL((k_lora_up_bwd<2>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext);
+#define HYC_GO(RT_, COPY_)                                                                                                   \
+  hipLaunchKernelGGL((k_lora_up_bwd<RT_, COPY_>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext)
+  if (M > 0) {
+    if (RC == 16) { if (cp) HYC_GO(1, true); else HYC_GO(1, false); }
+    else { if (cp) HYC_GO(2, true); else HYC_GO(2, false); }
+  }
+#undef HYC_GO
   if ((rc = check_launch("hyc_lora_up_bwd"))) return rc;
   const int64_t per = 256 / RC, token_blocks = (M + per - 1) / per, blocks = n * token_blocks + (rows + per - 1) / per;
   if (blocks >= ((int64_t)1 << 31)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: too many tokens");
