@@ -13,11 +13,17 @@
 #include <ATen/ATen.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <string>
 #include <vector>
 
 #include "../../../include/hyc_abi.h"
@@ -28,7 +34,7 @@ using at::Tensor;
 constexpr auto BF16 = at::kBFloat16;
 
 // torch.nn.Parameter, kernels.ChannelCompressed, ChannelPlan, ThresholdCompressed, SparseRows
-PyObject *t_parameter, *t_compressed, *t_plan, *t_threshold, *t_sparse;
+PyObject *t_parameter, *t_compressed, *t_plan, *t_threshold, *t_sparse, *t_namespace /* types.SimpleNamespace */;
 PyObject *s_H, *s_M, *s_S, *s_k, *s_idx, *s_plan, *s_scale_rule, *s_stored, *s_vals, *s_scales, *s_bits, *s_group, *s_row_ptr, *s_cols, *s_threshold,
     *s_scale, *s_L, *s_R;
 
@@ -53,11 +59,11 @@ auto unlocked(F&& f) {
 }
 
 // a dense GPU tensor of the exact type (a subclass may do anything on access, a functorch wrapper has no memory of its own)
+bool dense_gpu(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && !t.is_conj() && !t.is_neg(); }
 const Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o) && (PyObject*)Py_TYPE(o) != t_parameter) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.is_conj() || t.is_neg()) return nullptr;
-  return &t;
+  return dense_gpu(t) ? &t : nullptr;
 }
 const Tensor* bf16(PyObject* o) {
   const Tensor* t = plain(o);
@@ -135,35 +141,6 @@ bool get_plan(PyObject* o, int64_t H, c10::Device device, Plan* p) {
   return true;
 }
 
-// a compressed activation about to be written
-struct Out {
-  Tensor stored, vals, scales;
-  hyc_desc d;
-  Plan p;
-  PyObject *plan, *bits, *group;
-  int64_t M, H, b, g;
-  bool init(PyObject* plan_, PyObject* bits_, PyObject* group_, int64_t M_, int64_t H_, c10::Device device) {
-    plan = plan_; bits = bits_; group = group_; M = M_; H = H_;
-    if (!PyLong_CheckExact(bits) || !PyLong_CheckExact(group)) return false;
-    b = PyLong_AsLongLong(bits);
-    g = PyLong_AsLongLong(group);
-    if (hyc_check_shape(H, (int32_t)b, (int32_t)g, HYC_MODE_CHANNEL) != 0 || !get_plan(plan, H, device, &p)) return false;
-    p.describe(b, g, &d);
-    return true;
-  }
-  void alloc() {
-    const auto opt = at::TensorOptions().device(p.plan.device());
-    stored = at::empty({M, H * b / 8}, opt.dtype(b == 8 ? at::kChar : at::kByte));
-    vals = at::empty({M, p.k}, opt.dtype(BF16));
-    scales = at::empty({M, H / g}, opt.dtype(BF16));
-  }
-  PyObject* wrap() const {                                             // kernels.ChannelCompressed(stored, vals, scales, plan, bits, group, M, H)
-    Ref a(THPVariable_Wrap(stored)), b(THPVariable_Wrap(vals)), c(THPVariable_Wrap(scales)), m(PyLong_FromLongLong(M)), h(PyLong_FromLongLong(H));
-    if (!a.p || !b.p || !c.p || !m.p || !h.p) return nullptr;
-    PyObject* args[8] = {a.p, b.p, c.p, plan, bits, group, m.p, h.p};
-    return PyObject_Vectorcall(t_compressed, args, 8, nullptr);
-  }
-};
 // the threshold scheme's descriptor: a static scale read through two strides, a base of rank 0 or more
 struct Threshold {
   hyc_desc d;
@@ -198,52 +175,18 @@ const Tensor* attr_vec(const Ref& v, at::ScalarType type) {
 }
 Tensor empty_like_on(const Tensor& t, at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, at::TensorOptions().device(t.device()).dtype(type)); }
 
-// a compressed activation about to be read: of the channel scheme as it is, of the threshold scheme restored (ready())
-struct In {
-  Tensor stored, vals, scales, row_ptr, cols;
+// a compressed activation: of the channel scheme as it is read, of the threshold scheme restored first (ready()).  A value: a node of the graph
+// keeps one, and each pass over it works on a copy.
+struct Saved {
+  Tensor stored, vals, scales, row_ptr, cols, scale, L, R;
   Plan p;
-  Ref scale{nullptr}, L{nullptr}, R{nullptr};
   hyc_desc d;
-  int64_t M, H;
+  int64_t M = 0, H = 0, bits = 0, group = 0;
+  double threshold = 0.0;
   bool restore_first = false;
   const void* codes() const { return stored.data_ptr(); }
   const void* values() const { return vals.defined() ? vals.data_ptr() : nullptr; }
   const void* group_scales() const { return scales.defined() ? scales.data_ptr() : nullptr; }
-  bool init(PyObject* c) {
-    const bool thr = (PyObject*)Py_TYPE(c) == t_threshold;
-    if (!thr && (PyObject*)Py_TYPE(c) != t_compressed) return false;
-    bool ok = true;
-    M = attr_i64(c, s_M, &ok);
-    H = attr_i64(c, s_H, &ok);
-    const int64_t b = attr_i64(c, s_bits, &ok);
-    Ref st(PyObject_GetAttr(c, s_stored)), va(PyObject_GetAttr(c, s_vals));
-    const Tensor *ts = st.p ? plain(st.p) : nullptr, *tv = va.p ? plain(va.p) : nullptr;
-    if (!ok || !ts || !tv) { PyErr_Clear(); return false; }
-    stored = *ts; vals = *tv;
-    if (thr) {
-      const int64_t S = attr_i64(c, s_S, &ok);
-      Ref rp(PyObject_GetAttr(c, s_row_ptr)), co(PyObject_GetAttr(c, s_cols)), th(PyObject_GetAttr(c, s_threshold));
-      scale.p = PyObject_GetAttr(c, s_scale); L.p = PyObject_GetAttr(c, s_L); R.p = PyObject_GetAttr(c, s_R);
-      const Tensor *tr = attr_vec(rp, at::kInt), *tc = attr_vec(co, at::kInt);
-      Threshold t;
-      if (!ok || !tr || !tc || !th.p || !scale.p || !L.p || !R.p || !PyFloat_CheckExact(th.p) ||
-          !t.init(PyFloat_AS_DOUBLE(th.p), scale.p, b, S, H, L.p, R.p)) { PyErr_Clear(); return false; }
-      row_ptr = *tr; cols = *tc;
-      d = t.d;
-      d.csr_row_ptr = (decltype(d.csr_row_ptr))row_ptr.data_ptr();
-      d.csr_cols = cols.numel() ? (decltype(d.csr_cols))cols.data_ptr() : nullptr;
-      d.csr_vals = vals.numel() ? (decltype(d.csr_vals))vals.data_ptr() : nullptr;
-      restore_first = true;
-      return true;
-    }
-    const int64_t g = attr_i64(c, s_group, &ok);
-    Ref sc(PyObject_GetAttr(c, s_scales)), pl(PyObject_GetAttr(c, s_plan));
-    const Tensor* tc = sc.p ? plain(sc.p) : nullptr;
-    if (!ok || !tc || !pl.p || !get_plan(pl.p, H, ts->device(), &p)) { PyErr_Clear(); return false; }
-    scales = *tc;
-    p.describe(b, g, &d);
-    return true;
-  }
   // the dense x_hat [M, H]
   bool restore(Tensor* x) const {
     *x = empty_like_on(stored, {M, H}, BF16);
@@ -265,6 +208,90 @@ struct In {
   }
   // what a consumer kernel reads: the last thing before its launch
   bool ready() { return !restore_first || make_dense(); }
+  PyObject* wrap(PyObject* plan) const;                                // kernels.ChannelCompressed / ThresholdCompressed; plan: its plan, or null
+};
+struct In : Saved {
+  bool init(PyObject* c) {
+    const bool thr = (PyObject*)Py_TYPE(c) == t_threshold;
+    if (!thr && (PyObject*)Py_TYPE(c) != t_compressed) return false;
+    bool ok = true;
+    M = attr_i64(c, s_M, &ok);
+    H = attr_i64(c, s_H, &ok);
+    bits = attr_i64(c, s_bits, &ok);
+    Ref st(PyObject_GetAttr(c, s_stored)), va(PyObject_GetAttr(c, s_vals));
+    const Tensor *ts = st.p ? plain(st.p) : nullptr, *tv = va.p ? plain(va.p) : nullptr;
+    if (!ok || !ts || !tv) { PyErr_Clear(); return false; }
+    stored = *ts; vals = *tv;
+    if (thr) {
+      const int64_t S = attr_i64(c, s_S, &ok);
+      Ref rp(PyObject_GetAttr(c, s_row_ptr)), co(PyObject_GetAttr(c, s_cols)), th(PyObject_GetAttr(c, s_threshold)), sc(PyObject_GetAttr(c, s_scale)),
+          l(PyObject_GetAttr(c, s_L)), r(PyObject_GetAttr(c, s_R));
+      const Tensor *tr = attr_vec(rp, at::kInt), *tc = attr_vec(co, at::kInt);
+      Threshold t;
+      if (!ok || !tr || !tc || !th.p || !sc.p || !l.p || !r.p || !PyFloat_CheckExact(th.p) ||
+          !t.init(PyFloat_AS_DOUBLE(th.p), sc.p, bits, S, H, l.p, r.p)) { PyErr_Clear(); return false; }
+      row_ptr = *tr; cols = *tc;
+      scale = THPVariable_Unpack(sc.p);
+      if (THPVariable_Check(l.p)) L = THPVariable_Unpack(l.p);
+      if (THPVariable_Check(r.p)) R = THPVariable_Unpack(r.p);
+      threshold = PyFloat_AS_DOUBLE(th.p);
+      d = t.d;
+      d.csr_row_ptr = (decltype(d.csr_row_ptr))row_ptr.data_ptr();
+      d.csr_cols = cols.numel() ? (decltype(d.csr_cols))cols.data_ptr() : nullptr;
+      d.csr_vals = vals.numel() ? (decltype(d.csr_vals))vals.data_ptr() : nullptr;
+      restore_first = true;
+      return true;
+    }
+    group = attr_i64(c, s_group, &ok);
+    Ref sc(PyObject_GetAttr(c, s_scales)), pl(PyObject_GetAttr(c, s_plan));
+    const Tensor* tc = sc.p ? plain(sc.p) : nullptr;
+    if (!ok || !tc || !pl.p || !get_plan(pl.p, H, ts->device(), &p)) { PyErr_Clear(); return false; }
+    scales = *tc;
+    p.describe(bits, group, &d);
+    return true;
+  }
+};
+PyObject* wrap_or_none(const Tensor& t) {
+  if (t.defined()) return THPVariable_Wrap(t);
+  Py_RETURN_NONE;
+}
+PyObject* Saved::wrap(PyObject* plan) const {
+  if (restore_first) {                                                 // (stored, row_ptr, cols, vals, threshold, scale, L, R, bits, M, H, S)
+    Ref args(Py_BuildValue("NNNNdNNNLLLL", wrap_or_none(stored), wrap_or_none(row_ptr), wrap_or_none(cols), wrap_or_none(vals), threshold,
+                           wrap_or_none(scale), wrap_or_none(L), wrap_or_none(R), (long long)bits, (long long)M, (long long)H, (long long)d.S));
+    return args.p ? PyObject_CallObject(t_threshold, args.p) : nullptr;
+  }
+  Ref made(nullptr);
+  if (!plan) {                                                         // (H, k, idx, plan, scale_rule)
+    Ref args(Py_BuildValue("LLNNs", (long long)p.H, (long long)p.k, wrap_or_none(p.idx), wrap_or_none(p.plan),
+                           p.rule == HYC_SCALE_ABSMAX ? "absmax" : "range"));
+    if (!args.p || !(plan = made.p = PyObject_CallObject(t_plan, args.p))) return nullptr;
+  }
+  Ref a(THPVariable_Wrap(stored)), b(THPVariable_Wrap(vals)), c(THPVariable_Wrap(scales)), w(PyLong_FromLongLong(bits)), g(PyLong_FromLongLong(group)),
+      m(PyLong_FromLongLong(M)), h(PyLong_FromLongLong(H));
+  if (!a.p || !b.p || !c.p || !w.p || !g.p || !m.p || !h.p) return nullptr;
+  PyObject* args[8] = {a.p, b.p, c.p, plan, w.p, g.p, m.p, h.p};      // (stored, vals, scales, plan, bits, group, M, H)
+  return PyObject_Vectorcall(t_compressed, args, 8, nullptr);
+}
+// one of the channel scheme about to be written
+struct Out : Saved {
+  PyObject* plan;
+  bool init(PyObject* plan_, PyObject* bits_, PyObject* group_, int64_t M_, int64_t H_, c10::Device device) {
+    plan = plan_; M = M_; H = H_;
+    if (!PyLong_CheckExact(bits_) || !PyLong_CheckExact(group_)) return false;
+    bits = PyLong_AsLongLong(bits_);
+    group = PyLong_AsLongLong(group_);
+    if (hyc_check_shape(H, (int32_t)bits, (int32_t)group, HYC_MODE_CHANNEL) != 0 || !get_plan(plan, H, device, &p)) return false;
+    p.describe(bits, group, &d);
+    return true;
+  }
+  void alloc() {
+    const auto opt = at::TensorOptions().device(p.plan.device());
+    stored = at::empty({M, H * bits / 8}, opt.dtype(bits == 8 ? at::kChar : at::kByte));
+    vals = at::empty({M, p.k}, opt.dtype(BF16));
+    scales = at::empty({M, H / group}, opt.dtype(BF16));
+  }
+  PyObject* wrap() const { return Saved::wrap(plan); }
 };
 
 PyObject* none() { Py_RETURN_NONE; }
@@ -316,53 +343,81 @@ PyObject* decompress(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 }
 
 // ---- norms -----------------------------------------------------------------------------------------------------
-bool norm_weight(PyObject* o, int64_t H, const Tensor** w, int* dtype) {
-  *w = plain(o);
-  if (!*w || !(*w)->is_contiguous() || (*w)->numel() != H) return false;
-  if ((*w)->scalar_type() == at::kFloat) *dtype = HYC_DTYPE_F32;
-  else if ((*w)->scalar_type() == BF16) *dtype = HYC_DTYPE_BF16;
+bool weight_dtype(const Tensor& w, int64_t H, int* dtype) {
+  if (!w.is_contiguous() || w.numel() != H) return false;
+  if (w.scalar_type() == at::kFloat) *dtype = HYC_DTYPE_F32;
+  else if (w.scalar_type() == BF16) *dtype = HYC_DTYPE_BF16;
   else return false;
   return true;
 }
+bool norm_weight(PyObject* o, int64_t H, const Tensor** w, int* dtype) {
+  *w = plain(o);
+  return *w && weight_dtype(**w, H, dtype);
+}
+struct NormOut {
+  const Tensor *x, *w, *bias = nullptr;
+  Out o;
+  Tensor y, rstd, mean;
+  // (x [..., H], w, bias or None, layer_norm, eps, plan, bits, group); false: not the plain case, or an error that is set
+  bool init(PyObject* const* a) {
+    int64_t M, H;
+    x = bf16(a[0]);
+    if (!x || !rows_of(*x, &M, &H) || !norm_weight(a[1], H, &w, &dtype)) return false;
+    if (a[2] != Py_None) {
+      bias = plain(a[2]);
+      if (!bias || !bias->is_contiguous() || bias->numel() != H || bias->scalar_type() != w->scalar_type()) return false;
+    }
+    ln = a[3] == Py_True;
+    eps = PyFloat_AsDouble(a[4]);
+    return !PyErr_Occurred() && o.init(a[5], a[6], a[7], M, H, x->device());
+  }
+  int launch() {
+    o.alloc();
+    y = at::empty(x->sizes(), x->options());
+    rstd = empty_like_on(*x, {o.M}, at::kFloat);
+    if (!ln)
+      return hyc_rmsnorm_fwd_compress(x->data_ptr(), w->data_ptr(), dtype, (float)eps, o.M, o.H, &o.d, y.data_ptr(), (float*)rstd.data_ptr(),
+                                      o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(), nullptr, stream());
+    mean = empty_like_on(*x, {o.M}, at::kFloat);
+    return hyc_layernorm_fwd_compress(x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, dtype, (float)eps, o.M, o.H, &o.d, y.data_ptr(),
+                                      (float*)mean.data_ptr(), (float*)rstd.data_ptr(), o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(),
+                                      nullptr, stream());
+  }
+  int dtype;
+  bool ln;
+  double eps;
+};
 // norm_fwd(x [..., H], w, bias or None, layer_norm, eps, plan, bits, group) -> (y like x, mean or None, rstd, ChannelCompressed)
 PyObject* norm_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   ARGS(8);
-  const Tensor *x = bf16(a[0]), *w, *bias = nullptr;
-  int64_t M, H;
-  int dtype;
-  if (!x || !rows_of(*x, &M, &H) || !norm_weight(a[1], H, &w, &dtype)) return none();
-  if (a[2] != Py_None) {
-    bias = plain(a[2]);
-    if (!bias || !bias->is_contiguous() || bias->numel() != H || bias->scalar_type() != w->scalar_type()) return none();
-  }
-  const bool ln = a[3] == Py_True;
-  const double eps = PyFloat_AsDouble(a[4]);
-  if (PyErr_Occurred()) return nullptr;
-  Out o;
-  if (!o.init(a[5], a[6], a[7], M, H, x->device())) return none();
-  Tensor y, rstd, mean;
-  OR_NONE(unlocked([&] {
-    o.alloc();
-    y = at::empty(x->sizes(), x->options());
-    rstd = empty_like_on(*x, {M}, at::kFloat);
-    if (!ln)
-      return hyc_rmsnorm_fwd_compress(x->data_ptr(), w->data_ptr(), dtype, (float)eps, M, H, &o.d, y.data_ptr(), (float*)rstd.data_ptr(),
-                                      o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(), nullptr, stream());
-    mean = empty_like_on(*x, {M}, at::kFloat);
-    return hyc_layernorm_fwd_compress(x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, dtype, (float)eps, M, H, &o.d, y.data_ptr(),
-                                      (float*)mean.data_ptr(), (float*)rstd.data_ptr(), o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(),
-                                      nullptr, stream());
-  }));
-  PyObject* c = o.wrap();
+  NormOut n;
+  if (!n.init(a)) return none_if_plain(nullptr);
+  OR_NONE(unlocked([&] { return n.launch(); }));
+  PyObject* c = n.o.wrap();
   if (!c) return nullptr;
   PyObject* t = PyTuple_New(4);
-  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(y));
-  PyTuple_SET_ITEM(t, 1, ln ? THPVariable_Wrap(mean) : none());
-  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(rstd));
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(n.y));
+  PyTuple_SET_ITEM(t, 1, wrap_or_none(n.mean));
+  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(n.rstd));
   PyTuple_SET_ITEM(t, 3, c);
   return t;
   END_HANDLE_TH_ERRORS
+}
+// the statistics of M rows
+bool row_stats(const Tensor& t, int64_t M) { return t.scalar_type() == at::kFloat && t.is_contiguous() && t.numel() == M; }
+int norm_backward(const Tensor& dy, Saved& in, const Tensor& w, int dtype, const Tensor& mean, const Tensor& rstd, bool quirk, Tensor* dx, Tensor* dw) {
+  const int64_t M = in.M, H = in.H;
+  if (!in.ready()) return -1;
+  const int64_t P = hyc_rmsnorm_bwd_partials(M, H);
+  const Tensor partials = empty_like_on(dy, {P > 1 ? P : 1, H}, at::kFloat);
+  *dx = at::empty(dy.sizes(), dy.options());
+  *dw = empty_like_on(dy, {H}, w.scalar_type());
+  if (mean.defined())
+    return hyc_layernorm_bwd(dy.data_ptr(), in.codes(), in.values(), in.group_scales(), w.data_ptr(), dtype, (const float*)mean.data_ptr(),
+                             (const float*)rstd.data_ptr(), M, H, &in.d, dx->data_ptr(), (float*)partials.data_ptr(), dw->data_ptr(), stream());
+  return hyc_rmsnorm_bwd(dy.data_ptr(), in.codes(), in.values(), in.group_scales(), w.data_ptr(), dtype, (const float*)rstd.data_ptr(), M, H, &in.d,
+                         quirk, dx->data_ptr(), (float*)partials.data_ptr(), dw->data_ptr(), stream());
 }
 // norm_bwd(dy [..., H], c, w, mean or None, rstd, quirk) -> (dx like dy, dw in w's dtype)
 PyObject* norm_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
@@ -373,28 +428,22 @@ PyObject* norm_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   int dtype;
   In in;
   if (!dy || !rows_of(*dy, &M, &H) || !norm_weight(a[2], H, &w, &dtype) || !in.init(a[1]) || in.M != M || in.H != H) return none();
-  auto stats = [&](const Tensor* t) { return t && t->scalar_type() == at::kFloat && t->is_contiguous() && t->numel() == M; };
-  if (!stats(rstd)) return none();
+  if (!rstd || !row_stats(*rstd, M)) return none();
   if (a[3] != Py_None) {
     mean = plain(a[3]);
-    if (!stats(mean)) return none();
+    if (!mean || !row_stats(*mean, M)) return none();
   }
   const bool quirk = a[5] == Py_True;
   Tensor dx, dw;
-  OR_NONE(unlocked([&] {
-    if (!in.ready()) return -1;
-    const int64_t P = hyc_rmsnorm_bwd_partials(M, H);
-    const Tensor partials = empty_like_on(*dy, {P > 1 ? P : 1, H}, at::kFloat);
-    dx = at::empty(dy->sizes(), dy->options());
-    dw = empty_like_on(*dy, {H}, w->scalar_type());
-    if (mean)
-      return hyc_layernorm_bwd(dy->data_ptr(), in.codes(), in.values(), in.group_scales(), w->data_ptr(), dtype, (const float*)mean->data_ptr(),
-                               (const float*)rstd->data_ptr(), M, H, &in.d, dx.data_ptr(), (float*)partials.data_ptr(), dw.data_ptr(), stream());
-    return hyc_rmsnorm_bwd(dy->data_ptr(), in.codes(), in.values(), in.group_scales(), w->data_ptr(), dtype, (const float*)rstd->data_ptr(), M, H, &in.d,
-                           quirk, dx.data_ptr(), (float*)partials.data_ptr(), dw.data_ptr(), stream());
-  }));
+  OR_NONE(unlocked([&] { return norm_backward(*dy, in, *w, dtype, mean ? *mean : Tensor(), *rstd, quirk, &dx, &dw); }));
   return tuple2(THPVariable_Wrap(dx), THPVariable_Wrap(dw));
   END_HANDLE_TH_ERRORS
+}
+int bias_backward(const Tensor& dy, int64_t M, int64_t H, bool f32, Tensor* db) {
+  const int64_t P = hyc_bias_grad_partials(M, H);
+  const Tensor partials = empty_like_on(dy, {P > 1 ? P : 1, H}, at::kFloat);
+  *db = empty_like_on(dy, {H}, f32 ? at::kFloat : BF16);
+  return hyc_bias_grad(dy.data_ptr(), M, H, (float*)partials.data_ptr(), db->data_ptr(), f32 ? HYC_DTYPE_F32 : HYC_DTYPE_BF16, stream());
 }
 // bias_grad(dy [..., H], fp32) -> db [H]
 PyObject* bias_grad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
@@ -405,12 +454,7 @@ PyObject* bias_grad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (!dy || !rows_of(*dy, &M, &H)) return none();
   const bool f32 = a[1] == Py_True;
   Tensor db;
-  OR_NONE(unlocked([&] {
-    const int64_t P = hyc_bias_grad_partials(M, H);
-    const Tensor partials = empty_like_on(*dy, {P > 1 ? P : 1, H}, at::kFloat);
-    db = empty_like_on(*dy, {H}, f32 ? at::kFloat : BF16);
-    return hyc_bias_grad(dy->data_ptr(), M, H, (float*)partials.data_ptr(), db.data_ptr(), f32 ? HYC_DTYPE_F32 : HYC_DTYPE_BF16, stream());
-  }));
+  OR_NONE(unlocked([&] { return bias_backward(*dy, M, H, f32, &db); }));
   return THPVariable_Wrap(db);
   END_HANDLE_TH_ERRORS
 }
@@ -549,7 +593,7 @@ PyObject* softmax_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 
 // ---- weight gradient, linear layer -------------------------------------------------------------------------------
 // dW [N, H] = dy^T x_hat from rows of dy `pitch` apart; staged: through a restored x_hat
-bool weight_grad(const void* dy, int64_t pitch, int64_t M, int64_t N, const Tensor& like, In& in, bool f32, bool staged, Tensor* out) {
+bool weight_grad(const void* dy, int64_t pitch, int64_t M, int64_t N, const Tensor& like, Saved& in, bool f32, bool staged, Tensor* out) {
   if (!(staged ? in.make_dense() : in.ready())) return false;
   *out = empty_like_on(like, {N, in.H}, f32 ? at::kFloat : BF16);
   const int64_t bytes = hyc_gradw_workspace_bytes(M, N, in.H);
@@ -585,30 +629,46 @@ bool thin(const Tensor& rows, const Tensor& w, int64_t M, bool input_grad) {
          rows.device() == w.device() && rows.device().index() == c10::hip::current_device() &&
          (!at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) == BF16);
 }
+// y = x w^T, into rows of its own shape (`view`: the library's result seen as that, or an alias of it that no view is tracked for)
+int linear_forward(const Tensor& x, const Tensor& w, int64_t M, int64_t K, bool view, Tensor* y) {
+  const auto sizes = with_last(x, w.size(0));
+  if (!thin(x, w, M, false)) {
+    *y = at::mm(x.view({M, K}), w.t());
+    *y = view ? y->view(sizes) : at::_unsafe_view(*y, sizes);
+    return 0;
+  }
+  *y = at::empty(sizes, x.options());
+  const void* factor = w.data_ptr();
+  return hyc_lora_down(x.data_ptr(), K, M, K, &factor, 1, (int32_t)w.size(0), y->data_ptr(), stream());
+}
+bool linear_operands(const Tensor* x, const Tensor* w, int64_t* M, int64_t* K) {
+  return x && w && x->dim() >= 2 && w->dim() == 2 && x->numel() && rows_of(*x, M, K) && w->size(1) == *K;
+}
 // linear_fwd(x [..., K], w [N, K], plan or None, bits, group) -> (x w^T, ChannelCompressed or None)
 PyObject* linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   ARGS(5);
   const Tensor *x = bf16(a[0]), *w = bf16(a[1]);
   int64_t M, K;
-  if (!x || !w || x->dim() < 2 || w->dim() != 2 || x->numel() == 0 || !rows_of(*x, &M, &K) || w->size(1) != K) return none();
+  if (!linear_operands(x, w, &M, &K)) return none();
   PyObject* c = Py_None;
   if (a[2] == Py_None) Py_INCREF(c);
   else if (!(c = compress_rows(*x, a[2], a[3], a[4]))) return none_if_plain(nullptr);
   Ref hold(c);
   Tensor y;
-  OR_NONE(unlocked([&] {
-    if (!thin(*x, *w, M, false)) {
-      y = at::mm(x->view({M, K}), w->t()).view(with_last(*x, w->size(0)));
-      return 0;
-    }
-    y = at::empty(with_last(*x, w->size(0)), x->options());
-    const void* factor = w->data_ptr();
-    return hyc_lora_down(x->data_ptr(), K, M, K, &factor, 1, (int32_t)w->size(0), y.data_ptr(), stream());
-  }));
+  OR_NONE(unlocked([&] { return linear_forward(*x, *w, M, K, true, &y); }));
   Py_INCREF(c);
   return tuple2(THPVariable_Wrap(y), c);
   END_HANDLE_TH_ERRORS
+}
+int linear_backward(const Tensor& g, const Tensor& w, int64_t M, int64_t N, Saved* in, bool need_x, bool staged, Tensor* dx, Tensor* dw) {
+  if (in && !weight_grad(g.data_ptr(), N, M, N, g, *in, false, staged, dw)) return -1;
+  if (need_x && thin(g, w, M, true)) {
+    *dx = at::empty(with_last(g, w.size(1)), g.options());
+    return hyc_thin_dx(g.data_ptr(), N, M, w.data_ptr(), (int32_t)N, w.size(1), dx->data_ptr(), stream());
+  }
+  if (need_x) *dx = at::mm(g.view({M, N}), w).view(with_last(g, w.size(1)));
+  return 0;
 }
 // linear_bwd(g [..., N], w [N, K], c or None, need_x, staged) -> (g w or None, dW bf16 or None)
 PyObject* linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
@@ -622,37 +682,45 @@ PyObject* linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   In in;
   const bool need_w = a[2] != Py_None, need_x = a[3] == Py_True, staged = a[4] == Py_True;
   if (need_w && (!in.init(a[2]) || in.M != M)) return none();
-  OR_NONE(unlocked([&] {
-    if (need_w && !weight_grad(g->data_ptr(), N, M, N, *g, in, false, staged, &dw)) return -1;
-    if (need_x && thin(*g, *w, M, true)) {
-      dx = at::empty(with_last(*g, w->size(1)), g->options());
-      return hyc_thin_dx(g->data_ptr(), N, M, w->data_ptr(), (int32_t)N, w->size(1), dx.data_ptr(), stream());
-    }
-    if (need_x) dx = at::mm(g->view({M, N}), *w).view(with_last(*g, w->size(1)));
-    return 0;
-  }));
-  return tuple2(dx.defined() ? THPVariable_Wrap(dx) : none(), dw.defined() ? THPVariable_Wrap(dw) : none());
+  OR_NONE(unlocked([&] { return linear_backward(*g, *w, M, N, need_w ? &in : nullptr, need_x, staged, &dx, &dw); }));
+  return tuple2(wrap_or_none(dx), wrap_or_none(dw));
   END_HANDLE_TH_ERRORS
 }
 
 // ---- activations ---------------------------------------------------------------------------------------------------
+struct ActOut {
+  const Tensor* x;
+  Out o;
+  Tensor y;
+  int32_t code;
+  bool init(PyObject* const* a) {                                      // (code, x [..., H], plan, bits, group)
+    int64_t M, H;
+    x = bf16(a[1]);
+    if (!x || !rows_of(*x, &M, &H) || !o.init(a[2], a[3], a[4], M, H, x->device())) return false;
+    code = (int32_t)PyLong_AsLong(a[0]);
+    return !PyErr_Occurred();
+  }
+  int launch() {
+    o.alloc();
+    y = at::empty(x->sizes(), x->options());
+    return hyc_act_fwd_compress(code, x->data_ptr(), o.H, o.M, o.H, &o.d, y.data_ptr(), o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(),
+                                stream());
+  }
+};
 // act_fwd(code, x [..., H], plan, bits, group) -> (y like x, ChannelCompressed)
 PyObject* act_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   ARGS(5);
-  const Tensor* x = bf16(a[1]);
-  int64_t M, H;
-  Out o;
-  if (!x || !rows_of(*x, &M, &H) || !o.init(a[2], a[3], a[4], M, H, x->device())) return none();
-  const int32_t code = (int32_t)PyLong_AsLong(a[0]);
-  Tensor y;
-  OR_NONE(unlocked([&] {
-    o.alloc();
-    y = at::empty(x->sizes(), x->options());
-    return hyc_act_fwd_compress(code, x->data_ptr(), H, M, H, &o.d, y.data_ptr(), o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(), stream());
-  }));
-  return tuple2(THPVariable_Wrap(y), o.wrap());
+  ActOut f;
+  if (!f.init(a)) return none_if_plain(nullptr);
+  OR_NONE(unlocked([&] { return f.launch(); }));
+  return tuple2(THPVariable_Wrap(f.y), f.o.wrap());
   END_HANDLE_TH_ERRORS
+}
+int act_backward(int32_t code, const Tensor& g, Saved& in, Tensor* dx) {
+  if (!in.ready()) return -1;
+  *dx = at::empty(g.sizes(), g.options());
+  return hyc_act_bwd(code, g.data_ptr(), in.codes(), in.values(), in.group_scales(), in.M, in.H, &in.d, dx->data_ptr(), stream());
 }
 // act_bwd(code, g [..., H], c) -> dx like g
 PyObject* act_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
@@ -664,40 +732,48 @@ PyObject* act_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   if (!g || !rows_of(*g, &M, &H) || !in.init(a[2]) || in.M != M || in.H != H) return none();
   const int32_t code = (int32_t)PyLong_AsLong(a[0]);
   Tensor dx;
-  OR_NONE(unlocked([&] {
-    if (!in.ready()) return -1;
-    dx = at::empty(g->sizes(), g->options());
-    return hyc_act_bwd(code, g->data_ptr(), in.codes(), in.values(), in.group_scales(), M, H, &in.d, dx.data_ptr(), stream());
-  }));
+  OR_NONE(unlocked([&] { return act_backward(code, *g, in, &dx); }));
   return THPVariable_Wrap(dx);
   END_HANDLE_TH_ERRORS
 }
+struct GatedOut {
+  const Tensor *gate, *up;
+  Out o[3];
+  Tensor h;
+  int32_t code;
+  int64_t pg, pu;
+  bool init(PyObject* const* a) {                                      // (code, gate [..., H], up, plan_act, plan_up, plan_gate, bits, group)
+    int64_t M, H, M2, H2;
+    gate = bf16(a[1]);
+    up = bf16(a[2]);
+    if (!gate || !up || gate->sizes() != up->sizes() || !spaced_rows(*gate, &M, &H, &pg) || !spaced_rows(*up, &M2, &H2, &pu)) return false;
+    for (int i = 0; i < 3; ++i)
+      if (!o[i].init(a[3 + i], a[6], a[7], M, H, gate->device())) return false;
+    code = (int32_t)PyLong_AsLong(a[0]);
+    return !PyErr_Occurred();
+  }
+  int launch() {
+    for (Out& out : o) out.alloc();
+    h = at::empty(gate->sizes(), gate->options());
+    return hyc_gated_act_fwd(code, gate->data_ptr(), pg, up->data_ptr(), pu, o[0].M, o[0].H, &o[0].d, &o[1].d, &o[2].d, h.data_ptr(),
+                             o[0].stored.data_ptr(), o[0].vals.data_ptr(), o[0].scales.data_ptr(), o[1].stored.data_ptr(), o[1].vals.data_ptr(),
+                             o[1].scales.data_ptr(), o[2].stored.data_ptr(), o[2].vals.data_ptr(), o[2].scales.data_ptr(), stream());
+  }
+};
 // gated_fwd(code, gate [..., H], up, plan_act, plan_up, plan_gate, bits, group) -> (h [..., H], (c_act, c_up, c_gate))
 PyObject* gated_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   ARGS(8);
-  const Tensor *gate = bf16(a[1]), *up = bf16(a[2]);
-  int64_t M, H, pg, M2, H2, pu;
-  if (!gate || !up || gate->sizes() != up->sizes() || !spaced_rows(*gate, &M, &H, &pg) || !spaced_rows(*up, &M2, &H2, &pu)) return none();
-  Out o[3];
-  for (int i = 0; i < 3; ++i)
-    if (!o[i].init(a[3 + i], a[6], a[7], M, H, gate->device())) return none();
-  const int32_t code = (int32_t)PyLong_AsLong(a[0]);
-  Tensor h;
-  OR_NONE(unlocked([&] {
-    for (Out& out : o) out.alloc();
-    h = at::empty(gate->sizes(), gate->options());
-    return hyc_gated_act_fwd(code, gate->data_ptr(), pg, up->data_ptr(), pu, M, H, &o[0].d, &o[1].d, &o[2].d, h.data_ptr(), o[0].stored.data_ptr(),
-                             o[0].vals.data_ptr(), o[0].scales.data_ptr(), o[1].stored.data_ptr(), o[1].vals.data_ptr(), o[1].scales.data_ptr(),
-                             o[2].stored.data_ptr(), o[2].vals.data_ptr(), o[2].scales.data_ptr(), stream());
-  }));
+  GatedOut f;
+  if (!f.init(a)) return none_if_plain(nullptr);
+  OR_NONE(unlocked([&] { return f.launch(); }));
   PyObject* cs = PyTuple_New(3);
   for (int i = 0; i < 3; ++i) {
-    PyObject* c = o[i].wrap();
+    PyObject* c = f.o[i].wrap();
     if (!c) { Py_DECREF(cs); return nullptr; }
     PyTuple_SET_ITEM(cs, i, c);
   }
-  return tuple2(THPVariable_Wrap(h), cs);
+  return tuple2(THPVariable_Wrap(f.h), cs);
   END_HANDLE_TH_ERRORS
 }
 // `n` matrices of [lead..., H] side by side in one [M, n H + room], or on their own (room < 0)
@@ -719,12 +795,20 @@ PyObject* wrap_parts(const std::vector<Tensor>& parts, const Tensor& both) {
   return t;
 }
 int64_t room_of(PyObject* o) { return o == Py_None ? -1 : PyLong_AsLongLong(o); }
+template <class S>
+int gated_backward(int32_t code, const Tensor& g, const S* in, int64_t room, Tensor* both, std::vector<Tensor>* d) {
+  int64_t pitch;
+  side_by_side(g, 2, in[0].M, in[0].H, room, both, d, &pitch);
+  return hyc_gated_act_bwd_rows(code, g.data_ptr(), in[0].codes(), in[0].values(), in[0].group_scales(), &in[0].d, in[1].codes(), in[1].values(),
+                                in[1].group_scales(), &in[1].d, in[2].codes(), in[2].values(), in[2].group_scales(), &in[2].d, in[0].M, in[0].H,
+                                (*d)[0].data_ptr(), pitch, (*d)[1].data_ptr(), pitch, stream());
+}
 // gated_bwd(code, g [..., H], c_act, c_up, c_gate, room or None) -> (d_gate, d_up, their common matrix or None)
 PyObject* gated_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   ARGS(6);
   const Tensor* g = bf16(a[1]);
-  int64_t M, H, pitch;
+  int64_t M, H;
   In in[3];
   if (!g || g->dim() < 2 || !rows_of(*g, &M, &H)) return none();
   for (int i = 0; i < 3; ++i)
@@ -733,12 +817,7 @@ PyObject* gated_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const int64_t room = room_of(a[5]);
   Tensor both;
   std::vector<Tensor> d;
-  OR_NONE(unlocked([&] {
-    side_by_side(*g, 2, M, H, room, &both, &d, &pitch);
-    return hyc_gated_act_bwd_rows(code, g->data_ptr(), in[0].codes(), in[0].values(), in[0].group_scales(), &in[0].d, in[1].codes(), in[1].values(),
-                                  in[1].group_scales(), &in[1].d, in[2].codes(), in[2].values(), in[2].group_scales(), &in[2].d, M, H, d[0].data_ptr(),
-                                  pitch, d[1].data_ptr(), pitch, stream());
-  }));
+  OR_NONE(unlocked([&] { return gated_backward(code, *g, in, room, &both, &d); }));
   return wrap_parts(d, both);
   END_HANDLE_TH_ERRORS
 }
@@ -1180,6 +1259,271 @@ PyObject* attn_kept_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// ---- an operator's backward, recorded natively ---------------------------------------------------------------------------
+// A short pass is bound by what torch.autograd.Function does around the calls above: the context and its attributes, argument tuples, the
+// interpreter's lock in the engine's thread.  The *_node functions run the forward and record one node of this kind instead (us a pass: rms norm of 45 x
+// 4096 82 -> 64, layer norm 31 x 117 x 1024 103 -> 81, LoRA-A 4096 x 4096 91 -> 69, the reference's rms norm 133 -> 104).  Like the
+// contexts it replaces it keeps its tensors as they are (no saved-tensor hooks, nothing let go after a pass).  It holds no object of the
+// interpreter, so that the engine's thread can run it and let go of it without the lock.  What the calls above do not cover, in a pass over it too
+// (create_graph, gradients in a batch, of another type or layout), goes through `interpreted`, the Function's own backward as a function of
+// (context, gradient), with a context made for it.
+struct Recorded : public torch::autograd::Node {
+  enum Kind { NORM, LINEAR, ACT, GATED } kind;
+  std::vector<Saved> saved;                                            // one activation; of the gated product act(gate), up and gate
+  Tensor w, bias, mean, rstd;
+  bool quirk = false, staged = false;
+  bool needs[3] = {false, false, false};
+  int32_t code = 0;
+  std::string act, label;
+  PyObject* interpreted = nullptr;                                     // lives as long as the process
+  explicit Recorded(Kind k) : kind(k) {}
+  std::string name() const override { return label; }
+
+  bool native(const Tensor& g, torch::autograd::variable_list& out) const {
+    int64_t M, H;
+    int dtype;
+    if (!dense_gpu(g) || g.scalar_type() != BF16 || g.unsafeGetTensorImpl()->is_python_dispatch() || !rows_of(g, &M, &H)) return false;
+    for (const Saved& c : saved)
+      if (M != c.M || (kind != LINEAR && H != c.H)) return false;
+    if (kind == GATED) {
+      Tensor both;
+      std::vector<Tensor> d;
+      if (g.dim() < 2 || gated_backward(code, g, saved.data(), -1, &both, &d) != 0) return false;
+      out[0] = d[0];
+      out[1] = d[1];
+      return true;
+    }
+    std::vector<Saved> in = saved;                                     // (what is read as a restored matrix becomes one)
+    if (kind == NORM) {
+      if (!dense_gpu(w) || !weight_dtype(w, H, &dtype) || norm_backward(g, in[0], w, dtype, mean, rstd, quirk, &out[0], &out[1])) return false;
+      return !bias.defined() || bias_backward(g, M, H, bias.scalar_type() != BF16, &out[2]) == 0;
+    }
+    if (kind == ACT) return act_backward(code, g, in[0], &out[0]) == 0;
+    return g.dim() >= 2 && g.numel() && dense_gpu(w) && w.scalar_type() == BF16 && w.dim() == 2 && w.size(0) == H &&
+           linear_backward(g, w, M, H, in.empty() ? nullptr : &in[0], needs[0], staged, &out[0], &out[1]) == 0;
+  }
+  torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+    torch::autograd::variable_list out(num_outputs());
+    if (!c10::GradMode::is_enabled() && !c10::impl::TorchDispatchModeTLS::any_modes_set() && native(grads[0], out)) return out;
+    const Tensor g = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
+    struct Lock {
+      PyGILState_STATE state = PyGILState_Ensure();
+      ~Lock() { PyGILState_Release(state); }
+    } lock;
+    Ref names(attributes()), none_(PyTuple_New(0)), ctx(names.p && none_.p ? PyObject_Call(t_namespace, none_.p, names.p) : nullptr),
+        dy(ctx.p ? THPVariable_Wrap(g) : nullptr), r(dy.p ? PyObject_CallFunctionObjArgs(interpreted, ctx.p, dy.p, nullptr) : nullptr);
+    if (!r.p || !PyTuple_Check(r.p) || PyTuple_GET_SIZE(r.p) < (Py_ssize_t)out.size()) {
+      if (r.p) PyErr_SetString(PyExc_RuntimeError, "a backward returned something else than its gradients");
+      python_error e;
+      e.persist();
+      throw e;
+    }
+    for (size_t i = 0; i < out.size(); ++i) {
+      PyObject* d = PyTuple_GET_ITEM(r.p, (Py_ssize_t)i);
+      out[i] = d == Py_None ? Tensor() : THPVariable_Unpack(d);
+    }
+    return out;
+  }
+  // what the Functions' contexts hold under these names
+  PyObject* attributes() const {
+    PyObject* c = kind == GATED ? Py_BuildValue("NNN", saved[0].wrap(nullptr), saved[1].wrap(nullptr), saved[2].wrap(nullptr))
+                  : saved.empty() ? none() : saved[0].wrap(nullptr);
+    if (!c) return nullptr;
+    return Py_BuildValue("{s:N,s:N,s:N,s:N,s:N,s:N,s:N,s:d,s:N,s:N,s:O,s:s}", "saved", c, "weight", wrap_or_none(w), "w", wrap_or_none(w), "bias",
+                         wrap_or_none(bias), "mean", wrap_or_none(mean), "rstd", wrap_or_none(rstd), "c2_quirk", PyBool_FromLong(quirk), "weight_offset",
+                         0.0, "use_bias", PyBool_FromLong(0), "needs_input_grad",
+                         Py_BuildValue("NNN", PyBool_FromLong(needs[0]), PyBool_FromLong(needs[1]), PyBool_FromLong(needs[2])), "grad_room", Py_None, "act",
+                         act.c_str());
+  }
+};
+// grad_fn.saved and the like
+PyObject* node_attribute(PyObject* self, PyObject* name) {
+  PyObject* v = PyObject_GenericGetAttr(self, name);
+  if (v || !PyErr_ExceptionMatches(PyExc_AttributeError)) return v;
+  const auto* node = dynamic_cast<Recorded*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get());
+  if (!node) return nullptr;
+  PyObject *type, *value, *trace;
+  PyErr_Fetch(&type, &value, &trace);
+  Ref all(node->attributes());
+  if (all.p && (v = PyDict_GetItemWithError(all.p, name))) {
+    Py_INCREF(v);
+    Py_XDECREF(type); Py_XDECREF(value); Py_XDECREF(trace);
+    return v;
+  }
+  PyErr_Clear();
+  PyErr_Restore(type, value, trace);
+  return nullptr;
+}
+PyTypeObject node_type;
+
+// whether a call on these may skip torch.autograd.Function: nothing watches it (a functorch transform, a trace, a dispatch mode) and no
+// input carries a tangent
+bool unwatched(std::initializer_list<const Tensor*> inputs) {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+      c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer))
+    return false;
+  for (const Tensor* t : inputs)
+    if (t && (t->unsafeGetTensorImpl()->is_python_dispatch() || t->_fw_grad(0).defined())) return false;
+  return true;
+}
+bool recording(std::initializer_list<const Tensor*> inputs) {
+  if (!c10::GradMode::is_enabled()) return false;
+  for (const Tensor* t : inputs)
+    if (t && t->requires_grad()) return true;
+  return false;
+}
+// functions of a module: there are a handful, and a node's reference must not need the interpreter's lock
+PyObject* for_ever(PyObject* f) {
+  static std::vector<PyObject*> known;
+  for (PyObject* k : known)
+    if (k == f) return f;
+  Py_INCREF(f);
+  known.push_back(f);
+  return f;
+}
+std::shared_ptr<Recorded> new_node(Recorded::Kind kind, std::initializer_list<const Tensor*> inputs, PyObject* interpreted, PyObject* label) {
+  std::shared_ptr<Recorded> node(new Recorded(kind), torch::autograd::deleteNode);
+  torch::autograd::variable_list in;
+  for (const Tensor* t : inputs) {
+    if (!t) continue;
+    node->needs[in.size()] = t->requires_grad();
+    in.push_back(*t);
+  }
+  node->set_next_edges(torch::autograd::collect_next_edges(in));
+  node->interpreted = for_ever(interpreted);
+  const char* s = PyUnicode_AsUTF8(label);
+  if (!s) throw python_error();
+  node->label = s;
+  return node;
+}
+// recordable(x, w, bias or None) -> True where norm_record can follow
+PyObject* recordable(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(3);
+  const Tensor *x = plain(a[0]), *w = plain(a[1]), *b = a[2] == Py_None ? nullptr : plain(a[2]);
+  if (!x || !w || (a[2] != Py_None && !b) || !unwatched({x, w, b})) return none();
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+// norm_record(y, x, w, bias or None, c, mean or None, rstd, quirk, interpreted, label) -> y, with its backward where one is recorded
+PyObject* norm_record(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(10);
+  const Tensor *y = bf16(a[0]), *x = bf16(a[1]), *w, *bias = a[3] == Py_None ? nullptr : plain(a[3]), *mean = a[5] == Py_None ? nullptr : plain(a[5]),
+               *rstd = plain(a[6]);
+  In in;
+  int dtype;
+  if (!y || !x || y->sizes() != x->sizes() || !in.init(a[4]) || !norm_weight(a[2], in.H, &w, &dtype) || !rstd || !row_stats(*rstd, in.M) ||
+      (a[5] != Py_None && (!mean || !row_stats(*mean, in.M))) ||
+      (a[3] != Py_None && (!bias || bias->scalar_type() != w->scalar_type())) || !unwatched({x, w, bias}))
+    return none();
+  if (recording({x, w, bias})) {
+    auto node = new_node(Recorded::NORM, {x, w, bias}, a[8], a[9]);
+    node->saved.push_back(in);
+    node->w = *w;
+    if (bias) node->bias = *bias;
+    if (mean) node->mean = *mean;
+    node->rstd = *rstd;
+    node->quirk = a[7] == Py_True;
+    torch::autograd::set_history(*y, node);
+  }
+  Py_INCREF(a[0]);
+  return a[0];
+  END_HANDLE_TH_ERRORS
+}
+// norm_node(norm_fwd's arguments, quirk, interpreted, label) -> y
+PyObject* norm_node(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(11);
+  NormOut n;
+  if (!n.init(a)) return none_if_plain(nullptr);
+  if (!unwatched({n.x, n.w, n.bias})) return none();
+  OR_NONE(unlocked([&] { return n.launch(); }));
+  if (recording({n.x, n.w, n.bias})) {
+    auto node = new_node(Recorded::NORM, {n.x, n.w, n.bias}, a[9], a[10]);
+    node->saved.push_back(n.o);
+    node->w = *n.w;
+    if (n.bias) node->bias = *n.bias;
+    node->mean = n.mean;
+    node->rstd = n.rstd;
+    node->quirk = a[8] == Py_True;
+    torch::autograd::set_history(n.y, node);
+  }
+  return THPVariable_Wrap(n.y);
+  END_HANDLE_TH_ERRORS
+}
+// linear_node(x [..., K], w [N, K], plan, bits, group, staged, interpreted, label) -> x w^T; x is kept where w has a gradient
+PyObject* linear_node(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(8);
+  const Tensor *x = bf16(a[0]), *w = bf16(a[1]);
+  int64_t M, K;
+  if (!linear_operands(x, w, &M, &K) || !unwatched({x, w})) return none();
+  const bool keep = w->requires_grad();
+  Out o;
+  if (keep && !o.init(a[2], a[3], a[4], M, K, x->device())) return none_if_plain(nullptr);
+  Tensor y;
+  OR_NONE(unlocked([&] {
+    c10::AutoGradMode off(false);
+    if (keep) {
+      o.alloc();
+      const int rc = hyc_compress_rows(x->data_ptr(), K, M, K, &o.d, o.stored.data_ptr(), o.vals.data_ptr(), o.scales.data_ptr(), nullptr, stream());
+      if (rc) return rc;
+    }
+    return linear_forward(*x, *w, M, K, false, &y);
+  }));
+  if (recording({x, w})) {
+    auto node = new_node(Recorded::LINEAR, {x, w}, a[6], a[7]);
+    if (keep) node->saved.push_back(o);
+    node->w = *w;
+    node->staged = a[5] == Py_True;
+    torch::autograd::set_history(y, node);
+  }
+  return THPVariable_Wrap(y);
+  END_HANDLE_TH_ERRORS
+}
+// act_node(act_fwd's arguments, act, interpreted, label) -> act(x)
+PyObject* act_node(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(8);
+  ActOut f;
+  if (!f.init(a)) return none_if_plain(nullptr);
+  if (!unwatched({f.x})) return none();
+  OR_NONE(unlocked([&] { return f.launch(); }));
+  if (recording({f.x})) {
+    auto node = new_node(Recorded::ACT, {f.x}, a[6], a[7]);
+    node->saved.push_back(f.o);
+    node->code = f.code;
+    const char* s = PyUnicode_AsUTF8(a[5]);
+    if (!s) return nullptr;
+    node->act = s;
+    torch::autograd::set_history(f.y, node);
+  }
+  return THPVariable_Wrap(f.y);
+  END_HANDLE_TH_ERRORS
+}
+
+// gated_node(gated_fwd's arguments, act, interpreted, label) -> act(gate) up
+PyObject* gated_node(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  ARGS(11);
+  GatedOut f;
+  if (!f.init(a)) return none_if_plain(nullptr);
+  if (!unwatched({f.gate, f.up})) return none();
+  OR_NONE(unlocked([&] { return f.launch(); }));
+  if (recording({f.gate, f.up})) {
+    auto node = new_node(Recorded::GATED, {f.gate, f.up}, a[9], a[10]);
+    node->saved.assign(f.o, f.o + 3);
+    node->code = f.code;
+    const char* s = PyUnicode_AsUTF8(a[8]);
+    if (!s) return nullptr;
+    node->act = s;
+    torch::autograd::set_history(f.h, node);
+  }
+  return THPVariable_Wrap(f.h);
+  END_HANDLE_TH_ERRORS
+}
+
 // rows(t [..., H]) -> (M, H, pitch) as spaced_rows has them, of a tensor on any device
 PyObject* rows(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -1206,7 +1550,8 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 PyMethodDef methods[] = {ENTRY(bind), ENTRY(rows), ENTRY(compress), ENTRY(decompress), ENTRY(norm_fwd), ENTRY(norm_bwd), ENTRY(bias_grad), ENTRY(gradw),
                          ENTRY(linear_fwd), ENTRY(linear_bwd), ENTRY(act_fwd), ENTRY(act_bwd), ENTRY(gated_fwd), ENTRY(gated_bwd), ENTRY(lora_forward),
                          ENTRY(lora_backward), ENTRY(rope_attn_fwd), ENTRY(attn_bwd), ENTRY(attn_kept), ENTRY(attn_kept_bwd),
-                         ENTRY(threshold_fwd), ENTRY(softmax_fwd), ENTRY(softmax_bwd), {nullptr, nullptr, 0, nullptr}};
+                         ENTRY(threshold_fwd), ENTRY(softmax_fwd), ENTRY(softmax_bwd), ENTRY(norm_node), ENTRY(norm_record), ENTRY(recordable), ENTRY(linear_node),
+                         ENTRY(act_node), ENTRY(gated_node), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hyc_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
@@ -1218,5 +1563,12 @@ PyMODINIT_FUNC PyInit__hyc_host() {
                                                       {&s_S, "S"}, {&s_row_ptr, "row_ptr"}, {&s_cols, "cols"}, {&s_threshold, "threshold"},
                                                       {&s_scale, "scale"}, {&s_L, "L"}, {&s_R, "R"}};
   for (auto& n : names) *n.to = PyUnicode_InternFromString(n.s);
+  HANDLE_TH_ERRORS
+  Ref types(PyImport_ImportModule("types"));
+  if (!types.p || !(t_namespace = PyObject_GetAttrString(types.p, "SimpleNamespace"))) return nullptr;
+  node_type.tp_getattro = node_attribute;
+  torch::autograd::_initFunctionPyTypeObject(node_type, "CalibratedBackward", nullptr, nullptr);
+  torch::autograd::registerCppFunction(typeid(Recorded), &node_type);
+  END_HANDLE_TH_ERRORS
   return PyModule_Create(&module);
 }

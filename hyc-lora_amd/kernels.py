@@ -318,6 +318,13 @@ class _Native:
 native = _Native()
 
 
+def node(name):
+    """the function `name` of csrc/host/host.cpp that also records the operator's backward natively, without a torch.autograd.Function
+    around it (None, or a None from it: the Function serves).  Whoever puts something else in the place of `native`, to count the calls
+    or to have the interpreted forms alone, sees every one of them: nothing is recorded past it."""
+    return getattr(native, name) if type(native) is _Native else None
+
+
 def alloc_channel(M, H, plan, bits, group, device):
     if plan.H != H:
         raise ValueError("the outlier-channel plan was made for %d channels, the activation has %d" % (plan.H, H))
@@ -444,6 +451,20 @@ def threshold_native(x, norm, w, bias, eps, S, threshold, scale, bits, L, R, bud
     y, mean, rstd, stored, row_ptr, cols, vals, total = done
     budget.watch(total, cap, M)
     return y, mean, rstd, ThresholdCompressed(stored, row_ptr, cols, vals, float(threshold), scale, L, R, bits, M, H, S)
+
+
+def threshold_norm(x, norm, w, bias, eps, static_value, bits, rank, quirk, interpreted, label):
+    """y of a calibrated norm of the reference's scheme with its backward recorded natively, or None: the Function serves"""
+    outlier, L, scale, R = static_value
+    possible = node("recordable")
+    if possible is None or not possible(x, w, bias):
+        return None
+    done = threshold_native(x, norm, w, bias, eps, x.shape[-2] if x.dim() >= 2 else 1, threshold_value(outlier), scale, bits,
+                            L if rank > 0 else None, R if rank > 0 else None, kept_budget(outlier))
+    if done is None:
+        return None
+    y, mean, rstd, c = done
+    return native.norm_record(y, x, w, bias, c, mean, rstd, quirk, interpreted, label)
 
 
 def compress_threshold(x2d, S, threshold, scale, bits, L=None, R=None, budget=None):

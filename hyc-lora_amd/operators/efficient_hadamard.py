@@ -107,6 +107,19 @@ def _row_view(t):
         return t.reshape(-1, H)
 
 
+def _gated_backward(ctx, grad_output):
+    grads = K.native.gated_bwd(K.ACT_CODES[ctx.act], grad_output, *ctx.saved, ctx.grad_room)
+    if grads is not None:
+        d_gate, d_up = grads[:2]
+    else:
+        g2, _ = as_rows(grad_output.to(torch.bfloat16))
+        grads = K.gated_act_bwd(ctx.act, g2, *ctx.saved, room=ctx.grad_room)
+        d_gate, d_up = (t.reshape(grad_output.shape) for t in grads[:2])
+    if ctx.grad_room is not None:
+        d_gate._hyc_rows = d_up._hyc_rows = grads[2]
+    return d_gate, d_up
+
+
 class _ChannelGatedActFunc(torch.autograd.Function):
     """h = act(gate) * up with the three activations EfficientMemorySiLU/GELU and EfficientMemoryHadamard would save
     (gate; act(gate) and up), and one backward pass over them."""
@@ -135,16 +148,7 @@ class _ChannelGatedActFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        grads = K.native.gated_bwd(K.ACT_CODES[ctx.act], grad_output, *ctx.saved, ctx.grad_room)
-        if grads is not None:
-            d_gate, d_up = grads[:2]
-        else:
-            g2, _ = as_rows(grad_output.to(torch.bfloat16))
-            grads = K.gated_act_bwd(ctx.act, g2, *ctx.saved, room=ctx.grad_room)
-            d_gate, d_up = (t.reshape(grad_output.shape) for t in grads[:2])
-        if ctx.grad_room is not None:
-            d_gate._hyc_rows = d_up._hyc_rows = grads[2]
-        return d_gate, d_up, None, None, None, None, None, None
+        return _gated_backward(ctx, grad_output) + (None,) * 6
 
 
 class EfficientMemoryGatedAct(torch.nn.Module):
@@ -171,7 +175,13 @@ class EfficientMemoryGatedAct(torch.nn.Module):
 
     def forward(self, gate, up, grad_room=None):
         grad_room = self.grad_room if grad_room is None else grad_room
-        out = _ChannelGatedActFunc.apply(gate, up, self.act, (self.site_act, self.site_up, self.site_gate), self.iteration,
-                                         self.sub_outlier_bit, self.group_size, grad_room)
+        sites, bits, group, out = (self.site_act, self.site_up, self.site_gate), self.sub_outlier_bit, self.group_size, None
+        if (grad_room is None and self.iteration >= 2 and all(site.plan is not None for site in sites)
+                and K.gated_act_fwd_supported(gate.shape[-1], bits, group)):
+            record = K.node("gated_node")
+            out = record and record(K.ACT_CODES[self.act], gate, up, *(site.plan for site in sites), bits, group, self.act, _gated_backward,
+                                    "_ChannelGatedActFuncBackward")
+        if out is None:
+            out = _ChannelGatedActFunc.apply(gate, up, self.act, sites, self.iteration, bits, group, grad_room)
         self.iteration += 1
         return out

@@ -135,9 +135,21 @@ class EfficientMemoryLayerNorm(torch.nn.LayerNorm):
     def forward(self, x):
         if self.mode == "hyc":
             plan = self.site.channel_plan(x, self.iteration)
-            y = _ChannelLayerNormFunc.apply(x, self.weight, self.bias, self.eps, plan, self.sub_outlier_bit, self.group_size)
+            weight, bias = self.weight, self.bias
+            record = K.node("norm_node") if K.layernorm_fwd_supported(x.shape[-1], self.sub_outlier_bit) else None
+            y = record and record(x, weight, bias, True, self.eps, plan, self.sub_outlier_bit, self.group_size, False, _backward,
+                                  "_ChannelLayerNormFuncBackward")
+            if y is None:
+                y = _ChannelLayerNormFunc.apply(x, weight, bias, self.eps, plan, self.sub_outlier_bit, self.group_size)
             self.iteration += 1
             return y
+        if (self.iteration >= 2 and x.dim() == 3 and self.sub_outlier_ratio > 0. and self.sub_outlier_bit != 16 and x.shape[-1] <= 32768
+                and K.layernorm_fwd_supported(x.shape[-1], self.sub_outlier_bit)):
+            y = K.threshold_norm(x, 2, self.weight, self.bias, self.eps, self.static_value, self.sub_outlier_bit, self.rank, False, _backward,
+                                 "EfficientMemoryLayerNormFuncBackward")
+            if y is not None:
+                self.iteration += 1
+                return y
         result, outlier, L, R, scale = EfficientMemoryLayerNormFunc.apply(
             x, self.normalized_shape, self.outlier_ratio, self.sub_outlier_ratio, self.sub_outlier_bit,
             self.sub_outlier_quantize_method, self.rank, self.weight, self.bias, self.eps, self.iteration,

@@ -53,6 +53,15 @@ class EfficientMemoryLinearFunc(torch.autograd.Function):
         return gi, gw, gb, None, None, None, None, None, None, None, None
 
 
+def _channel_backward(ctx, grad_output):
+    if not ctx.use_bias:
+        needs, w = ctx.needs_input_grad, ctx.w
+        done = K.native.linear_bwd(grad_output, w, ctx.saved if needs[1] else None, needs[0], K.gradw_staged_by_default(*w.shape))
+        if done is not None:
+            return done[0], done[1], None
+    return _linear_backward(grad_output, ctx.w.detach(), ctx.saved, ctx.use_bias, ctx.needs_input_grad[:3])
+
+
 class _ChannelLinearFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b, plan, bits, group):
@@ -74,13 +83,7 @@ class _ChannelLinearFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        if not ctx.use_bias:
-            needs, w = ctx.needs_input_grad, ctx.w
-            done = K.native.linear_bwd(grad_output, w, ctx.saved if needs[1] else None, needs[0], K.gradw_staged_by_default(*w.shape))
-            if done is not None:
-                return done[0], done[1], None, None, None, None
-        gi, gw, gb = _linear_backward(grad_output, ctx.w.detach(), ctx.saved, ctx.use_bias, ctx.needs_input_grad[:3])
-        return gi, gw, gb, None, None, None
+        return _channel_backward(ctx, grad_output) + (None, None, None)
 
 
 class EfficientMemoryLinear(torch.nn.Linear):
@@ -103,7 +106,12 @@ class EfficientMemoryLinear(torch.nn.Linear):
     def forward(self, input: torch.Tensor):
         if self.mode == "hyc":
             plan = self.site.channel_plan(input, self.iteration)
-            result = _ChannelLinearFunc.apply(input, self.weight, self.bias, plan, self.sub_outlier_bit, self.group_size)
+            weight, bias = self.weight, self.bias
+            record = K.node("linear_node") if bias is None else None
+            result = record and record(input, weight, plan, self.sub_outlier_bit, self.group_size, K.gradw_staged_by_default(*weight.shape),
+                                       _channel_backward, "_ChannelLinearFuncBackward")
+            if result is None:
+                result = _ChannelLinearFunc.apply(input, weight, bias, plan, self.sub_outlier_bit, self.group_size)
             self.iteration += 1
             return result
         result, outlier, L, R, scale = EfficientMemoryLinearFunc.apply(

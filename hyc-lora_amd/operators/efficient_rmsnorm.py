@@ -43,8 +43,7 @@ def _ref_forward(ctx, x, outlier_ratio, sub_outlier_ratio, sub_outlier_bit, sub_
     return y, outlier, L, R, scale
 
 
-def _ref_backward(ctx, dy):
-    dy = result_gradient(ctx, dy)
+def _backward(ctx, dy):
     if not ctx.weight_offset:
         done = K.native.norm_bwd(dy, ctx.saved, ctx.weight, None, ctx.rstd, bool(ctx.c2_quirk))
         if done is not None:
@@ -70,7 +69,7 @@ class EfficientMemoryRMSNormFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, grad_outlier, grad_L, grad_R, grad_scale):
-        dx, dw = _ref_backward(ctx, dy)
+        dx, dw = _backward(ctx, result_gradient(ctx, dy))
         return dx, None, None, None, None, None, None, dw, None, None, None, None
 
 
@@ -86,7 +85,7 @@ class _RMSNormFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy, grad_outlier, grad_L, grad_R, grad_scale):
-        dx, dw = _ref_backward(ctx, dy)
+        dx, dw = _backward(ctx, result_gradient(ctx, dy))
         return dx, None, None, None, None, None, None, dw, None, None, None, None, None, None
 
 
@@ -106,14 +105,7 @@ class _ChannelRMSNormFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        if not ctx.weight_offset:
-            done = K.native.norm_bwd(dy, ctx.saved, ctx.weight, None, ctx.rstd, bool(ctx.c2_quirk))
-            if done is not None:
-                return done[0], done[1], None, None, None, None, None, None
-        dy2, _ = as_rows(dy.to(torch.bfloat16))
-        dx, dw = K.rmsnorm_bwd(dy2, ctx.saved, _effective_weight(ctx.weight, ctx.weight_offset), ctx.rstd,
-                               c2_quirk=ctx.c2_quirk)
-        return dx.reshape(dy.shape), dw.to(ctx.weight.dtype), None, None, None, None, None, None
+        return _backward(ctx, dy) + (None,) * 6
 
 
 class EfficientMemoryRMSNorm(torch.nn.LayerNorm):
@@ -140,10 +132,21 @@ class EfficientMemoryRMSNorm(torch.nn.LayerNorm):
     def forward(self, x):
         if self.mode == "hyc":
             plan = self.site.channel_plan(x, self.iteration)
-            y = _ChannelRMSNormFunc.apply(x, self.weight, self.eps, plan, self.sub_outlier_bit, self.group_size,
-                                          self.ref_c2_quirk, self._func.weight_offset)
+            weight, offset = self.weight, self._func.weight_offset
+            record = None if offset else K.node("norm_node")
+            y = record and record(x, weight, None, False, self.eps, plan, self.sub_outlier_bit, self.group_size, bool(self.ref_c2_quirk),
+                                  _backward, "_ChannelRMSNormFuncBackward")
+            if y is None:
+                y = _ChannelRMSNormFunc.apply(x, weight, self.eps, plan, self.sub_outlier_bit, self.group_size, self.ref_c2_quirk, offset)
             self.iteration += 1
             return y
+        if (self.iteration >= 2 and not self._func.weight_offset and self.bias is None and self.sub_outlier_ratio and self.sub_outlier_bit != 16
+                and x.shape[-1] <= 32768):
+            y = K.threshold_norm(x, 1, self.weight, None, self.eps, self.static_value, self.sub_outlier_bit, self.rank,
+                                 bool(self.ref_c2_quirk), _backward, "_RMSNormFuncBackward")
+            if y is not None:
+                self.iteration += 1
+                return y
         result, outlier, L, R, scale = _RMSNormFunc.apply(
             x, self.normalized_shape, self.outlier_ratio, self.sub_outlier_ratio, self.sub_outlier_bit,
             self.sub_outlier_quantize_method, self.rank, self.weight, self.bias, self.eps, self.iteration,

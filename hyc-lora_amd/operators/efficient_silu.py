@@ -51,6 +51,14 @@ class EfficientMemorySiLUFunc(torch.autograd.Function):
         return _ref_backward(ctx, "silu", grad_output), None, None, None, None, None, None, None
 
 
+def _channel_backward(ctx, grad_output):
+    dx = K.native.act_bwd(K.ACT_CODES[ctx.act], grad_output, ctx.saved)
+    if dx is None:
+        g2, _ = as_rows(grad_output.to(torch.bfloat16))
+        dx = K.act_bwd(ctx.act, g2, ctx.saved).reshape(grad_output.shape)
+    return (dx,)
+
+
 class _ChannelActFunc(torch.autograd.Function):
     """channel-mode twin: apply(x, act, plan, bits, group) -> act(x); x saved as ChannelCompressed"""
 
@@ -71,11 +79,7 @@ class _ChannelActFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        dx = K.native.act_bwd(K.ACT_CODES[ctx.act], grad_output, ctx.saved)
-        if dx is not None:
-            return dx, None, None, None, None
-        g2, _ = as_rows(grad_output.to(torch.bfloat16))
-        return K.act_bwd(ctx.act, g2, ctx.saved).reshape(grad_output.shape), None, None, None, None
+        return _channel_backward(ctx, grad_output) + (None,) * 4
 
 
 class _ActModule(torch.nn.Module):
@@ -101,7 +105,11 @@ class _ActModule(torch.nn.Module):
     def forward(self, input):
         if self.mode == "hyc":
             plan = self.site.channel_plan(input, self.iteration)
-            result = _ChannelActFunc.apply(input, self._act, plan, self.sub_outlier_bit, self.group_size)
+            bits, group = self.sub_outlier_bit, self.group_size
+            record = K.node("act_node") if K.act_fwd_compress_supported(input.shape[-1], bits, group) else None
+            result = record and record(K.ACT_CODES[self._act], input, plan, bits, group, self._act, _channel_backward, "_ChannelActFuncBackward")
+            if result is None:
+                result = _ChannelActFunc.apply(input, self._act, plan, bits, group)
             self.iteration += 1
             return result
         result, outlier, L, R, scale = self._func.apply(
