@@ -256,10 +256,12 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
     @staticmethod
     def _grad_A(ctx, dh, A):
         """dA_i = dh_i^T @ x_hat: the projections of a group read the same saved activation, so their dh go through the
-        weight-gradient kernel side by side (32 output rows per call, the widest its LoRA-shaped form takes) and x_hat is
-        decoded once per call instead of once per projection"""
+        weight-gradient kernel side by side (up to 128 output rows a call, what its form for few of them takes in tiles of 32): one
+        launch, and one that adds up the partial results, for the whole group.  With 32 rows a call and 8-bit codes, two or three
+        calls -> one, us: 48 rows at 157 x 2048 11.4 -> 6.7, 2048 x 4096 19.2 -> 13.9, 4096 x 4096 22.7 -> 15.2, 8192 x 2048
+        23.5 -> 16.3; 64 rows 13.0 -> 6.7, 21.3 -> 15.1, 24.7 -> 15.3, 24.7 -> 16.7; 96 rows 19.4 -> 6.8 to 37.4 -> 19.8"""
         r, dA = A[0].shape[0], []
-        per_call = max(1, 32 // r) * r
+        per_call = max(1, 128 // r) * r
         for c0 in range(0, dh.shape[1], per_call):
             block = K.gradw_gemm(dh[:, c0:c0 + per_call], ctx.saved_x, out_dtype=A[0].dtype)
             dA.extend(block[j:j + r] for j in range(0, block.shape[0], r))
