@@ -96,6 +96,9 @@ SIGNATURES = {
     "hyc_lora_down": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i32, c_i32, c_ptr, c_ptr]),
     "hyc_thin_covers": (c_i32, [c_i64, c_i64, c_i64, c_i32]),
     "hyc_thin_dx": (c_i32, [c_ptr, c_i64, c_i64, c_ptr, c_i32, c_i64, c_ptr, c_ptr]),
+    "hyc_few_rows_covers": (c_i32, [c_i64, c_i64, c_i64, c_i32]),
+    "hyc_few_rows_nf4": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i32, c_i32, c_f32, c_ptr, c_ptr]),
+    "hyc_few_rows": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i64, c_ptr, c_ptr]),
     "hyc_lora_up": (c_i32, [c_ptr, c_i64, c_ptr, c_ptr, c_i32, c_i32, c_f32, c_ptr, c_ptr]),
     "hyc_lora_weight_t": (c_i32, [c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_i32, c_i32, c_i64, c_ptr, c_ptr]),
     "hyc_lora_up_bwd_workspace_bytes": (c_i64, [c_i64, c_ptr, c_i32, c_i32]),

@@ -908,14 +908,21 @@ PyObject* lora_forward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   Out o;
   const bool keep = a[8] != Py_None;
   if (keep && !o.init(a[8], a[9], a[10], M, K, x->device())) return none();
+  bool few = hyc_few_rows_covers(M, K, total, 0);                      // kernels.few_rows_base
+  for (int i = 0; i < A.n; ++i) few = few && outs[i] % 16 == 0;
+  few = few && aligned16(packed->data_ptr()) && aligned16(absmax->data_ptr());
   Tensor x2, h, y;
   OR_NONE(unlocked([&] {
     x2 = x->view({M, K});
     h = empty_like_on(*x, {M, A.n * r}, BF16);
     y = empty_like_on(*x, {M, total}, BF16);
     int rc = hyc_lora_down(x->data_ptr(), K, M, K, A.p, A.n, (int32_t)r, h.data_ptr(), stream());
-    if (!rc) rc = hyc_lora_up(h.data_ptr(), M, B.p, outs, B.n, (int32_t)r, (float)scale, y.data_ptr(), stream());
-    if (!rc) {                                                         // (the weight's room is free again for the codes)
+    if (!rc && few)
+      rc = hyc_few_rows_nf4(x->data_ptr(), K, M, K, packed->data_ptr(), (const float*)absmax->data_ptr(), h.data_ptr(), B.p, outs, B.n, (int32_t)r,
+                            (float)scale, y.data_ptr(), stream());
+    else if (!rc)
+      rc = hyc_lora_up(h.data_ptr(), M, B.p, outs, B.n, (int32_t)r, (float)scale, y.data_ptr(), stream());
+    if (!rc && !few) {                                                 // (the weight's room is free again for the codes)
       const Tensor w = empty_like_on(*x, {total, K}, BF16);
       rc = hyc_nf4_dequantize(packed->data_ptr(), (const float*)absmax->data_ptr(), total * K, w.data_ptr(), stream());
       if (!rc) accumulate(y, x2, w, parts);
@@ -1007,7 +1014,10 @@ PyObject* lora_backward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const Tensor wt = empty_like_on(*h, {K, total + room}, BF16);
     dx = empty_like_on(*h, {M, K}, BF16);
     rc = hyc_lora_weight_t(packed->data_ptr(), (const float*)absmax->data_ptr(), K, A.p, outs, n, (int32_t)r, room, wt.data_ptr(), stream());
-    if (!rc) product(dx, ext, wt, cut);
+    if (!rc && hyc_few_rows_covers(M, total + room, K, 1))
+      rc = hyc_few_rows(ext.data_ptr(), total + room, M, total + room, wt.data_ptr(), K, dx.data_ptr(), stream());
+    else if (!rc)
+      product(dx, ext, wt, cut);
     return rc;
   }));
   PyObject* t = PyTuple_New(1 + 2 * n);

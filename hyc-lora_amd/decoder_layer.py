@@ -157,11 +157,14 @@ def _parts(M, N):
 
 
 def _product(out, a, b, accumulate=False):
-    """out [M, N] (+)= a @ b^T, both operands contiguous along the reduction, in one product or more (_cut_columns, _parts)"""
+    """out [M, N] (+)= a @ b^T, both operands contiguous along the reduction, in one product or more (_cut_columns, _parts); over few
+    rows by the package's own (kernels.few_rows)"""
     M, N = out.shape
     if accumulate:
         for c0, c1, r0, r1 in _parts(M, N):
             out[r0:r1, c0:c1].addmm_(a[r0:r1], b[c0:c1].t())
+        return
+    if K.few_rows(out, a, b):
         return
     cut = _cut_columns(M, N)
     for lo, hi in (((0, cut), (cut, N)) if cut else ((0, N),)):
@@ -193,9 +196,9 @@ def _kernel_rows(t):
 
 
 class _LoRAProjectionsFunc(torch.autograd.Function):
-    """A group is one library product each way: forward y = s h B^T (h = x A^T), onto which the base product accumulates in
-    its epilogue (in parts, see _parts); backward dX = [dY | s dY B] [W^T | A^T]^T with the rank-r terms as further columns of the
-    reduction (kernels.lora_down / lora_up / lora_up_bwd / lora_weight_t)."""
+    """A group is one product each way: forward y = s h B^T (h = x A^T), onto which the base product accumulates in its epilogue (in
+    parts, see _parts; over few tokens both in one launch from the codes, kernels.few_rows_base); backward dX = [dY | s dY B] [W^T |
+    A^T]^T with the rank-r terms as further columns of the reduction (kernels.lora_down / lora_up / lora_up_bwd / lora_weight_t)."""
 
     @staticmethod
     def forward(ctx, x, mod, plan, *ab):
@@ -215,8 +218,10 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
                     return ys
         x2 = _kernel_rows(x)
         h = K.lora_down(x2, A)
-        y_all = K.lora_up(h, B, mod.scaling, mod.out_features)
-        _product(y_all, x2, K.nf4_dequantize(mod.base_all), accumulate=True)
+        y_all = K.few_rows_base(x2, mod.base_all, h, B, mod.scaling, mod.out_features)
+        if y_all is None:
+            y_all = K.lora_up(h, B, mod.scaling, mod.out_features)
+            _product(y_all, x2, K.nf4_dequantize(mod.base_all), accumulate=True)
         outs, row = [], 0
         for out in mod.out_features:                            # column slices: no copies, consumers take the pitch
             outs.append(y_all[:, row:row + out].unflatten(0, x.shape[:-1]))

@@ -1200,6 +1200,38 @@ def lora_up(h, B, scale, outs=None):
     return y
 
 
+def few_rows_base(x2, base, h, B, scale, outs):
+    """y [M, sum(outs)] = scale * h_i B_i^T + x W^T in one launch from the codes of W, or None where the products take other forms
+    (hyc_few_rows_covers, and what the launch reads)"""
+    (M, H), n, total = x2.shape, len(outs), sum(outs)
+    r, pitch = h.shape[-1] // n, x2.stride(0) if M > 1 else H
+    if not M or any(o % 16 for o in outs) or not _lora_kernels_cover(M, n, r, H, tuple(outs)) or h.shape != (M, n * r):
+        return None
+    if (x2.dtype != BF16 or not x2.is_cuda or x2.data_ptr() % 16 or x2.stride(1) != 1 or pitch < H or pitch % 8 or M * pitch >= 1 << 30
+            or any(t.dtype != dt or t.numel() * per != total * H or t.device != x2.device or not t.is_contiguous() or t.data_ptr() % 16
+                   for t, dt, per in ((base.packed, torch.uint8, 2), (base.absmax, torch.float32, 64)))):
+        return None
+    lib = _abi.load()
+    if not lib.hyc_few_rows_covers(M, H, total, 0) or not _lora_factors(B, [(o, r) for o in outs], x2.device, "B"):
+        return None
+    _need(h, BF16, "h")
+    y = torch.empty((M, total), dtype=BF16, device=x2.device)
+    check(lib.hyc_few_rows_nf4(_p(x2), pitch, M, H, _p(base.packed), _p(base.absmax), _p(h), _ptrs(B), _i64s(outs), n, r, float(scale), _p(y), _stream()))
+    return y
+
+
+def few_rows(out, a, b):
+    """out [M, N] = a @ b^T in one launch where that is better than a library product (hyc_few_rows_covers); whether it was"""
+    (M, H), N = a.shape, b.shape[0]
+    if any(t.dtype != BF16 or not t.is_cuda or not t.is_contiguous() or t.data_ptr() % 16 for t in (out, a, b)):
+        return False
+    lib = _abi.load()
+    if not lib.hyc_few_rows_covers(M, H, N, 1):
+        return False
+    check(lib.hyc_few_rows(_p(a), H, M, H, _p(b), N, _p(out), _stream()))
+    return True
+
+
 def lora_up_bwd(gs, B, h, scale, room, ext=None):
     """(ext, dh, [dB_i]) from the gradients gs[i] [M, out_i] of a group: dB_i = scale * gs[i]^T h_i, dh = scale * gs[i] B_i
     side by side [M, n r] and, with zeros behind them, as the columns [sum(outs), + room) of ext.  ext: the buffer the gs

@@ -350,6 +350,9 @@ int hyc_rope_from_heads(const void* g, const void* cosv, const void* sinv, int64
  *   hyc_thin_covers    1 where x w^T (hyc_lora_down with w as its one factor) or, with input_grad, g w (hyc_thin_dx) of a
  *                      linear layer with N output features is better taken by these kernels than by a library product
  *   hyc_lora_up        y bf16 [M, sum n_out] = scale * h_i B_i^T side by side (the base product accumulates onto it)
+ *   hyc_few_rows_nf4   y = bf16(scale * h_i B_i^T) + x W^T in one launch, W = the base as its codes (N a multiple of 16, as each n_out)
+ *   hyc_few_rows       y bf16 [M, N] = x w^T for w bf16 [N, K] (K a multiple of 64, N of 16)
+ *   hyc_few_rows_covers  1 where the first (input_grad 0) or the second is better than a library product over [M, K] and [N, K]
  *   hyc_lora_up_bwd    from one read of dY_i [M, n_out_i] (rows ldg[i] apart): dh = bf16(scale * dY_i B_i) to dh [M, n r] and,
  *                      with zeros behind them, to the `room` columns [sum n_out, + room) of ext (rows ld_ext apart);
  *                      dB_i = scale * dY_i^T h_i; with copy_dy the dY_i side by side to the first sum n_out columns of ext.
@@ -363,6 +366,10 @@ int32_t hyc_thin_covers(int64_t M, int64_t K, int64_t N, int32_t input_grad);
 int hyc_thin_dx(const void* g, int64_t ldg, int64_t M, const void* w, int32_t N, int64_t K, void* dx, void* stream);
 int hyc_lora_up(const void* h, int64_t M, const void* const* B, const int64_t* n_out, int32_t n, int32_t r, float scale, void* y,
                 void* stream);
+int32_t hyc_few_rows_covers(int64_t M, int64_t K, int64_t N, int32_t input_grad);
+int hyc_few_rows_nf4(const void* x, int64_t ldx, int64_t M, int64_t K, const void* packed, const float* absmax, const void* h, const void* const* B,
+                     const int64_t* n_out, int32_t n, int32_t r, float scale, void* y, void* stream);
+int hyc_few_rows(const void* x, int64_t ldx, int64_t M, int64_t K, const void* w, int64_t N, void* y, void* stream);
 int64_t hyc_lora_up_bwd_workspace_bytes(int64_t M, const int64_t* n_out, int32_t n, int32_t r);
 int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const int64_t* n_out, const void* const* B, const void* h,
                     int32_t n, int32_t r, float scale, void* dh, void* ext, int64_t ld_ext, int64_t room, int32_t copy_dy, void* const* dB,
