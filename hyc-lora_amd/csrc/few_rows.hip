@@ -6,7 +6,7 @@
 // Over a few hundred tokens a product is a walk over the weight, and the library's call costs the host more (20 to 25 us) than the walk
 // costs the GPU; the decoded weight, written and read again, is a second launch, and y = s h B^T a third.  What bounds the walk is how
 // fast operands reach a CU; with fragments loaded as the matrix operands want them, neighbouring lanes in different rows, 157 tokens x
-// 2048 -> 2048 / 6144 / 11264 took 15.7 / 34.5 / 51.1 us instead of 8.3 / 17.4 / 25.7.
+// 2048 -> 2048 / 6144 / 11264 took 15.7 / 34.5 / 51.1 us instead of 8.2 / 15.9 / 25.5.
 #include "abi_util.hpp"
 #include "nf4_levels.hpp"
 
@@ -17,7 +17,6 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 #define HYC_MFMA16(a_, b_, c_) __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_, b_, c_, 0, 0, 0)
 
 constexpr int FR_MAX = 4;                                // projections of a group
-constexpr int FR_MT = 5;                                 // token tiles of 16 a workgroup takes at most
 
 struct FewRows {
   const uint16_t* x;                                     // [M, K], rows ldx apart
@@ -193,15 +192,23 @@ k_few_rows(FewRows a) {
   }
 }
 
+// Tokens in tiles of 4 or 5 a workgroup, whichever pads less; features in 1, 2 or 4, the fewest with which the workgroups are resident at
+// once, one of eight waves a CU; past that, 4 features' tiles and workgroups of four waves, two a CU (so are those of a weight that goes
+// through LDS).
 template <bool NF4>
 static void few_rows_launch(const FewRows& a, hipStream_t st) {
-  const int tiles = (a.M + 15) / 16, down = (tiles + FR_MT - 1) / FR_MT, mt = (tiles + down - 1) / down;
-  const int across = a.N / 16, nt = across * down > 512 ? 2 : 1;
+  const int tiles = (a.M + 15) / 16, across = a.N / 16;
+  const int mt = tiles <= 4 ? tiles : (tiles + 4) / 5 * 5 < (tiles + 3) / 4 * 4 ? 5 : 4, down = (tiles + mt - 1) / mt;
+  // (2048 -> 2048 over 512 tokens with 1 / 2 / 4 tiles of features, us: 17.0 / 14.9 / 13.4; over 256 26.2 in four waves / 9.2 / 12.8)
+  const int nt = across * down <= 256 ? 1 : (across + 1) / 2 * down <= 256 ? 2 : 4;
   const dim3 grid((unsigned)((across + nt - 1) / nt), (unsigned)down);
+  const bool four = nt == 4 && (!NF4 || grid.x * grid.y > 256);
 #define HYC_GO(MT_)                                                                                        \
   do {                                                                                                     \
-    if (nt == 2) hipLaunchKernelGGL((k_few_rows<MT_, 2, NF4, 4>), grid, dim3(256), 0, st, a);               \
-    else hipLaunchKernelGGL((k_few_rows<MT_, 1, NF4, 8>), grid, dim3(512), 0, st, a);                       \
+    if (nt == 1) hipLaunchKernelGGL((k_few_rows<MT_, 1, NF4, 8>), grid, dim3(512), 0, st, a);               \
+    else if (nt == 2) hipLaunchKernelGGL((k_few_rows<MT_, 2, NF4, 8>), grid, dim3(512), 0, st, a);          \
+    else if (four) hipLaunchKernelGGL((k_few_rows<MT_, 4, NF4, 4>), grid, dim3(256), 0, st, a);             \
+    else if constexpr (NF4) hipLaunchKernelGGL((k_few_rows<MT_, 4, NF4, 8>), grid, dim3(512), 0, st, a);    \
   } while (0)
   switch (mt) {
     case 1: HYC_GO(1); break;
@@ -221,30 +228,32 @@ extern "C" {
 
 // Where these products are taken.  GPU time, us, library with its decoding and k_lora_up (forward) or alone (dX) -> one launch here; a
 // library call costs the host 21 to 30 us beside it, one of these 5.
-//   forward K -> N      16 tokens      157            256            512            1024
-//   1024 -> 1024        11.6 -> 3.5    16.6 -> 5.5    17.6 -> 5.3    18.0 -> 9.8    19.0 -> 11.0
-//   1024 -> 5632        18.2 -> 4.7    25.4 -> 11.0   28.1 -> 13.0   32.9 -> 23.6   40.7 -> 40.4
-//   2048 -> 6144        28.1 -> 6.6    36.7 -> 17.4   40.1 -> 20.8   39.4 -> 43.9   47.3 -> 69.2
-//   2048 -> 11264       28.0 -> 9.8    40.6 -> 25.7   43.7 -> 36.0   52.7 -> 69.2   75.7 -> 120
-//   5632 -> 2048        24.7 -> 7.3    34.4 -> 17.2   33.0 -> 24.3   35.0 -> 36.5   48.3 -> 67.5
-//   4096 -> 12288       45.7 -> 20.1   59.1 -> 42.8   68.9 -> 65.9   81.1 -> 134
-//   11008 -> 4096       49.1 -> 15.5   59.6 -> 54.7   62.1 -> 62.2   84.9 -> 124
-//   dX N -> K           16             157            256            512            1024
-//   1024 -> 1024        5.6 -> 2.8     5.5 -> 4.8     5.6 -> 4.7     6.6 -> 8.6     7.9 -> 9.3
-//   3072 -> 1024        10.0 -> 4.0    10.7 -> 8.3    13.4 -> 7.7    16.2 -> 16.2   19.1 -> 19.3
-//   2048 -> 2048        8.7 -> 3.9     9.7 -> 7.3     13.4 -> 10.4   14.1 -> 13.8   16.0 -> 24.4
-//   11264 -> 2048       30.4 -> 11.4   37.1 -> 25.5   38.5 -> 40.4   47.3 -> 55.9
-//   2048 -> 5632        11.2 -> 6.3    14.7 -> 14.0   19.4 -> 17.0   20.7 -> 31.4
-//   12288 -> 4096       33.4 -> 16.7   46.6 -> 54.3   49.8 -> 52.9   71.4 -> 117
-//   4096 -> 11008       27.0 -> 16.6   30.5 -> 37.2   38.9 -> 61.9
-// A workgroup's tiles share its operands with no other one, so what a launch reads grows with the products of the sides; the library
-// wins where that outweighs what a launch costs it.  Over a long reduction into few features it has too few workgroups for longer.
+//   forward K -> N      16 tokens      157            256            512            1024           2048
+//   1024 -> 1024        11.8 -> 3.5    16.6 -> 5.5    17.5 -> 5.2    18.0 -> 6.7    19.2 -> 9.5    21.8 -> 14.9
+//   1024 -> 5632        17.2 -> 4.5    25.3 -> 11.2   28.6 -> 14.3   32.9 -> 22.0   41.5 -> 37.1   54.7 -> 64.8
+//   2048 -> 2048        17.2 -> 4.4    21.1 -> 8.2    25.2 -> 9.5    27.4 -> 13.3   31.4 -> 22.9   37.1 -> 41.7
+//   2048 -> 6144        29.0 -> 6.3    37.1 -> 15.9   40.0 -> 22.8   38.9 -> 33.2   46.7 -> 58.7
+//   2048 -> 11264       27.8 -> 11.5   39.4 -> 25.5   43.3 -> 32.9   52.2 -> 57.7   75.3 -> 102
+//   5632 -> 2048        24.6 -> 7.3    33.9 -> 17.0   32.8 -> 19.1   34.1 -> 27.7   47.7 -> 49.5
+//   4096 -> 12288       45.4 -> 19.9   58.9 -> 42.9   69.2 -> 56.6   80.0 -> 104
+//   11008 -> 4096       49.2 -> 15.5   59.4 -> 36.4   61.8 -> 48.0   86.7 -> 90.5
+//   dX N -> K           16             157            256            512            1024           2048
+//   1024 -> 1024        5.5 -> 2.8     5.5 -> 4.8     5.6 -> 4.7     6.6 -> 5.7     7.9 -> 7.6     10.4 -> 12.3
+//   3072 -> 1024        10.0 -> 4.0    10.7 -> 8.3    13.5 -> 7.7    16.3 -> 9.7    19.2 -> 13.9   21.7 -> 24.4
+//   2048 -> 2048        8.7 -> 3.5     9.6 -> 7.1     13.5 -> 7.4    14.1 -> 10.7   16.0 -> 17.1   22.0 -> 30.8
+//   11264 -> 2048       30.5 -> 11.4   37.0 -> 25.4   38.4 -> 25.7   46.7 -> 37.9   66.6 -> 67.2
+//   2048 -> 5632        11.2 -> 5.9    14.6 -> 11.8   19.4 -> 16.5   19.4 -> 23.8   29.2 -> 42.5
+//   12288 -> 4096       33.4 -> 16.7   46.8 -> 35.5   49.5 -> 40.8   71.1 -> 75.8
+//   4096 -> 11008       27.2 -> 16.7   30.5 -> 38.7   38.9 -> 54.6
+// A workgroup's tiles share their operands with no other one, so what a launch reads grows with the products of the sides.  dX is
+// better while its result is at most one tile of 64 x 64 a CU, whatever the reduction (at 1.25 of that 0.93 to 1.08 of the
+// library's speed, at 1.5 of it 0.7 to 0.9); the forward, which saves a pass over the decoded weight as well, up to 256 tokens and beyond them
+// until about 6e9 multiplications.
 int32_t hyc_few_rows_covers(int64_t M, int64_t K, int64_t N, int32_t input_grad) {
   if (M <= 0 || K <= 0 || N <= 0 || K % 64 != 0 || N % 16 != 0 || K > (1 << 24) || N > (1 << 24)) return 0;
   if (M * K >= ((int64_t)1 << 30) || N * K >= ((int64_t)1 << 30)) return 0;
-  const int64_t work = M * K * N;
-  if (!input_grad) return M <= 160 || (M <= 2048 && work <= (int64_t)1 << 32) ? 1 : 0;
-  return M <= 64 || (M <= 1024 && work <= (int64_t)1 << 31) || (M <= 160 && N * K <= (1 << 25) && K >= 2 * N) ? 1 : 0;
+  if (input_grad) return M <= 1024 && M * N <= (1 << 20) ? 1 : 0;
+  return M <= 256 || (M <= 2048 && M * K * N <= (int64_t)6000000000) ? 1 : 0;
 }
 
 static int few_rows_args(const char* who, const void* x, int64_t ldx, int64_t M, int64_t K, int64_t N, const void* w, const void* y) {

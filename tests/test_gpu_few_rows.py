@@ -22,7 +22,7 @@ def near(got, want, size, roundings):
 
 
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 79, 81, 160, 161, 257])
-@pytest.mark.parametrize("Kf,outs,r", [(64, [16], 8), (192, [48, 16], 16), (576, [272, 16, 32], 24), (1088, [64], 32), (128, [8208], 16)])
+@pytest.mark.parametrize("Kf,outs,r", [(64, [16], 8), (192, [48, 16], 16), (576, [272, 16, 32], 24), (1088, [64], 32), (128, [8208], 16), (128, [4784], 8)])
 def test_base_product_with_its_rank_term(K, M, Kf, outs, r):
     n, N, s = len(outs), sum(outs), 1.5
     if not K._abi.load().hyc_few_rows_covers(M, Kf, N, 0):
@@ -43,7 +43,7 @@ def test_base_product_with_its_rank_term(K, M, Kf, outs, r):
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 80, 81, 161, 400])
-@pytest.mark.parametrize("Kf,N", [(64, 16), (192, 64), (1088, 80), (128, 8208), (512, 512)])
+@pytest.mark.parametrize("Kf,N", [(64, 16), (192, 64), (1088, 80), (128, 8208), (512, 512), (128, 4784), (64, 2608)])
 def test_product(K, M, Kf, N):
     if not K._abi.load().hyc_few_rows_covers(M, Kf, N, 1):
         pytest.skip("left to the library")
@@ -65,7 +65,7 @@ def test_product(K, M, Kf, N):
 def test_what_is_left_to_the_library(K, hyc):
     covers = K._abi.load().hyc_few_rows_covers
     assert covers(157, 2048, 11264, 0) and covers(157, 11264 + 64, 2048, 1) and covers(16, 4096, 22016, 0) and covers(16, 22080, 4096, 1)
-    for M, Kf, N, grad in ((4096, 4096, 4096, 0), (4096, 4096, 4096, 1), (2049, 64, 16, 0), (0, 64, 16, 0), (8, 96, 16, 0), (8, 64, 24, 1),
+    for M, Kf, N, grad in ((4096, 4096, 4096, 0), (4096, 4096, 4096, 1), (2049, 64, 16, 0), (1025, 64, 16, 1), (257, 4096, 4096, 1), (0, 64, 16, 0), (8, 96, 16, 0), (8, 64, 24, 1),
                            (64, 1 << 24, 16, 0), (16, 64, 1 << 24, 1)):
         assert not covers(M, Kf, N, grad)
     mk = lambda *shape: torch.randn(*shape, device="cuda").to(BF16)
