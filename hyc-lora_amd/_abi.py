@@ -96,6 +96,8 @@ SIGNATURES = {
     "hyc_lora_down": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i32, c_i32, c_ptr, c_ptr]),
     "hyc_thin_covers": (c_i32, [c_i64, c_i64, c_i64, c_i32]),
     "hyc_thin_dx": (c_i32, [c_ptr, c_i64, c_i64, c_ptr, c_i32, c_i64, c_ptr, c_ptr]),
+    "hyc_softmax_csr_slab": (c_i32, [c_ptr, c_i64, c_i64, c_f32, c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),
+    "hyc_ref_outlier_csr_slab": (c_i32, [c_ptr, c_i64, c_i64, ctypes.POINTER(HycDesc), c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),
     "hyc_few_rows_covers": (c_i32, [c_i64, c_i64, c_i64, c_i32]),
     "hyc_few_rows_nf4": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i32, c_i32, c_f32, c_ptr, c_ptr]),
     "hyc_few_rows": (c_i32, [c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i64, c_ptr, c_ptr]),

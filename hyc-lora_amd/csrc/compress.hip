@@ -4,6 +4,7 @@
 
 #include "abi_util.hpp"
 #include "row_kernels.hpp"
+#include "softmax_slab.hpp"
 #include "threshold.hpp"
 #include "wave_scan.hpp"
 
@@ -318,24 +319,33 @@ k_outlier_count(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a,
 }
 
 // slab (may be null): rows of at most `cap` kept elements are copied from there (threshold.hip), x is read for the others only
+// OFFSETS: row_ptr is made here (csr_rows4), otherwise read.
+template <bool OFFSETS>
 __global__ void __launch_bounds__(256)
-k_outlier_fill(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a, const int32_t* __restrict__ row_ptr,
+k_outlier_fill(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a, int32_t* __restrict__ row_ptr,
                int32_t* __restrict__ cols, uint16_t* __restrict__ vals, const int32_t* __restrict__ counts,
-               const uint32_t* __restrict__ slab, int cap) {
+               const uint32_t* __restrict__ slab, int cap, int64_t capacity, int64_t* __restrict__ total) {
   __shared__ uint32_t stage_all[4][STAGE_CAP];
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  RowRoom room;
+  if constexpr (OFFSETS) room = csr_rows4(counts, M, capacity, row_ptr, total);
   if (row >= M) return;                                  // whole waves leave together
   uint32_t* stage = stage_all[threadIdx.x >> 6];
   const uint16_t* xr = x + row * H;
   const int64_t s_pos = row % a.S;
   const int64_t nch = H / 8;
-  const int64_t base = row_ptr[row];
-  const int limit = (int)(row_ptr[row + 1] - base);        // the row's room in cols / vals
+  if constexpr (!OFFSETS) {
+    room.base = row_ptr[row];
+    room.limit = (int)(row_ptr[row + 1] - room.base);
+    room.n = slab ? counts[row] : 0;
+  }
+  const int64_t base = room.base;
+  const int limit = room.limit;                          // the row's room in cols / vals
   int32_t* cols_row = cols + base;
   uint16_t* vals_row = vals + base;
   if (slab) {
-    const int n = counts[row];
+    const int n = room.n;
     if (n <= cap) {
       const int m = n < limit ? n : limit;
       for (int e = lane; e < m; e += 64) {
@@ -574,8 +584,9 @@ static int outlier_fill(const char* who, const void* x, int64_t M, int64_t H, co
   if (M == 0) return HYC_OK;
   if (!x || !row_ptr) return fail(HYC_EFAULT, "%s: null buffer", who);
   if (!aligned16(x)) return fail(HYC_EINVAL, "%s: x must be 16-byte aligned", who);
-  hipLaunchKernelGGL(k_outlier_fill, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, begin_launch(stream),
-                     static_cast<const uint16_t*>(x), M, H, a, row_ptr, cols, static_cast<uint16_t*>(vals), counts, slab, (int)cap);
+  hipLaunchKernelGGL(k_outlier_fill<false>, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, begin_launch(stream),
+                     static_cast<const uint16_t*>(x), M, H, a, const_cast<int32_t*>(row_ptr), cols, static_cast<uint16_t*>(vals), counts, slab, (int)cap,
+                     (int64_t)0, static_cast<int64_t*>(nullptr));
   return check_launch(who);
 }
 
@@ -589,6 +600,24 @@ int hyc_ref_outlier_fill_slab(const void* x, int64_t M, int64_t H, const hyc_des
   if (cap <= 0 || cap > H) return fail(HYC_EINVAL, "hyc_ref_outlier_fill_slab: cap=%lld must be in 1..H=%lld", (long long)cap, (long long)H);
   if (M > 0 && (!counts || !slab)) return fail(HYC_EFAULT, "hyc_ref_outlier_fill_slab: null buffer");
   return outlier_fill("hyc_ref_outlier_fill_slab", x, M, H, d, counts, slab, cap, row_ptr, cols, vals, stream);
+}
+
+int hyc_ref_outlier_csr_slab(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* counts, const uint32_t* slab, int64_t cap,
+                             int64_t capacity, int32_t* row_ptr, int64_t* total, int32_t* cols, void* vals, void* stream) {
+  if (M <= 0 || M > SLAB_OFFSETS_MAX || !aligned16(counts)) {
+    const int rc = hyc_csr_offsets(counts, M, capacity, row_ptr, total, stream);
+    return rc ? rc : hyc_ref_outlier_fill_slab(x, M, H, d, counts, slab, cap, row_ptr, cols, vals, stream);
+  }
+  ThrArgs a;
+  int rc = outlier_args("hyc_ref_outlier_csr_slab", x, M, H, d, &a);
+  if (rc) return rc;
+  if (cap <= 0 || cap > H) return fail(HYC_EINVAL, "hyc_ref_outlier_csr_slab: cap=%lld must be in 1..H=%lld", (long long)cap, (long long)H);
+  if (!x || !counts || !slab || !row_ptr) return fail(HYC_EFAULT, "hyc_ref_outlier_csr_slab: null buffer");
+  if (!aligned16(x)) return fail(HYC_EINVAL, "hyc_ref_outlier_csr_slab: x must be 16-byte aligned");
+  if (capacity < 0 || capacity > 0x7FFFFFFFll) capacity = 0x7FFFFFFFll;          // row_ptr is int32
+  hipLaunchKernelGGL(k_outlier_fill<true>, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, begin_launch(stream),
+                     static_cast<const uint16_t*>(x), M, H, a, row_ptr, cols, static_cast<uint16_t*>(vals), counts, slab, (int)cap, capacity, total);
+  return check_launch("hyc_ref_outlier_csr_slab");
 }
 
 }  // extern "C"

@@ -462,13 +462,18 @@ PyObject* bias_grad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 // ---- the threshold scheme and kept probabilities: side data sized ahead of time ------------------------------------------
 struct Csr {
   Tensor row_ptr, cols, vals, total;
-  // offsets of the counts, cut off at `cap` entries, and room for them
-  bool offsets(const Tensor& counts, int64_t rows, int64_t cap) {
+  // room for `cap` entries
+  void alloc(const Tensor& counts, int64_t rows, int64_t cap) {
     row_ptr = empty_like_on(counts, {rows + 1}, at::kInt);
     total = empty_like_on(counts, {}, at::kLong);
     cols = empty_like_on(counts, {cap}, at::kInt);
     vals = empty_like_on(counts, {cap}, BF16);
-    return hyc_csr_offsets((const int32_t*)counts.data_ptr(), rows, cap, (int32_t*)row_ptr.data_ptr(), (int64_t*)total.data_ptr(), stream()) == 0;
+  }
+  int64_t* all() const { return (int64_t*)total.data_ptr(); }
+  // and offsets of the counts, cut off at that
+  bool offsets(const Tensor& counts, int64_t rows, int64_t cap) {
+    alloc(counts, rows, cap);
+    return hyc_csr_offsets((const int32_t*)counts.data_ptr(), rows, cap, rp(), all(), stream()) == 0;
   }
   int32_t* rp() const { return (int32_t*)row_ptr.data_ptr(); }
   int32_t* co() const { return (int32_t*)cols.data_ptr(); }
@@ -529,10 +534,14 @@ PyObject* threshold_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                                     nullptr, nullptr, n, stream());
     else if (general)
       rc = hyc_compress(x->data_ptr(), M, H, &t.d, stored.data_ptr(), nullptr, nullptr, n, stream());
-    if (rc != 0 || !csr.offsets(counts, M, cap)) return -1;
-    if (general) return hyc_ref_outlier_fill(x->data_ptr(), M, H, &t.d, csr.rp(), csr.co(), csr.vals.data_ptr(), stream());
-    return hyc_ref_outlier_fill_slab(x->data_ptr(), M, H, &t.d, n, (const uint32_t*)slab.data_ptr(), slab_cap, csr.rp(), csr.co(), csr.vals.data_ptr(),
-                                     stream());
+    if (rc != 0) return -1;
+    if (general) {
+      if (!csr.offsets(counts, M, cap)) return -1;
+      return hyc_ref_outlier_fill(x->data_ptr(), M, H, &t.d, csr.rp(), csr.co(), csr.vals.data_ptr(), stream());
+    }
+    csr.alloc(counts, M, cap);
+    return hyc_ref_outlier_csr_slab(x->data_ptr(), M, H, &t.d, n, (const uint32_t*)slab.data_ptr(), slab_cap, cap, csr.rp(), csr.all(), csr.co(),
+                                    csr.vals.data_ptr(), stream());
   }));
   return wrap_all({y, mean, rstd, stored, csr.row_ptr, csr.cols, csr.vals, csr.total});
   END_HANDLE_TH_ERRORS
@@ -555,8 +564,9 @@ PyObject* softmax_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     int32_t* n = (int32_t*)counts.data_ptr();
     uint32_t* sl = (uint32_t*)slab.data_ptr();
     const int rc = hyc_softmax_fwd_slab(x->data_ptr(), M, N, 0, (float)thr, y.data_ptr(), n, sl, slab_cap, stream());
-    if (rc != 0 || !csr.offsets(counts, M, cap)) return -1;
-    return hyc_softmax_fill_slab(y.data_ptr(), M, N, (float)thr, n, sl, slab_cap, csr.rp(), csr.co(), csr.vals.data_ptr(), stream());
+    if (rc != 0) return -1;
+    csr.alloc(counts, M, cap);
+    return hyc_softmax_csr_slab(y.data_ptr(), M, N, (float)thr, n, sl, slab_cap, cap, csr.rp(), csr.all(), csr.co(), csr.vals.data_ptr(), stream());
   }));
   return wrap_all({y, csr.row_ptr, csr.cols, csr.vals, csr.total});
   END_HANDLE_TH_ERRORS

@@ -340,16 +340,24 @@ k_csr_offsets_multi(const int32_t* __restrict__ counts, int64_t rows, int64_t ca
 
 // The kept entries from the forward's slab, one wave per row: a copy of a few words.  A row that kept more than the slab
 // holds is read again, as k_softmax_fill does (without a y it is left to the caller).
+// OFFSETS: row_ptr is made here (csr_rows4), otherwise read.
+template <bool OFFSETS>
 __global__ void __launch_bounds__(256)
 k_softmax_fill_slab(const uint16_t* __restrict__ y, int64_t rows, int64_t N, float thr, const int32_t* __restrict__ counts,
-                    const uint32_t* __restrict__ slab, int cap, const int32_t* __restrict__ row_ptr, int32_t* __restrict__ cols,
-                    uint16_t* __restrict__ vals) {
+                    const uint32_t* __restrict__ slab, int cap, int32_t* __restrict__ row_ptr, int64_t capacity, int64_t* __restrict__ total,
+                    int32_t* __restrict__ cols, uint16_t* __restrict__ vals) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  RowRoom room;
+  if constexpr (OFFSETS) room = csr_rows4(counts, rows, capacity, row_ptr, total);
   if (row >= rows) return;
-  const int n = counts[row];
-  const int64_t base = row_ptr[row];
-  const int limit = row_ptr[row + 1] - (int)base;           // the row's room in cols / vals
+  if constexpr (!OFFSETS) {
+    room.base = row_ptr[row];
+    room.limit = row_ptr[row + 1] - (int)room.base;
+    room.n = counts[row];
+  }
+  const int64_t base = room.base;
+  const int limit = room.limit, n = room.n;                 // the row's room in cols / vals
   if (n <= cap) {
     const int m = n < limit ? n : limit;
     for (int e = lane; e < m; e += 64) {
@@ -516,8 +524,9 @@ k_softmax_rows(const uint16_t* g, int64_t rows, int64_t N, const int32_t* __rest
 
 void launch_slab_copy(int64_t rows, const int32_t* counts, const uint32_t* slab, int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals,
                       hipStream_t stream) {
-  hipLaunchKernelGGL(k_softmax_fill_slab, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, static_cast<const uint16_t*>(nullptr), rows,
-                     (int64_t)0, 0.f, counts, slab, (int)cap, row_ptr, cols, static_cast<uint16_t*>(vals));
+  hipLaunchKernelGGL(k_softmax_fill_slab<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, static_cast<const uint16_t*>(nullptr),
+                     rows, (int64_t)0, 0.f, counts, slab, (int)cap, const_cast<int32_t*>(row_ptr), (int64_t)0, static_cast<int64_t*>(nullptr), cols,
+                     static_cast<uint16_t*>(vals));
 }
 
 static int softmax_shape(const char* who, int64_t rows, int64_t N) {
@@ -628,10 +637,28 @@ int hyc_softmax_fill_slab(const void* y, int64_t rows, int64_t N, float threshol
   if (rows == 0) return HYC_OK;
   if (!y || !counts || !slab || !row_ptr) return fail(HYC_EFAULT, "hyc_softmax_fill_slab: null buffer");
   if (!aligned16(y)) return fail(HYC_EINVAL, "hyc_softmax_fill_slab: y must be 16-byte aligned");
-  hipLaunchKernelGGL(k_softmax_fill_slab, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, begin_launch(stream),
-                     static_cast<const uint16_t*>(y), rows, N, round_to_bf16(threshold), counts, slab, (int)cap, row_ptr, cols,
-                     static_cast<uint16_t*>(vals));
+  hipLaunchKernelGGL(k_softmax_fill_slab<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, begin_launch(stream),
+                     static_cast<const uint16_t*>(y), rows, N, round_to_bf16(threshold), counts, slab, (int)cap, const_cast<int32_t*>(row_ptr),
+                     (int64_t)0, static_cast<int64_t*>(nullptr), cols, static_cast<uint16_t*>(vals));
   return check_launch("hyc_softmax_fill_slab");
+}
+
+int hyc_softmax_csr_slab(const void* y, int64_t rows, int64_t N, float threshold, const int32_t* counts, const uint32_t* slab, int64_t cap,
+                         int64_t capacity, int32_t* row_ptr, int64_t* total, int32_t* cols, void* vals, void* stream) {
+  if (rows <= 0 || rows > SLAB_OFFSETS_MAX || !aligned16(counts)) {
+    const int rc = hyc_csr_offsets(counts, rows, capacity, row_ptr, total, stream);
+    return rc ? rc : hyc_softmax_fill_slab(y, rows, N, threshold, counts, slab, cap, row_ptr, cols, vals, stream);
+  }
+  int rc = softmax_shape("hyc_softmax_csr_slab", rows, N);
+  if (rc) return rc;
+  if (cap <= 0 || cap > N) return fail(HYC_EINVAL, "hyc_softmax_csr_slab: cap=%lld must be in 1..N=%lld", (long long)cap, (long long)N);
+  if (!y || !counts || !slab || !row_ptr) return fail(HYC_EFAULT, "hyc_softmax_csr_slab: null buffer");
+  if (!aligned16(y)) return fail(HYC_EINVAL, "hyc_softmax_csr_slab: y must be 16-byte aligned");
+  if (capacity < 0 || capacity > 0x7FFFFFFFll) capacity = 0x7FFFFFFFll;          // row_ptr is int32
+  hipLaunchKernelGGL(k_softmax_fill_slab<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, begin_launch(stream),
+                     static_cast<const uint16_t*>(y), rows, N, round_to_bf16(threshold), counts, slab, (int)cap, row_ptr, capacity, total, cols,
+                     static_cast<uint16_t*>(vals));
+  return check_launch("hyc_softmax_csr_slab");
 }
 
 int hyc_csr_offsets(const int32_t* counts, int64_t rows, int64_t capacity, int32_t* row_ptr, int64_t* total, void* stream) {

@@ -174,6 +174,9 @@ int hyc_threshold_fwd(int32_t norm, const void* x, const void* w, const void* bi
                       void* stream);
 int hyc_ref_outlier_fill_slab(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* counts, const uint32_t* slab,
                               int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals, void* stream);
+/* hyc_csr_offsets (row_ptr and *total are written) and hyc_ref_outlier_fill_slab, in one launch over few rows */
+int hyc_ref_outlier_csr_slab(const void* x, int64_t M, int64_t H, const hyc_desc* d, const int32_t* counts, const uint32_t* slab, int64_t cap,
+                             int64_t capacity, int32_t* row_ptr, int64_t* total, int32_t* cols, void* vals, void* stream);
 
 /* ---- RMSNorm ----------------------------------------------------------------------------------- */
 /* y = bf16((x*rstd)*w), rstd = 1/sqrt(mean(x^2)+eps) [M] fp32, and x compressed as hyc_compress does. */
@@ -300,6 +303,9 @@ int hyc_softmax_fill_slab(const void* y, int64_t rows, int64_t N, float threshol
  * what lets a calibrated caller size cols / vals ahead of time (e.g. 1.25 x the kept fraction it measured) instead of
  * reading the total back before it allocates, as the reference's to_sparse() does (compress_function.py:153, :269). */
 int hyc_csr_offsets(const int32_t* counts, int64_t rows, int64_t capacity, int32_t* row_ptr, int64_t* total, void* stream);
+/* hyc_csr_offsets and hyc_softmax_fill_slab, in one launch over few rows */
+int hyc_softmax_csr_slab(const void* y, int64_t rows, int64_t N, float threshold, const int32_t* counts, const uint32_t* slab, int64_t cap,
+                         int64_t capacity, int32_t* row_ptr, int64_t* total, int32_t* cols, void* vals, void* stream);
 /* the kept probabilities as CSR: row_ptr int32 [rows+1] (exclusive prefix sums of counts, or hyc_csr_offsets), cols
  * ascending per row; row r receives its first row_ptr[r+1] - row_ptr[r] kept entries */
 int hyc_softmax_fill(const void* y, int64_t rows, int64_t N, float threshold, const int32_t* row_ptr, int32_t* cols,
