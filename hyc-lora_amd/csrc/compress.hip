@@ -63,16 +63,16 @@ k_decompress_chan(const uint8_t* __restrict__ stored, const uint16_t* __restrict
   }
 }
 
-// Fast paths: every lane owns exactly one chunk per segment (CPS == blockDim.x), the group width is a template
+// Fast paths: every lane owns exactly one chunk per segment (long rows: row_parts), the group width is a template
 // parameter, plan words are loaded once, pointers advance by a constant and the next row is requested before the
 // current one is processed.
 template <int BITS, int LPGT, int MAXT, int RULE>
 __global__ void __launch_bounds__(MAXT)
-k_compress_chan_fast(const uint16_t* __restrict__ x, int64_t M, int64_t H /* row pitch of x */, int CPS, ChanArgs a,
+k_compress_chan_fast(const uint16_t* __restrict__ x, int64_t M, int64_t H /* row pitch of x */, int CPS, int cps_wg, ChanArgs a,
                      uint8_t* __restrict__ stored, uint16_t* __restrict__ vals, uint16_t* __restrict__ scales) {
   constexpr int NSEG = Q<BITS>::NSEG;
-  const int c = threadIdx.x;
-  if (c >= CPS) return;                                 // tail of the last wave; scale groups never straddle it
+  const int c = (int)blockIdx.y * cps_wg + (int)threadIdx.x;   // (gridDim.y workgroups of cps_wg chunks share a long row)
+  if ((int)threadIdx.x >= cps_wg || c >= CPS) return;   // tail of the last wave; scale groups never straddle it
   const int64_t SEG = (int64_t)CPS * 8;
   const bool leader = (c & (LPGT - 1)) == 0;
   const int seg_groups = CPS >> a.chunk_to_group_shift;
@@ -137,11 +137,11 @@ k_compress_chan_fast(const uint16_t* __restrict__ x, int64_t M, int64_t H /* row
 template <int BITS, int MAXT>
 __global__ void __launch_bounds__(MAXT)
 k_decompress_chan_fast(const uint8_t* __restrict__ stored, const uint16_t* __restrict__ vals,
-                       const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, ChanArgs a,
+                       const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, int cps_wg, ChanArgs a,
                        uint16_t* __restrict__ xhat) {
   constexpr int NSEG = Q<BITS>::NSEG;
-  const int c = threadIdx.x;
-  if (c >= CPS) return;
+  const int c = (int)blockIdx.y * cps_wg + (int)threadIdx.x;   // (gridDim.y workgroups of cps_wg chunks share a long row)
+  if ((int)threadIdx.x >= cps_wg || c >= CPS) return;
   const int64_t SEG = (int64_t)CPS * 8;
   const int seg_groups = CPS >> a.chunk_to_group_shift;
   uint32_t plan[NSEG];
@@ -397,6 +397,19 @@ static int long_input_grid(int64_t M, int dflt) {
   return g > dflt ? (int)g : dflt;
 }
 
+// Rows of more than 1024 chunks per segment (more than 8192 channels of 8-bit codes, 16384 of 4-bit) are shared by workgroups of at most 768
+// chunks, a whole number of `unit` each: nothing in the fast kernels looks beyond a scale group.  The kernels that walk such a row in turns
+// wait for every load before the next one is asked for; shared, 8-bit codes in groups of 128 went (compress | decompress, us)
+//   300 x 11008 5.4 -> 4.7 | 4.9 -> 4.7, 4096 x 11008 29.1 -> 23.9 | 40.2 -> 21.5, 9000 x 11008 73.2 -> 49.7 | 80.3 -> 45.2,
+//   4096 x 13824 31.4 -> 30.5 | 42.4 -> 26.8, 2048 x 65536 83.6 -> 80.9 | 78.5 -> 59.0; no size was slower.
+// What still takes the kernels with turns: 1-bit codes, and compressing in groups of other widths than 64 and 128.
+struct RowParts { int parts, cps_wg, threads; };
+static RowParts row_parts(const RowGeom& g, int unit) {
+  if (g.iters == 1) return {1, g.cps, g.threads};
+  const int parts = (g.cps + 767) / 768, cps_wg = ((g.cps + unit - 1) / unit + parts - 1) / parts * unit;
+  return {parts, cps_wg, (cps_wg + 63) / 64 * 64};
+}
+
 #define HYC_DISPATCH_BITS(BITS_, ...)            \
   switch (BITS_) {                               \
     case 1: { constexpr int B = 1; __VA_ARGS__; } break; \
@@ -432,19 +445,18 @@ int hyc_compress_rows(const void* x, int64_t ldx, int64_t M, int64_t H, const hy
     if (M == 0) return HYC_OK;
     if (!x || !stored || !scales || (d->k > 0 && !vals)) return fail(HYC_EFAULT, "hyc_compress: null buffer");
     if (!aligned16(x) || !aligned8(stored)) return fail(HYC_EINVAL, "hyc_compress: x must be 16-byte and stored 8-byte aligned");
-    const int grid = row_grid(M, g.threads);
-    if (g.iters == 1 && (lpg == 8 || lpg == 16) && d->bits != 1) {
+    if ((lpg == 8 || lpg == 16) && d->bits != 1) {
+      const RowParts p = row_parts(g, lpg);
+      const dim3 grid((unsigned)long_input_grid(M, row_grid(M, p.threads)), (unsigned)p.parts);
 #define HYC_CF_R(B_, L_, R_)                                                                                       \
   do {                                                                                                             \
-    if (g.threads <= 256)                                                                                          \
-      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 256, R_>),                                                  \
-                         dim3(long_input_grid(M, grid)), dim3(g.threads), 0, st, \
-                         static_cast<const uint16_t*>(x), M, ldx, g.cps, a, static_cast<uint8_t*>(stored),               \
+    if (p.threads <= 256)                                                                                          \
+      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 256, R_>), grid, dim3(p.threads), 0, st,                    \
+                         static_cast<const uint16_t*>(x), M, ldx, g.cps, p.cps_wg, a, static_cast<uint8_t*>(stored), \
                          static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                            \
     else                                                                                                           \
-      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 1024, R_>),                                                 \
-                         dim3(long_input_grid(M, grid)), dim3(g.threads), 0, st, \
-                         static_cast<const uint16_t*>(x), M, ldx, g.cps, a, static_cast<uint8_t*>(stored),               \
+      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 1024, R_>), grid, dim3(p.threads), 0, st,                   \
+                         static_cast<const uint16_t*>(x), M, ldx, g.cps, p.cps_wg, a, static_cast<uint8_t*>(stored), \
                          static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                            \
   } while (0)
 #define HYC_CF(B_, L_)                                           \
@@ -465,7 +477,7 @@ int hyc_compress_rows(const void* x, int64_t ldx, int64_t M, int64_t H, const hy
       return check_launch("hyc_compress");
     }
     HYC_DISPATCH_BITS(d->bits,
-      hipLaunchKernelGGL((k_compress_chan<B>), dim3(grid), dim3(g.threads), 0, st,
+      hipLaunchKernelGGL((k_compress_chan<B>), dim3(row_grid(M, g.threads)), dim3(g.threads), 0, st,
                          static_cast<const uint16_t*>(x), M, ldx, g.cps, g.iters, lpg, a, static_cast<uint8_t*>(stored),
                          static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales)));
     return check_launch("hyc_compress");
@@ -503,20 +515,19 @@ int hyc_decompress(const void* stored, const void* vals, const void* scales, int
     if (M == 0) return HYC_OK;
     if (!stored || !xhat || !scales || (d->k > 0 && !vals)) return fail(HYC_EFAULT, "hyc_decompress: null buffer");
     if (!aligned16(xhat) || !aligned8(stored)) return fail(HYC_EINVAL, "hyc_decompress: xhat must be 16-byte and stored 8-byte aligned");
-    const int grid = row_grid(M, g.threads);
-    if (g.iters == 1 && d->bits != 1) {
+    if (d->bits != 1) {
+      const RowParts p = row_parts(g, 64);
+      const dim3 grid((unsigned)long_input_grid(M, row_grid(M, p.threads)), (unsigned)p.parts);
 #define HYC_DF(B_)                                                                                                 \
   do {                                                                                                             \
-    if (g.threads <= 256)                                                                                          \
-      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 256>),                                                        \
-                         dim3(long_input_grid(M, grid)), dim3(g.threads), 0, st, \
+    if (p.threads <= 256)                                                                                          \
+      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 256>), grid, dim3(p.threads), 0, st,                          \
                          static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                  \
-                         static_cast<const uint16_t*>(scales), M, H, g.cps, a, static_cast<uint16_t*>(xhat));         \
+                         static_cast<const uint16_t*>(scales), M, H, g.cps, p.cps_wg, a, static_cast<uint16_t*>(xhat)); \
     else                                                                                                           \
-      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 1024>),                                                       \
-                         dim3(long_input_grid(M, grid)), dim3(g.threads), 0, st, \
+      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 1024>), grid, dim3(p.threads), 0, st,                         \
                          static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                  \
-                         static_cast<const uint16_t*>(scales), M, H, g.cps, a, static_cast<uint16_t*>(xhat));         \
+                         static_cast<const uint16_t*>(scales), M, H, g.cps, p.cps_wg, a, static_cast<uint16_t*>(xhat)); \
   } while (0)
       if (d->bits == 2) HYC_DF(2);
       else if (d->bits == 4) HYC_DF(4);
@@ -525,7 +536,7 @@ int hyc_decompress(const void* stored, const void* vals, const void* scales, int
       return check_launch("hyc_decompress");
     }
     HYC_DISPATCH_BITS(d->bits,
-      hipLaunchKernelGGL((k_decompress_chan<B>), dim3(grid), dim3(g.threads), 0, st,
+      hipLaunchKernelGGL((k_decompress_chan<B>), dim3(row_grid(M, g.threads)), dim3(g.threads), 0, st,
                          static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),
                          static_cast<const uint16_t*>(scales), M, H, g.cps, g.iters, a, static_cast<uint16_t*>(xhat)));
     return check_launch("hyc_decompress");
