@@ -190,11 +190,11 @@ __device__ __forceinline__ bool lut_grad8(const uint16_t* lut, const uint4& xr, 
   return true;
 }
 
-// fast path: channel source, every lane owns one chunk per segment, next row requested ahead
+// fast path: channel source, every lane owns one chunk per segment (long rows: row_parts), next row requested ahead
 template <int BITS, int ACT, int MAXT>
 __global__ void __launch_bounds__(MAXT)
 k_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__ stored, const uint16_t* __restrict__ vals,
-               const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, ChanArgs ca,
+               const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, int cps_wg, ChanArgs ca,
                uint16_t* __restrict__ dx, int use_lut) {
   constexpr int NSEG = Q<BITS>::NSEG;
   constexpr bool HAS_LUT = ACT == HYC_ACT_SILU || ACT == HYC_ACT_GELU_TANH;
@@ -203,8 +203,8 @@ k_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__ store
     lut_fill<ACT>(lut);
     __syncthreads();
   }
-  const int c = threadIdx.x;
-  if (c >= CPS) return;                                 // tail of the last wave
+  const int c = (int)blockIdx.y * cps_wg + (int)threadIdx.x;   // (gridDim.y workgroups of cps_wg chunks share a long row)
+  if ((int)threadIdx.x >= cps_wg || c >= CPS) return;   // tail of the last wave
   const int64_t SEG = (int64_t)CPS * 8;
   const int seg_groups = CPS >> ca.chunk_to_group_shift;
   uint32_t plan[NSEG];
@@ -843,6 +843,14 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
   // 17.6 -> 15.2 us, and 232 -> 221 us at 65 536 rows; H = 5120, 320 threads, 2048 -> 768: 36.0 -> 21.2 / 24.6 -> 18.6 us)
   // Rows of eight waves or more (one workgroup per CU at a time): about eight rows per workgroup, in whole rounds of the
   // 256 CUs (2048 x 11008: GELU 24.5 -> 20.5 us, 4096 rows: 38.9 -> 37.5, 16 384 rows: SiLU 160.7 -> 152.3).
+  // Rows that two or more workgroups share (more than 1024 chunks, row_parts) fill a table in each: one workgroup a CU below 768 rows, then
+  // by rows again, at most four a CU and part.  Against the kernel that walks such rows in turns (SiLU | GELU, us): 100 x 13824 6.7 -> 5.1 |
+  // 7.8 -> 6.5, 300 x 11008 8.1 -> 6.6 | 11.1 -> 8.0, 1000 x 13824 18.8 -> 13.1 | 24.2 -> 15.3, 4096 x 13824 57.1 -> 47.1 | 64.1 -> 49.9,
+  // 9000 x 11008 146 -> 88 | 157 -> 84; no size was slower.
+  if (ACT != ACT_MUL && geo.iters > 1 && d->mode == HYC_MODE_CHANNEL && d->bits != 1) {
+    const int64_t by_rows = (M / 8 / 256) * 256, fewer = M < 768 ? 128 : by_rows < 256 ? 256 : by_rows > 1024 ? 1024 : by_rows;
+    grid = (int)(M < fewer ? M : fewer);
+  }
   if (ACT != ACT_MUL && geo.iters == 1) {
     int fewer = geo.threads <= 128 ? 1024 : geo.threads <= 256 ? 512 : 768;
     if (geo.threads >= 512) {
@@ -853,19 +861,21 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
     if (grid > fewer) grid = fewer;
   }
   hipStream_t st = begin_launch(stream);
-  const int use_lut = lut_pays(M, grid, geo.threads * geo.iters, LUT_PAYS_BWD);
-  if (d->mode == HYC_MODE_CHANNEL && geo.iters == 1 && d->bits != 1) {
+  if (d->mode == HYC_MODE_CHANNEL && d->bits != 1) {
+    const RowParts p = row_parts(geo, 64);
+    const dim3 wgs((unsigned)grid, (unsigned)p.parts);
+    const int use_lut = lut_pays(M, grid, p.threads, LUT_PAYS_BWD);
 #define HYC_ACT_FAST(B_)                                                                                       \
   do {                                                                                                         \
-    if (geo.threads <= 256)                                                                                    \
-      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 256>), dim3(grid), dim3(geo.threads), 0, st,                 \
+    if (p.threads <= 256)                                                                                    \
+      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 256>), wgs, dim3(p.threads), 0, st,                 \
                          static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                 \
-                         static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, ca, \
+                         static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, p.cps_wg, ca, \
                          static_cast<uint16_t*>(dx), use_lut);                                                 \
     else                                                                                                       \
-      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 1024>), dim3(grid), dim3(geo.threads), 0, st,                \
+      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 1024>), wgs, dim3(p.threads), 0, st,                \
                          static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                 \
-                         static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, ca, \
+                         static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, p.cps_wg, ca, \
                          static_cast<uint16_t*>(dx), use_lut);                                                 \
   } while (0)
     if (d->bits == 2) HYC_ACT_FAST(2);
@@ -874,6 +884,7 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
 #undef HYC_ACT_FAST
     return check_launch(who);
   }
+  const int use_lut = lut_pays(M, grid, geo.threads * geo.iters, LUT_PAYS_BWD);
 #define HYC_ACT_LAUNCH(B_, S_)                                                                            \
   hipLaunchKernelGGL((k_act_bwd<B_, S_, ACT>), dim3(grid), dim3(geo.threads), 0, st,                      \
                      static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                \

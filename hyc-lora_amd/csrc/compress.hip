@@ -397,19 +397,11 @@ static int long_input_grid(int64_t M, int dflt) {
   return g > dflt ? (int)g : dflt;
 }
 
-// Rows of more than 1024 chunks per segment (more than 8192 channels of 8-bit codes, 16384 of 4-bit) are shared by workgroups of at most 768
-// chunks, a whole number of `unit` each: nothing in the fast kernels looks beyond a scale group.  The kernels that walk such a row in turns
+// Long rows are shared by workgroups (row_parts): nothing in the fast kernels looks beyond a scale group.  The kernels that walk such a row in turns
 // wait for every load before the next one is asked for; shared, 8-bit codes in groups of 128 went (compress | decompress, us)
-//   300 x 11008 5.4 -> 4.7 | 4.9 -> 4.7, 4096 x 11008 29.1 -> 23.9 | 40.2 -> 21.5, 9000 x 11008 73.2 -> 49.7 | 80.3 -> 45.2,
-//   4096 x 13824 31.4 -> 30.5 | 42.4 -> 26.8, 2048 x 65536 83.6 -> 80.9 | 78.5 -> 59.0; no size was slower.
+//   500 x 13824 6.5 -> 5.5 | 5.8 -> 5.4, 4096 x 11008 29.1 -> 23.9 | 40.2 -> 21.5, 9000 x 11008 73.2 -> 49.7 | 80.3 -> 45.2,
+//   4096 x 13824 31.1 -> 29.8 | 41.9 -> 27.4, 4096 x 65536 188.8 -> 176.1 | 284.4 -> 175.2; no size was slower.
 // What still takes the kernels with turns: 1-bit codes, and compressing in groups of other widths than 64 and 128.
-struct RowParts { int parts, cps_wg, threads; };
-static RowParts row_parts(const RowGeom& g, int unit) {
-  if (g.iters == 1) return {1, g.cps, g.threads};
-  const int parts = (g.cps + 767) / 768, cps_wg = ((g.cps + unit - 1) / unit + parts - 1) / parts * unit;
-  return {parts, cps_wg, (cps_wg + 63) / 64 * 64};
-}
-
 #define HYC_DISPATCH_BITS(BITS_, ...)            \
   switch (BITS_) {                               \
     case 1: { constexpr int B = 1; __VA_ARGS__; } break; \
