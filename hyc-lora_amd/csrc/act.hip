@@ -190,8 +190,9 @@ __device__ __forceinline__ bool lut_grad8(const uint16_t* lut, const uint4& xr, 
   return true;
 }
 
-// fast path: channel source, every lane owns one chunk per segment (long rows: row_parts), next row requested ahead
-template <int BITS, int ACT, int MAXT>
+// fast path: channel source, every lane owns one chunk per segment (SHARED: of a long row's
+// blockIdx.y-th part, row_parts), next row requested ahead
+template <int BITS, int ACT, int MAXT, bool SHARED>
 __global__ void __launch_bounds__(MAXT)
 k_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__ stored, const uint16_t* __restrict__ vals,
                const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, int cps_wg, ChanArgs ca,
@@ -203,8 +204,8 @@ k_act_bwd_fast(const uint16_t* __restrict__ g, const uint8_t* __restrict__ store
     lut_fill<ACT>(lut);
     __syncthreads();
   }
-  const int c = (int)blockIdx.y * cps_wg + (int)threadIdx.x;   // (gridDim.y workgroups of cps_wg chunks share a long row)
-  if ((int)threadIdx.x >= cps_wg || c >= CPS) return;   // tail of the last wave
+  const int c = (SHARED ? (int)blockIdx.y * cps_wg : 0) + (int)threadIdx.x;
+  if ((SHARED && (int)threadIdx.x >= cps_wg) || c >= CPS) return;   // tail of the last wave
   const int64_t SEG = (int64_t)CPS * 8;
   const int seg_groups = CPS >> ca.chunk_to_group_shift;
   uint32_t plan[NSEG];
@@ -865,18 +866,23 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
     const RowParts p = row_parts(geo, 64);
     const dim3 wgs((unsigned)grid, (unsigned)p.parts);
     const int use_lut = lut_pays(M, grid, p.threads, LUT_PAYS_BWD);
-#define HYC_ACT_FAST(B_)                                                                                       \
-  do {                                                                                                         \
-    if (p.threads <= 256)                                                                                    \
-      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 256>), wgs, dim3(p.threads), 0, st,                 \
-                         static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                 \
+#define HYC_ACT_FAST(B_)                                                                                                        \
+  do {                                                                                                                          \
+    if (p.parts > 1)                                                                                                            \
+      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 1024, true>), wgs, dim3(p.threads), 0, st,                                    \
+                         static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                                  \
                          static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, p.cps_wg, ca, \
-                         static_cast<uint16_t*>(dx), use_lut);                                                 \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 1024>), wgs, dim3(p.threads), 0, st,                \
-                         static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                 \
+                         static_cast<uint16_t*>(dx), use_lut);                                                                  \
+    else if (p.threads <= 256)                                                                                                  \
+      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 256, false>), wgs, dim3(p.threads), 0, st,                                    \
+                         static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                                  \
                          static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, p.cps_wg, ca, \
-                         static_cast<uint16_t*>(dx), use_lut);                                                 \
+                         static_cast<uint16_t*>(dx), use_lut);                                                                  \
+    else                                                                                                                        \
+      hipLaunchKernelGGL((k_act_bwd_fast<B_, ACT, 1024, false>), wgs, dim3(p.threads), 0, st,                                   \
+                         static_cast<const uint16_t*>(g), static_cast<const uint8_t*>(stored),                                  \
+                         static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, p.cps_wg, ca, \
+                         static_cast<uint16_t*>(dx), use_lut);                                                                  \
   } while (0)
     if (d->bits == 2) HYC_ACT_FAST(2);
     else if (d->bits == 4) HYC_ACT_FAST(4);

@@ -1,5 +1,6 @@
 // Standalone compress / decompress of a [M, H] bf16 activation, and the element-threshold outliers as CSR.
 // One workgroup walks rows (grid-stride); within a row the chunk mapping of row_codec.hpp applies.
+#include <type_traits>
 #include <stdlib.h>
 
 #include "abi_util.hpp"
@@ -63,16 +64,16 @@ k_decompress_chan(const uint8_t* __restrict__ stored, const uint16_t* __restrict
   }
 }
 
-// Fast paths: every lane owns exactly one chunk per segment (long rows: row_parts), the group width is a template
+// Fast paths: every lane owns exactly one chunk per segment (SHARED: of a long row's blockIdx.y-th part, row_parts), the group width is a template
 // parameter, plan words are loaded once, pointers advance by a constant and the next row is requested before the
 // current one is processed.
-template <int BITS, int LPGT, int MAXT, int RULE>
+template <int BITS, int LPGT, int MAXT, int RULE, bool SHARED>
 __global__ void __launch_bounds__(MAXT)
 k_compress_chan_fast(const uint16_t* __restrict__ x, int64_t M, int64_t H /* row pitch of x */, int CPS, int cps_wg, ChanArgs a,
                      uint8_t* __restrict__ stored, uint16_t* __restrict__ vals, uint16_t* __restrict__ scales) {
   constexpr int NSEG = Q<BITS>::NSEG;
-  const int c = (int)blockIdx.y * cps_wg + (int)threadIdx.x;   // (gridDim.y workgroups of cps_wg chunks share a long row)
-  if ((int)threadIdx.x >= cps_wg || c >= CPS) return;   // tail of the last wave; scale groups never straddle it
+  const int c = (SHARED ? (int)blockIdx.y * cps_wg : 0) + (int)threadIdx.x;
+  if ((SHARED && (int)threadIdx.x >= cps_wg) || c >= CPS) return;   // tail of the last wave; scale groups never straddle it
   const int64_t SEG = (int64_t)CPS * 8;
   const bool leader = (c & (LPGT - 1)) == 0;
   const int seg_groups = CPS >> a.chunk_to_group_shift;
@@ -134,14 +135,14 @@ k_compress_chan_fast(const uint16_t* __restrict__ x, int64_t M, int64_t H /* row
   }
 }
 
-template <int BITS, int MAXT>
+template <int BITS, int MAXT, bool SHARED>
 __global__ void __launch_bounds__(MAXT)
 k_decompress_chan_fast(const uint8_t* __restrict__ stored, const uint16_t* __restrict__ vals,
                        const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, int cps_wg, ChanArgs a,
                        uint16_t* __restrict__ xhat) {
   constexpr int NSEG = Q<BITS>::NSEG;
-  const int c = (int)blockIdx.y * cps_wg + (int)threadIdx.x;   // (gridDim.y workgroups of cps_wg chunks share a long row)
-  if ((int)threadIdx.x >= cps_wg || c >= CPS) return;
+  const int c = (SHARED ? (int)blockIdx.y * cps_wg : 0) + (int)threadIdx.x;
+  if ((SHARED && (int)threadIdx.x >= cps_wg) || c >= CPS) return;
   const int64_t SEG = (int64_t)CPS * 8;
   const int seg_groups = CPS >> a.chunk_to_group_shift;
   uint32_t plan[NSEG];
@@ -322,9 +323,9 @@ k_outlier_count(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a,
 // OFFSETS: row_ptr is made here (csr_rows4), otherwise read.
 template <bool OFFSETS>
 __global__ void __launch_bounds__(256)
-k_outlier_fill(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a, int32_t* __restrict__ row_ptr,
-               int32_t* __restrict__ cols, uint16_t* __restrict__ vals, const int32_t* __restrict__ counts,
-               const uint32_t* __restrict__ slab, int cap, int64_t capacity, int64_t* __restrict__ total) {
+k_outlier_fill(const uint16_t* __restrict__ x, int64_t M, int64_t H, ThrArgs a,
+               std::conditional_t<OFFSETS, int32_t*, const int32_t*> __restrict__ row_ptr, int32_t* __restrict__ cols,
+               uint16_t* __restrict__ vals, const int32_t* __restrict__ counts, const uint32_t* __restrict__ slab, int cap, int64_t capacity, int64_t* __restrict__ total) {
   __shared__ uint32_t stage_all[4][STAGE_CAP];
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -440,16 +441,20 @@ int hyc_compress_rows(const void* x, int64_t ldx, int64_t M, int64_t H, const hy
     if ((lpg == 8 || lpg == 16) && d->bits != 1) {
       const RowParts p = row_parts(g, lpg);
       const dim3 grid((unsigned)long_input_grid(M, row_grid(M, p.threads)), (unsigned)p.parts);
-#define HYC_CF_R(B_, L_, R_)                                                                                       \
-  do {                                                                                                             \
-    if (p.threads <= 256)                                                                                          \
-      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 256, R_>), grid, dim3(p.threads), 0, st,                    \
+#define HYC_CF_R(B_, L_, R_)                                                                                         \
+  do {                                                                                                               \
+    if (p.parts > 1)                                                                                                 \
+      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 1024, R_, true>), grid, dim3(p.threads), 0, st,               \
                          static_cast<const uint16_t*>(x), M, ldx, g.cps, p.cps_wg, a, static_cast<uint8_t*>(stored), \
-                         static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                            \
-    else                                                                                                           \
-      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 1024, R_>), grid, dim3(p.threads), 0, st,                   \
+                         static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                              \
+    else if (p.threads <= 256)                                                                                       \
+      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 256, R_, false>), grid, dim3(p.threads), 0, st,               \
                          static_cast<const uint16_t*>(x), M, ldx, g.cps, p.cps_wg, a, static_cast<uint8_t*>(stored), \
-                         static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                            \
+                         static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                              \
+    else                                                                                                             \
+      hipLaunchKernelGGL((k_compress_chan_fast<B_, L_, 1024, R_, false>), grid, dim3(p.threads), 0, st,              \
+                         static_cast<const uint16_t*>(x), M, ldx, g.cps, p.cps_wg, a, static_cast<uint8_t*>(stored), \
+                         static_cast<uint16_t*>(vals), static_cast<uint16_t*>(scales));                              \
   } while (0)
 #define HYC_CF(B_, L_)                                           \
   do {                                                           \
@@ -510,15 +515,19 @@ int hyc_decompress(const void* stored, const void* vals, const void* scales, int
     if (d->bits != 1) {
       const RowParts p = row_parts(g, 64);
       const dim3 grid((unsigned)long_input_grid(M, row_grid(M, p.threads)), (unsigned)p.parts);
-#define HYC_DF(B_)                                                                                                 \
-  do {                                                                                                             \
-    if (p.threads <= 256)                                                                                          \
-      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 256>), grid, dim3(p.threads), 0, st,                          \
-                         static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                  \
+#define HYC_DF(B_)                                                                                                      \
+  do {                                                                                                                  \
+    if (p.parts > 1)                                                                                                    \
+      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 1024, true>), grid, dim3(p.threads), 0, st,                        \
+                         static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                       \
                          static_cast<const uint16_t*>(scales), M, H, g.cps, p.cps_wg, a, static_cast<uint16_t*>(xhat)); \
-    else                                                                                                           \
-      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 1024>), grid, dim3(p.threads), 0, st,                         \
-                         static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                  \
+    else if (p.threads <= 256)                                                                                          \
+      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 256, false>), grid, dim3(p.threads), 0, st,                        \
+                         static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                       \
+                         static_cast<const uint16_t*>(scales), M, H, g.cps, p.cps_wg, a, static_cast<uint16_t*>(xhat)); \
+    else                                                                                                                \
+      hipLaunchKernelGGL((k_decompress_chan_fast<B_, 1024, false>), grid, dim3(p.threads), 0, st,                       \
+                         static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),                       \
                          static_cast<const uint16_t*>(scales), M, H, g.cps, p.cps_wg, a, static_cast<uint16_t*>(xhat)); \
   } while (0)
       if (d->bits == 2) HYC_DF(2);
@@ -588,7 +597,7 @@ static int outlier_fill(const char* who, const void* x, int64_t M, int64_t H, co
   if (!x || !row_ptr) return fail(HYC_EFAULT, "%s: null buffer", who);
   if (!aligned16(x)) return fail(HYC_EINVAL, "%s: x must be 16-byte aligned", who);
   hipLaunchKernelGGL(k_outlier_fill<false>, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, begin_launch(stream),
-                     static_cast<const uint16_t*>(x), M, H, a, const_cast<int32_t*>(row_ptr), cols, static_cast<uint16_t*>(vals), counts, slab, (int)cap,
+                     static_cast<const uint16_t*>(x), M, H, a, row_ptr, cols, static_cast<uint16_t*>(vals), counts, slab, (int)cap,
                      (int64_t)0, static_cast<int64_t*>(nullptr));
   return check_launch(who);
 }

@@ -4,6 +4,7 @@
 //   backward  dx = (g - sum_j g_j*yh_j) * yh, yh = the kept probabilities, zero elsewhere
 //   dense     yh as a dense matrix (what true_decompress_softmax returns)
 // Reference: operators/efficient_softmax.py:10-45, operators/compress_function.py:264-275.
+#include <type_traits>
 #include "abi_util.hpp"
 #include "softmax_slab.hpp"
 #include "wave_scan.hpp"
@@ -344,17 +345,17 @@ k_csr_offsets_multi(const int32_t* __restrict__ counts, int64_t rows, int64_t ca
 template <bool OFFSETS>
 __global__ void __launch_bounds__(256)
 k_softmax_fill_slab(const uint16_t* __restrict__ y, int64_t rows, int64_t N, float thr, const int32_t* __restrict__ counts,
-                    const uint32_t* __restrict__ slab, int cap, int32_t* __restrict__ row_ptr, int64_t capacity, int64_t* __restrict__ total,
-                    int32_t* __restrict__ cols, uint16_t* __restrict__ vals) {
+                    const uint32_t* __restrict__ slab, int cap, std::conditional_t<OFFSETS, int32_t*, const int32_t*> __restrict__ row_ptr,
+                    int64_t capacity, int64_t* __restrict__ total, int32_t* __restrict__ cols, uint16_t* __restrict__ vals) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   RowRoom room;
   if constexpr (OFFSETS) room = csr_rows4(counts, rows, capacity, row_ptr, total);
   if (row >= rows) return;
   if constexpr (!OFFSETS) {
+    room.n = counts[row];
     room.base = row_ptr[row];
     room.limit = row_ptr[row + 1] - (int)room.base;
-    room.n = counts[row];
   }
   const int64_t base = room.base;
   const int limit = room.limit, n = room.n;                 // the row's room in cols / vals
@@ -525,7 +526,7 @@ k_softmax_rows(const uint16_t* g, int64_t rows, int64_t N, const int32_t* __rest
 void launch_slab_copy(int64_t rows, const int32_t* counts, const uint32_t* slab, int64_t cap, const int32_t* row_ptr, int32_t* cols, void* vals,
                       hipStream_t stream) {
   hipLaunchKernelGGL(k_softmax_fill_slab<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, static_cast<const uint16_t*>(nullptr),
-                     rows, (int64_t)0, 0.f, counts, slab, (int)cap, const_cast<int32_t*>(row_ptr), (int64_t)0, static_cast<int64_t*>(nullptr), cols,
+                     rows, (int64_t)0, 0.f, counts, slab, (int)cap, row_ptr, (int64_t)0, static_cast<int64_t*>(nullptr), cols,
                      static_cast<uint16_t*>(vals));
 }
 
@@ -638,7 +639,7 @@ int hyc_softmax_fill_slab(const void* y, int64_t rows, int64_t N, float threshol
   if (!y || !counts || !slab || !row_ptr) return fail(HYC_EFAULT, "hyc_softmax_fill_slab: null buffer");
   if (!aligned16(y)) return fail(HYC_EINVAL, "hyc_softmax_fill_slab: y must be 16-byte aligned");
   hipLaunchKernelGGL(k_softmax_fill_slab<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, begin_launch(stream),
-                     static_cast<const uint16_t*>(y), rows, N, round_to_bf16(threshold), counts, slab, (int)cap, const_cast<int32_t*>(row_ptr),
+                     static_cast<const uint16_t*>(y), rows, N, round_to_bf16(threshold), counts, slab, (int)cap, row_ptr,
                      (int64_t)0, static_cast<int64_t*>(nullptr), cols, static_cast<uint16_t*>(vals));
   return check_launch("hyc_softmax_fill_slab");
 }
