@@ -1013,8 +1013,8 @@ PyObject* lora_backward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
                            copy ? 1 : 0, pB, ws.data_ptr(), stream());
     }
     if (rc) return rc;
-    // the dh of a group go through the weight gradient side by side, up to 128 rows of dA a call
-    const int64_t per_call = (128 / r > 1 ? 128 / r : 1) * r;
+    // the dh of a group go through the weight gradient side by side, in as few calls as leave its sums in one order
+    const int64_t per_call = hyc_gradw_rows_per_call(M, n * r, r, K, &in.d);
     for (int64_t c0 = 0; c0 < n * r; c0 += per_call) {
       const int64_t cols = c0 + per_call <= n * r ? per_call : n * r - c0;
       Tensor block;

@@ -261,12 +261,16 @@ class _LoRAProjectionsFunc(torch.autograd.Function):
     @staticmethod
     def _grad_A(ctx, dh, A):
         """dA_i = dh_i^T @ x_hat: the projections of a group read the same saved activation, so their dh go through the
-        weight-gradient kernel side by side (up to 128 output rows a call, what its form for few of them takes in tiles of 32): one
-        launch, and one that adds up the partial results, for the whole group.  With 32 rows a call and 8-bit codes, two or three
-        calls -> one, us: 48 rows at 157 x 2048 11.4 -> 6.7, 2048 x 4096 19.2 -> 13.9, 4096 x 4096 22.7 -> 15.2, 8192 x 2048
-        23.5 -> 16.3; 64 rows 13.0 -> 6.7, 21.3 -> 15.1, 24.7 -> 15.3, 24.7 -> 16.7; 96 rows 19.4 -> 6.8 to 37.4 -> 19.8"""
+        weight-gradient kernel side by side, up to 128 rows a call where its sums keep the order they have with up to 32
+        (kernels.gradw_rows_per_call; otherwise they lose precision): one launch, and one that adds up the partial results, for the
+        whole group.  Two or three calls of up to 32 rows -> one, us, codes of 2 | 4 | 8 bits | dense:
+        48 rows of 157 x 2048 13.9 -> 6.9 | 13.9 -> 7.0 | 11.6 -> 7.0 | 12.9 -> 9.7, 1000 x 1024 17.7 -> 8.9 | 17.7 -> 8.9 |
+        16.0 -> 8.9 | 14.3 -> 10.6, 157 x 11008 14.1 -> 7.2 | 14.1 -> 7.2 | 11.9 -> 7.2 | 14.7 -> 11.9; 96 rows of 157 x 2048
+        19.4 -> 7.0 | 19.5 -> 7.1 | 19.6 -> 7.1 | 19.8 -> 10.6.  From about 2000 tokens on codes take 32 rows a call (dense sources
+        keep their order, 48 and 96 rows of 4096 x 4096 28.1 -> 27.2 and 45.9 -> 32.3): one call would be faster there too, 48
+        rows of 2048 x 4096 20.1 -> 13.8, 4096 x 4096 23.2 -> 14.6, 4096 x 11008 38.1 -> 26.0 (2 bits)."""
         r, dA = A[0].shape[0], []
-        per_call = max(1, 128 // r) * r
+        per_call = K.gradw_rows_per_call(dh.shape[0], dh.shape[1], r, ctx.saved_x)
         for c0 in range(0, dh.shape[1], per_call):
             block = K.gradw_gemm(dh[:, c0:c0 + per_call], ctx.saved_x, out_dtype=A[0].dtype)
             dA.extend(block[j:j + r] for j in range(0, block.shape[0], r))

@@ -871,6 +871,13 @@ def gradw_gemm(dy2d, src, out_dtype=BF16, alpha=1.0, out=None, beta=0.0, staged=
     return out
 
 
+def gradw_rows_per_call(M, N_out, unit, src):
+    """how many of N_out rows of dW, whole groups of `unit`, gradw_gemm takes at a time without another order of its sums (src as there)"""
+    H = src.H if isinstance(src, ChannelCompressed) else src.shape[-1]
+    d = _source(src, M, H)[3]
+    return int(_abi.load().hyc_gradw_rows_per_call(M, N_out, unit, H, ctypes.byref(d)))
+
+
 # ----------------------------------------------------------------------------------------------------
 # softmax
 # ----------------------------------------------------------------------------------------------------

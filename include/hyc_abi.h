@@ -322,6 +322,9 @@ int hyc_softmax_dense(int64_t rows, int64_t N, const int32_t* row_ptr, const int
  * x_hat dequantised on the fly (channel mode) or read as bf16 (HYC_MODE_DENSE); out [N_out, H] bf16 or fp32.
  * workspace: hyc_gradw_workspace_bytes() bytes of device memory, 16-byte aligned (may be 0 -> NULL). */
 int64_t hyc_gradw_workspace_bytes(int64_t M, int64_t N_out, int64_t H);
+/* N_out rows of out in calls of this many, a whole number of `unit`: up to 128 where every element is then added up in the order that
+ * calls of up to 32 add it up in, else up to 32 */
+int64_t hyc_gradw_rows_per_call(int64_t M, int64_t N_out, int64_t unit, int64_t H, const hyc_desc* d);
 int hyc_gradw_gemm(const void* dy, int64_t ldy, const void* stored, const void* vals, const void* scales, int64_t M,
                    int64_t N_out, int64_t H, const hyc_desc* d, float alpha, float beta, void* out, int32_t out_dtype,
                    void* workspace, void* stream);
