@@ -119,34 +119,40 @@ struct Plan {
     d->chan_idx = k ? (decltype(d->chan_idx))idx.data_ptr() : nullptr;
     d->scale_rule = rule;
   }
+  // what kernels._check_plan asks of a plan, for an activation of n channels on `device`
+  bool usable(int64_t n, c10::Device device) const {
+    return H == n && k >= 0 && dense_gpu(idx) && dense_gpu(plan) && idx.scalar_type() == at::kInt && plan.scalar_type() == at::kInt &&
+           idx.is_contiguous() && plan.is_contiguous() && idx.numel() == k && plan.numel() == H / 8 && idx.device() == device && plan.device() == device;
+  }
 };
-// what kernels._check_plan asks of a plan, for an activation of H channels on `device`
 bool get_plan(PyObject* o, int64_t H, c10::Device device, Plan* p) {
   if ((PyObject*)Py_TYPE(o) != t_plan) return false;
   bool ok = true;
   p->H = attr_i64(o, s_H, &ok);
   p->k = attr_i64(o, s_k, &ok);
-  if (!ok || p->H != H || p->k < 0) return false;
+  if (!ok) return false;
   Ref idx(PyObject_GetAttr(o, s_idx)), plan(PyObject_GetAttr(o, s_plan)), rule(PyObject_GetAttr(o, s_scale_rule));
   if (!idx.p || !plan.p || !rule.p) { PyErr_Clear(); return false; }
   const Tensor *ti = plain(idx.p), *tp = plain(plan.p);
-  if (!ti || !tp || ti->scalar_type() != at::kInt || tp->scalar_type() != at::kInt || !ti->is_contiguous() || !tp->is_contiguous() ||
-      ti->numel() != p->k || tp->numel() != H / 8 || ti->device() != device || tp->device() != device || !PyUnicode_Check(rule.p))
-    return false;
+  if (!ti || !tp || !PyUnicode_Check(rule.p)) return false;
   if (PyUnicode_CompareWithASCIIString(rule.p, "absmax") == 0) p->rule = HYC_SCALE_ABSMAX;
   else if (PyUnicode_CompareWithASCIIString(rule.p, "range") == 0) p->rule = HYC_SCALE_RANGE;
   else return false;
   p->idx = *ti;
   p->plan = *tp;
-  return true;
+  return p->usable(H, device);
 }
 
 // the threshold scheme's descriptor: a static scale read through two strides, a base of rank 0 or more
 struct Threshold {
   hyc_desc d;
+  static bool readable(const Tensor* t) { return t && dense_gpu(*t) && t->scalar_type() == BF16 && t->is_contiguous(); }
   bool init(double threshold, PyObject* scale, int64_t bits, int64_t S, int64_t H, PyObject* L, PyObject* R) {
-    const Tensor* sc = bf16(scale);
-    if (!sc || !sc->is_contiguous()) return false;
+    const Tensor *l = L != Py_None ? bf16(L) : nullptr, *r = L != Py_None ? bf16(R) : nullptr;
+    return (L == Py_None || (l && r)) && init(threshold, bf16(scale), bits, S, H, l, r);
+  }
+  bool init(double threshold, const Tensor* sc, int64_t bits, int64_t S, int64_t H, const Tensor* l, const Tensor* r) {
+    if (!readable(sc)) return false;
     std::memset(&d, 0, sizeof d);
     d.mode = HYC_MODE_THRESHOLD;
     d.bits = (int32_t)bits;
@@ -158,9 +164,8 @@ struct Threshold {
     else if (sc->dim() >= 2 && sc->size(-1) == 1 && n == S) { d.scale_stride_token = 1; d.scale_stride_channel = 0; }
     else return false;
     d.S = S;
-    if (L != Py_None) {
-      const Tensor *l = bf16(L), *r = bf16(R);
-      if (!l || !r || !l->is_contiguous() || !r->is_contiguous() || l->dim() != 2 || r->dim() != 2 || l->size(0) < S || l->size(1) != r->size(0) || r->size(1) != H)
+    if (l) {
+      if (!readable(l) || !readable(r) || l->dim() != 2 || r->dim() != 2 || l->size(0) < S || l->size(1) != r->size(0) || r->size(1) != H)
         return false;                                                  // (fewer rows than S: padded by the general form)
       d.rank = (int32_t)l->size(1);
       if (d.rank) { d.L = (decltype(d.L))l->data_ptr(); d.R = (decltype(d.R))r->data_ptr(); }
@@ -168,22 +173,41 @@ struct Threshold {
     return true;
   }
 };
+bool vec(const Tensor& t, at::ScalarType type) { return dense_gpu(t) && t.scalar_type() == type && t.is_contiguous(); }
 const Tensor* attr_vec(const Ref& v, at::ScalarType type) {
   const Tensor* t = v.p ? plain(v.p) : nullptr;
   if (!v.p) PyErr_Clear();
-  return t && t->scalar_type() == type && t->is_contiguous() ? t : nullptr;
+  return t && vec(*t, type) ? t : nullptr;
 }
 Tensor empty_like_on(const Tensor& t, at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, at::TensorOptions().device(t.device()).dtype(type)); }
 
 // a compressed activation: of the channel scheme as it is read, of the threshold scheme restored first (ready()).  A value: a node of the graph
-// keeps one, and each pass over it works on a copy.
+// keeps one, and each pass over it works on a copy whose descriptor is made anew (a tensor may have been given other memory since).
 struct Saved {
   Tensor stored, vals, scales, row_ptr, cols, scale, L, R;
   Plan p;
   hyc_desc d;
-  int64_t M = 0, H = 0, bits = 0, group = 0;
+  int64_t M = 0, H = 0, S = 0, bits = 0, group = 0;
   double threshold = 0.0;
   bool restore_first = false;
+  // the descriptor, from where the tensors lie now; false: not as the kernels read them
+  bool describe() {
+    if (!dense_gpu(stored) || !dense_gpu(vals)) return false;
+    if (!restore_first) {
+      if (!dense_gpu(scales) || !p.usable(H, stored.device())) return false;
+      p.describe(bits, group, &d);
+      return true;
+    }
+    Threshold t;
+    if (!vec(row_ptr, at::kInt) || !vec(cols, at::kInt) ||
+        !t.init(threshold, &scale, bits, S, H, L.defined() ? &L : nullptr, R.defined() ? &R : nullptr))
+      return false;
+    d = t.d;
+    d.csr_row_ptr = (decltype(d.csr_row_ptr))row_ptr.data_ptr();
+    d.csr_cols = cols.numel() ? (decltype(d.csr_cols))cols.data_ptr() : nullptr;
+    d.csr_vals = vals.numel() ? (decltype(d.csr_vals))vals.data_ptr() : nullptr;
+    return true;
+  }
   const void* codes() const { return stored.data_ptr(); }
   const void* values() const { return vals.defined() ? vals.data_ptr() : nullptr; }
   const void* group_scales() const { return scales.defined() ? scales.data_ptr() : nullptr; }
@@ -223,32 +247,28 @@ struct In : Saved {
     if (!ok || !ts || !tv) { PyErr_Clear(); return false; }
     stored = *ts; vals = *tv;
     if (thr) {
-      const int64_t S = attr_i64(c, s_S, &ok);
+      S = attr_i64(c, s_S, &ok);
       Ref rp(PyObject_GetAttr(c, s_row_ptr)), co(PyObject_GetAttr(c, s_cols)), th(PyObject_GetAttr(c, s_threshold)), sc(PyObject_GetAttr(c, s_scale)),
           l(PyObject_GetAttr(c, s_L)), r(PyObject_GetAttr(c, s_R));
-      const Tensor *tr = attr_vec(rp, at::kInt), *tc = attr_vec(co, at::kInt);
-      Threshold t;
-      if (!ok || !tr || !tc || !th.p || !sc.p || !l.p || !r.p || !PyFloat_CheckExact(th.p) ||
-          !t.init(PyFloat_AS_DOUBLE(th.p), sc.p, bits, S, H, l.p, r.p)) { PyErr_Clear(); return false; }
-      row_ptr = *tr; cols = *tc;
-      scale = THPVariable_Unpack(sc.p);
-      if (THPVariable_Check(l.p)) L = THPVariable_Unpack(l.p);
-      if (THPVariable_Check(r.p)) R = THPVariable_Unpack(r.p);
+      const Tensor *tr = attr_vec(rp, at::kInt), *tc = attr_vec(co, at::kInt), *ts = sc.p ? plain(sc.p) : nullptr,
+                   *tl = l.p && l.p != Py_None ? plain(l.p) : nullptr, *tR = r.p && r.p != Py_None ? plain(r.p) : nullptr;
+      if (!ok || !tr || !tc || !ts || !th.p || !l.p || !r.p || !PyFloat_CheckExact(th.p) || (l.p != Py_None && (!tl || !tR))) {
+        PyErr_Clear();
+        return false;
+      }
+      row_ptr = *tr; cols = *tc; scale = *ts;
+      if (tl) L = *tl;
+      if (tR) R = *tR;
       threshold = PyFloat_AS_DOUBLE(th.p);
-      d = t.d;
-      d.csr_row_ptr = (decltype(d.csr_row_ptr))row_ptr.data_ptr();
-      d.csr_cols = cols.numel() ? (decltype(d.csr_cols))cols.data_ptr() : nullptr;
-      d.csr_vals = vals.numel() ? (decltype(d.csr_vals))vals.data_ptr() : nullptr;
       restore_first = true;
-      return true;
+      return describe();
     }
     group = attr_i64(c, s_group, &ok);
     Ref sc(PyObject_GetAttr(c, s_scales)), pl(PyObject_GetAttr(c, s_plan));
     const Tensor* tc = sc.p ? plain(sc.p) : nullptr;
-    if (!ok || !tc || !pl.p || !get_plan(pl.p, H, ts->device(), &p)) { PyErr_Clear(); return false; }
+    if (!ok || !tc || !pl.p || !get_plan(pl.p, H, stored.device(), &p)) { PyErr_Clear(); return false; }
     scales = *tc;
-    p.describe(bits, group, &d);
-    return true;
+    return describe();
   }
 };
 PyObject* wrap_or_none(const Tensor& t) {
@@ -258,7 +278,7 @@ PyObject* wrap_or_none(const Tensor& t) {
 PyObject* Saved::wrap(PyObject* plan) const {
   if (restore_first) {                                                 // (stored, row_ptr, cols, vals, threshold, scale, L, R, bits, M, H, S)
     Ref args(Py_BuildValue("NNNNdNNNLLLL", wrap_or_none(stored), wrap_or_none(row_ptr), wrap_or_none(cols), wrap_or_none(vals), threshold,
-                           wrap_or_none(scale), wrap_or_none(L), wrap_or_none(R), (long long)bits, (long long)M, (long long)H, (long long)d.S));
+                           wrap_or_none(scale), wrap_or_none(L), wrap_or_none(R), (long long)bits, (long long)M, (long long)H, (long long)S));
     return args.p ? PyObject_CallObject(t_threshold, args.p) : nullptr;
   }
   Ref made(nullptr);
@@ -1303,19 +1323,20 @@ struct Recorded : public torch::autograd::Node {
     int64_t M, H;
     int dtype;
     if (!dense_gpu(g) || g.scalar_type() != BF16 || g.unsafeGetTensorImpl()->is_python_dispatch() || !rows_of(g, &M, &H)) return false;
-    for (const Saved& c : saved)
-      if (M != c.M || (kind != LINEAR && H != c.H)) return false;
+    std::vector<Saved> in = saved;                                     // (what is read as a restored matrix becomes one)
+    for (Saved& c : in)
+      if (M != c.M || (kind != LINEAR && H != c.H) || !c.describe()) return false;
     if (kind == GATED) {
       Tensor both;
       std::vector<Tensor> d;
-      if (g.dim() < 2 || gated_backward(code, g, saved.data(), -1, &both, &d) != 0) return false;
+      if (g.dim() < 2 || gated_backward(code, g, in.data(), -1, &both, &d) != 0) return false;
       out[0] = d[0];
       out[1] = d[1];
       return true;
     }
-    std::vector<Saved> in = saved;                                     // (what is read as a restored matrix becomes one)
     if (kind == NORM) {
-      if (!dense_gpu(w) || !weight_dtype(w, H, &dtype) || norm_backward(g, in[0], w, dtype, mean, rstd, quirk, &out[0], &out[1])) return false;
+      if (!dense_gpu(w) || !weight_dtype(w, H, &dtype) || !dense_gpu(rstd) || !row_stats(rstd, M) ||
+          (mean.defined() && (!dense_gpu(mean) || !row_stats(mean, M))) || norm_backward(g, in[0], w, dtype, mean, rstd, quirk, &out[0], &out[1])) return false;
       return !bias.defined() || bias_backward(g, M, H, bias.scalar_type() != BF16, &out[2]) == 0;
     }
     if (kind == ACT) return act_backward(code, g, in[0], &out[0]) == 0;
