@@ -544,21 +544,30 @@ static int lora_group(const char* who, const void* const* factors, const int64_t
 // workgroup's share of the walk shortest, rounds included, the fewest (each is one more partial dB).  A workgroup's start and end
 // count as LU_FIXED tiles.  One workgroup too many is a round of its own: us with 10 / 12 ranges of 4096 x 3 x 4096 26.8 / 31.2, with
 // 5 / 6 of 4096 x 2 x 11008 40.6 / 47.4.  At most 32, unless that leaves a range more than 32768 tokens (its offsets into dY are
-// 31-bit numbers of bytes up to row pitches of 32760).
-constexpr int64_t LU_FIXED = 3;
-static int64_t lora_up_tokens(int64_t M, int64_t fblocks) {
+// 31-bit numbers of bytes up to row pitches of 32760).  Where the rows of dY are so far apart (`pitch` elements) that such a range
+// would not fit its 31 bits, as many ranges as it takes workgroups to reach 512, which may be one more.
+constexpr int64_t LU_FIXED = 3, LU_RANGE = (int64_t)1 << 30;     // (elements)
+static int64_t lora_up_tokens(int64_t M, int64_t fblocks, int64_t pitch) {
   const int64_t tiles = (M + LU_M - 1) / LU_M, least = (M + 32767) / 32768;
   int64_t best = 0, best_cost = 0;
   for (int64_t n = 1; n <= 32 && n <= tiles; ++n) {
     const int64_t each = (tiles + n - 1) / n, used = (tiles + each - 1) / each, cost = (fblocks * used + 511) / 512 * (each + LU_FIXED);
     if (!best || cost < best_cost) { best = each; best_cost = cost; }
   }
-  const int64_t most = least > 0 ? (tiles + least - 1) / least : 1;
-  return LU_M * (best < most ? (best > 0 ? best : 1) : most);
+  int64_t most = least > 0 ? (tiles + least - 1) / least : 1;
+  if (best < most) most = best > 0 ? best : 1;
+  if (LU_M * most * pitch >= LU_RANGE) {
+    int64_t n = (512 + fblocks - 1) / fblocks;
+    if (n > 32) n = 32;
+    const int64_t each = (tiles + n - 1) / n;
+    if (each > 0 && each < most) most = each;
+  }
+  return LU_M * most;
 }
-static int lora_up_ranges(int64_t M, int fblocks) {
-  const int64_t tokens = lora_up_tokens(M, fblocks);
-  return M > 0 ? (int)((M + tokens - 1) / tokens) : 1;
+// partial results of dB a call may have: either rule's
+static int64_t lora_up_ranges(int64_t M, int64_t fblocks) {
+  const int64_t tokens = lora_up_tokens(M, fblocks, LU_RANGE);
+  return M > 0 ? (M + tokens - 1) / tokens : 1;
 }
 static int lora_up_blocks(const int64_t* n_out, int n) {
   int64_t b = 0;
@@ -677,7 +686,7 @@ int64_t hyc_lora_up_bwd_workspace_bytes(int64_t M, const int64_t* n_out, int32_t
   for (int i = 0; i < n; ++i) rows += n_out[i];
   const int fblocks = lora_up_blocks(n_out, n);
   const int64_t RC = r <= 16 ? 16 : 32;
-  return 4 * RC * ((int64_t)fblocks * M + (int64_t)lora_up_ranges(M, fblocks) * rows);
+  return 4 * RC * ((int64_t)fblocks * M + lora_up_ranges(M, fblocks) * rows);
 }
 
 int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const int64_t* n_out, const void* const* B, const void* h,
@@ -708,15 +717,21 @@ int hyc_lora_up_bwd(const void* const* dy, const int64_t* ldg, int64_t M, const 
     a.row0[i + 1] = a.row0[i] + (int)n_out[i];
   }
   const int fblocks = a.fb0[n];
-  const int64_t tokens = lora_up_tokens(M, fblocks);
-  for (int i = 0; i < n; ++i)
-    if (tokens * ldg[i] >= ((int64_t)1 << 30)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: a token range of dy must stay below 2 GiB");
-  if (copy_dy && ld_ext >= ((int64_t)1 << 29)) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: rows %lld apart", (long long)ld_ext);
+  int64_t pitch = 0;
+  for (int i = 0; i < n; ++i) pitch = ldg[i] > pitch ? ldg[i] : pitch;
+  const int64_t tokens = lora_up_tokens(M, fblocks, pitch);
+  if (tokens * pitch >= LU_RANGE) return fail(HYC_ENOTSUP, "hyc_lora_up_bwd: a token range of dy must stay below 2 GiB");
   const int used = M ? (int)((M + tokens - 1) / tokens) : 0;   // (no tokens: the sums below are empty and dB is zero)
   const int RC = r <= 16 ? 16 : 32;
   float *dhp = static_cast<float*>(workspace), *dbp = dhp + (int64_t)fblocks * M * RC;
-  uint16_t* cp = copy_dy ? static_cast<uint16_t*>(ext) : nullptr;
+  // (the kernel's copy counts 32-bit bytes from one row to the next; rows that far apart are few and go one by one)
+  const bool by_rows = copy_dy && ld_ext >= ((int64_t)1 << 29);
+  uint16_t* cp = copy_dy && !by_rows ? static_cast<uint16_t*>(ext) : nullptr;
   hipStream_t st = begin_launch(stream);
+  for (int i = 0; i < n && by_rows; ++i)
+    for (int64_t m = 0; m < M; ++m)
+      if (hipMemcpyAsync(static_cast<uint16_t*>(ext) + m * ld_ext + a.row0[i], a.g[i] + m * ldg[i], 2 * (size_t)n_out[i], hipMemcpyDeviceToDevice, st) != hipSuccess)
+        return fail(HYC_ELAUNCH, "hyc_lora_up_bwd: a row of dy could not be copied");
   const dim3 grid((unsigned)fblocks, (unsigned)used);
 #define HYC_GO(RT_, COPY_)                                                                                                   \
   hipLaunchKernelGGL((k_lora_up_bwd<RT_, COPY_>), grid, dim3(256), 0, st, a, M, static_cast<const uint16_t*>(h), (int)tokens, dhp, dbp, cp, ld_ext)
