@@ -192,16 +192,23 @@ k_few_rows(FewRows a) {
   }
 }
 
-// Tokens in tiles of 4 or 5 a workgroup, whichever pads less; features in 1, 2 or 4, the fewest with which the workgroups are resident at
+// Tokens in tiles of up to 4, or of 4 or 5, a workgroup, whichever pads less; features in 1, 2 or 4, the fewest with which the workgroups are resident at
 // once, one of eight waves a CU; past that, 4 features' tiles and workgroups of four waves, two a CU (so are those of a weight that goes
 // through LDS).
-template <bool NF4>
-static void few_rows_launch(const FewRows& a, hipStream_t st) {
-  const int tiles = (a.M + 15) / 16, across = a.N / 16;
+struct FewTiles { int mt, nt, across, down; };           // tiles of a workgroup, workgroups
+static FewTiles few_rows_tiles(int64_t M, int64_t N) {
+  const int tiles = (int)((M + 15) / 16), across = (int)(N / 16);
   const int mt = tiles <= 4 ? tiles : (tiles + 4) / 5 * 5 < (tiles + 3) / 4 * 4 ? 5 : 4, down = (tiles + mt - 1) / mt;
   // (2048 -> 2048 over 512 tokens with 1 / 2 / 4 tiles of features, us: 17.0 / 14.9 / 13.4; over 256 26.2 in four waves / 9.2 / 12.8)
-  const int nt = across * down <= 256 ? 1 : (across + 1) / 2 * down <= 256 ? 2 : 4;
-  const dim3 grid((unsigned)((across + nt - 1) / nt), (unsigned)down);
+  const int64_t all = (int64_t)across * down, half = (int64_t)((across + 1) / 2) * down;
+  const int nt = all <= 256 ? 1 : half <= 256 ? 2 : 4;
+  return {mt, nt, (across + nt - 1) / nt, down};
+}
+template <bool NF4>
+static void few_rows_launch(const FewRows& a, hipStream_t st) {
+  const FewTiles t = few_rows_tiles(a.M, a.N);
+  const int mt = t.mt, nt = t.nt;
+  const dim3 grid((unsigned)t.across, (unsigned)t.down);
   const bool four = nt == 4 && (!NF4 || grid.x * grid.y > 256);
 #define HYC_GO(MT_)                                                                                        \
   do {                                                                                                     \
@@ -246,13 +253,27 @@ extern "C" {
 //   12288 -> 4096       33.4 -> 16.7   46.8 -> 35.5   49.5 -> 40.8   71.1 -> 75.8
 //   4096 -> 11008       27.2 -> 16.7   30.5 -> 38.7   38.9 -> 54.6
 // A workgroup's tiles share their operands with no other one, so what a launch reads grows with the products of the sides.  dX is
-// better while its result is at most one tile of 64 x 64 a CU, whatever the reduction (at 1.25 of that 0.93 to 1.08 of the
-// library's speed, at 1.5 of it 0.7 to 0.9); the forward, which saves a pass over the decoded weight as well, up to 256 tokens and beyond them
-// until about 6e9 multiplications.
+// better, whatever the reduction, while its workgroups are resident at once, one a CU, and its result has at most 2^20 elements.  One
+// more block of tokens is a second round, us, library -> here, just below | just above:
+//   N 11008, K 4160     80 tokens 27.1 -> 19.0 | 81 26.2 -> 34.2, 95 26.4 -> 34.7
+//   N 5632, K 2112      160       15.6 -> 11.6 | 161 15.0 -> 15.7, 186 15.1 -> 15.8
+//   N 2816, K 1088      320       7.9 -> 7.7   | 321 8.9 -> 10.0, 350 8.8 -> 10.2
+//   N 1536, K 4160                             | 680 25.0 -> 25.9
+// A single block of tokens pays past that too (N 22016, K 4160: 16 tokens 67.7 -> 38.4, 40 45.8 -> 45.2; 32768: 16 60.0 -> 46.8, 32 50.8
+// -> 48.9): every weight row is read by one workgroup.
+// The forward, which saves a pass over the decoded weight as well, is taken up to 256 tokens, whatever the weight, and beyond them until
+// about 6e9 multiplications.  From 193 tokens on the library comes level at a few widths: 4096 -> 22016 over 157 / 192 / 224 / 256 tokens
+// 89.2 -> 65.9 / 95.6 -> 87.1 / 97.9 -> 97.3 / 101.5 -> 102.5, 5120 -> 15360 over 224 / 241 / 256 94.8 -> 79.2 / 84.9 -> 90.5 / 95.1 -> 88.4, 3072 ->
+// 16384 over 241 62.0 -> 63.0; beside them 4096 -> 28672 over 256 148 -> 127, 5120 -> 27648 180 -> 155, 13824 -> 5120 138 -> 107, 8192 ->
+// 57344 over 16 / 157 / 256 479 -> 133 / 508 -> 303 / 518 -> 516, 28672 -> 8192 over 256 453 -> 247.
 int32_t hyc_few_rows_covers(int64_t M, int64_t K, int64_t N, int32_t input_grad) {
   if (M <= 0 || K <= 0 || N <= 0 || K % 64 != 0 || N % 16 != 0 || K > (1 << 24) || N > (1 << 24)) return 0;
   if (M * K >= ((int64_t)1 << 30) || N * K >= ((int64_t)1 << 30)) return 0;
-  if (input_grad) return M <= 1024 && M * N <= (1 << 20) ? 1 : 0;
+  if (input_grad) {
+    if (M > 1024 || M * N > (1 << 20)) return 0;
+    const FewTiles t = few_rows_tiles(M, N);
+    return t.down == 1 || (int64_t)t.across * t.down <= 256 ? 1 : 0;
+  }
   return M <= 256 || (M <= 2048 && M * K * N <= (int64_t)6000000000) ? 1 : 0;
 }
 
