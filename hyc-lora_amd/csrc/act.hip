@@ -844,13 +844,24 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
   // 17.6 -> 15.2 us, and 232 -> 221 us at 65 536 rows; H = 5120, 320 threads, 2048 -> 768: 36.0 -> 21.2 / 24.6 -> 18.6 us)
   // Rows of eight waves or more (one workgroup per CU at a time): about eight rows per workgroup, in whole rounds of the
   // 256 CUs (2048 x 11008: GELU 24.5 -> 20.5 us, 4096 rows: 38.9 -> 37.5, 16 384 rows: SiLU 160.7 -> 152.3).
-  // Rows that two or more workgroups share (more than 1024 chunks, row_parts) fill a table in each: one workgroup a CU below 768 rows, then
-  // by rows again, at most four a CU and part.  Against the kernel that walks such rows in turns (SiLU | GELU, us): 100 x 13824 6.7 -> 5.1 |
-  // 7.8 -> 6.5, 300 x 11008 8.1 -> 6.6 | 11.1 -> 8.0, 1000 x 13824 18.8 -> 13.1 | 24.2 -> 15.3, 4096 x 13824 57.1 -> 47.1 | 64.1 -> 49.9,
-  // 9000 x 11008 146 -> 88 | 157 -> 84; no size was slower.
-  if (ACT != ACT_MUL && geo.iters > 1 && d->mode == HYC_MODE_CHANNEL && d->bits != 1) {
-    const int64_t by_rows = (M / 8 / 256) * 256, fewer = M < 768 ? 128 : by_rows < 256 ? 256 : by_rows > 1024 ? 1024 : by_rows;
+  // Rows that two or more workgroups share (more than 1024 chunks, row_parts) fill a table in each: one workgroup a CU, all parts
+  // together, where rows are few, then by rows again, at most four a CU and part.  Against the kernel that walks such rows in turns (SiLU |
+  // GELU, us): 100 x 13824 6.7 -> 5.1 | 7.8 -> 6.5, 300 x 11008 8.1 -> 6.6 | 11.1 -> 8.0, 1000 x 13824 18.8 -> 13.1 | 24.2 -> 15.3, 4096 x 13824
+  // 57.1 -> 47.1 | 64.1 -> 49.9, 9000 x 11008 146 -> 88 | 157 -> 84; of three parts 200 x 24576 8.6 -> 7.7 | 9.9 -> 8.9 (with 128 workgroups a
+  // part 8.9 | 11.4), of eight 100 x 65536 19.6 -> 8.6 | 21.1 -> 9.8 (11.7 | 16.5).  Of 255 sizes from 1 x 8320 to 2500 x 49152 and 65536
+  // channels two are slower by more than 3 %, 447 and 1500 x 65536 of 2 bits (GELU 30.5 -> 31.8 and 82 -> 85).
+  const RowParts p = row_parts(geo, 64);
+  if (ACT != ACT_MUL && p.parts > 1 && d->mode == HYC_MODE_CHANNEL && d->bits != 1) {
+    const int64_t by_rows = (M / 8 / 256) * 256;
+    const int64_t fewer = p.parts > 2 && M * p.parts < 1024 ? 256 / p.parts : M < 768 ? 128 : by_rows < 256 ? 256 : by_rows > 1024 ? 1024 : by_rows;
     grid = (int)(M < fewer ? M : fewer);
+  }
+  // The product has no table: 256 workgroups a part for 448 to 1023 rows, 128 for fewer rows of two parts, so that each has a next row to
+  // ask for (both products of a Hadamard backward, us, one row each -> so, walked: 200 x 13824 9.6 -> 8.8, 9.6; 500 x 8320 10.4 -> 9.7, 10.6;
+  // 500 x 13824 14.4 -> 12.4, 13.9; 768 x 65536 of 4 bits 75.9 -> 69.0, 77.4).
+  if (ACT == ACT_MUL && p.parts > 1 && d->mode == HYC_MODE_CHANNEL && d->bits != 1 && M < 1024) {
+    if (M >= 448) grid = 256;
+    else if (M >= 160 && p.parts == 2) grid = 128;
   }
   if (ACT != ACT_MUL && geo.iters == 1) {
     int fewer = geo.threads <= 128 ? 1024 : geo.threads <= 256 ? 512 : 768;
@@ -863,7 +874,6 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
   }
   hipStream_t st = begin_launch(stream);
   if (d->mode == HYC_MODE_CHANNEL && d->bits != 1) {
-    const RowParts p = row_parts(geo, 64);
     const dim3 wgs((unsigned)grid, (unsigned)p.parts);
     const int use_lut = lut_pays(M, grid, p.threads, LUT_PAYS_BWD);
 #define HYC_ACT_FAST(B_)                                                                                                        \
