@@ -400,9 +400,29 @@ static int long_input_grid(int64_t M, int dflt) {
 
 // Long rows are shared by workgroups (row_parts): nothing in the fast kernels looks beyond a scale group.  The kernels that walk such a row in turns
 // wait for every load before the next one is asked for; shared, 8-bit codes in groups of 128 went (compress | decompress, us)
-//   500 x 13824 6.5 -> 5.5 | 5.8 -> 5.4, 4096 x 11008 29.1 -> 23.9 | 40.2 -> 21.5, 9000 x 11008 73.2 -> 49.7 | 80.3 -> 45.2,
-//   4096 x 13824 31.1 -> 29.8 | 41.9 -> 27.4, 4096 x 65536 188.8 -> 176.1 | 284.4 -> 175.2; no size was slower.
-// What still takes the kernels with turns: 1-bit codes, and compressing in groups of other widths than 64 and 128.
+//   500 x 13824 6.9 -> 5.4 | 6.0 -> 5.2, 4096 x 11008 29.1 -> 23.9 | 40.2 -> 21.5, 9000 x 11008 73.2 -> 49.7 | 80.3 -> 45.2,
+//   4096 x 13824 31.1 -> 29.8 | 41.9 -> 27.4, 4096 x 65536 188.8 -> 176.1 | 284.4 -> 175.2.
+// Of 255 sizes from 1 x 8320 to 2500 x 49152 and 65536 channels of 2 to 8 bits, restoring 447 to 500 x 65536 of 2 bits is slower (13.6 -> 15.3).
+// What still takes the kernels with turns: 1-bit codes, compressing in groups of other widths than 64 and 128, and what compress_walks()
+// names.
+//
+// Compressing: whole rounds of the 256 CUs over the rows (2000 x 32768 of 4 bits: 1000 workgroups a part 32.5 us, walked 30.7;
+// 2500 x 8320: 1250 13.6, 1024 11.2).  Restoring a few hundred 8-bit rows of two parts: 256 workgroups a part, so that each has a next row to ask for
+// (500 x 13824 5.9 -> 5.2, walked 5.7; 768 x 11008 7.2 -> 6.0, 8.1).
+static dim3 compress_grid(int64_t M, const RowParts& p) {
+  const int few = row_grid(M, p.threads), most = long_input_grid(M, few), rounds = most / 256 * 256;
+  return dim3((unsigned)(p.parts > 1 && most > few ? (rounds > few ? rounds : few) : most), (unsigned)p.parts);
+}
+static dim3 restore_grid(int64_t M, int bits, const RowParts& p) {
+  return dim3((unsigned)(p.parts == 2 && bits == 8 && M >= 448 && M < 1024 ? 256 : long_input_grid(M, row_grid(M, p.threads))), (unsigned)p.parts);
+}
+// 8-bit rows of 32768 channels and more, so many that they fill a good part of the last-level cache (256 MB) with their codes, but not
+// more: workgroups on many short parts of them compete for it where the walk streams.  Walked | shared, us: 1500 x 32768 26.0 | 27.1,
+// 1500 x 49152 38.0 | 40.4, 768 x 65536 26.4 | 28.5, 1200 x 65536 41.5 | 43.8; outside 1000 x 32768 20.3 | 18.8, 600 x 65536 25.0 | 22.6,
+// 2500 x 32768 48.9 | 44.3, 1500 x 65536 64.3 | 53.7.
+static bool compress_walks(int64_t M, int64_t H, int bits) {
+  return bits == 8 && H >= 32768 && M >= 640 && M * H >= 33000000 && M * H < 80000000;
+}
 #define HYC_DISPATCH_BITS(BITS_, ...)            \
   switch (BITS_) {                               \
     case 1: { constexpr int B = 1; __VA_ARGS__; } break; \
@@ -438,9 +458,9 @@ int hyc_compress_rows(const void* x, int64_t ldx, int64_t M, int64_t H, const hy
     if (M == 0) return HYC_OK;
     if (!x || !stored || !scales || (d->k > 0 && !vals)) return fail(HYC_EFAULT, "hyc_compress: null buffer");
     if (!aligned16(x) || !aligned8(stored)) return fail(HYC_EINVAL, "hyc_compress: x must be 16-byte and stored 8-byte aligned");
-    if ((lpg == 8 || lpg == 16) && d->bits != 1) {
+    if ((lpg == 8 || lpg == 16) && d->bits != 1 && !compress_walks(M, H, d->bits)) {
       const RowParts p = row_parts(g, lpg);
-      const dim3 grid((unsigned)long_input_grid(M, row_grid(M, p.threads)), (unsigned)p.parts);
+      const dim3 grid = compress_grid(M, p);
 #define HYC_CF_R(B_, L_, R_)                                                                                         \
   do {                                                                                                               \
     if (p.parts > 1)                                                                                                 \
@@ -514,7 +534,7 @@ int hyc_decompress(const void* stored, const void* vals, const void* scales, int
     if (!aligned16(xhat) || !aligned8(stored)) return fail(HYC_EINVAL, "hyc_decompress: xhat must be 16-byte and stored 8-byte aligned");
     if (d->bits != 1) {
       const RowParts p = row_parts(g, 64);
-      const dim3 grid((unsigned)long_input_grid(M, row_grid(M, p.threads)), (unsigned)p.parts);
+      const dim3 grid = restore_grid(M, d->bits, p);
 #define HYC_DF(B_)                                                                                                      \
   do {                                                                                                                  \
     if (p.parts > 1)                                                                                                    \
