@@ -907,12 +907,7 @@ static int launch_act(const void* g, const void* stored, const void* vals, const
                      static_cast<const uint16_t*>(vals), static_cast<const uint16_t*>(scales), M, H, geo.cps, \
                      geo.iters, ca, static_cast<uint16_t*>(dx), use_lut)
   if (d->mode == HYC_MODE_CHANNEL) {
-    switch (d->bits) {
-      case 1: HYC_ACT_LAUNCH(1, 0); break;
-      case 2: HYC_ACT_LAUNCH(2, 0); break;
-      case 4: HYC_ACT_LAUNCH(4, 0); break;
-      default: HYC_ACT_LAUNCH(8, 0); break;
-    }
+    HYC_ACT_LAUNCH(1, 0);                                 // (wider codes: above)
   } else {
     switch (d->bits) {
       case 1: HYC_ACT_LAUNCH(1, 2); break;

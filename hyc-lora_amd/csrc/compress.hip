@@ -39,12 +39,12 @@ k_compress_chan(const uint16_t* __restrict__ x, int64_t M, int64_t H /* row pitc
   }
 }
 
-template <int BITS>
+// 1-bit codes (wider ones: k_decompress_chan_fast)
 __global__ void __launch_bounds__(1024)
 k_decompress_chan(const uint8_t* __restrict__ stored, const uint16_t* __restrict__ vals,
                   const uint16_t* __restrict__ scales, int64_t M, int64_t H, int CPS, int iters, ChanArgs a,
                   uint16_t* __restrict__ xhat) {
-  constexpr int NSEG = Q<BITS>::NSEG;
+  constexpr int BITS = 1, NSEG = Q<BITS>::NSEG;
   const int64_t SEG = (int64_t)CPS * 8;
   for (int64_t row = blockIdx.x; row < M; row += gridDim.x) {
     const uint8_t* sr = stored + row * SEG;
@@ -556,10 +556,9 @@ int hyc_decompress(const void* stored, const void* vals, const void* scales, int
 #undef HYC_DF
       return check_launch("hyc_decompress");
     }
-    HYC_DISPATCH_BITS(d->bits,
-      hipLaunchKernelGGL((k_decompress_chan<B>), dim3(row_grid(M, g.threads)), dim3(g.threads), 0, st,
-                         static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),
-                         static_cast<const uint16_t*>(scales), M, H, g.cps, g.iters, a, static_cast<uint16_t*>(xhat)));
+    hipLaunchKernelGGL(k_decompress_chan, dim3(row_grid(M, g.threads)), dim3(g.threads), 0, st,
+                       static_cast<const uint8_t*>(stored), static_cast<const uint16_t*>(vals),
+                       static_cast<const uint16_t*>(scales), M, H, g.cps, g.iters, a, static_cast<uint16_t*>(xhat));
     return check_launch("hyc_decompress");
   }
   if (d->mode == HYC_MODE_THRESHOLD) {
