@@ -22,6 +22,7 @@
 #include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <atomic>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -1306,7 +1307,12 @@ PyObject* attn_kept_bwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 // contexts it replaces it keeps its tensors as they are (no saved-tensor hooks, nothing let go after a pass).  It holds no object of the
 // interpreter, so that the engine's thread can run it and let go of it without the lock.  What the calls above do not cover, in a pass over it too
 // (create_graph, gradients in a batch, of another type or layout), goes through `interpreted`, the Function's own backward as a function of
-// (context, gradient), with a context made for it.
+// (context, gradient), with a context made for it.  Whoever looks at what it keeps (grad_fn.saved and the like) or writes to it has it as a
+// Function's context from then on: the same objects each time, and passes that go by them.
+struct Lock {                                                          // the interpreter's lock
+  PyGILState_STATE state = PyGILState_Ensure();
+  ~Lock() { PyGILState_Release(state); }
+};
 struct Recorded : public torch::autograd::Node {
   enum Kind { NORM, LINEAR, ACT, GATED } kind;
   std::vector<Saved> saved;                                            // one activation; of the gated product act(gate), up and gate
@@ -1316,7 +1322,13 @@ struct Recorded : public torch::autograd::Node {
   int32_t code = 0;
   std::string act, label;
   PyObject* interpreted = nullptr;                                     // lives as long as the process
+  std::atomic<PyObject*> seen{nullptr};                                // a dict, once somebody has looked
   explicit Recorded(Kind k) : kind(k) {}
+  ~Recorded() override {
+    if (!seen.load() || !Py_IsInitialized()) return;
+    Lock lock;
+    Py_DECREF(seen.load());
+  }
   std::string name() const override { return label; }
 
   bool native(const Tensor& g, torch::autograd::variable_list& out) const {
@@ -1345,13 +1357,10 @@ struct Recorded : public torch::autograd::Node {
   }
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     torch::autograd::variable_list out(num_outputs());
-    if (!c10::GradMode::is_enabled() && !c10::impl::TorchDispatchModeTLS::any_modes_set() && native(grads[0], out)) return out;
+    if (!c10::GradMode::is_enabled() && !c10::impl::TorchDispatchModeTLS::any_modes_set() && !seen.load() && native(grads[0], out)) return out;
     const Tensor g = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
-    struct Lock {
-      PyGILState_STATE state = PyGILState_Ensure();
-      ~Lock() { PyGILState_Release(state); }
-    } lock;
-    Ref names(attributes()), none_(PyTuple_New(0)), ctx(names.p && none_.p ? PyObject_Call(t_namespace, none_.p, names.p) : nullptr),
+    Lock lock;
+    Ref names(seen.load() ? (Py_INCREF(seen.load()), seen.load()) : attributes()), none_(PyTuple_New(0)), ctx(names.p && none_.p ? PyObject_Call(t_namespace, none_.p, names.p) : nullptr),
         dy(ctx.p ? THPVariable_Wrap(g) : nullptr), r(dy.p ? PyObject_CallFunctionObjArgs(interpreted, ctx.p, dy.p, nullptr) : nullptr);
     if (!r.p || !PyTuple_Check(r.p) || PyTuple_GET_SIZE(r.p) < (Py_ssize_t)out.size()) {
       if (r.p) PyErr_SetString(PyExc_RuntimeError, "a backward returned something else than its gradients");
@@ -1376,24 +1385,47 @@ struct Recorded : public torch::autograd::Node {
                          Py_BuildValue("NNN", PyBool_FromLong(needs[0]), PyBool_FromLong(needs[1]), PyBool_FromLong(needs[2])), "grad_room", Py_None, "act",
                          act.c_str());
   }
+  // them as somebody sees them, for `name` or, to write to, whatever it is; null without an error: there is none of the name
+  PyObject* look(PyObject* name, bool write) {
+    if (PyObject* d = seen.load()) return d;
+    Ref all(attributes());
+    if (!all.p) return nullptr;
+    if (!write) {
+      const int has = PyDict_Contains(all.p, name);
+      if (has <= 0) return nullptr;
+    }
+    Py_INCREF(all.p);
+    seen.store(all.p);
+    return all.p;
+  }
 };
+Recorded* node_of(PyObject* self) { return dynamic_cast<Recorded*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get()); }
 // grad_fn.saved and the like
 PyObject* node_attribute(PyObject* self, PyObject* name) {
   PyObject* v = PyObject_GenericGetAttr(self, name);
   if (v || !PyErr_ExceptionMatches(PyExc_AttributeError)) return v;
-  const auto* node = dynamic_cast<Recorded*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get());
+  Recorded* node = node_of(self);
   if (!node) return nullptr;
   PyObject *type, *value, *trace;
   PyErr_Fetch(&type, &value, &trace);
-  Ref all(node->attributes());
-  if (all.p && (v = PyDict_GetItemWithError(all.p, name))) {
-    Py_INCREF(v);
-    Py_XDECREF(type); Py_XDECREF(value); Py_XDECREF(trace);
-    return v;
+  PyObject* all = node->look(name, false);
+  if (all && (v = PyDict_GetItemWithError(all, name))) Py_INCREF(v);
+  if (!v && !PyErr_Occurred()) {
+    PyErr_Restore(type, value, trace);
+    return nullptr;
   }
-  PyErr_Clear();
-  PyErr_Restore(type, value, trace);
-  return nullptr;
+  Py_XDECREF(type); Py_XDECREF(value); Py_XDECREF(trace);
+  return v;
+}
+int set_node_attribute(PyObject* self, PyObject* name, PyObject* value) {
+  Recorded* node = node_of(self);
+  if (!node || PyObject_HasAttr((PyObject*)Py_TYPE(self), name)) return PyObject_GenericSetAttr(self, name, value);
+  PyObject* all = node->look(name, true);
+  if (!all) return -1;
+  if (value) return PyDict_SetItem(all, name, value);
+  if (PyDict_DelItem(all, name) == 0) return 0;
+  if (PyErr_ExceptionMatches(PyExc_KeyError)) PyErr_SetObject(PyExc_AttributeError, name);
+  return -1;
 }
 PyTypeObject node_type;
 
@@ -1608,6 +1640,7 @@ PyMODINIT_FUNC PyInit__hyc_host() {
   Ref types(PyImport_ImportModule("types"));
   if (!types.p || !(t_namespace = PyObject_GetAttrString(types.p, "SimpleNamespace"))) return nullptr;
   node_type.tp_getattro = node_attribute;
+  node_type.tp_setattro = set_node_attribute;
   torch::autograd::_initFunctionPyTypeObject(node_type, "CalibratedBackward", nullptr, nullptr);
   torch::autograd::registerCppFunction(typeid(Recorded), &node_type);
   END_HANDLE_TH_ERRORS
