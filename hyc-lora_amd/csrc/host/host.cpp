@@ -1004,7 +1004,7 @@ PyObject* lora_backward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     M = m;
     dy[i] = g->data_ptr();
     if (!i) g0 = g;
-    const int64_t range = (M < 32768 ? M : 32768) + 63;
+    const int64_t range = (M < 32768 ? M : 32768) + 63;                // kernels._lora_range_fits
     if (range / 64 * 64 * pitches[i] >= ((int64_t)1 << 30)) return none();
   }
   if (h->size(0) != M || h->size(1) != n * r || room < n * r || !base_weight(a[8], a[9], *h, total * K, &packed, &absmax)) return none();

@@ -1126,8 +1126,8 @@ def _lora_kernels_cover(M, n, r, K, outs):
 
 
 def _lora_range_fits(M, pitch):
-    """a token range of hyc_lora_up_bwd (whole tiles of 64 tokens, at most 32768) stays below 2 GiB of rows `pitch` apart, however
-    many ranges there are"""
+    """a token range of hyc_lora_up_bwd (at most 32768 tokens; rounded up to 64, twice its tile: a margin) stays below 2 GiB of rows
+    `pitch` apart, however many ranges there are"""
     return (min(M, 32768) + 63) // 64 * 64 * pitch < 1 << 30
 
 
